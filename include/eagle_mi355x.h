@@ -49,6 +49,7 @@ enum eagle_status {
                                 two mask words and the entry points that say so */
 #define EAGLE_MAX_TREE_SLOTS 64 /* tree tokens the tree-layout kernels take (root + 63 nodes; the reference's
                                    default is 39 nodes, mlx_eagle.py:390,510) */
+#define EAGLE_MAX_SEGMENTS 16 /* pieces of a list that the tree layout reads where they are */
 #define EAGLE_MAX_CHUNK 2048 /* rows of one causal pass over a prompt chunk */
 #define EAGLE_MAX_M 32       /* rows of x accepted by the quantised matmul */
 
@@ -132,6 +133,8 @@ int eagle_qmv_w4g64_f16(const void* x, const uint32_t* wq, const void* scales, c
  * qmv.py:226-241); x [M, K], out [M, N].  Measured against the matrix-tile kernel at M = 2, 4, 8
  * by `bench.py --small-m`. */
 int eagle_qmv_rows_supported(int M, int N, int K);
+/* 1 where this form is the faster one for M rows of x. */
+int eagle_qmv_preferred(int M, int N, int K);
 int eagle_qmv_rows_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
                              const void* biases, const void* bias, void* out, int M, int N, int K,
                              int group_size, int bits, eagle_stream_t stream);
@@ -429,6 +432,18 @@ int eagle_process_draft_tree(const void* scores, const int32_t* tokens,
                              int32_t* mask_index, int32_t* draft_tokens,
                              uint32_t* tree_mask_bits, eagle_stream_t stream);
 
+/* The same from the per-level lists as the expansion leaves them (mlx_eagle.py:217-226): HOST arrays of
+ * `n` device pointers to scores (fp16) and tokens with `counts` entries each, `parents_n` pointers to
+ * parents with `parent_counts` entries each (at least C / k in all), read where they are.  The root token
+ * is an int32 or (sampled_is_64bit) an int64; the mask comes out as the additive matrix [T,T] in bf16
+ * (0 visible, -inf elsewhere). */
+int eagle_process_draft_tree_lists(const void* const* scores, const int32_t* const* tokens,
+                                   const int* counts, int n, const uint32_t* const* parents,
+                                   const int* parent_counts, int parents_n,
+                                   const void* sampled_token_dev, int sampled_is_64bit, int k, int total,
+                                   int32_t* tree_position_ids, int32_t* mask_index,
+                                   int32_t* draft_tokens, void* tree_mask_bf16, eagle_stream_t stream);
+
 /* post_process_draft_tree (mlx_eagle.py:254-295) without the host round trip:
  * retrieve_indices [64,64] int32 (row r = path of the r-th leaf, -1 padded; EAGLE_MAX_TREE_SLOTS
  * rows and columns whatever the tree size),
@@ -436,6 +451,12 @@ int eagle_process_draft_tree(const void* scores, const int32_t* tokens,
 int eagle_post_process_draft_tree(const int32_t* tree_position_ids, const int32_t* mask_index,
                                   int total, int32_t* retrieve_indices, int32_t* shape_out,
                                   eagle_stream_t stream);
+/* The same with the rows packed: leaf_num rows of max_depth + 1 entries, nothing between them
+ * (retrieve_indices still holds 64 * 64 entries).  shape_out may be pinned host memory, for a
+ * caller that waits for the stream to learn the shape. */
+int eagle_post_process_draft_tree_packed(const int32_t* tree_position_ids, const int32_t* mask_index,
+                                         int total, int32_t* retrieve_indices, int32_t* shape_out,
+                                         eagle_stream_t stream);
 
 /* Greedy acceptance (evaluate_posterior_greedy, mlx_eagle.py:311-326, with the
  * gathers of :582-589).  node_argmax [T] is the argmax token of each tree node's

@@ -12,6 +12,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libeagle_mi355x.so")
 
 _lib = None
+_host = None
 
 # name -> (restype, argtypes); must list every symbol the header declares
 SIGNATURES = {
@@ -30,6 +31,7 @@ SIGNATURES = {
     "eagle_qmv_supported": (c_int, [c_int] * 2),
     "eagle_qmv_w4g64_f16": (c_int, [c_void_p] * 6 + [c_int] * 4 + [c_void_p]),
     "eagle_qmv_rows_supported": (c_int, [c_int] * 3),
+    "eagle_qmv_preferred": (c_int, [c_int] * 3),
     "eagle_qmv_rows_w4g64_f16": (c_int, [c_void_p] * 6 + [c_int] * 5 + [c_void_p]),
     "eagle_qmm_plan": (c_int, [c_int, c_int, c_int, c_void_p]),
     "eagle_qmm_swiglu_w4g64_f16": (c_int, [c_void_p] * 6 + [c_int] * 5 + [c_void_p, c_size_t, c_void_p]),
@@ -88,6 +90,9 @@ SIGNATURES = {
     "eagle_argmax_rows_f16": (c_int, [c_void_p] * 2 + [c_int, c_long, c_void_p, c_size_t, c_void_p]),
     "eagle_process_draft_tree": (c_int, [c_void_p] * 4 + [c_int] * 3 + [c_void_p] * 5),
     "eagle_post_process_draft_tree": (c_int, [c_void_p] * 2 + [c_int] + [c_void_p] * 3),
+    "eagle_process_draft_tree_lists": (c_int, [c_void_p] * 3 + [c_int] + [c_void_p] * 2 + [c_int, c_void_p]
+                                       + [c_int] * 3 + [c_void_p] * 5),
+    "eagle_post_process_draft_tree_packed": (c_int, [c_void_p] * 2 + [c_int] + [c_void_p] * 3),
     "eagle_greedy_accept": (c_int, [c_void_p] * 4 + [c_int] + [c_void_p] * 3),
     "eagle_kv_compact_f16": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_long, c_void_p]),
     "eagle_fill_i32": (c_int, [c_void_p, c_int32, c_long, c_void_p]),
@@ -115,6 +120,22 @@ def lib():
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+def host():
+    """The native host path of the operators (csrc/host.cpp), on top of the library."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise EagleLibraryMissing(f"the native host module cannot be loaded ({e}): build the HIP extension first "
+                                      "(python -m mlx_eagle_spec_decoding_tree_amd.build)") from e
+        from . import ops
+        module.init(ops.workspace)
+        _host = module
+    return _host
 
 
 def status_string(rc):

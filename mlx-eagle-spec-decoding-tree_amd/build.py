@@ -20,6 +20,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libeagle_mi355x.so")
+HOST = os.path.join(HERE, "_host.so")
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -88,11 +89,40 @@ def sources():
     return sorted(glob.glob(os.path.join(CSRC, "*.hip")))
 
 
+def start_host(objdir):
+    """Start the compile of csrc/host.cpp, the native host path of the operators (no device code): a
+    Python module on torch's C++ interface.  Returns (process, object)."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    obj = os.path.join(objdir, "host.cpp.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{d}" for d in cpp_extension.include_paths()), "-isystem/opt/rocm/include",
+           f"-isystem{sysconfig.get_paths()['include']}", "-c", os.path.join(CSRC, "host.cpp"), "-o", obj]
+    return subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT), obj
+
+
+def link_host(obj):
+    from torch.utils import cpp_extension
+    libs = cpp_extension.library_paths()
+    tmp = HOST + ".tmp"
+    cmd = ["g++", "-shared", obj, "-o", tmp, *(f"-L{d}" for d in libs), "-L/opt/rocm/lib", f"-L{HERE}",
+           "-l:libeagle_mi355x.so", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+           "-lamdhip64", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
+    if r.returncode != 0:
+        raise RuntimeError("link of the host module failed:\n" + r.stdout.decode(errors="replace"))
+    os.replace(tmp, HOST)
+
+
 def build(verbose=False, jobs=8):
-    """Compile every csrc/*.hip to an object (in parallel) and link the library."""
+    """Compile every csrc/*.hip to an object (in parallel) and link the library, then the host
+    module on top of it."""
     cc = hipcc()
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
+    host, host_obj = start_host(objdir)
     procs = []
     objs = []
     flags = [f for f in FLAGS if f != "-shared"]
@@ -129,6 +159,10 @@ def build(verbose=False, jobs=8):
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stdout.decode(errors="replace"))
     os.replace(tmp, LIB)
+    out, _ = host.communicate()
+    if host.returncode != 0:
+        raise RuntimeError("g++ failed on csrc/host.cpp:\n" + out.decode(errors="replace"))
+    link_host(host_obj)
     return LIB
 
 

@@ -10,49 +10,82 @@ namespace {
 constexpr int MAXT = EAGLE_MAX_TREE_SLOTS;   // 64: tree tokens the kernels of this file lay out
 constexpr int MAXC = 1024;             // draft candidates (k + k*k*depth)
 
-// mlx_eagle.py:217-250 (with topk :24-58 and search_sorted :61-93).
-__global__ __launch_bounds__(256) void process_draft_tree_kernel(
-    const half_t* __restrict__ scores, const int32_t* __restrict__ tokens,
-    const uint32_t* __restrict__ parents_list, const int32_t* __restrict__ sampled,
-    int C, int k, int total, int32_t* __restrict__ pos_ids, int32_t* __restrict__ mask_index,
-    int32_t* __restrict__ draft_tokens, uint32_t* __restrict__ bits_out) {
-  __shared__ float sc[MAXC];
-  __shared__ unsigned char picked[MAXC];
+// The candidates as they come from the expansion: a list of per-level pieces for each of scores,
+// tokens and parents (or one piece each), read where they are instead of concatenated first.
+struct TreeLists {
+  const half_t* scores[EAGLE_MAX_SEGMENTS];
+  const int32_t* tokens[EAGLE_MAX_SEGMENTS];
+  const uint32_t* parents[EAGLE_MAX_SEGMENTS];
+  int end[EAGLE_MAX_SEGMENTS];        // candidates up to and including piece i
+  int pend[EAGLE_MAX_SEGMENTS];       // parents up to and including piece i
+  const void* root;                   // the root token, int32 or int64
+  int n, pn, root64;
+};
+
+template <typename T>
+__device__ inline T list_at(const T* const (&ptr)[EAGLE_MAX_SEGMENTS], const int (&end)[EAGLE_MAX_SEGMENTS], int n, int i) {
+  int s = 0;
+  while (s + 1 < n && i >= end[s]) ++s;
+  return ptr[s][s ? i - end[s - 1] : i];
+}
+
+constexpr int TREE_THREADS = 512;
+
+// mlx_eagle.py:217-250 (with topk :24-58 and search_sorted :61-93).  One workgroup; bound by the
+// chain of its phases, so none of them is a loop of one thread: the picked candidates are counted
+// with ballots and every token walks up to the root by itself (one thread that ORed the rows in
+// order took longer than the rest of the kernel: 18 -> 7 us for 39 of 328 candidates).
+__global__ __launch_bounds__(TREE_THREADS) void process_draft_tree_kernel(
+    TreeLists in, int C, int k, int total, int32_t* __restrict__ pos_ids, int32_t* __restrict__ mask_index,
+    int32_t* __restrict__ draft_tokens, uint32_t* __restrict__ bits_out, uint16_t* __restrict__ mask_out) {
+  __shared__ __attribute__((aligned(16))) float sc[MAXC];
+  __shared__ int wave_picked[MAXC / 64];
   __shared__ int sel[MAXT];
   __shared__ int midx[MAXT];
   __shared__ unsigned long long bits[MAXT];
   const int tid = threadIdx.x;
   // a NaN score ranks as -inf: with the index tie rule the order below is then total, so
   // exactly `total` candidates are picked whatever the scores hold
-  for (int i = tid; i < C; i += blockDim.x) {
-    const float v = (float)scores[i];
+  const int C4 = (C + 3) / 4 * 4;
+  for (int i = tid; i < C4; i += TREE_THREADS) {
+    const float v = i < C ? (float)list_at(in.scores, in.end, in.n, i) : -INFINITY;
     sc[i] = v != v ? -INFINITY : v;
   }
   __syncthreads();
   // rank in the stable descending order: candidates ahead of i are those with a larger
   // score, or an equal score and a lower flat index
-  for (int i = tid; i < C; i += blockDim.x) {
-    const float si = sc[i];
+  bool picked[MAXC / TREE_THREADS];
+#pragma unroll
+  for (int r = 0; r < MAXC / TREE_THREADS; ++r) {
+    const int i = tid + r * TREE_THREADS;
+    const float si = sc[i < C ? i : 0];
     int rank = 0;
-    for (int j = 0; j < C; ++j) {
-      const float sj = sc[j];
-      rank += (sj > si) || (sj == si && j < i);
+    if (r * TREE_THREADS < C) {
+      for (int j = 0; j < C4; j += 4) {
+        const float4_t s4 = *reinterpret_cast<const float4_t*>(sc + j);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rank += (s4[e] > si) || (s4[e] == si && j + e < i);
+      }
     }
-    picked[i] = rank < total;
+    picked[r] = i < C && rank < total;
+    const unsigned long long m = __ballot(picked[r]);
+    if ((tid & 63) == 0) wave_picked[i >> 6] = __popcll(m);
   }
   __syncthreads();
   // the picked candidates in ascending flat index
-  for (int i = tid; i < C; i += blockDim.x) {
-    if (!picked[i]) continue;
-    int before = 0;
-    for (int j = 0; j < i; ++j) before += picked[j];
-    if (before < total) sel[before] = i;
+#pragma unroll
+  for (int r = 0; r < MAXC / TREE_THREADS; ++r) {
+    const int i = tid + r * TREE_THREADS;
+    const unsigned long long m = __ballot(picked[r]);
+    int before = __popcll(m & ((1ull << (tid & 63)) - 1ull));
+    for (int w = 0; w < (i >> 6); ++w) before += wave_picked[w];
+    if (picked[r] && before < total) sel[before] = i;
   }
   __syncthreads();
   if (tid < total) {
     const int c = sel[tid];
-    draft_tokens[tid + 1] = tokens[c];
-    const uint32_t dp = parents_list[c / k];
+    draft_tokens[tid + 1] = list_at(in.tokens, in.end, in.n, c);
+    const uint32_t dp = list_at(in.parents, in.pend, in.pn, c / k);
     // fixed-step left binary search for the flat id dp - 1 (uint32 arithmetic, wraps for dp == 0)
     const uint32_t target = dp - 1u;
     uint32_t low = 0, high = (uint32_t)total;
@@ -69,44 +102,56 @@ __global__ __launch_bounds__(256) void process_draft_tree_kernel(
     midx[tid] = mi;
     mask_index[tid] = mi;
   }
-  if (tid == 0) draft_tokens[0] = sampled[0];
-  __syncthreads();
-  if (tid == 0) {
-    // identity rows first, then the sequential OR of mlx_eagle.py:239-243 (a parent slot ahead
-    // of its child, which only poisoned scores can produce, then reads an identity row, as the
-    // reference's loop over an identity matrix does)
-    for (int i = 0; i <= total; ++i) bits[i] = 1ull << i;
-    for (int i = 0; i < total; ++i) {
-      const int par = midx[i] < 0 ? 0 : (midx[i] > total ? total : midx[i]);
-      bits[i + 1] |= bits[par];
-    }
-  }
+  if (tid == 0)
+    draft_tokens[0] = in.root64 ? (int32_t)*static_cast<const int64_t*>(in.root) : *static_cast<const int32_t*>(in.root);
   __syncthreads();
   if (tid <= total) {
-    // one mask word per row for trees of at most 32 tokens, two (low, high) above that
-    if (total + 1 <= 32) {
-      bits_out[tid] = (uint32_t)bits[tid];
-    } else {
-      bits_out[2 * tid] = (uint32_t)bits[tid];
-      bits_out[2 * tid + 1] = (uint32_t)(bits[tid] >> 32);
+    // identity rows ORed in ascending order (mlx_eagle.py:239-243): a row inherits its parent's
+    // finished row where the parent comes earlier, and the bare identity row of a parent slot at or
+    // after its child (which only poisoned scores can produce), where the walk therefore ends
+    unsigned long long row = 1ull << tid;
+    int cur = tid;
+    while (cur > 0) {
+      const int m = midx[cur - 1];
+      const int par = m < 0 ? 0 : (m > total ? total : m);
+      row |= 1ull << par;
+      if (par >= cur) break;
+      cur = par;
     }
-    pos_ids[tid] = __popcll(bits[tid]) - 1;
+    bits[tid] = row;
+    // one mask word per row for trees of at most 32 tokens, two (low, high) above that
+    if (bits_out) {
+      if (total + 1 <= 32) {
+        bits_out[tid] = (uint32_t)row;
+      } else {
+        bits_out[2 * tid] = (uint32_t)row;
+        bits_out[2 * tid + 1] = (uint32_t)(row >> 32);
+      }
+    }
+    pos_ids[tid] = __popcll(row) - 1;
   }
+  if (!mask_out) return;
+  // the additive mask of the module path, bf16: 0 where visible, -inf elsewhere
+  __syncthreads();
+  const int T = total + 1;
+  for (int i = tid; i < T * T; i += TREE_THREADS)
+    mask_out[i] = (bits[i / T] >> (i % T)) & 1ull ? 0u : 0xff80u;
 }
 
-// mlx_eagle.py:254-295.  retrieve [64][64], shape {leaf_num, max_depth + 1}.
-__global__ __launch_bounds__(128) void post_process_kernel(const int32_t* __restrict__ pos_ids,
-                                                          const int32_t* __restrict__ mask_index,
-                                                          int total, int32_t* __restrict__ retrieve,
-                                                          int32_t* __restrict__ shape) {
+// mlx_eagle.py:254-295 in one wave (a lane per token, T <= 64).  retrieve [64][64], shape {leaf_num,
+// max_depth + 1}; PACKED: rows of max_depth + 1 entries, leaf_num of them, without padding.
+template <bool PACKED>
+__global__ __launch_bounds__(64) void post_process_kernel(const int32_t* __restrict__ pos_ids,
+                                                         const int32_t* __restrict__ mask_index,
+                                                         int total, int32_t* __restrict__ retrieve,
+                                                         int32_t* __restrict__ shape) {
   __shared__ int inner[MAXT + 1];
-  __shared__ int depth[MAXT];
   __shared__ int par[MAXT];
   const int tid = threadIdx.x;
   const int T = total + 1;
-  if (tid <= MAXT) inner[tid] = 0;
-  for (int i = tid; i < MAXT * MAXT; i += blockDim.x) retrieve[i] = -1;
-  if (tid < T) depth[tid] = pos_ids[tid];
+  inner[tid] = 0;
+  if (tid == 0) inner[MAXT] = 0;
+  const int depth = tid < T ? pos_ids[tid] : 0;
   if (tid < total) par[tid] = mask_index[tid];
   __syncthreads();
   if (tid < total) {
@@ -114,22 +159,31 @@ __global__ __launch_bounds__(128) void post_process_kernel(const int32_t* __rest
     if (p >= 0 && p <= MAXT) inner[p] = 1;   // benign race: all writers store 1
   }
   __syncthreads();
+  const unsigned long long inner_mask = __ballot(inner[tid] != 0);
+  const int n_inner = __popcll(inner_mask) + inner[MAXT];
+  int md = depth;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const int other = __shfl_xor(md, o, 64);
+    md = other > md ? other : md;
+  }
+  const int leaves = total - (n_inner - 1), cols = md + 1;
+  if (tid == 0) {
+    shape[0] = leaves;
+    shape[1] = cols;
+  }
+  const int ld = PACKED ? (cols < 1 ? 1 : (cols > MAXT ? MAXT : cols)) : MAXT;
+  const int rows = PACKED ? (leaves < 1 ? 1 : (leaves > MAXT ? MAXT : leaves)) : MAXT;
+  for (int i = tid; i < rows * ld; i += 64) retrieve[i] = -1;
+  __syncthreads();
   if (tid < T && !inner[tid]) {
-    int r = 0;
-    for (int j = 0; j < tid; ++j) r += !inner[j];
+    const int r = __popcll(~inner_mask & ((1ull << tid) - 1ull));
     int cur = tid;
-    for (int col = depth[tid]; col >= 0; --col) {
-      if (col < MAXT) retrieve[r * MAXT + col] = cur;
+    for (int col = depth; col >= 0; --col) {
+      if (col < ld && r < rows) retrieve[r * ld + col] = cur;
       cur = (cur == 0) ? par[total - 1] : par[cur - 1];
       cur = cur < 0 ? 0 : (cur > total ? total : cur);
     }
-  }
-  if (tid == 0) {
-    int n_inner = 0, md = 0;
-    for (int j = 0; j <= MAXT; ++j) n_inner += inner[j];
-    for (int j = 0; j < T; ++j) md = depth[j] > md ? depth[j] : md;
-    shape[0] = total - (n_inner - 1);
-    shape[1] = md + 1;
   }
 }
 
@@ -240,6 +294,16 @@ __global__ void advance_len_kernel(int32_t* len_dev, int delta) {
 
 }  // namespace
 
+static int process_tree(const TreeLists& in, int C, int k, int total, int32_t* tree_position_ids, int32_t* mask_index,
+                        int32_t* draft_tokens, uint32_t* bits, void* mask, eagle_stream_t stream) {
+  if (k < 1 || C < 1 || C > MAXC || (C % k) != 0 || total < 1 || total >= MAXT || total > C)
+    return EAGLE_ERR_SHAPE;
+  hipLaunchKernelGGL(process_draft_tree_kernel, dim3(1), dim3(TREE_THREADS), 0, static_cast<hipStream_t>(stream),
+                     in, C, k, total, tree_position_ids, mask_index, draft_tokens, bits,
+                     static_cast<uint16_t*>(mask));
+  return eagle_launch_status();
+}
+
 EAGLE_EXPORT int eagle_process_draft_tree(const void* scores, const int32_t* tokens,
                                           const uint32_t* parents_list,
                                           const int32_t* sampled_token_dev, int C, int k,
@@ -249,12 +313,60 @@ EAGLE_EXPORT int eagle_process_draft_tree(const void* scores, const int32_t* tok
   if (!scores || !tokens || !parents_list || !sampled_token_dev || !tree_position_ids ||
       !mask_index || !draft_tokens || !tree_mask_bits)
     return EAGLE_ERR_NULL;
-  if (k < 1 || C < 1 || C > MAXC || (C % k) != 0 || total < 1 || total >= MAXT || total > C)
-    return EAGLE_ERR_SHAPE;
-  hipLaunchKernelGGL(process_draft_tree_kernel, dim3(1), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), (const half_t*)scores, tokens, parents_list,
-                     sampled_token_dev, C, k, total, tree_position_ids, mask_index, draft_tokens,
-                     tree_mask_bits);
+  TreeLists in = {};
+  in.scores[0] = static_cast<const half_t*>(scores);
+  in.tokens[0] = tokens;
+  in.parents[0] = parents_list;
+  in.end[0] = in.pend[0] = MAXC;
+  in.n = in.pn = 1;
+  in.root = sampled_token_dev;
+  return process_tree(in, C, k, total, tree_position_ids, mask_index, draft_tokens, tree_mask_bits, nullptr, stream);
+}
+
+EAGLE_EXPORT int eagle_process_draft_tree_lists(const void* const* scores, const int32_t* const* tokens,
+                                                const int* counts, int n, const uint32_t* const* parents,
+                                                const int* parent_counts, int parents_n,
+                                                const void* sampled_token_dev, int sampled_is_64bit, int k,
+                                                int total, int32_t* tree_position_ids, int32_t* mask_index,
+                                                int32_t* draft_tokens, void* tree_mask_bf16,
+                                                eagle_stream_t stream) {
+  if (!scores || !tokens || !counts || !parents || !parent_counts || !sampled_token_dev || !tree_position_ids ||
+      !mask_index || !draft_tokens || !tree_mask_bf16)
+    return EAGLE_ERR_NULL;
+  if (n < 1 || n > EAGLE_MAX_SEGMENTS || parents_n < 1 || parents_n > EAGLE_MAX_SEGMENTS) return EAGLE_ERR_SHAPE;
+  TreeLists in = {};
+  int C = 0, P = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!scores[i] || !tokens[i]) return EAGLE_ERR_NULL;
+    if (counts[i] < 1 || counts[i] > MAXC) return EAGLE_ERR_SHAPE;
+    in.scores[i] = static_cast<const half_t*>(scores[i]);
+    in.tokens[i] = tokens[i];
+    in.end[i] = C += counts[i];
+  }
+  for (int i = 0; i < parents_n; ++i) {
+    if (!parents[i]) return EAGLE_ERR_NULL;
+    if (parent_counts[i] < 1 || parent_counts[i] > MAXC) return EAGLE_ERR_SHAPE;
+    in.parents[i] = parents[i];
+    in.pend[i] = P += parent_counts[i];
+  }
+  if (k < 1 || P < C / k) return EAGLE_ERR_SHAPE;
+  in.n = n;
+  in.pn = parents_n;
+  in.root = sampled_token_dev;
+  in.root64 = sampled_is_64bit;
+  return process_tree(in, C, k, total, tree_position_ids, mask_index, draft_tokens, nullptr, tree_mask_bf16, stream);
+}
+
+static int post_process(const int32_t* tree_position_ids, const int32_t* mask_index, int total,
+                        int32_t* retrieve_indices, int32_t* shape_out, bool packed, eagle_stream_t stream) {
+  if (!tree_position_ids || !mask_index || !retrieve_indices || !shape_out) return EAGLE_ERR_NULL;
+  if (total < 1 || total >= MAXT) return EAGLE_ERR_SHAPE;
+  if (packed)
+    hipLaunchKernelGGL(post_process_kernel<true>, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream),
+                       tree_position_ids, mask_index, total, retrieve_indices, shape_out);
+  else
+    hipLaunchKernelGGL(post_process_kernel<false>, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream),
+                       tree_position_ids, mask_index, total, retrieve_indices, shape_out);
   return eagle_launch_status();
 }
 
@@ -262,11 +374,14 @@ EAGLE_EXPORT int eagle_post_process_draft_tree(const int32_t* tree_position_ids,
                                                const int32_t* mask_index, int total,
                                                int32_t* retrieve_indices, int32_t* shape_out,
                                                eagle_stream_t stream) {
-  if (!tree_position_ids || !mask_index || !retrieve_indices || !shape_out) return EAGLE_ERR_NULL;
-  if (total < 1 || total >= MAXT) return EAGLE_ERR_SHAPE;
-  hipLaunchKernelGGL(post_process_kernel, dim3(1), dim3(128), 0, static_cast<hipStream_t>(stream),
-                     tree_position_ids, mask_index, total, retrieve_indices, shape_out);
-  return eagle_launch_status();
+  return post_process(tree_position_ids, mask_index, total, retrieve_indices, shape_out, false, stream);
+}
+
+EAGLE_EXPORT int eagle_post_process_draft_tree_packed(const int32_t* tree_position_ids,
+                                                      const int32_t* mask_index, int total,
+                                                      int32_t* retrieve_indices, int32_t* shape_out,
+                                                      eagle_stream_t stream) {
+  return post_process(tree_position_ids, mask_index, total, retrieve_indices, shape_out, true, stream);
 }
 
 EAGLE_EXPORT int eagle_greedy_accept(const int32_t* node_argmax, const int32_t* draft_tokens,

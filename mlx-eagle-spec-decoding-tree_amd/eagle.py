@@ -169,6 +169,9 @@ def process_draft_tree_device(scores, tokens, parents_list, sampled_token_id, k,
 def process_draft_tree(scores_list, ss_token, parents_list, sampled_token_id, k, total_tokens):
     """mlx_eagle.py:217-250.  Lists of per-level tensors in, and
     (tree_position_ids [T], mask_index [V], draft_tokens [1,T], tree_mask [T,T] bf16) out."""
+    r = ops._native().process_draft_tree(scores_list, ss_token, parents_list, sampled_token_id, k, total_tokens)
+    if r is not None:      # fp16 scores and int32 tokens and parents of one sequence, read where they are
+        return r
     scores = torch.cat([s.reshape(s.shape[0], -1) for s in scores_list], dim=1).flatten()
     tokens = torch.cat([t.reshape(t.shape[0], -1) for t in ss_token], dim=1).flatten()
     parents = torch.cat([p.flatten() for p in parents_list], dim=0)
@@ -195,6 +198,9 @@ def post_process_draft_tree_device(tree_position_ids, total_tokens, mask_index, 
 def post_process_draft_tree(tree_position_ids, total_tokens, mask_index):
     """mlx_eagle.py:254-295: retrieve_indices [leaf_num, max_depth+1]; like the reference
     this form synchronises with the host (to learn the shape)."""
+    r = ops._native().post_process_draft_tree(tree_position_ids, mask_index, total_tokens)
+    if r is not None:
+        return r
     full, shape = post_process_draft_tree_device(tree_position_ids.to(torch.int32).contiguous(),
                                                  total_tokens,
                                                  mask_index.to(torch.int32).contiguous())

@@ -11,6 +11,7 @@ import torch
 
 from . import _lib
 
+_H = None       # the native host module, loaded by the first operator call
 _WS = {}        # (device index, tag) -> workspace tensor
 _RETIRED = []   # outgrown workspaces, kept allocated (see workspace())
 
@@ -21,6 +22,13 @@ def _stream():
 
 def _ptr(t):
     return None if t is None else t.data_ptr()
+
+
+def _native():
+    global _H
+    if _H is None:
+        _H = _lib.host()
+    return _H
 
 
 def _need_cuda(*ts):
@@ -67,13 +75,19 @@ def as_packed_u32(w_q):
 def quantized_matmul(x, w_q, scales, biases, transpose=True, group_size=64, bits=4, bias=None,
                      out=None, tuned=None, gemm=None):
     """`mx.quantized_matmul(x, w, scales, biases, transpose=True, group_size=64, bits=4)`
-    (any leading dims, flattened as qmm_kernel.py:99-100,136): the streaming kernel for 1..32
-    rows of x, two passes of it for 33..64 rows (a tree above 32 tokens; faster there than the
-    GEMM's few long-running workgroups: 21 against 31 us for 40 x 4608 x 3584, 44 against 185 us
-    for 40 x 3584 x 18944), a tiled GEMM above that.
-    `bias` ([N] fp16) is added after rounding, as the patched linear layer does
+    (any leading dims, flattened as qmm_kernel.py:99-100,136): the vector-ALU kernel for one row (or
+    two) where `qmv_preferred` says so, the streaming kernel for up to 32 rows of x, two passes of it
+    for 33..64 rows (a tree above 32 tokens; faster there than the GEMM's few long-running workgroups:
+    21 against 31 us for 40 x 4608 x 3584, 44 against 185 us for 40 x 3584 x 18944), a tiled GEMM above
+    that.  `bias` ([N] fp16) is added after rounding, as the patched linear layer does
     (mlx_model_fwd_bench.py:70-71).  `tuned` forces a launch shape of the streaming kernel,
-    `gemm=True` the tiled GEMM whatever the row count."""
+    `gemm=True` the tiled GEMM whatever the row count.  The default path is native code
+    (csrc/host.cpp)."""
+    default = transpose and group_size == 64 and bits == 4 and tuned is None and not gemm
+    if default:
+        r = _native().quantized_matmul(x, w_q, scales, biases, bias, out)
+        if r is not None:
+            return r
     if not transpose:
         raise ValueError("only transpose=True (x @ dequant(w).T) is implemented")
     _need_cuda(x, w_q, scales, biases, bias)
@@ -90,40 +104,23 @@ def quantized_matmul(x, w_q, scales, biases, transpose=True, group_size=64, bits
         bias = _f16(bias, "bias")
         if tuple(bias.shape) != (N,):
             raise ValueError("bias must have shape [N]")
+    if default:                      # the arguments in plain form now
+        r = _native().quantized_matmul(x, w_q, scales, biases, bias, out)
+        if r is None:
+            raise ValueError(f"out must be a contiguous float16 tensor of {M} x {N} elements" if M > 0 else "x is empty")
+        return r
     if out is None:
         out = torch.empty((*lead, N), dtype=torch.float16, device=x.device)
     L = _lib.lib()
+    if group_size != 64 or bits != 4:
+        _lib.check(4, "quantized_matmul")
     if M > 32 and tuned is not None:
         raise ValueError("launch shapes can be forced for at most 32 rows")
-    if ROW_PASS < M <= 2 * ROW_PASS and not gemm:
-        x2, out2 = x.reshape(M, K), out.view(M, N)
-        for r0 in range(0, M, ROW_PASS):
-            quantized_matmul(x2[r0:r0 + ROW_PASS], w_q, scales, biases, group_size=group_size, bits=bits,
-                             bias=bias, out=out2[r0:r0 + ROW_PASS])
-        return out
-    if M > 32 or gemm:
-        # many rows (the prompt pass): the tiled GEMM form
+    if gemm:
         rc = L.eagle_qmm_gemm_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias),
                                         _ptr(out), M, N, K, group_size, bits, _stream())
-        _lib.check(rc, "quantized_matmul")
-        return out
-    if tuned is None and M <= QMV_MAX_ROWS and qmv_preferred(N, K, M) and group_size == 64 and bits == 4:
-        # one row (or the few rows `qmv_preferred` takes): the vector-ALU kernel, faster than a 16-row
-        # matrix tile with most rows idle wherever the matrix has enough rows to fill the GPU with
-        # short K
-        rc = L.eagle_qmv_rows_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias),
-                                        _ptr(out), M, N, K, group_size, bits, _stream())
-        _lib.check(rc, "quantized_matmul")
-        return out
-    if tuned is None:
-        ws = workspace("qmm", L.eagle_qmm_workspace_bytes(M, N, K), x.device)
-        rc = L.eagle_qmm_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias),
-                                   _ptr(out), M, N, K, group_size, bits, _ptr(ws), ws.numel(),
-                                   _stream())
     else:
         # tuned = (nw, phases, splits, ranges[, unit_cols]): forced launch shape
-        if group_size != 64 or bits != 4:
-            raise ValueError("only group_size=64, bits=4 is supported")
         nw, phases, splits, ranges = (int(v) for v in tuned[:4])
         unit_cols = int(tuned[4]) if len(tuned) > 4 else 0
         need = L.eagle_qmm_workspace_bytes_tuned(M, N, splits)
@@ -477,23 +474,10 @@ def qkv_rope_small(x, w_q, scales, biases, bias, rope_cs, q_rot, k_cache, v_cach
     return q_rot
 
 
-# rows of x up to which `quantized_matmul` considers the vector-ALU kernel (`bench.py --small-m`
-# has the measurements behind QMV_MAX_ROWS and `qmv_preferred`)
-QMV_MAX_ROWS = 2
-
-
 def qmv_preferred(N, K, M=1):
-    """True where the vector-ALU kernel is the faster form for M rows of x.  Measured on the
-    projection shapes of the 7B model, vector ALU against matrix tiles, us per launch:
-      M = 1: 5.8 / 8.5 (3584 x 3584), 4.4 / 6.7 (512 x 3584), 12.6 / 16.1 (18944 x 3584), 5.3 / 7.1
-             (8192 x 2048); a long K over few rows (3584 x 18944: 28.3 / 18.9) and the vocabulary
-             projection (66.6 / 63.2) stay on the matrix kernel;
-      M = 2: 7.2 / 8.5, 5.8 / 6.9, 16.3 / 15.9, 6.6 / 7.2: the vector ALU up to a few thousand rows;
-      M = 4: 9.4 / 8.6, 8.4 / 7.0, 28.7 / 16.1, 8.9 / 7.3; M = 8: 15.1 / 8.7, 14.3 / 7.1, 44.2 / 16.1,
-             14.2 / 7.4: matrix tiles everywhere (5 + 4 M vector instructions per packed word)."""
-    if M > QMV_MAX_ROWS or not _lib.lib().eagle_qmv_rows_supported(M, N, K) or K > 4096:
-        return False
-    return N <= 65536 if M == 1 else N <= 16384
+    """True where the vector-ALU kernel is the faster form for M rows of x (the measurements behind the
+    rule are in csrc/qmv.hip; `bench.py --small-m` repeats them)."""
+    return bool(_lib.lib().eagle_qmv_preferred(int(M), int(N), int(K)))
 
 
 def quantized_matvec(x, w_q, scales, biases, bias=None, out=None):
@@ -568,18 +552,10 @@ def rope_kv_append(q_lin, k_lin, v_lin, positions, inv_freqs, scaling_factor, q_
     """Rotate q and k at `positions`, write q as [H,T,hd] and append k, v to the caches.
     row_stride > 0: q_lin, k_lin, v_lin are column blocks of one [T,row_stride] matrix.
     rope_cs: the `rope_table` of these positions (then positions / inv_freqs are not read)."""
-    T = q_lin.shape[0]
-    if rope_cs is not None:
-        rc = _lib.lib().eagle_rope_kv_append_table_f16(
-            _ptr(q_lin), _ptr(k_lin), _ptr(v_lin), _ptr(rope_cs), _ptr(q_out), _ptr(k_cache),
-            _ptr(v_cache), _ptr(cache_len_dev), T, H, G, hd, k_cache.shape[1], int(row_stride), _stream())
-        _lib.check(rc, "rope_kv_append")
-        return
-    rc = _lib.lib().eagle_rope_kv_append_f16(
-        _ptr(q_lin), _ptr(k_lin), _ptr(v_lin), _ptr(positions), _ptr(inv_freqs),
-        float(scaling_factor), _ptr(q_out), _ptr(k_cache), _ptr(v_cache), _ptr(cache_len_dev),
-        T, H, G, hd, k_cache.shape[1], int(row_stride), _stream())
-    _lib.check(rc, "rope_kv_append")
+    if _native().rope_kv_append(q_lin, k_lin, v_lin, positions, inv_freqs, scaling_factor, q_out, k_cache, v_cache,
+                                cache_len_dev, H, G, hd, row_stride, rope_cs) is None:
+        _need_cuda(q_lin, k_lin, v_lin, q_out, k_cache, v_cache, cache_len_dev)
+        raise ValueError("rope_kv_append takes device tensors, caches [G, capacity, head_dim] and positions or a table")
 
 
 def rope_kv_append_slabs(partial, slabs, bias, rope_cs, q_out, k_cache, v_cache, cache_len_dev, T, H, G, hd):
@@ -609,30 +585,12 @@ def tree_attention(q, k_cache, v_cache, tree_mask_bits, cache_len_dev, scale, ma
     """q [H,T,hd]; k_cache, v_cache [G,capacity,hd] holding *cache_len_dev prefix rows
     followed by the T tree rows; tree_mask_bits [T] int32, or [T,2] (`mask_to_words`) for
     trees of up to 64 tokens.  Returns [T, H*hd]."""
-    _need_cuda(q, k_cache, v_cache, tree_mask_bits, cache_len_dev)
-    H, T, hd = q.shape
-    G, cap, _ = k_cache.shape
-    if max_len is None:
-        max_len = cap
-    if out is None:
-        out = torch.empty((T, H * hd), dtype=torch.float16, device=q.device)
-    L = _lib.lib()
-    if tree_mask_bits.dim() == 2:
-        if tree_mask_bits.shape != (T, 2):
-            raise ValueError("two mask words per tree token")
-        ws = workspace("attn", L.eagle_tree_attention_wide_workspace_bytes(T, H, hd, max_len), q.device)
-        rc = L.eagle_tree_attention_wide_f16(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(tree_mask_bits),
-                                             _ptr(cache_len_dev), _ptr(out), T, T, H, G, hd, cap, max_len,
-                                             float(scale), _ptr(ws), ws.numel(), _stream())
-        _lib.check(rc, "tree_attention")
-        return out
-    need = L.eagle_tree_attention_workspace_bytes(H, hd, max_len)
-    ws = workspace("attn", need, q.device)
-    rc = L.eagle_tree_attention_f16(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(tree_mask_bits),
-                                    _ptr(cache_len_dev), _ptr(out), T, H, G, hd, cap, max_len,
-                                    float(scale), _ptr(ws), ws.numel(), _stream())
-    _lib.check(rc, "tree_attention")
-    return out
+    r = _native().tree_attention(q, k_cache, v_cache, tree_mask_bits, cache_len_dev, scale, max_len, out)
+    if r is None:
+        _need_cuda(q, k_cache, v_cache, tree_mask_bits, cache_len_dev, out)
+        raise ValueError("tree_attention takes q [H,T,hd], caches [G,capacity,hd], one mask word per tree token or "
+                         "two, and a contiguous float16 out")
+    return r
 
 
 def rope_table(positions, inv_freqs, scaling_factor=1.0, out=None):
