@@ -49,6 +49,7 @@ enum eagle_status {
                                 two mask words and the entry points that say so */
 #define EAGLE_MAX_TREE_SLOTS 64 /* tree tokens the tree-layout kernels take (root + 63 nodes; the reference's
                                    default is 39 nodes, mlx_eagle.py:390,510) */
+#define EAGLE_MAX_TILE_PARTS 4  /* row-major matrices that one tiled copy is made of */
 #define EAGLE_MAX_SEGMENTS 16 /* pieces of a list that the tree layout reads where they are */
 #define EAGLE_MAX_CHUNK 2048 /* rows of one causal pass over a prompt chunk */
 #define EAGLE_MAX_M 32       /* rows of x accepted by the quantised matmul */
@@ -252,6 +253,14 @@ int eagle_qmm_tiled_supported(int M, int N, int K);
 size_t eagle_qmm_tiled_sb_bytes(int N, int K);
 int eagle_qmm_tile_w4g64(const uint32_t* wq, const void* scales, const void* biases, uint32_t* wt,
                          void* sbt, int N, int K, int group_size, int bits, eagle_stream_t stream);
+/* The same from `parts` row-major matrices of rows[i] rows each (HOST arrays), stacked in order (q, k and
+ * v as one projection) or, with interleave != 0 and two parts of equal size, alternating in 16-row tiles
+ * (gate and up, as eagle_qmm_swiglu_w4g64_f16 takes them).  max_scale_bits (device, may be NULL): raised
+ * to the largest |scale| seen, as the bit pattern of a non-negative float. */
+int eagle_qmm_tile_parts_w4g64(const uint32_t* const* wq, const void* const* scales,
+                               const void* const* biases, const int* rows, int parts, int interleave,
+                               uint32_t* wt, void* sbt, int N, int K, unsigned* max_scale_bits,
+                               eagle_stream_t stream);
 int eagle_qmm_slab_partial_tiled_w4g64(const void* x, const uint32_t* wt, const void* sbt,
                                        float* partial, size_t partial_bytes, int M, int N, int K,
                                        int steps_per_slab, int small_scales, eagle_stream_t stream);
@@ -279,6 +288,34 @@ int eagle_slab_sum_f16(const float* partial, int slabs, const void* bias, void* 
 int eagle_embed_w4g64_f16(const int32_t* ids, const uint32_t* wq, const void* scales,
                           const void* biases, void* out, int T, int D, int V,
                           eagle_stream_t stream);
+
+/* Everything a pass through a decoder needs before its first product, one launch: the embedding rows h
+ * (eagle_embed_w4g64_f16), their RMSNorm hn (eagle_rmsnorm_f16, same arithmetic), the positions and the
+ * (cos, sin) table of eagle_rope_table_f32, the mask words, and the cache lengths the later launches read.
+ * Rows T .. R - 1 are padding (token 0, positions continuing). */
+typedef struct eagle_pass_begin {
+  const void* ids;             /* [T] token ids, int32 or (ids64) int64 */
+  const uint32_t* wq;          /* embedding [V, D/8] with scales, biases [V, D/64] */
+  const void *scales, *biases;
+  const void* norm_w;          /* [D] */
+  void *h, *hn;                /* [R, D]; hn may be NULL (no norm) */
+  const void* positions;       /* [T] int32 or (pos64) int64, or NULL: 0 for every row */
+  const int32_t* base_len;     /* device scalar added to every position, or NULL */
+  const float* inv_freqs;      /* [half] */
+  int32_t* positions_out;      /* [R] or NULL */
+  float* rope_cs;              /* [R, half, 2] or NULL */
+  const void* mask;            /* additive mask [T, Tk] (row stride mask_ld elements), or NULL: causal */
+  uint32_t* words;             /* [T, 2] mask words over the last Tk <= 64 rows, or NULL */
+  int32_t* lens;               /* {write_len, attn_len}, or NULL */
+  int32_t* piece_len;          /* [R / 32] = write_len + 32 j, or NULL */
+  long mask_ld;
+  float eps, scaling_factor;
+  int ids64, pos64, mask_bits; /* mask_bits: 16 (any 16-bit float) or 32 */
+  int T, R, D, V, half, Tk;
+  int pos_add, pos_step;       /* position of row t = positions[t] + *base_len + pos_add + pos_step * t */
+  int write_len, attn_len;
+} eagle_pass_begin;
+int eagle_pass_begin_f16(const eagle_pass_begin* args, eagle_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * RoPE with one position per (batch, token), half-split pairing, fp32 math.

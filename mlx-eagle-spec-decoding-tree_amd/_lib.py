@@ -47,6 +47,7 @@ SIGNATURES = {
     "eagle_qmm_tiled_supported": (c_int, [c_int] * 3),
     "eagle_qmm_tiled_sb_bytes": (c_size_t, [c_int] * 2),
     "eagle_qmm_tile_w4g64": (c_int, [c_void_p] * 5 + [c_int] * 4 + [c_void_p]),
+    "eagle_qmm_tile_parts_w4g64": (c_int, [c_void_p] * 4 + [c_int] * 2 + [c_void_p] * 2 + [c_int] * 2 + [c_void_p] * 2),
     "eagle_qmm_slab_partial_tiled_w4g64": (c_int, [c_void_p] * 4 + [c_size_t] + [c_int] * 5 + [c_void_p]),
     "eagle_qmm_slab_swiglu_tiled_w4g64_f16": (c_int, [c_void_p] * 5 + [c_int] * 4 + [c_void_p]),
     "eagle_qmm_rows_tiled_supported": (c_int, [c_int] * 3),
@@ -60,6 +61,7 @@ SIGNATURES = {
     "eagle_rope_kv_append_slabs_f16": (c_int, [c_void_p, c_int] + [c_void_p] * 6 + [c_int] * 4
                                        + [c_long, c_void_p]),
     "eagle_embed_w4g64_f16": (c_int, [c_void_p] * 5 + [c_int] * 3 + [c_void_p]),
+    "eagle_pass_begin_f16": (c_int, [c_void_p] * 2),
     "eagle_rope_arrayed_f16": (c_int, [c_void_p] * 3 + [c_float, c_void_p] + [c_int] * 4 + [c_void_p]),
     "eagle_rope_kv_append_f16": (c_int, [c_void_p] * 5 + [c_float] + [c_void_p] * 4 + [c_int] * 4
                                  + [c_long, c_long, c_void_p]),

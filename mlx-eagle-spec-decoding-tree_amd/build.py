@@ -90,24 +90,33 @@ def sources():
 
 
 def start_host(objdir):
-    """Start the compile of csrc/host.cpp, the native host path of the operators (no device code): a
-    Python module on torch's C++ interface.  Returns (process, object)."""
+    """Start the compiles of csrc/*.cpp, the native host path of the operators (no device code): a
+    Python module on torch's C++ interface.  Returns [(source, object, process)]."""
     import sysconfig
     import torch
     from torch.utils import cpp_extension
-    obj = os.path.join(objdir, "host.cpp.o")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *(f"-isystem{d}" for d in cpp_extension.include_paths()), "-isystem/opt/rocm/include",
-           f"-isystem{sysconfig.get_paths()['include']}", "-c", os.path.join(CSRC, "host.cpp"), "-o", obj]
-    return subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT), obj
+    out = []
+    for src in sorted(glob.glob(os.path.join(CSRC, "*.cpp"))):
+        obj = os.path.join(objdir, os.path.basename(src) + ".o")
+        cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+               *(f"-isystem{d}" for d in cpp_extension.include_paths()), "-isystem/opt/rocm/include",
+               f"-isystem{sysconfig.get_paths()['include']}", "-c", src, "-o", obj]
+        out.append((src, obj, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
+    return out
 
 
-def link_host(obj):
+def link_host(compiles):
     from torch.utils import cpp_extension
+    objs = []
+    for src, obj, p in compiles:
+        out, _ = p.communicate()
+        if p.returncode != 0:
+            raise RuntimeError(f"g++ failed on {src}:\n" + out.decode(errors="replace"))
+        objs.append(obj)
     libs = cpp_extension.library_paths()
     tmp = HOST + ".tmp"
-    cmd = ["g++", "-shared", obj, "-o", tmp, *(f"-L{d}" for d in libs), "-L/opt/rocm/lib", f"-L{HERE}",
+    cmd = ["g++", "-shared", *objs, "-o", tmp, *(f"-L{d}" for d in libs), "-L/opt/rocm/lib", f"-L{HERE}",
            "-l:libeagle_mi355x.so", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
            "-lamdhip64", "-Wl,-rpath,$ORIGIN"]
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
@@ -122,7 +131,7 @@ def build(verbose=False, jobs=8):
     cc = hipcc()
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
-    host, host_obj = start_host(objdir)
+    host = start_host(objdir)
     procs = []
     objs = []
     flags = [f for f in FLAGS if f != "-shared"]
@@ -159,10 +168,7 @@ def build(verbose=False, jobs=8):
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stdout.decode(errors="replace"))
     os.replace(tmp, LIB)
-    out, _ = host.communicate()
-    if host.returncode != 0:
-        raise RuntimeError("g++ failed on csrc/host.cpp:\n" + out.decode(errors="replace"))
-    link_host(host_obj)
+    link_host(host)
     return LIB
 
 

@@ -8,53 +8,31 @@
 // Every function returns None when an argument is not in the plain form (a device tensor of the expected
 // type, contiguous, of matching shape): the Python caller then normalises the arguments, or raises the
 // error it always raised, and calls again.
-#include <torch/csrc/autograd/python_variable.h>
-#include <ATen/ATen.h>
-#include <c10/hip/HIPStream.h>
+#include "host.h"
 
-#include "../../include/eagle_mi355x.h"
+using namespace eagle_host;
 
 namespace {
-
 PyObject* g_workspace = nullptr;     // ops.workspace(tag, nbytes, device)
-
-struct Slot {
-  void* ptr = nullptr;
-  size_t bytes = 0;
-};
 constexpr int MAX_DEVICES = 64;
 Slot g_qmm_ws[MAX_DEVICES];
+}  // namespace
 
-inline void* stream_of(const at::Tensor& t) {
-  return static_cast<void*>(c10::hip::getCurrentHIPStream(t.device().index()).stream());
-}
-
-// nullptr where the object is not a tensor
-inline const at::Tensor* tensor(PyObject* o) {
-  return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr;
-}
-inline bool plain(const at::Tensor* t, at::ScalarType dt) {
-  return t && t->is_cuda() && t->scalar_type() == dt && t->is_contiguous();
-}
-inline bool packed(const at::Tensor* t) {
-  return t && t->is_cuda() && t->is_contiguous() && t->dim() == 2 &&
-         (t->scalar_type() == at::kInt || t->scalar_type() == at::kUInt32);
-}
-inline at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dt, const at::Tensor& like) {
-  return at::empty(sizes, like.options().dtype(dt));
-}
+namespace eagle_host {
 
 PyObject* fail(int rc, const char* what) {
-  PyErr_Format(rc >= EAGLE_ERR_NULL && rc <= EAGLE_ERR_WORKSPACE ? PyExc_ValueError : PyExc_RuntimeError,
-               "%s: %s (status %d)", what, eagle_status_string(rc), rc);
+  if (rc >= 0)
+    PyErr_Format(rc >= EAGLE_ERR_NULL && rc <= EAGLE_ERR_WORKSPACE ? PyExc_ValueError : PyExc_RuntimeError,
+                 "%s: %s (status %d)", what, eagle_status_string(rc), rc);
   return nullptr;
 }
 
-// The split-K workspace of the streaming matmul (ops.workspace keeps it: zeroed counters that every call
-// leaves zero, never released once a captured graph may hold its address).
 bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out) {
   const int dev = like.device().index();
-  if (dev < 0 || dev >= MAX_DEVICES) return false;
+  if (dev < 0 || dev >= MAX_DEVICES) {
+    PyErr_SetString(PyExc_RuntimeError, "device index out of range");
+    return false;
+  }
   Slot& s = g_qmm_ws[dev];
   if (s.bytes < need) {
     PyObject* d = THPVariable_Wrap(like);
@@ -72,9 +50,8 @@ bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out) {
   return true;
 }
 
-// The product of M rows: which form runs is the rule of ops.quantized_matmul (its docstring).
-int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias,
-           void* out, int M, int N, int K, void* st, bool* python_error) {
+int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
+           int M, int N, int K, void* st) {
   const uint32_t* wq = static_cast<const uint32_t*>(w);
   if (M > 2 * EAGLE_MAX_M) return eagle_qmm_gemm_w4g64_f16(x, wq, s, b, bias, out, M, N, K, 64, 4, st);
   for (int r0 = 0; r0 < M; r0 += EAGLE_MAX_M) {
@@ -86,16 +63,17 @@ int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, 
       rc = eagle_qmv_rows_w4g64_f16(xr, wq, s, b, bias, outr, m, N, K, 64, 4, st);
     } else {
       Slot ws;
-      if (!qmm_workspace(like, eagle_qmm_workspace_bytes(m, N, K), &ws)) {
-        *python_error = PyErr_Occurred() != nullptr;
-        return EAGLE_ERR_WORKSPACE;
-      }
+      if (!qmm_workspace(like, eagle_qmm_workspace_bytes(m, N, K), &ws)) return -1;
       rc = eagle_qmm_w4g64_f16(xr, wq, s, b, bias, outr, m, N, K, 64, 4, ws.ptr, ws.bytes, st);
     }
     if (rc != EAGLE_OK) return rc;
   }
   return EAGLE_OK;
 }
+
+}  // namespace eagle_host
+
+namespace {
 
 // quantized_matmul(x, w_q, scales, biases, bias, out)
 PyObject* py_quantized_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -122,10 +100,8 @@ PyObject* py_quantized_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
   }
   const at::Tensor& o = a[5] == Py_None ? made : *out;
-  bool python_error = false;
   const int rc = matmul(*x, x->data_ptr(), w->data_ptr(), s->data_ptr(), b->data_ptr(), bias ? bias->data_ptr() : nullptr,
-                        o.data_ptr(), (int)M, (int)N, (int)K, stream_of(*x), &python_error);
-  if (python_error) return nullptr;
+                        o.data_ptr(), (int)M, (int)N, (int)K, stream_of(*x));
   if (rc != EAGLE_OK) return fail(rc, "quantized_matmul");
   if (a[5] == Py_None) return THPVariable_Wrap(std::move(made));
   Py_INCREF(a[5]);
@@ -294,6 +270,41 @@ PyObject* py_post_process_draft_tree(PyObject*, PyObject* const* a, Py_ssize_t n
   return THPVariable_Wrap(full.narrow(0, 0, leaves * cols).view({leaves, cols}));
 }
 
+// tile_parts(weights, scales, biases, interleave, wt, sbt, max_scale): one tiled copy of a list of matrices
+// (eagle_qmm_tile_parts_w4g64), max_scale a float32 scalar on the device
+PyObject* py_tile_parts(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 7 || !PyList_Check(a[0]) || !PyList_Check(a[1]) || !PyList_Check(a[2])) {
+    PyErr_SetString(PyExc_TypeError, "tile_parts takes three lists and four more arguments");
+    return nullptr;
+  }
+  const Py_ssize_t parts = PyList_GET_SIZE(a[0]);
+  const at::Tensor *wt = tensor(a[4]), *sbt = tensor(a[5]), *mx = tensor(a[6]);
+  if (parts < 1 || parts > EAGLE_MAX_TILE_PARTS || PyList_GET_SIZE(a[1]) != parts || PyList_GET_SIZE(a[2]) != parts ||
+      !wt || !wt->is_cuda() || !wt->is_contiguous() || !plain(sbt, at::kHalf) || !plain(mx, at::kFloat))
+    Py_RETURN_NONE;
+  const uint32_t* w[EAGLE_MAX_TILE_PARTS];
+  const void *s[EAGLE_MAX_TILE_PARTS], *b[EAGLE_MAX_TILE_PARTS];
+  int rows[EAGLE_MAX_TILE_PARTS];
+  int64_t N = 0, K = 0;
+  for (Py_ssize_t i = 0; i < parts; ++i) {
+    const at::Tensor *wi = tensor(PyList_GET_ITEM(a[0], i)), *si = tensor(PyList_GET_ITEM(a[1], i)),
+                     *bi = tensor(PyList_GET_ITEM(a[2], i));
+    if (!packed(wi) || !plain(si, at::kHalf) || !plain(bi, at::kHalf)) Py_RETURN_NONE;
+    if (i == 0) K = wi->size(1) * 8;
+    if (wi->size(1) * 8 != K || si->numel() * 64 != wi->size(0) * K || bi->numel() * 64 != wi->size(0) * K) Py_RETURN_NONE;
+    w[i] = static_cast<const uint32_t*>(wi->data_ptr());
+    s[i] = si->data_ptr();
+    b[i] = bi->data_ptr();
+    rows[i] = (int)wi->size(0);
+    N += wi->size(0);
+  }
+  if (wt->numel() * wt->element_size() < N * K / 2 || sbt->numel() < N * (K / 64) * 2) Py_RETURN_NONE;
+  const int rc = eagle_qmm_tile_parts_w4g64(w, s, b, rows, (int)parts, PyObject_IsTrue(a[3]), static_cast<uint32_t*>(wt->data_ptr()),
+                                            sbt->data_ptr(), (int)N, (int)K, static_cast<unsigned*>(mx->data_ptr()), stream_of(*wt));
+  if (rc != EAGLE_OK) return fail(rc, "tile_weights");
+  Py_RETURN_TRUE;
+}
+
 // init(workspace): ops.workspace, which keeps the buffers that outlive a call
 PyObject* py_init(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 1 || !PyCallable_Check(a[0])) {
@@ -322,6 +333,10 @@ PyMethodDef methods[] = {EAGLE_PY(init),
                          EAGLE_PY(tree_attention),
                          EAGLE_PY(process_draft_tree),
                          EAGLE_PY(post_process_draft_tree),
+                         EAGLE_PY(tile_parts),
+                         EAGLE_PY(decoder_new),
+                         EAGLE_PY(decoder_current),
+                         EAGLE_PY(decoder_forward),
                          {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods};

@@ -1,0 +1,52 @@
+// Shared by the native host path (host.cpp, decoder.cpp): torch tensors in, C-ABI calls out.
+#pragma once
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+
+#include "../../include/eagle_mi355x.h"
+
+namespace eagle_host {
+
+struct Slot {
+  void* ptr = nullptr;
+  size_t bytes = 0;
+};
+
+inline void* stream_of(const at::Tensor& t) {
+  return static_cast<void*>(c10::hip::getCurrentHIPStream(t.device().index()).stream());
+}
+
+// nullptr where the object is not a tensor
+inline const at::Tensor* tensor(PyObject* o) {
+  return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr;
+}
+inline bool plain(const at::Tensor* t, at::ScalarType dt) {
+  return t && t->is_cuda() && t->scalar_type() == dt && t->is_contiguous();
+}
+inline bool packed(const at::Tensor* t) {
+  return t && t->is_cuda() && t->is_contiguous() && t->dim() == 2 &&
+         (t->scalar_type() == at::kInt || t->scalar_type() == at::kUInt32);
+}
+inline at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dt, const at::Tensor& like) {
+  return at::empty(sizes, like.options().dtype(dt));
+}
+
+// raises what _lib.check raises
+PyObject* fail(int rc, const char* what);
+
+// The split-K workspace of the streaming matmul on the device of `like` (ops.workspace keeps it: zeroed
+// counters that every call leaves zero, never released once a captured graph may hold its address).
+// False with a Python error set.
+bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out);
+
+// The product of M rows: which form runs is the rule of ops.quantized_matmul (its docstring).  A negative
+// result: a Python error is set.
+int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
+           int M, int N, int K, void* st);
+
+PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n);
+PyObject* py_decoder_current(PyObject*, PyObject* const* a, Py_ssize_t n);
+PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n);
+
+}  // namespace eagle_host

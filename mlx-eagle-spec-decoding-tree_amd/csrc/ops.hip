@@ -343,6 +343,98 @@ __global__ void embed_kernel(const int32_t* __restrict__ ids, const uint32_t* __
 }
 
 // ------------------------------------------------------------------------------------
+// The start of a pass (eagle_pass_begin): a workgroup per row.  Six launches of a few microseconds
+// each (positions, mask words, table, embedding, norm and the length scalars) with nothing to do but
+// wait for one another; here a row's chain is: token id -> packed words -> row sum.
+// ------------------------------------------------------------------------------------
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void pass_begin_kernel(eagle_pass_begin a) {
+  constexpr int NV = 256 * RMS_MAXV / BLOCK;
+  __shared__ float red[BLOCK / 64];
+  const int r = blockIdx.x, tid = threadIdx.x;
+  int id = 0;
+  if (r < a.T) {
+    const long v = a.ids64 ? static_cast<const int64_t*>(a.ids)[r] : (long)static_cast<const int32_t*>(a.ids)[r];
+    id = v < 0 ? 0 : (v >= a.V ? a.V - 1 : (int)v);   // as the embedding gather: stay in bounds
+  }
+  const long src = r < a.T ? r : a.T - 1;
+  int pos = a.pos_add + a.pos_step * r;
+  if (a.positions)
+    pos += a.pos64 ? (int)static_cast<const int64_t*>(a.positions)[src] : static_cast<const int32_t*>(a.positions)[src];
+  if (a.base_len) pos += *a.base_len;
+
+  // embedding row and its norm, vector c of the row in thread c % BLOCK as in rmsnorm_kernel
+  const int nvec = a.D >> 3;
+  const half_t* nw = static_cast<const half_t*>(a.norm_w);
+  half8_t v[NV], w8[NV];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = tid + i * BLOCK;
+    if (c < nvec) {
+      if (a.hn) w8[i] = *reinterpret_cast<const half8_t*>(nw + c * 8);
+      const uint32_t word = a.wq[(long)id * nvec + c];
+      const float sc = (float)static_cast<const half_t*>(a.scales)[(long)id * (a.D >> 6) + (c >> 3)];
+      const float bi = (float)static_cast<const half_t*>(a.biases)[(long)id * (a.D >> 6) + (c >> 3)];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[i][j] = (half_t)__builtin_fmaf(sc, (float)((word >> (4 * j)) & 15u), bi);
+      *reinterpret_cast<half8_t*>(static_cast<half_t*>(a.h) + (long)r * a.D + c * 8) = v[i];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss += (float)v[i][j] * (float)v[i][j];
+    }
+  }
+
+  if (a.rope_cs)
+    for (int i = tid; i < a.half; i += BLOCK) {
+      const float lf = a.scaling_factor * a.inv_freqs[i];
+      float sn, cs;
+      sincosf(lf * (float)pos, &sn, &cs);
+      *reinterpret_cast<float2_t*>(a.rope_cs + ((long)r * a.half + i) * 2) = float2_t{cs, sn};
+    }
+  if (tid == 0) {
+    if (a.positions_out) a.positions_out[r] = pos;
+    if (r == 0 && a.lens) {
+      a.lens[0] = a.write_len;
+      a.lens[1] = a.attn_len;
+    }
+    if (a.piece_len && (r & 31) == 0) a.piece_len[r >> 5] = a.write_len + r;
+  }
+  if (a.words && r < a.T && tid < 64) {
+    // lane j: is row j of the last Tk visible to this query (an additive mask is 0 there)
+    bool vis = false;
+    if (tid < a.Tk) {
+      if (!a.mask)
+        vis = tid <= a.Tk - a.T + r;
+      else if (a.mask_bits == 32)
+        vis = (static_cast<const uint32_t*>(a.mask)[r * a.mask_ld + tid] & 0x7fffffffu) == 0u;
+      else
+        vis = (static_cast<const uint16_t*>(a.mask)[r * a.mask_ld + tid] & 0x7fffu) == 0u;
+    }
+    const unsigned long long m = __ballot(vis);
+    if (tid < 2) a.words[2 * r + tid] = (uint32_t)(m >> (32 * tid));
+  }
+
+  if (!a.hn) return;
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  float tot = 0.f;
+#pragma unroll
+  for (int k = 0; k < BLOCK / 64; ++k) tot += red[k];
+  const float rinv = 1.0f / sqrtf(tot / (float)a.D + a.eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = tid + i * BLOCK;
+    if (c < nvec) {
+      half8_t o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (half_t)((float)w8[i][j] * ((float)v[i][j] * rinv));
+      *reinterpret_cast<half8_t*>(static_cast<half_t*>(a.hn) + (long)r * a.D + c * 8) = o;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------
 // Row argmax, first maximum.  Stage 1: grid (chunks, rows); stage 2: one wave per row.
 // ------------------------------------------------------------------------------------
 struct ValIdx {
@@ -577,6 +669,26 @@ EAGLE_EXPORT int eagle_embed_w4g64_f16(const int32_t* ids, const uint32_t* wq, c
   hipLaunchKernelGGL(embed_kernel, dim3(blocks_for(total, 256)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), ids, wq, (const half_t*)scales,
                      (const half_t*)biases, (half_t*)out, T, D, V);
+  return eagle_launch_status();
+}
+
+EAGLE_EXPORT int eagle_pass_begin_f16(const eagle_pass_begin* args, eagle_stream_t stream) {
+  if (!args) return EAGLE_ERR_NULL;
+  const eagle_pass_begin& a = *args;
+  if (!a.ids || !a.wq || !a.scales || !a.biases || !a.h || (a.hn && !a.norm_w) || (a.rope_cs && !a.inv_freqs))
+    return EAGLE_ERR_NULL;
+  if (a.T < 1 || a.R < a.T || a.R > EAGLE_MAX_CHUNK || a.V < 1 || a.D < 64 || (a.D % 64) != 0 ||
+      a.D > 256 * 8 * RMS_MAXV || (a.rope_cs && a.half < 1) ||
+      (a.words && (a.Tk < 1 || a.Tk > 64 || (!a.mask && a.Tk < a.T))) || (a.mask && a.mask_bits != 16 && a.mask_bits != 32))
+    return EAGLE_ERR_SHAPE;
+  if (!eagle_aligned16(a.h) || (a.hn && (!eagle_aligned16(a.hn) || !eagle_aligned16(a.norm_w))) ||
+      (a.rope_cs && (reinterpret_cast<uintptr_t>(a.rope_cs) & 7u)))
+    return EAGLE_ERR_ALIGN;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (a.D > 256 * 8)     // the block of rmsnorm_kernel, so that both give the same bits
+    hipLaunchKernelGGL(pass_begin_kernel<512>, dim3(a.R), dim3(512), 0, st, a);
+  else
+    hipLaunchKernelGGL(pass_begin_kernel<256>, dim3(a.R), dim3(256), 0, st, a);
   return eagle_launch_status();
 }
 

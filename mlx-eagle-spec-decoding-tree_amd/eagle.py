@@ -9,8 +9,9 @@ import math
 
 import torch
 
-from . import _lib, ops
+from . import _lib, native, ops
 from .layer import emit_layer
+from .llama import Model
 
 MAXT = 32            # tree tokens per matmul launch and per mask word; larger trees: two of each
 TREE_SLOTS = 64      # tree tokens the tree-layout kernels, the module path and the fused step take
@@ -223,6 +224,12 @@ def evaluate_posterior_greedy(logits, candidates):
 def tree_decoding(token_ids, tree_mask, tree_position_ids, base_model, cache):
     """mlx_eagle.py:329-346."""
     offset = cache[0].offset
+    if isinstance(base_model, Model) and isinstance(tree_mask, torch.Tensor) and tree_mask.dim() == 2:
+        # the mask covers the tree's own rows, everything before them is visible: no [T, S] mask is built
+        out = native.forward(base_model, token_ids, cache, mask=tree_mask, Tk=tree_mask.shape[1],
+                             positions=tree_position_ids, pos_add=offset)
+        if out is not None:
+            return out
     T = tree_mask.shape[0]
     mask = torch.zeros((1, 1, T, offset), dtype=tree_mask.dtype, device=tree_mask.device)
     mask = torch.cat((mask, tree_mask[None, None]), dim=-1)
@@ -400,6 +407,46 @@ def fuse_projections(model, swiglu):
     return qkv_w, gu_w
 
 
+def tile_model(model):
+    """The q|k|v, o, gate|up (interleaved) and down matrices of every layer as `ops.TiledWeights`, with the
+    bias of the product (q|k|v, gate|up) or None: one [(tiled, bias) x 4] per layer.  One set per model,
+    rebuilt when a source tensor was exchanged or written to; the copies are slices of two allocations."""
+    sources, layers = [], []
+    for layer in model.model.layers:
+        at, mlp = layer.self_attn, layer.mlp
+        groups = ([at.q_proj, at.k_proj, at.v_proj], [at.o_proj], [mlp.gate_proj, mlp.up_proj], [mlp.down_proj])
+        layers.append(groups)
+        sources += [(t.data_ptr(), 0 if t.is_inference() else t._version) for g in groups for lin in g
+                    for t in (lin.weight, lin.scales, lin.biases, lin.bias) if t is not None]
+    done = model.__dict__.get("_tiled_model")
+    if done is not None and done[0] == sources:
+        return done[1]
+    dev = model.model.layers[0].self_attn.q_proj.weight.device
+    sizes = [(sum(lin.weight.shape[0] for lin in g), g[0].weight.shape[1] * 8) for groups in layers for g in groups]
+    wt = torch.empty(sum(n * k // 8 for n, k in sizes), dtype=torch.int32, device=dev)
+    sbt = torch.empty(sum(n * k // 32 for n, k in sizes), dtype=torch.float16, device=dev)
+    worst = torch.zeros(len(sizes), dtype=torch.float32, device=dev)
+    made, w0, s0 = [], 0, 0
+    for i, (g, (n, k)) in enumerate(zip((g for groups in layers for g in groups), sizes)):
+        w1, s1 = w0 + n * k // 8, s0 + n * k // 32
+        made.append(ops.tile_parts(g, len(g) == 2, wt[w0:w1].view(n // 32, k // 64, 64, 4),
+                                   sbt[s0:s1].view(n // 32, k // 512, 64, 8), worst[i:i + 1]))
+        w0, s0 = w1, s1
+    for t, m in zip(made, worst.tolist()):
+        t.small = m < ops.TILED_SMALL_SCALE
+
+    def bias_of(g):
+        if all(lin.bias is None for lin in g):
+            return None
+        parts = [lin.bias if lin.bias is not None else torch.zeros(lin.weight.shape[0], dtype=torch.float16, device=dev)
+                 for lin in g]
+        return ops.interleave_gate_up(*parts) if len(g) == 2 else torch.cat(parts)
+
+    out = [[(t, bias_of(g)) for t, g in zip(made[4 * i:4 * i + 4], groups)] for i, groups in enumerate(layers)]
+    model.__dict__["_tiled_model"] = (sources, out)
+    return out
+
+
 def tiled_projections(model, qkv_w, gu_w, plan, swiglu):
     """`ops.TiledWeights` copies of the projections a pass of up to 32 rows runs through the slab
     kernels: q|k|v, o and down where `plan` sends them there, and the interleaved gate|up when
@@ -416,6 +463,12 @@ def tiled_projections(model, qkv_w, gu_w, plan, swiglu):
         n, k = w.shape[0], w.shape[1] * 8
         return ops.tile_weights(w, sc, bi) if ops.tiled_supported(32, n, k) else None
 
+    if all(key) and all(ops.tiled_supported(32, w[0].shape[0], w[0].shape[1] * 8) for w in (
+            qkv_w[0], gu_w[0], (model.model.layers[0].self_attn.o_proj.weight,),
+            (model.model.layers[0].mlp.down_proj.weight,))):
+        sets = tile_model(model)
+        done[key] = {name: [entry[j][0] for entry in sets] for j, name in enumerate(("qkv", "o", "gu", "down"))}
+        return done[key]
     out = {"qkv": [], "o": [], "down": [], "gu": []}
     for i, layer in enumerate(model.model.layers):
         at, mlp = layer.self_attn, layer.mlp

@@ -6,15 +6,17 @@ fp16 roundings fall in the same places; every operator runs as a HIP kernel
 behind the C ABI.  `patch_model(model, kernel)` is the plug-in seam of
 mlx_model_fwd_bench.py:43-86.
 
-The kernels serve at most 32 rows per linear layer.  Passes without a mask are causal
-(mlx_llama.py:275-276); longer ones (the prompt) run as consecutive 32-token passes.
+A pass runs as one native call where `native` takes the model and the arguments; the modules below
+are the same pass operator by operator (patched layers, other caches).  There the kernels serve at
+most 32 rows per linear layer.  Passes without a mask are causal (mlx_llama.py:275-276); longer ones
+(the prompt) run as consecutive 32-token passes.
 """
 from functools import reduce
 
 import numpy as np
 import torch
 
-from . import ops
+from . import native, ops
 from .synth import ModelArgs, inv_freqs
 
 
@@ -23,6 +25,16 @@ CAUSAL_CHUNK = 32
 
 class Module:
     """Minimal module base: attribute containers that can be walked and patched."""
+
+    epoch = 0        # attribute assignments on any module so far: what the native decoders are checked against
+
+    def __setattr__(self, name, value):
+        Module.epoch += 1
+        object.__setattr__(self, name, value)
+
+    def __delattr__(self, name):
+        Module.epoch += 1
+        object.__delattr__(self, name)
 
     def children(self):
         for name, value in vars(self).items():
@@ -215,7 +227,20 @@ class Model(Module):
             tensors[k] = torch.from_numpy(np.ascontiguousarray(v)).to(device)
         return cls(args, tensors, device)
 
+    def _native_pass(self, inputs, cache, mask, position_ids, flat_rope):
+        """The pass as one native call (csrc/decoder.cpp), or None where that does not take the arguments."""
+        if cache is None or (mask is None and inputs.shape[1] > CAUSAL_CHUNK
+                             and (position_ids is not None or flat_rope)):
+            return None
+        if isinstance(position_ids, torch.Tensor):
+            return native.forward(self, inputs, cache, mask, positions=position_ids)
+        start = cache[0].offset if position_ids is None else int(position_ids)
+        return native.forward(self, inputs, cache, mask, pos_add=start, pos_step=0 if flat_rope else 1)
+
     def __call__(self, inputs, cache=None, mask=None, position_ids=None, flat_rope=False):
+        out = self._native_pass(inputs, cache, mask, position_ids, flat_rope)
+        if out is not None:
+            return out
         if mask is None and inputs.shape[1] > CAUSAL_CHUNK:
             # a long causal pass (prompt prefill, mlx_eagle.py:522-533) as consecutive passes of
             # at most 32 tokens: the kernels of this path take at most 32 rows

@@ -1,0 +1,145 @@
+"""The native form of a decoder (csrc/decoder.cpp): built once per model from its layers, used by
+`Model.__call__`, `tree_decoding` and the draft expansion for every pass that it takes.
+
+A decoder is rebuilt when an attribute of a module changed, a layer was exchanged, or somebody wrote
+to a weight tensor.  Models it does not take (a patched layer, another group size, CPU tensors) run
+the Python operators of the module path."""
+import torch
+
+from . import ops
+from .cache import KVCache
+
+PLAIN, FUSED, TILED = 0, 1, 2
+
+# Below this hidden size the layers keep one launch per projection on the checkpoint's own tensors: their
+# weights (under 4 MB per layer) are a few microseconds of reading either way, and no copy of them is made.
+FUSE_HIDDEN = 768
+
+
+class _State:
+    def __init__(self, epoch, handle):
+        self.epoch, self.handle = epoch, handle
+
+
+def decoder(model):
+    """The decoder of `model` (a handle for `forward`), or None where the native form does not take it."""
+    from .llama import Module
+    st = model.__dict__.get("_native")
+    if st is not None:
+        if st.epoch == Module.epoch and (st.handle is None or ops._native().decoder_current(st.handle)):
+            return st.handle
+    epoch = Module.epoch
+    handle = _build(model)
+    model.__dict__["_native"] = _State(epoch if Module.epoch == epoch else Module.epoch, handle)
+    return handle
+
+
+def forward(model, ids, cache, mask=None, words=None, Tk=0, positions=None, pos_add=0, pos_step=0, head=2):
+    """One pass (see decoder_forward in csrc/decoder.cpp): logits [1, rows, V], True with head=0, or None
+    where this path does not take the arguments (nothing has been done then)."""
+    handle = decoder(model)
+    if handle is None:
+        return None
+    return ops._native().decoder_forward(handle, ids, cache, mask, words, Tk, positions, pos_add, pos_step, head)
+
+
+def _leaf(lin):
+    return lin.weight, lin.scales, lin.biases, lin.bias
+
+
+def _plain_leaf(lin, n, k, device):
+    from .llama import QuantizedLinear
+    if type(lin) is not QuantizedLinear or lin.group_size != 64 or lin.bits != 4:
+        return False
+    ts = [t for t in _leaf(lin) if t is not None]
+    return (all(isinstance(t, torch.Tensor) and t.device == device and t.is_contiguous() for t in ts)
+            and lin.weight.dtype in (torch.int32, torch.uint32) and tuple(lin.weight.shape) == (n, k // 8)
+            and all(t.dtype == torch.float16 for t in ts[1:]) and all(t.data_ptr() % 16 == 0 for t in ts)
+            and tuple(lin.scales.shape) == tuple(lin.biases.shape) == (n, k // 64)
+            and (lin.bias is None or tuple(lin.bias.shape) == (n,)))
+
+
+def _build(model):
+    from .llama import Attention, LlamaModel, MLP, QuantizedEmbedding, RMSNorm, TransformerBlock
+    args, m = model.args, model.model
+    if type(m) is not LlamaModel or not isinstance(m.layers, list) or not m.layers or type(m.norm) is not RMSNorm:
+        return None
+    D, I, V = args.hidden_size, args.intermediate_size, args.vocab_size
+    H, G, hd = args.num_attention_heads, args.num_key_value_heads, args.head_dim
+    emb = m.embed_tokens
+    if type(emb) is not QuantizedEmbedding or emb.group_size != 64 or emb.bits != 4 or not emb.weight.is_cuda:
+        return None
+    dev = emb.weight.device
+    # what the kernels of every form take
+    if hd not in (64, 128) or H % G or H // G > 8 or D % 64 or I % 64 or (H * hd) % 64 or V % 8 or D > 8192:
+        return None
+    shapes = {"q": (H * hd, D), "k": (G * hd, D), "v": (G * hd, D), "o": (D, H * hd), "gate": (I, D), "up": (I, D),
+              "down": (D, I)}
+    if any(n % 8 or k % 64 for n, k in shapes.values()):
+        return None
+    norms = [m.norm]
+    layers = []
+    for layer in m.layers:
+        if type(layer) is not TransformerBlock or type(layer.self_attn) is not Attention or type(layer.mlp) is not MLP:
+            return None
+        at, mlp = layer.self_attn, layer.mlp
+        lins = dict(q=at.q_proj, k=at.k_proj, v=at.v_proj, o=at.o_proj, gate=mlp.gate_proj, up=mlp.up_proj,
+                    down=mlp.down_proj)
+        if not all(_plain_leaf(lin, *shapes[name], dev) for name, lin in lins.items()):
+            return None
+        norms += [layer.input_layernorm, layer.post_attention_layernorm]
+        layers.append(lins)
+    if not all(type(n) is RMSNorm and n.eps == args.rms_norm_eps and n.weight.device == dev and n.weight.dtype == torch.float16
+               and n.weight.is_contiguous() and tuple(n.weight.shape) == (D,) and n.weight.data_ptr() % 16 == 0 for n in norms):
+        return None
+    head = emb if args.tie_word_embeddings else model.lm_head
+    head_w = (head.weight, head.scales, head.biases, None if head is emb else head.bias)
+    emb_w = (emb.weight, emb.scales, emb.biases, None)
+    for w in (emb_w, head_w):
+        if w[0].dtype not in (torch.int32, torch.uint32) or tuple(w[0].shape) != (V, D // 8) \
+                or not all(t is None or (t.device == dev and t.is_contiguous()) for t in w):
+            return None
+    if head is not emb and not _plain_leaf(head, V, D, dev):
+        return None
+    at0 = m.layers[0].self_attn
+    if any(l.self_attn._inv_freqs is not at0._inv_freqs and not torch.equal(l.self_attn._inv_freqs, at0._inv_freqs)
+           or l.self_attn._scaling_factor != at0._scaling_factor or l.self_attn.scale != at0.scale for l in m.layers):
+        return None
+    if at0._inv_freqs.numel() != hd // 2 or not at0._inv_freqs.is_cuda or at0._inv_freqs.dtype != torch.float32:
+        return None
+
+    form, small, derived, thead = _derive(model, layers, head_w, shapes, I, D, V, H, G, hd)
+    described = []
+    for i, lins in enumerate(layers):
+        layer = m.layers[i]
+        leaves = [_leaf(lin) for lin in (layer.self_attn.q_proj, layer.self_attn.k_proj, layer.self_attn.v_proj,
+                                         layer.self_attn.o_proj, layer.mlp.gate_proj, layer.mlp.up_proj, layer.mlp.down_proj)]
+        described.append((*leaves, *derived[i], layer.input_layernorm.weight, layer.post_attention_layernorm.weight))
+    return ops._native().decoder_new(
+        (D, I, H, G, hd, V, form, int(small)), (args.rms_norm_eps, float(at0._scaling_factor), float(at0.scale)), emb_w, head_w,
+        thead, m.norm.weight, at0._inv_freqs, described, m.layers, KVCache)
+
+
+def _derive(model, layers, head_w, shapes, I, D, V, H, G, hd):
+    """(form, scales small enough for the small-row products, per layer (qkv, gu, four tiled copies), tiled head)."""
+    from . import eagle
+    none = (None,) * 6
+    if D < FUSE_HIDDEN:
+        return PLAIN, False, [none] * len(layers), None
+    W = (H + 2 * G) * hd
+    products = {"qkv": (W, D), "o": shapes["o"], "down": shapes["down"]}
+    tiled = all(ops.slab_steps(32, n, k) and ops.tiled_supported(32, n, k) for n, k in products.values()) \
+        and ops.tiled_supported(32, 2 * I, D) and I % 16 == 0 \
+        and all(lins["o"].bias is None and lins["down"].bias is None for lins in layers)
+    if tiled:
+        sets = eagle.tile_model(model)
+        derived = [(None, None, *((t.wt, t.sbt, t.N, t.K, t.small, b) for t, b in entry)) for entry in sets]
+        th = eagle.tiled_head(model) if head_w[3] is None else None
+        return TILED, False, derived, None if th is None else (th.wt, th.sbt, th.N, th.K, th.small, None)
+    if not ops.swiglu_supported(32, I, D) or W % 16 or D % 16:
+        return PLAIN, False, [none] * len(layers), None
+    qkv_w, gu_w = eagle.fuse_projections(model, True)
+    worst = torch.stack([t.abs().amax() for i, lins in enumerate(layers)
+                         for t in (qkv_w[i][1], lins["o"].scales, gu_w[i][1], lins["down"].scales)]).amax()
+    small = bool(worst.item() < ops.SMALL_SCALE_LIMIT)
+    return FUSED, small, [(qkv_w[i], gu_w[i], None, None, None, None) for i in range(len(layers))], None

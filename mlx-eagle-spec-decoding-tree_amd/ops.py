@@ -388,6 +388,18 @@ def tiled_supported(M, N, K):
     return bool(_lib.lib().eagle_qmm_tiled_supported(int(M), int(N), int(K)))
 
 
+def tile_parts(linears, interleave, wt, sbt, max_scale):
+    """One tiled copy, in `wt` and `sbt`, of the matrices of `linears` (anything with weight, scales and biases in
+    the MLX layout) stacked in order or, `interleave`, of two of them alternating in 16-row tiles
+    (`interleave_gate_up`).  max_scale (float32 [1], zeroed) takes the largest |scale|; the caller sets
+    `small` from it."""
+    w = [as_packed_u32(lin.weight) for lin in linears]
+    s, b = [_f16(lin.scales, "scales") for lin in linears], [_f16(lin.biases, "biases") for lin in linears]
+    if _native().tile_parts(w, s, b, interleave, wt, sbt, max_scale) is None:
+        raise ValueError("tile_parts: matrices [N, K] on the GPU with N % 32 == 0 in all and K % 512 == 0, and room for the copy")
+    return TiledWeights(wt, sbt, sum(t.shape[0] for t in w), w[0].shape[1] * 8, False)
+
+
 def tile_weights(w_q, scales, biases):
     """Re-lay a weight matrix in the MLX layout (`w_q` [N, K/8] uint32, `scales`, `biases`
     [N, K/64] fp16) out as `TiledWeights` (one device launch; the inputs are left as they are)."""
@@ -395,16 +407,14 @@ def tile_weights(w_q, scales, biases):
     w_q = as_packed_u32(w_q)
     scales, biases = _f16(scales, "scales"), _f16(biases, "biases")
     N, K = w_q.shape[0], w_q.shape[1] * 8
-    L = _lib.lib()
-    nsb = L.eagle_qmm_tiled_sb_bytes(N, K)
-    if not nsb or tuple(scales.shape) != (N, K // 64) or tuple(biases.shape) != (N, K // 64):
+    if not _lib.lib().eagle_qmm_tiled_sb_bytes(N, K) or tuple(scales.shape) != (N, K // 64) or tuple(biases.shape) != (N, K // 64):
         raise ValueError(f"the tiled layout takes N % 32 == 0 and K % 512 == 0, got [{N}, {K}]")
     wt = torch.empty((N // 32, K // 64, 64, 4), dtype=torch.int32, device=w_q.device)
     sbt = torch.empty((N // 32, K // 512, 64, 8), dtype=torch.float16, device=w_q.device)
-    rc = L.eagle_qmm_tile_w4g64(_ptr(w_q), _ptr(scales), _ptr(biases), _ptr(wt), _ptr(sbt), N, K, 64, 4, _stream())
-    _lib.check(rc, "tile_weights")
-    small = bool(scales.abs().max().item() < TILED_SMALL_SCALE)
-    return TiledWeights(wt, sbt, N, K, small)
+    worst = torch.zeros(1, dtype=torch.float32, device=w_q.device)
+    if _native().tile_parts([w_q], [scales], [biases], False, wt, sbt, worst) is None:
+        raise ValueError("tile_weights: unexpected argument types")
+    return TiledWeights(wt, sbt, N, K, worst.item() < TILED_SMALL_SCALE)
 
 
 SMALL_SCALE_LIMIT = 0.2499       # |scale| * 2^18 has to stay a finite fp16 (the small-row kernels)

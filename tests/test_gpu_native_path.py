@@ -3,9 +3,10 @@ import numpy as np
 import pytest
 import torch
 
-from mlx_eagle_spec_decoding_tree_amd import eagle, ops
+from mlx_eagle_spec_decoding_tree_amd import eagle, llama, native, ops, synth
+from mlx_eagle_spec_decoding_tree_amd.cache import make_prompt_cache
 from oracle import tree_oracle as to
-from util import to_dev
+from util import MODEL_TOL, rel_err, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +40,101 @@ def test_tree_layout_from_lists(dev, depth, total, root_dtype):
     want = to.post_process_draft_tree(pos, total, midx)
     got = eagle.post_process_draft_tree(to_dev(pos, dev), total, to_dev(midx, dev))
     assert got.is_contiguous() and np.array_equal(got.cpu().numpy(), want)
+
+
+FORMS = {       # one launch per projection; fused products (K not a multiple of 512); tiled copies
+    "plain": dict(hidden=256, inter=512, heads=4, kv_heads=2, head_dim=64),
+    "fused": dict(hidden=896, inter=1152, heads=14, kv_heads=2, head_dim=64),
+    "tiled": dict(hidden=1024, inter=1536, heads=8, kv_heads=2, head_dim=128),
+}
+
+
+def small_model(dev, form, bias=True):
+    args = synth.tiny(layers=2, vocab=1000, attention_bias=bias, **FORMS[form])
+    return llama.Model.from_numpy(args, synth.make_model_weights(args, seed=3), dev)
+
+
+def filled_cache(model, P, cap, seed=1):
+    rng = np.random.default_rng(seed)
+    cache = make_prompt_cache(model, capacity=cap)
+    for c in cache:
+        for buf in (c.keys, c.values):
+            buf[0, :, :P] = to_dev(rng.standard_normal((buf.shape[1], P, buf.shape[3])).astype(np.float16), buf.device)
+        c.offset = P
+    return cache
+
+
+def by_operators(model, *a, **kw):
+    """The module path operator by operator."""
+    keep = model.__dict__.get("_native")
+    model.__dict__["_native"] = native._State(llama.Module.epoch, None)
+    try:
+        return model(*a, **kw)
+    finally:
+        model.__dict__["_native"] = keep
+
+
+def same_pass(model, ids, P, cap, **kw):
+    """One pass both ways; the native one must have run."""
+    a, b = filled_cache(model, P, cap), filled_cache(model, P, cap)
+    got = model._native_pass(ids, a, kw.get("mask"), kw.get("position_ids"), kw.get("flat_rope", False))
+    assert got is not None
+    want = by_operators(model, ids, b, **kw)
+    assert got.shape == want.shape and a[0].offset == b[0].offset == P + ids.shape[1]
+    assert rel_err(got.cpu().numpy(), want.cpu().numpy()) <= MODEL_TOL
+    for x, y in zip(a, b):
+        n = x.offset
+        assert rel_err(x.keys[0, :, :n].cpu().numpy(), y.keys[0, :, :n].cpu().numpy()) <= MODEL_TOL
+        assert rel_err(x.values[0, :, :n].cpu().numpy(), y.values[0, :, :n].cpu().numpy()) <= MODEL_TOL
+    return got
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("T", [1, 16, 17, 32, 33, 64])
+def test_native_tree_pass(dev, form, T):
+    model, P = small_model(dev, form), 45
+    rng = np.random.default_rng(T)
+    depth, vis, _ = synth.tree_arrays(synth.random_tree(rng, T))
+    ids = to_dev(rng.integers(0, 1000, (1, T)), dev)
+    print(f"{form} T={T}", flush=True)
+    mask = np.concatenate([np.zeros((T, P)), np.where(vis, 0.0, -np.inf)], axis=1).astype(np.float32)
+    pos = to_dev((depth + P).astype(np.int32), dev)
+    for dtype in (torch.float32, torch.bfloat16):
+        got = same_pass(model, ids, P, P + T, mask=to_dev(mask, dev)[None, None].to(dtype), position_ids=pos[None])
+    tree = to_dev(np.where(vis, 0.0, -np.inf).astype(np.float32), dev).to(torch.bfloat16)
+    cache = filled_cache(model, P, P + T)
+    again = eagle.tree_decoding(ids, tree, to_dev(depth.astype(np.int64), dev), model, cache)
+    assert rel_err(again.cpu().numpy(), got.cpu().numpy()) <= MODEL_TOL and cache[1].offset == P + T
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("T,P", [(1, 0), (32, 7), (64, 0), (65, 3), (96, 40), (130, 0)])
+def test_native_causal_pass(dev, form, T, P):
+    model = small_model(dev, form, bias=False)
+    print(f"{form} T={T} P={P}", flush=True)
+    ids = to_dev(np.random.default_rng(T).integers(0, 1000, (1, T)), dev)
+    same_pass(model, ids, P, P + (T + 31) // 32 * 32)
+    if T <= 32:
+        same_pass(model, ids, P, P + T, position_ids=5, flat_rope=True)
+
+
+def test_native_decoder_follows_the_weights(dev):
+    """Weights written to, exchanged layers and patched layers reach the next pass; arguments the native
+    path does not take (no room for the padding of a chunk) still run."""
+    model, ids = small_model(dev, "tiled"), torch.arange(6, device=dev)[None]
+    first = same_pass(model, ids, 3, 16)
+    model.layers[1].mlp.down_proj.scales.mul_(0.5)
+    second = same_pass(model, ids, 3, 16)
+    assert not torch.equal(first, second)
+    q = model.layers[0].self_attn.q_proj
+    model.layers[0].self_attn.q_proj = llama.QuantizedLinear(q.weight, q.scales * 0.5, q.biases * 0.5, q.bias)
+    third = same_pass(model, ids, 3, 16)
+    assert not torch.equal(second, third)
+    model.layers[0], model.layers[1] = model.layers[1], model.layers[0]
+    assert not torch.equal(third, same_pass(model, ids, 3, 16))
+    cache = filled_cache(model, 3, 100)
+    long = torch.arange(97, device=dev)[None]
+    assert model._native_pass(long, cache, None, None, False) is None and cache[0].offset == 3
+    assert model(long, cache).shape == (1, 97, 1000) and cache[0].offset == 100
+    llama.patch_model(model, lambda *a: ops.matmul(*a)[0])
+    assert native.decoder(model) is None
