@@ -196,6 +196,16 @@ int eagle_qmm_gemm_swiglu_w4g64_f16(const void* x, const uint32_t* wq, const voi
                                     const void* biases, const void* bias, void* out, int M, int N,
                                     int K, int group_size, int bits, eagle_stream_t stream);
 
+/* Either of the two with a workspace for products whose grid would leave most of the GPU idle (few rows, few
+ * weight rows, a long K): several workgroups then share an output block, each over a part of K, and a second
+ * launch adds their fp32 sums in order.  The library decides; workspace bytes 0: no split.  Same
+ * roundings; workspace 16-byte aligned. */
+size_t eagle_qmm_gemm_workspace_bytes(int M, int N, int K, int swiglu);
+int eagle_qmm_gemm_split_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
+                                   const void* biases, const void* bias, void* out, int M, int N,
+                                   int K, int group_size, int bits, int swiglu, void* workspace,
+                                   size_t workspace_bytes, eagle_stream_t stream);
+
 /* The same product for 1..64 rows in the slab form, with the result left as fp32 partial sums:
  * every workgroup owns 128 weight rows and one K slab of `steps_per_slab` quantisation groups
  * (a multiple of 8), moves x through LDS eight groups at a time and expands the weights to fp16

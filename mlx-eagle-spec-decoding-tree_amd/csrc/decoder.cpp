@@ -182,7 +182,7 @@ struct Pass {
   int swiglu(const Mat& m, const void* x, void* out) {
     if (eagle_qmm_slab_swiglu_preferred(R, m.N, m.K))
       return eagle_qmm_slab_swiglu_w4g64_f16(x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, 64, 4, st);
-    if (R > 2 * EAGLE_MAX_M) return eagle_qmm_gemm_swiglu_w4g64_f16(x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, 64, 4, st);
+    if (R > 2 * EAGLE_MAX_M) return gemm(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);
     for (int r0 = 0; r0 < R; r0 += EAGLE_MAX_M) {
       const int rows = std::min(R - r0, EAGLE_MAX_M);
       Slot ws;

@@ -132,11 +132,13 @@ struct StepIndex {
 // SWI: the weight rows are gate and up rows interleaved in 16-row tiles (rows 0..15 of a 32-row
 // matrix tile gate, 16..31 the matching up rows: the same accumulator lane holds both); the
 // result is silu(g) * u, [M, N / 2].
-template <int NTW, int MT, int SBW, int KGRP = 1, bool SWI = false>
+// SPLITK: gridDim.z workgroups share an output block, each over its own part of K, and leave fp32 partial
+// sums in `partial` [z][M][N] for gemm_sum_kernel.
+template <int NTW, int MT, int SBW, int KGRP = 1, bool SWI = false, bool SPLITK = false>
 __global__ __launch_bounds__(256 * KGRP, (KGRP == 1 ? 2 : 1)) void qmm_gemm_w4g64_kernel(
     const half_t* __restrict__ x, const uint32_t* __restrict__ w, const half_t* __restrict__ s,
     const half_t* __restrict__ b, const half_t* __restrict__ bias, half_t* __restrict__ out, int M,
-    int N, int K) {
+    int N, int K, float* __restrict__ partial) {
   // NTW = 32-row weight tiles per wave (1 or 2); the four waves sit side by side along the
   // weight rows, each over all x rows of the block: no weight row is loaded or expanded twice,
   // and with NTW = 2 every x operand read from LDS serves two matrix instructions
@@ -157,8 +159,15 @@ __global__ __launch_bounds__(256 * KGRP, (KGRP == 1 ? 2 : 1)) void qmm_gemm_w4g6
   const int m0 = blockIdx.y * BMT;
   const int KW = K >> 3;                    // packed words per weight row
   const int KG = K >> 6;                    // groups per weight row
-  const int steps = K / BK / KGRP;          // of this group
-  const int kbase = grp * steps * BK;       // its first column
+  int steps = K / BK / KGRP;                // of this group
+  int kbase = grp * steps * BK;             // its first column
+  if (SPLITK) {
+    // chunks of SBW steps dealt over the splits as evenly as they go
+    const int all = K / BK / SBW, z = blockIdx.z, nz = gridDim.z;
+    const int lo = (int)((long)all * z / nz), hi = (int)((long)all * (z + 1) / nz);
+    steps = (hi - lo) * SBW;
+    kbase = lo * SBW * BK;
+  }
   x += kbase;
   w += kbase >> 3;
   s += kbase >> 6;
@@ -364,7 +373,32 @@ __global__ __launch_bounds__(256 * KGRP, (KGRP == 1 ? 2 : 1)) void qmm_gemm_w4g6
     __syncthreads();                                     // the sums are in registers: LDS is free again
     if (grp != 0) return;
   }
-  if (SWI) {
+  if (SPLITK) {
+    // 32 rows of x at a time through the wave's region of LDS, out as whole row segments
+    constexpr int ROWF = 32 * NTW + 4;                   // floats per staged row (padded)
+    float* stage = reinterpret_cast<float*>(xs_all) + wave * (32 * ROWF);
+    float* dst = partial + (size_t)blockIdx.z * M * N;
+    constexpr int LPR = 8 * NTW;                         // lanes per row (16 bytes each)
+    constexpr int RPI = 64 / LPR;
+    const int pr = lane / LPR, pc = (lane % LPR) * 4;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+          *reinterpret_cast<float4_t*>(stage + ql * ROWF + nt * 32 + 8 * i4 + 4 * hb) =
+              float4_t{acc[nt][mt][4 * i4], acc[nt][mt][4 * i4 + 1], acc[nt][mt][4 * i4 + 2], acc[nt][mt][4 * i4 + 3]};
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int r0 = 0; r0 < 32; r0 += RPI) {
+        const int m = m0 + mt * 32 + r0 + pr, n = n0 + pc;
+        const float4_t v = *reinterpret_cast<const float4_t*>(stage + (r0 + pr) * ROWF + pc);
+        if (m < M && n < N) *reinterpret_cast<float4_t*>(dst + (size_t)m * N + n) = v;
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  } else if (SWI) {
     // 16 output columns per 32-row tile: accumulator registers 0..7 are gate rows 8 (i / 4) + 4 hb +
     // i % 4, registers 8..15 the up rows 16 further on
     constexpr int ROWB = 32 * NTW + 16;
@@ -433,9 +467,46 @@ __global__ __launch_bounds__(256 * KGRP, (KGRP == 1 ? 2 : 1)) void qmm_gemm_w4g6
   }
 }
 
-template <int NTW, int MT, int SBW, int KGRP = 1, bool SWI = false>
+// The partial sums of a split GEMM added in split order: fp16 (+ bias), or silu(g) * u of interleaved gate|up rows
+// (SWI).  Eight consecutive outputs per thread, every load in flight before the first add.
+template <bool SWI>
+__global__ __launch_bounds__(256) void gemm_sum_kernel(const float* __restrict__ partial, int splits,
+                                                       const half_t* __restrict__ bias, half_t* __restrict__ out, int M,
+                                                       int N) {
+  const int per_row = (SWI ? N >> 1 : N) >> 3;
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (long)M * per_row) return;
+  const int m = (int)(idx / per_row), o8 = (int)(idx % per_row) * 8;
+  // SWI: output columns o .. o + 7 are gate rows 32 (o / 16) + o % 16 .. and the up rows 16 further on
+  const int n = SWI ? (o8 >> 4) * 32 + (o8 & 15) : o8;
+  const size_t stride = (size_t)M * N;
+  const half8_t g = eagle_slab_sum8(partial, splits, stride, (size_t)m * N + n, nullptr);
+  half8_t r = g;
+  if (SWI) {
+    const half8_t u = eagle_slab_sum8(partial, splits, stride, (size_t)m * N + n + 16, nullptr);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      half_t ge = g[e], ue = u[e];
+      if (bias) {
+        ge = ge + bias[n + e];
+        ue = ue + bias[n + 16 + e];
+      }
+      const float gf = (float)ge;
+      const half_t a = (half_t)(gf / (1.0f + expf(-gf)));
+      r[e] = (half_t)((float)a * (float)ue);
+    }
+    *reinterpret_cast<half8_t*>(out + (size_t)m * (N >> 1) + o8) = r;
+  } else {
+    if (bias)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) r[e] = r[e] + bias[n + e];
+    *reinterpret_cast<half8_t*>(out + (size_t)m * N + o8) = r;
+  }
+}
+
+template <int NTW, int MT, int SBW, int KGRP = 1, bool SWI = false, bool SPLITK = false>
 int launch_gemm(const half_t* x, const uint32_t* w, const half_t* s, const half_t* b, const half_t* bias,
-                half_t* out, int M, int N, int K, hipStream_t st) {
+                half_t* out, int M, int N, int K, hipStream_t st, int splits = 1, float* partial = nullptr) {
   constexpr int BMT = 32 * MT;
   constexpr int BN = 128 * NTW;
   static_assert(256 % BMT == 0 && BMT >= 32, "block load mapping");
@@ -444,16 +515,18 @@ int launch_gemm(const half_t* x, const uint32_t* w, const half_t* s, const half_
   const size_t lds_red = KGRP > 1 ? 4 * (size_t)NTW * MT * 4 * 64 * sizeof(float4_t) : 0;
   size_t lds = lds_x > lds_out ? lds_x : lds_out;
   lds = lds > lds_red ? lds : lds_red;
+  const size_t lds_part = SPLITK ? 4 * 32 * (size_t)(32 * NTW + 4) * sizeof(float) : 0;
+  lds = lds > lds_part ? lds : lds_part;
   static bool configured = false;
   if (!configured) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&qmm_gemm_w4g64_kernel<NTW, MT, SBW, KGRP, SWI>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&qmm_gemm_w4g64_kernel<NTW, MT, SBW, KGRP, SWI, SPLITK>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return EAGLE_ERR_HIP;
     configured = true;
   }
-  const dim3 grid((N + BN - 1) / BN, (M + BMT - 1) / BMT);
-  hipLaunchKernelGGL((qmm_gemm_w4g64_kernel<NTW, MT, SBW, KGRP, SWI>), grid, dim3(256 * KGRP), lds, st, x, w, s, b,
-                     bias, out, M, N, K);
+  const dim3 grid((N + BN - 1) / BN, (M + BMT - 1) / BMT, splits);
+  hipLaunchKernelGGL((qmm_gemm_w4g64_kernel<NTW, MT, SBW, KGRP, SWI, SPLITK>), grid, dim3(256 * KGRP), lds, st, x, w, s, b,
+                     bias, out, M, N, K, partial);
   return eagle_launch_status();
 }
 
@@ -1649,9 +1722,96 @@ EAGLE_EXPORT int eagle_qmm_rows_tiled_w4g64_f16(const void* x, const uint32_t* w
                       : launch_rows_tiled<10, false>(xh, wt, sb, bh, oh, M, N, K, st);
 }
 
+// Block shape and K splits of the many-row product.
+//
+// Block: 64 x 128, 128 x 128 or 128 x 256 (x rows x weight rows).  The compute unit with the
+// most workgroups sets the time, and a workgroup's work goes with its block (bigger
+// blocks do a little less per output: 0.55 / 1 / 1.85); the estimate below reproduced the
+// faster choice for every projection shape of the 7B / 8B / 0.5B models at 512 and 2048 rows.
+//
+// Splits: a grid of a few dozen workgroups walks a long K one step after the other (0.4 - 1.1 us a step
+// whatever the grid), so several workgroups share an output block, each over a part of K, and a second
+// launch adds their fp32 sums.  `gemm_cost` is fitted to 900 forced launches (65 .. 2048 rows, K 896 .. 18944,
+// N 896 .. 37888): us per K step of a workgroup alone on its compute unit and of two that share one, 3.5 us
+// and the traffic of the partial sums for the second launch.  A split is taken where it is estimated at least
+// a tenth faster.  Measured, us without and with: 65 x 3584 x 18944 104 / 32, 128 x 896 x 4864 27 / 13,
+// 512 x 2896 x 9344 71 / 52, 128 x 3584 x 3584 20 / 16; 512 x 14336 x 4096 stays whole (66).
+struct GemmPlan {
+  int block;      // 0: 64 x 128, 1: 128 x 128, 2: 128 x 256
+  int kgrp;       // K groups inside a workgroup
+  int splits;     // workgroups along K
+  int sbw;        // scale groups per fetch
+};
+
+static double gemm_cost(int block, long wgs, double steps) {
+  static const double alone[3] = {0.40, 0.64, 1.08}, pair[3] = {0.68, 1.14, 2.05};
+  const double c = (double)wgs / NUM_CU;
+  if (c <= 1.) return 4. + steps * alone[block];
+  const long full = (long)c / 2;                       // whole pairs on the busiest compute unit
+  const double rest = c - 2. * full;
+  return 4. + steps * (pair[block] * full + (rest > 1. ? pair[block] : rest > 0. ? alone[block] : 0.));
+}
+
+static GemmPlan gemm_plan(int M, int N, int K, const void* scales, const void* biases, bool swiglu, bool may_split) {
+  auto most = [](long blocks) { return (double)((blocks + NUM_CU - 1) / NUM_CU); };
+  const long nb = (N + 127) / 128, wgs_of[3] = {nb * ((M + 63) / 64), nb * ((M + 127) / 128),
+                                                ((N + 255) / 256) * (long)((M + 127) / 128)};
+  const double cost_norm = most(wgs_of[1]);
+  const double cost_small = M > 64 && !swiglu ? 0.55 * most(wgs_of[0]) : 1e30;
+  const double cost_big = 1.85 * most(wgs_of[2]);
+  GemmPlan p;
+  p.block = cost_small < cost_norm && cost_small <= cost_big ? 0 : cost_big < cost_norm ? 2 : 1;
+  // scales and biases per fetch: as many groups as divide a row and as the base addresses are
+  // aligned for
+  const uintptr_t sb_addr = reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases);
+  p.sbw = (K % 512) == 0 && (sb_addr & 15u) == 0 ? 8
+          : (K % 256) == 0 && (sb_addr & 7u) == 0 ? 4
+          : (K % 128) == 0 && (sb_addr & 3u) == 0 ? 2
+                                                  : 1;
+  // (the SwiGLU epilogue of the 128 x 256 block is built for eight groups only)
+  if (swiglu && p.block == 2 && p.sbw != 8) p.block = 1;
+  // two K groups per workgroup where the grid would leave a compute unit with one workgroup
+  p.kgrp = !swiglu && p.sbw == 8 && (K % 1024) == 0 && p.block != 2 && wgs_of[p.block] <= GEMM_SPLIT_WGS ? 2 : 1;
+  p.splits = 1;
+  if (!may_split) return p;
+  const double steps = K / 64;
+  double best = p.kgrp == 2 ? 4. + steps / 2 * (p.block == 0 ? 0.70 : 1.15) * (wgs_of[p.block] > NUM_CU ? 2 : 1)
+                            : gemm_cost(p.block, wgs_of[p.block], steps);
+  best *= 0.9;
+  static const int tried[] = {2, 3, 4, 6, 8, 12, 16, 24};
+  for (int b = 0; b < 3; ++b)
+    for (int z : tried) {
+      const int unit = b == 2 && p.sbw == 8 ? 4 : p.sbw;     // steps are dealt in fetches of scales
+      const int units = K / 64 / unit;
+      if (z > units || wgs_of[b] * z > 6 * NUM_CU) continue;
+      const double c = gemm_cost(b, wgs_of[b] * z, (double)((units + z - 1) / z * unit)) + 3.5 +
+                       8e-6 / 4.5 * z * (double)M * N;
+      if (c < best) {
+        best = c;
+        p.block = b;
+        p.splits = z;
+        p.kgrp = 1;
+      }
+    }
+  return p;
+}
+
+EAGLE_EXPORT size_t eagle_qmm_gemm_workspace_bytes(int M, int N, int K, int swiglu) {
+  if (M < 1 || N < 8 || K < 64 || (K % 64) != 0) return 0;
+  // (the fetch width, which depends on the addresses, only moves the split: the largest of the two)
+  size_t need = 0;
+  for (uintptr_t addr = 0; addr <= 2; addr += 2) {
+    const void* a = reinterpret_cast<const void*>(addr);
+    const GemmPlan p = gemm_plan(M, N, K, a, a, swiglu != 0, true);
+    const size_t bytes = p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
+    need = bytes > need ? bytes : need;
+  }
+  return need;
+}
+
 static int gemm_dispatch(const void* x, const uint32_t* wq, const void* scales, const void* biases,
                          const void* bias, void* out, int M, int N, int K, int group_size, int bits,
-                         bool swiglu, eagle_stream_t stream) {
+                         bool swiglu, void* workspace, size_t workspace_bytes, eagle_stream_t stream) {
   if (!x || !wq || !scales || !biases || !out) return EAGLE_ERR_NULL;
   if (group_size != 64 || bits != 4) return EAGLE_ERR_UNSUPPORTED;
   if (M < 1 || N < 8 || (N % 8) != 0 || K < 64 || (K % 64) != 0) return EAGLE_ERR_SHAPE;
@@ -1660,72 +1820,84 @@ static int gemm_dispatch(const void* x, const uint32_t* wq, const void* scales, 
   if (!eagle_aligned16(x) || !eagle_aligned16(wq) || !eagle_aligned16(out) ||
       (bias && (reinterpret_cast<uintptr_t>(bias) & 7u)))
     return EAGLE_ERR_ALIGN;
+  if (workspace && !eagle_aligned16(workspace)) return EAGLE_ERR_ALIGN;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const half_t* xh = static_cast<const half_t*>(x);
   const half_t* sh = static_cast<const half_t*>(scales);
   const half_t* bh = static_cast<const half_t*>(biases);
   const half_t* bi = static_cast<const half_t*>(bias);
   half_t* oh = static_cast<half_t*>(out);
-  // Block shape: 64 x 128, 128 x 128 or 128 x 256 (x rows x weight rows).  The compute unit with
-  // the most workgroups sets the time, and a workgroup's work goes with its block (bigger
-  // blocks do a little less per output: 0.55 / 1 / 1.85); the estimate below reproduced the
-  // faster choice for every projection shape of the 7B / 8B / 0.5B models at 512 and 2048 rows.
-  auto most = [](long blocks) { return (double)((blocks + NUM_CU - 1) / NUM_CU); };
-  const long nb = (N + 127) / 128;
-  const double cost_norm = most(nb * ((M + 127) / 128));
-  const double cost_small = M > 64 ? 0.55 * most(nb * ((M + 63) / 64)) : 1e30;
-  const double cost_big = 1.85 * most(((N + 255) / 256) * (long)((M + 127) / 128));
-  const bool small = cost_small < cost_norm && cost_small <= cost_big;
-  const bool big = !small && cost_big < cost_norm;
-  // scales and biases per fetch: as many groups as divide a row and as the base addresses are
-  // aligned for
-  const uintptr_t sb_addr = reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases);
-  const int sbw = (K % 512) == 0 && (sb_addr & 15u) == 0 ? 8
-                : (K % 256) == 0 && (sb_addr & 7u) == 0  ? 4
-                : (K % 128) == 0 && (sb_addr & 3u) == 0  ? 2
-                                                         : 1;
-#define EAGLE_GEMM_SHAPE(NTW, MT)                                                              \
-  switch (sbw) {                                                                               \
-    case 8: return launch_gemm<NTW, MT, 8>(xh, wq, sh, bh, bi, oh, M, N, K, st);               \
-    case 4: return launch_gemm<NTW, MT, 4>(xh, wq, sh, bh, bi, oh, M, N, K, st);               \
-    case 2: return launch_gemm<NTW, MT, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st);               \
-    default: return launch_gemm<NTW, MT, 1>(xh, wq, sh, bh, bi, oh, M, N, K, st);              \
+  GemmPlan p = gemm_plan(M, N, K, scales, biases, swiglu, workspace != nullptr);
+  if (p.splits > 1 && workspace_bytes < (size_t)p.splits * M * N * sizeof(float)) return EAGLE_ERR_WORKSPACE;
+  if (p.splits > 1) {
+    float* part = static_cast<float*>(workspace);
+    int rc = EAGLE_ERR_UNSUPPORTED;
+#define EAGLE_GEMM_SPLIT(NTW, MT)                                                                                       \
+  switch (p.sbw) {                                                                                                      \
+    case 8: rc = launch_gemm<NTW, MT, (NTW == 2 ? 4 : 8), 1, false, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break; \
+    case 4: rc = launch_gemm<NTW, MT, 4, 1, false, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break;   \
+    case 2: rc = launch_gemm<NTW, MT, 2, 1, false, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break;   \
+    default: rc = launch_gemm<NTW, MT, 1, 1, false, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break;  \
   }
-  // two K groups per workgroup where the grid would leave a compute unit with one workgroup
-  const long wgs = small ? nb * ((M + 63) / 64) : big ? ((N + 255) / 256) * (long)((M + 127) / 128) : nb * ((M + 127) / 128);
+    if (p.block == 0) { EAGLE_GEMM_SPLIT(1, 2) } else if (p.block == 1) { EAGLE_GEMM_SPLIT(1, 4) } else { EAGLE_GEMM_SPLIT(2, 4) }
+#undef EAGLE_GEMM_SPLIT
+    if (rc != EAGLE_OK) return rc;
+    const long total = (long)M * ((swiglu ? N / 2 : N) / 8);
+    const dim3 grid((unsigned)((total + 255) / 256));
+    if (swiglu)
+      hipLaunchKernelGGL(gemm_sum_kernel<true>, grid, dim3(256), 0, st, part, p.splits, bi, oh, M, N);
+    else
+      hipLaunchKernelGGL(gemm_sum_kernel<false>, grid, dim3(256), 0, st, part, p.splits, bi, oh, M, N);
+    return eagle_launch_status();
+  }
   if (swiglu) {
     // the wide gate|up matrix: the 128 x 256 block where it pays, else 128 x 128
-    switch (sbw) {
-      case 8: return big ? launch_gemm<2, 4, 4, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st)
-                         : launch_gemm<1, 4, 8, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st);
+    switch (p.sbw) {
+      case 8: return p.block == 2 ? launch_gemm<2, 4, 4, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st)
+                                  : launch_gemm<1, 4, 8, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st);
       case 4: return launch_gemm<1, 4, 4, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st);
       case 2: return launch_gemm<1, 4, 2, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st);
       default: return launch_gemm<1, 4, 1, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st);
     }
   }
-  const bool split_k = sbw == 8 && (K % 1024) == 0 && wgs <= GEMM_SPLIT_WGS;
-  if (split_k) {
-    if (small) return launch_gemm<1, 2, 8, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st);
-    if (!big) return launch_gemm<1, 4, 8, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st);
+#define EAGLE_GEMM_SHAPE(NTW, MT)                                                              \
+  switch (p.sbw) {                                                                             \
+    case 8: return launch_gemm<NTW, MT, 8>(xh, wq, sh, bh, bi, oh, M, N, K, st);               \
+    case 4: return launch_gemm<NTW, MT, 4>(xh, wq, sh, bh, bi, oh, M, N, K, st);               \
+    case 2: return launch_gemm<NTW, MT, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st);               \
+    default: return launch_gemm<NTW, MT, 1>(xh, wq, sh, bh, bi, oh, M, N, K, st);              \
   }
-  if (small) { EAGLE_GEMM_SHAPE(1, 2) }
+  if (p.kgrp == 2)
+    return p.block == 0 ? launch_gemm<1, 2, 8, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st)
+                        : launch_gemm<1, 4, 8, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st);
+  if (p.block == 0) { EAGLE_GEMM_SHAPE(1, 2) }
+  if (p.block == 1) { EAGLE_GEMM_SHAPE(1, 4) }
   // (the 128 x 256 block takes its scales four groups per fetch at most: with eight it spills
   // twenty registers and is no faster, 149-153 us against 143-152 us for 512 x 28672 x 4096)
-  if (big && sbw == 8) return launch_gemm<2, 4, 4>(xh, wq, sh, bh, bi, oh, M, N, K, st);
-  if (big) { EAGLE_GEMM_SHAPE(2, 4) }
-  EAGLE_GEMM_SHAPE(1, 4)
+  if (p.sbw >= 4) return launch_gemm<2, 4, 4>(xh, wq, sh, bh, bi, oh, M, N, K, st);
+  return p.sbw == 2 ? launch_gemm<2, 4, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st)
+                    : launch_gemm<2, 4, 1>(xh, wq, sh, bh, bi, oh, M, N, K, st);
 #undef EAGLE_GEMM_SHAPE
 }
 
 EAGLE_EXPORT int eagle_qmm_gemm_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
                                           const void* biases, const void* bias, void* out, int M, int N,
                                           int K, int group_size, int bits, eagle_stream_t stream) {
-  return gemm_dispatch(x, wq, scales, biases, bias, out, M, N, K, group_size, bits, false, stream);
+  return gemm_dispatch(x, wq, scales, biases, bias, out, M, N, K, group_size, bits, false, nullptr, 0, stream);
 }
 
 EAGLE_EXPORT int eagle_qmm_gemm_swiglu_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
                                                  const void* biases, const void* bias, void* out, int M,
                                                  int N, int K, int group_size, int bits,
                                                  eagle_stream_t stream) {
-  return gemm_dispatch(x, wq, scales, biases, bias, out, M, N, K, group_size, bits, true, stream);
+  return gemm_dispatch(x, wq, scales, biases, bias, out, M, N, K, group_size, bits, true, nullptr, 0, stream);
+}
+
+EAGLE_EXPORT int eagle_qmm_gemm_split_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
+                                                const void* biases, const void* bias, void* out, int M,
+                                                int N, int K, int group_size, int bits, int swiglu,
+                                                void* workspace, size_t workspace_bytes,
+                                                eagle_stream_t stream) {
+  return gemm_dispatch(x, wq, scales, biases, bias, out, M, N, K, group_size, bits, swiglu != 0, workspace,
+                       workspace_bytes, stream);
 }

@@ -50,10 +50,20 @@ bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out) {
   return true;
 }
 
+int gemm(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out, int M,
+         int N, int K, bool swiglu, void* st) {
+  // the partial sums go back to torch's allocator with the launches in the stream
+  const size_t need = eagle_qmm_gemm_workspace_bytes(M, N, K, swiglu);
+  at::Tensor ws;
+  if (need) ws = empty({(int64_t)need}, at::kByte, like);
+  return eagle_qmm_gemm_split_w4g64_f16(x, static_cast<const uint32_t*>(w), s, b, bias, out, M, N, K, 64, 4, swiglu,
+                                        need ? ws.data_ptr() : nullptr, need, st);
+}
+
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
            int M, int N, int K, void* st) {
   const uint32_t* wq = static_cast<const uint32_t*>(w);
-  if (M > 2 * EAGLE_MAX_M) return eagle_qmm_gemm_w4g64_f16(x, wq, s, b, bias, out, M, N, K, 64, 4, st);
+  if (M > 2 * EAGLE_MAX_M) return gemm(like, x, w, s, b, bias, out, M, N, K, false, st);
   for (int r0 = 0; r0 < M; r0 += EAGLE_MAX_M) {
     const int m = M - r0 < EAGLE_MAX_M ? M - r0 : EAGLE_MAX_M;
     const void* xr = static_cast<const char*>(x) + (size_t)r0 * K * 2;

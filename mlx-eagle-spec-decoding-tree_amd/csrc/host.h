@@ -45,6 +45,10 @@ bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out);
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
            int M, int N, int K, void* st);
 
+// The many-row product, split over K where the library says so (SwiGLU: interleaved gate|up rows)
+int gemm(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out, int M,
+         int N, int K, bool swiglu, void* st);
+
 PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* py_decoder_current(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n);

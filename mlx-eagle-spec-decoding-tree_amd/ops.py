@@ -354,9 +354,12 @@ def quantized_matmul_swiglu(x, w_q, scales, biases, bias=None, out=None, gemm=No
                                     out=out2[r0:r0 + ROW_PASS])
         return out
     if M > 32 or gemm:
-        # many rows (a prompt chunk): the tiled GEMM with the same epilogue
-        rc = L.eagle_qmm_gemm_swiglu_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias),
-                                               _ptr(out), M, N, K, 64, 4, _stream())
+        # many rows (a prompt chunk): the tiled GEMM with the same epilogue, split over K where that fills
+        # the GPU better
+        need = L.eagle_qmm_gemm_workspace_bytes(M, N, K, 1) if not gemm else 0
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+        rc = L.eagle_qmm_gemm_split_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias),
+                                              _ptr(out), M, N, K, 64, 4, 1, _ptr(ws), need, _stream())
         _lib.check(rc, "quantized_matmul_swiglu")
         return out
     ws = workspace("qmm", L.eagle_qmm_workspace_bytes(M, N, K), x.device)
