@@ -59,6 +59,46 @@ __global__ __launch_bounds__(QMV_WAVES * 64) void qmv_w4g64_kernel(
   const int tid = threadIdx.x;
   const int nthr = QMV_WAVES * 64;
   const int KC = K / 32;
+  const int wave = tid >> 6, lane = tid & 63;
+  const int l16 = lane & 15, rg = lane >> 4;
+  const int steps = K >> 9;                    // 512 columns per step
+  const int G = K >> 6, KW = K >> 3;
+  const long stride = (long)gridDim.x * (QMV_WAVES * 4);
+  const long first = (long)blockIdx.x * (QMV_WAVES * 4) + wave * 4 + rg;   // this lane's row in round 0
+  const int rounds = (int)(((long)N - (long)blockIdx.x * (QMV_WAVES * 4) + stride - 1) / stride);
+
+  // The steps of all rounds of rows are one sequence; the next QMV_RING of them are in flight, the first ones
+  // requested before x is staged (the two barriers of the staging cost a microsecond, which the weights now
+  // travel through: 6.4 -> 5.5 us for 3584 x 3584, 20.9 -> 19.3 for 4096 x 32768).
+  uint4_t ring[QMV_RING];
+  half_t sr[QMV_RING], br[QMV_RING];
+  int l_round = 0, l_st = 0;                   // the next step to request
+  const uint32_t* wp;
+  const half_t *sp, *bp;
+  auto locate = [&]() {
+    long n = first + l_round * stride;
+    if (n > N - 1) n = N - 1;                  // rows past the end are never stored
+    wp = w + n * KW + l16 * 4;
+    sp = s + n * G + (l16 >> 1);
+    bp = b + n * G + (l16 >> 1);
+  };
+  locate();
+  auto request = [&](int r) {
+    ring[r] = *reinterpret_cast<const uint4_t*>(wp + l_st * 64);
+    sr[r] = sp[l_st * 8];
+    br[r] = bp[l_st * 8];
+    if (l_st + 1 < steps) {
+      ++l_st;
+    } else if (l_round + 1 < rounds) {         // (the last step of all is requested again)
+      ++l_round;
+      l_st = 0;
+      locate();
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < QMV_RING; ++r) request(r);
+  __builtin_amdgcn_sched_barrier(0);
+
   // stage x: thread t handles words of 8 columns (rows past M repeat the last one; never stored)
   for (int c = tid; c < MR * (K / 8); c += nthr) {
     const int m = c / (K / 8), cc = c % (K / 8);
@@ -81,76 +121,58 @@ __global__ __launch_bounds__(QMV_WAVES * 64) void qmv_w4g64_kernel(
   }
   __syncthreads();
 
-  const int wave = tid >> 6, lane = tid & 63;
-  const int l16 = lane & 15, rg = lane >> 4;
-  const int steps = K >> 9;                    // 512 columns per step
-  const int G = K >> 6, KW = K >> 3;
-  const int rows_per_wg = QMV_WAVES * 4;
   const uint32_t magic_lo = 0x64006400u, magic_hi = 0x54005400u;
-  for (long base = (long)blockIdx.x * rows_per_wg; base < N; base += (long)gridDim.x * rows_per_wg) {
-    long n = base + wave * 4 + rg;
-    const bool live = n < N;
-    if (!live) n = N - 1;
-    const uint32_t* wp = w + n * KW + l16 * 4;
-    const half_t* sp = s + n * G + (l16 >> 1);
-    const half_t* bp = b + n * G + (l16 >> 1);
-    uint4_t ring[QMV_RING];
-    half_t sr[QMV_RING], br[QMV_RING];
+  const int total = rounds * steps;
+  int round = 0, st = 0;
+  float acc[MR];
+#pragma unroll
+  for (int m = 0; m < MR; ++m) acc[m] = 0.f;
+  for (int it0 = 0; it0 < total; it0 += QMV_RING) {
 #pragma unroll
     for (int r = 0; r < QMV_RING; ++r) {
-      const int st = r < steps ? r : steps - 1;
-      ring[r] = *reinterpret_cast<const uint4_t*>(wp + st * 64);
-      sr[r] = sp[st * 8];
-      br[r] = bp[st * 8];
-    }
-    float acc[MR];
+      if (it0 + r >= total) break;
+      const uint4_t wv = ring[r];
+      const float sc = (float)sr[r], bi = (float)br[r];
+      request(r);
+      const int col = st * 512 + l16 * 32;
+      float d[MR];
 #pragma unroll
-    for (int m = 0; m < MR; ++m) acc[m] = 0.f;
-    for (int st0 = 0; st0 < steps; st0 += QMV_RING) {
+      for (int m = 0; m < MR; ++m) d[m] = 0.f;
 #pragma unroll
-      for (int r = 0; r < QMV_RING; ++r) {
-        const int st = st0 + r;
-        if (st >= steps) break;
-        const uint4_t wv = ring[r];
-        const float sc = (float)sr[r], bi = (float)br[r];
-        const int nx = st + QMV_RING < steps ? st + QMV_RING : steps - 1;
-        ring[r] = *reinterpret_cast<const uint4_t*>(wp + nx * 64);
-        sr[r] = sp[nx * 8];
-        br[r] = bp[nx * 8];
-        const int col = st * 512 + l16 * 32;
-        float d[MR];
-#pragma unroll
-        for (int m = 0; m < MR; ++m) d[m] = 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t v = wv[j], v2 = v >> 8;
-          // (1024 + q0, 1024 + q4), (64 + q1 .. as 16 q1 in the low mantissa bits of 64: the
-          // nibble sits four bits up, so the value is 64 + q), (1024 + q2, 1024 + q6), (64 + q3, 64 + q7)
-          const uint32_t e0 = qmv_and_or(v, 0x000f000fu, magic_lo), e1 = qmv_and_or(v, 0x00f000f0u, magic_hi);
-          const uint32_t e2 = qmv_and_or(v2, 0x000f000fu, magic_lo), e3 = qmv_and_or(v2, 0x00f000f0u, magic_hi);
-#pragma unroll
-          for (int m = 0; m < MR; ++m) {
-            const half8_t xv = *reinterpret_cast<const half8_t*>(xl + (long)m * K + col + j * 8);
-            d[m] = dot2(e0, half2_t{xv[0], xv[1]}, d[m]);
-            d[m] = dot2(e1, half2_t{xv[2], xv[3]}, d[m]);
-            d[m] = dot2(e2, half2_t{xv[4], xv[5]}, d[m]);
-            d[m] = dot2(e3, half2_t{xv[6], xv[7]}, d[m]);
-          }
-        }
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t v = wv[j], v2 = v >> 8;
+        // (1024 + q0, 1024 + q4), (64 + q1 .. as 16 q1 in the low mantissa bits of 64: the
+        // nibble sits four bits up, so the value is 64 + q), (1024 + q2, 1024 + q6), (64 + q3, 64 + q7)
+        const uint32_t e0 = qmv_and_or(v, 0x000f000fu, magic_lo), e1 = qmv_and_or(v, 0x00f000f0u, magic_hi);
+        const uint32_t e2 = qmv_and_or(v2, 0x000f000fu, magic_lo), e3 = qmv_and_or(v2, 0x00f000f0u, magic_hi);
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
-          const float* cp = corr + ((long)m * KC + (col >> 5)) * 3;
-          acc[m] += sc * (d[m] - 1024.f * cp[1] - 64.f * cp[2]) + bi * cp[0];
+          const half8_t xv = *reinterpret_cast<const half8_t*>(xl + (long)m * K + col + j * 8);
+          d[m] = dot2(e0, half2_t{xv[0], xv[1]}, d[m]);
+          d[m] = dot2(e1, half2_t{xv[2], xv[3]}, d[m]);
+          d[m] = dot2(e2, half2_t{xv[4], xv[5]}, d[m]);
+          d[m] = dot2(e3, half2_t{xv[6], xv[7]}, d[m]);
         }
       }
-    }
 #pragma unroll
-    for (int m = 0; m < MR; ++m) {
-      const float a = row_sum16(acc[m]);
-      if (live && l16 == 0 && m < M) {
-        half_t o = (half_t)a;
-        if (bias) o = o + bias[n];
-        out[(long)m * N + n] = o;
+      for (int m = 0; m < MR; ++m) {
+        const float* cp = corr + ((long)m * KC + (col >> 5)) * 3;
+        acc[m] += sc * (d[m] - 1024.f * cp[1] - 64.f * cp[2]) + bi * cp[0];
+      }
+      if (++st == steps) {
+        const long n = first + round * stride;
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+          const float a = row_sum16(acc[m]);
+          acc[m] = 0.f;
+          if (n < N && l16 == 0 && m < M) {
+            half_t o = (half_t)a;
+            if (bias) o = o + bias[n];
+            out[(long)m * N + n] = o;
+          }
+        }
+        st = 0;
+        ++round;
       }
     }
   }
