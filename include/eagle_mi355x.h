@@ -94,10 +94,11 @@ int eagle_qmm_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
  * launches of eagle_qmm_w4g64_f16 / eagle_qmm_slab_partial_w4g64 and eagle_rmsnorm_f16 /
  * eagle_rmsnorm_slabs_f16 of such a pass.
  * Constraints (eagle_qmm_small_supported): T <= 16; K a multiple of 128, up to 6144 (the waves of
- * a workgroup hold all of x between them); N a multiple of 16 (32 with SwiGLU); every scale
- * below 0.2499 in magnitude (the nibbles are expanded through fp16 subnormals times
- * scale * 2^18); x must not alias out; x, norm_w, wq, residual, out 16-byte aligned. */
+ * a workgroup hold all of x between them); N a multiple of 8 (32 with SwiGLU); x must not alias
+ * out; x, norm_w, wq, residual, out 16-byte, bias 8-byte, scales and biases 4-byte aligned.
+ * eagle_qmm_small_preferred: whether it is the fastest form of a plain or SwiGLU product of M rows. */
 int eagle_qmm_small_supported(int T, int N, int K, int norm, int swiglu);
+int eagle_qmm_small_preferred(int M, int N, int K);
 int eagle_qmm_small_w4g64_f16(const void* x, const void* norm_w, float eps, const uint32_t* wq,
                               const void* scales, const void* biases, const void* bias,
                               const void* residual, void* out, int T, int N, int K,
@@ -112,7 +113,7 @@ int eagle_qmm_small_w4g64_f16(const void* x, const void* norm_w, float eps, cons
  *   x [T, D] fp16; rope_cs [T, hd / 2, 2] fp32; q_out [H, T, hd] fp16; k_cache, v_cache
  *   [G, capacity, hd] fp16 (rows *cache_len_dev + t are written; rows at or past capacity are not).
  * Constraints (eagle_qkv_rope_small_supported): T <= 16, D a multiple of 128 up to 6144, hd a
- * multiple of 32, scales below 0.2499 in magnitude. */
+ * multiple of 32. */
 int eagle_qkv_rope_small_supported(int T, int D, int H, int G, int hd);
 int eagle_qkv_rope_small_w4g64_f16(const void* x, const void* norm_w, float eps, const uint32_t* wq,
                                    const void* scales, const void* biases, const void* bias,

@@ -38,8 +38,8 @@ SCRATCH_ALLOWED = [
     (r"qmm_gemm_w4g64_kernelILi2ELi4E", "prompt GEMM, 128 x 256 blocks"),
     # sixteen waves (K above 3072) leave a wave 128 registers: too few with a second weight tile
     # (SwiGLU, rope) or with the norm weights of three chunks; the drafter's K is 896 there
-    (r"qmm_small_kernelILi16ELi\dELi[12]E", "small-row kernel, sixteen waves, two tiles"),
-    (r"qmm_small_kernelILi16ELi\dELi0ELb1E", "small-row kernel, sixteen waves, norm folded in"),
+    (r"qmm_small_kernelILi1[346]ELi[23]ELi\dELi[12]E", "small-row kernel, sixteen waves, two tiles"),
+    (r"qmm_small_kernelILi1[36]ELi3ELi\dELi0ELb1E", "small-row kernel, sixteen waves, norm folded in"),
     # one query head per KV group at head dimension 128 on a tree above 32 tokens
     (r"tree_attn_split_kernelILi128ELb1ELi8ELi1ELi1E", "attention split, eight vectors per thread"),
 ]

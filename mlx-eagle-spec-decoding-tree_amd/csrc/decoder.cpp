@@ -40,7 +40,7 @@ struct Layer {
 };
 
 struct Decoder {
-  int D, I, H, G, hd, V, form, small;      // small: the weights allow the small-row products
+  int D, I, H, G, hd, V, form;
   float eps, rope_factor, scale;
   Mat emb, head;
   Tiles thead;
@@ -144,7 +144,7 @@ struct Pass {
     chunk = T > 2 * EAGLE_MAX_TREE;
     tiled = d.form == TILED && !chunk;
     fused = d.form == FUSED;
-    folded = fused && d.small && T <= 16 && eagle_qkv_rope_small_supported(T, d.D, d.H, d.G, d.hd) &&
+    folded = fused && T <= 16 && eagle_qkv_rope_small_supported(T, d.D, d.H, d.G, d.hd) &&
              eagle_qmm_small_supported(T, d.D, d.H * d.hd, 0, 0) && eagle_qmm_small_supported(T, 2 * d.I, d.D, 1, 1) &&
              eagle_qmm_small_supported(T, d.D, d.I, 0, 0);
     const size_t f16 = 2, rows = (size_t)R;
@@ -180,6 +180,9 @@ struct Pass {
   }
 
   int swiglu(const Mat& m, const void* x, void* out) {
+    if (eagle_qmm_small_preferred(R, m.N, m.K) && eagle_qmm_small_supported(R, m.N, m.K, 0, 1) &&
+        small_aligned(x, m.s, m.b, m.bias, out))
+      return eagle_qmm_small_w4g64_f16(x, nullptr, 0.f, m.w, m.s, m.b, m.bias, nullptr, out, R, m.N, m.K, 64, 4, 1, st);
     if (eagle_qmm_slab_swiglu_preferred(R, m.N, m.K))
       return eagle_qmm_slab_swiglu_w4g64_f16(x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, 64, 4, st);
     if (R > 2 * EAGLE_MAX_M) return gemm(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);
@@ -292,18 +295,18 @@ PyObject* str(const char* s) { return PyUnicode_InternFromString(s); }
 }  // namespace
 
 // decoder_new(ints, floats, emb, head, thead, norm, inv_freqs, layers, layer_list, cache_type) -> capsule
-//   ints: (D, I, H, G, hd, V, form, small); floats: (eps, rope_factor, scale); layers: per layer (seven projections, qkv, gu,
+//   ints: (D, I, H, G, hd, V, form); floats: (eps, rope_factor, scale); layers: per layer (seven projections, qkv, gu,
 //   four tiled copies, two norms)
 PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  int v[8];
+  int v[7];
   float f[3];
-  if (n != 10 || !PyArg_ParseTuple(a[0], "iiiiiiii", v, v + 1, v + 2, v + 3, v + 4, v + 5, v + 6, v + 7) ||
+  if (n != 10 || !PyArg_ParseTuple(a[0], "iiiiiii", v, v + 1, v + 2, v + 3, v + 4, v + 5, v + 6) ||
       !PyArg_ParseTuple(a[1], "fff", f, f + 1, f + 2) || !PyList_Check(a[7]) || !PyList_Check(a[8])) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "decoder_new takes ten arguments");
     return nullptr;
   }
   std::unique_ptr<Decoder> d(new Decoder());
-  d->D = v[0]; d->I = v[1]; d->H = v[2]; d->G = v[3]; d->hd = v[4]; d->V = v[5]; d->form = v[6]; d->small = v[7];
+  d->D = v[0]; d->I = v[1]; d->H = v[2]; d->G = v[3]; d->hd = v[4]; d->V = v[5]; d->form = v[6];
   d->eps = f[0]; d->rope_factor = f[1]; d->scale = f[2];
   d->emb = take_mat(d.get(), a[2]);
   d->head = take_mat(d.get(), a[3]);

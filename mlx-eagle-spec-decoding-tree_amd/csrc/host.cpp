@@ -60,6 +60,12 @@ int gemm(const at::Tensor& like, const void* x, const void* w, const void* s, co
                                         need ? ws.data_ptr() : nullptr, need, st);
 }
 
+// what the small-row kernel asks of its operands beyond the other forms
+bool small_aligned(const void* x, const void* s, const void* b, const void* bias, const void* out) {
+  auto low = [](const void* p, uintptr_t bits) { return reinterpret_cast<uintptr_t>(p) & bits; };
+  return !low(x, 15) && !low(out, 15) && !low(s, 3) && !low(b, 3) && !low(bias, 7) && x != out;
+}
+
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
            int M, int N, int K, void* st) {
   const uint32_t* wq = static_cast<const uint32_t*>(w);
@@ -69,7 +75,9 @@ int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, 
     const void* xr = static_cast<const char*>(x) + (size_t)r0 * K * 2;
     void* outr = static_cast<char*>(out) + (size_t)r0 * N * 2;
     int rc;
-    if (eagle_qmv_preferred(m, N, K)) {
+    if (eagle_qmm_small_preferred(m, N, K) && small_aligned(xr, s, b, bias, outr)) {
+      rc = eagle_qmm_small_w4g64_f16(xr, nullptr, 0.f, wq, s, b, bias, nullptr, outr, m, N, K, 64, 4, 0, st);
+    } else if (eagle_qmv_preferred(m, N, K)) {
       rc = eagle_qmv_rows_w4g64_f16(xr, wq, s, b, bias, outr, m, N, K, 64, 4, st);
     } else {
       Slot ws;

@@ -40,6 +40,9 @@ PyObject* fail(int rc, const char* what);
 // False with a Python error set.
 bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out);
 
+// Whether the operands have the alignment that the small-row kernel asks for
+bool small_aligned(const void* x, const void* s, const void* b, const void* bias, const void* out);
+
 // The product of M rows: which form runs is the rule of ops.quantized_matmul (its docstring).  A negative
 // result: a Python error is set.
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,

@@ -17,12 +17,10 @@
 //     in flight together; there is no loop over K.
 //   * The norm is folded into the load of x: each wave sums the squares of its columns, the row
 //     sums are added across the waves in LDS; no launch and no pass over memory for it.  Every
-//     workgroup repeats it, so it is kept short: v_dot2 for the sums, x / rms rounded to fp16 and
-//     then multiplied by the norm weight in packed fp16 (two roundings where the norm launch has
-//     one).
-//   * Expansion of the nibbles through fp16 subnormals (a masked nibble pair at mantissa bits
-//     6..9 is q * 2^-18 exactly; one packed fma with (s * 2^18, b)): fp16(s q + b), single
-//     rounding; scales below 0.2499.
+//     workgroup repeats it, so it is kept short: v_dot2 for the sums, mixed-precision products.
+//   * The weights are never rounded: the matrix instructions multiply x with the integers q (exact in
+//     fp16, through the fp8 conversion) a quantisation group at a time, and with ones for the group's
+//     sum of x; scale and bias are applied to the two sums in fp32.
 //
 // Measured on the way (8 rows, the 0.5B drafter's shapes, launches back to back in a graph):
 //   - one wave per tile over the whole K: 2500 instructions on one wave per SIMD, 15 us per launch;
@@ -43,25 +41,22 @@ namespace {
 
 typedef __attribute__((address_space(3))) float4_t sp_lds_float4;
 
+// x in the order of the expanded weights below
 __device__ inline half8_t sp_permute8(half8_t v) {
-  return half8_t{v[0], v[4], v[1], v[5], v[2], v[6], v[3], v[7]};
+  return half8_t{v[0], v[2], v[4], v[6], v[1], v[3], v[5], v[7]};
 }
 
-// eight nibbles -> fp16(s q + b), in the order q0 q4 q1 q5 q2 q6 q3 q7
-__device__ inline half8_t sp_dequant(uint32_t w, half2_t s18, half2_t b2) {
-  union { uint32_t u; half2_t h; } c[4];
-  c[0].u = (w << 6) & 0x03c003c0u;
-  c[1].u = (w << 2) & 0x03c003c0u;
-  c[2].u = (w >> 2) & 0x03c003c0u;
-  c[3].u = (w >> 6) & 0x03c003c0u;
-  half8_t o;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const half2_t v = __builtin_elementwise_fma(c[i].h, s18, b2);
-    o[2 * i] = v[0];
-    o[2 * i + 1] = v[1];
-  }
-  return o;
+// eight nibbles -> fp16 q, in the order q0 q2 q4 q6 q1 q3 q5 q7.  A byte that holds a nibble is, read as OCP
+// e4m3, q * 2^-9 exactly (subnormals up to 7, the first exponent up to 15), so the fp8 conversion gives the
+// fp16 values of q two at a time: seven instructions.
+__device__ inline half8_t sp_expand(uint32_t w) {
+  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
+  union { half2_t h2[4]; half8_t h8; } o;
+  o.h2[0] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, false);
+  o.h2[1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, true);
+  o.h2[2] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, false);
+  o.h2[3] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, true);
+  return o.h8;
 }
 
 struct SmallArgs {
@@ -88,13 +83,17 @@ struct SmallArgs {
 
 enum { SMALL_PLAIN = 0, SMALL_SWIGLU = 1, SMALL_ROPE = 2 };
 
-// NW waves per workgroup, at most SMALL_MAXC chunks of 128 columns per wave, RP passes of four x rows
+// NW waves per workgroup, at most MAXC chunks of 128 columns per wave (a wave requests MAXC whatever it owns:
+// the smallest number that serves K), RP passes of four x rows
 // (2: T <= 8, 4: T <= 16).  MODE: one tile per workgroup (plain / residual), a (gate, up) tile pair
 // 16 rows apart with the SwiGLU epilogue, or two tiles of one head half a head apart (the two
 // halves a rotation pairs) with the rope epilogue.  Lane (r = lane % 16, kq = lane / 16) of a wave
-// holds, per chunk, weight row r columns 32 kq .. + 32 (one 16-byte load, four packed words, one
-// per matrix instruction) and x row r at the same columns; the accumulator of lane (m, q4) is
-// weight rows 4 q4 .. + 4 of x row m.
+// loads, per chunk, weight row r columns 32 kq .. + 32 (one 16-byte load, four packed words): two lanes
+// per quantisation group.  Two half-wave swaps of words deal them so that a word is of one group in all
+// four lanes of a row: after them word 2 g + j of lane (r, kq) is columns 64 g + 32 (kq % 2) +
+// 16 (kq / 2) + 8 j of the chunk, and x row r is read at the same columns.  x is the A operand, the
+// weights are B: the accumulator of lane (r, kq) is x rows 4 kq .. + 4 of weight row r, whose scale and
+// bias are one value per lane.
 //
 // What bounds this kernel is the number of cache lines its load instructions touch per compute
 // unit, so every request is shaped for few lines: x is read with whole rows of a chunk per
@@ -102,15 +101,17 @@ enum { SMALL_PLAIN = 0, SMALL_SWIGLU = 1, SMALL_ROPE = 2 };
 // buffer; the two scales (biases) of a chunk come as one 4-byte load for the three chunks of a
 // wave at once and are handed to the lanes that need them with a lane shuffle.
 constexpr int SMALL_MAXC = 3;
+constexpr int SMALL_RED = 64 + 4;          // floats per four weight rows of a wave's tile
 constexpr int SMALL_XROW = 256 + 16;       // bytes per staged x row: 128 columns, padded against bank conflicts
 
-template <int NW, int RP, int MODE, bool NORM>
+template <int NW, int MAXC, int RP, int MODE, bool NORM>
 __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
   constexpr int NT = MODE == SMALL_PLAIN ? 1 : 2;
-  constexpr int MAXC = SMALL_MAXC;
-  __shared__ __attribute__((aligned(16))) float4_t red[NW][NT][64];
-  __shared__ __attribute__((aligned(16))) unsigned char xstage[NW][RP * 4 * SMALL_XROW];
-  __shared__ float ssq[NW][16];
+  // a slice per wave: first its x, then (written by the same wave) its tiles
+  constexpr int SLICE = RP * 4 * SMALL_XROW;
+  static_assert(NT * 16 * SMALL_RED <= SLICE, "a wave's tiles do not fit over its x");
+  __shared__ __attribute__((aligned(16))) unsigned char slices[NW][SLICE];
+  __shared__ float ssq[NORM ? NW : 1][16];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 15, kq = lane >> 4;
   const int K = a.K, KW = K >> 3, G = K >> 6;
@@ -134,18 +135,7 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
   // join, which puts the requests of a wave one behind the other): chunks the wave does not own
   // and rows past T read a valid address again and their values are never used.
   const int kb = nch > 0 ? k0 : 0;
-  uint4_t wv[NT][MAXC];
-  uint32_t spair[NT], bpair[NT];          // lane (r, c): the two scales (biases) of row r in chunk c
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const long row = row0 + second * t + r;
-    const uint32_t* wp = a.w + row * KW + (kb >> 3) + kq * 4;
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) wv[t][c] = *reinterpret_cast<const uint4_t*>(wp + (c < nch ? c : 0) * 16);
-    const int cpair = kq < nch ? kq : 0;
-    spair[t] = *reinterpret_cast<const uint32_t*>(a.s + row * G + (kb >> 6) + cpair * 2);
-    bpair[t] = *reinterpret_cast<const uint32_t*>(a.b + row * G + (kb >> 6) + cpair * 2);
-  }
+  const int xcol = 4 * (kq & 1) + 2 * (kq >> 1);      // this lane's first 8 columns of a group, in eights
   // x: lane l reads 16 bytes of row 4 p + l / 16 at byte 16 (l % 16) of the chunk's 256
   uint4_t xg[MAXC][RP];
   {
@@ -161,11 +151,25 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
   }
   half8_t nw[MAXC][4];
   if (NORM && a.norm_w) {
-    const half_t* np = a.norm_w + kb + kq * 32;
+    const half_t* np = a.norm_w + kb + xcol * 8;
 #pragma unroll
     for (int c = 0; c < MAXC; ++c)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) nw[c][i] = *reinterpret_cast<const half8_t*>(np + (c < nch ? c : 0) * 128 + i * 8);
+      for (int i = 0; i < 4; ++i) nw[c][i] = *reinterpret_cast<const half8_t*>(np + (c < nch ? c : 0) * 128 + (i >> 1) * 64 + (i & 1) * 8);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  uint4_t wv[NT][MAXC];
+  uint32_t spair[NT], bpair[NT];          // lane (r, c): the two scales (biases) of row r in chunk c
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    long row = row0 + second * t + r;
+    if (MODE == SMALL_PLAIN && row > a.N - 1) row = a.N - 1;         // (N a multiple of 8: never stored)
+    const uint32_t* wp = a.w + row * KW + (kb >> 3) + kq * 4;
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) wv[t][c] = *reinterpret_cast<const uint4_t*>(wp + (c < nch ? c : 0) * 16);
+    const int cpair = kq < nch ? kq : 0;
+    spair[t] = *reinterpret_cast<const uint32_t*>(a.s + row * G + (kb >> 6) + cpair * 2);
+    bpair[t] = *reinterpret_cast<const uint32_t*>(a.b + row * G + (kb >> 6) + cpair * 2);
   }
   // what the epilogue of wave 0 adds (bias, residual, the rotation's cos / sin, the cache length)
   // is requested here with everything else, not after the product: a load behind the product is
@@ -176,7 +180,7 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
   long e_len = 0;
   const int e_rope_head = MODE == SMALL_ROPE ? row0 / a.hd : 0;
   if (wave == 0) {
-    const int bn = row0 + 4 * kq;
+    const int bn = MODE == SMALL_PLAIN && row0 + 4 * kq >= a.N ? 0 : row0 + 4 * kq;
     if (a.bias) {
       e_bias0 = *reinterpret_cast<const half4_t*>(a.bias + bn);
       if (NT == 2) e_bias1 = *reinterpret_cast<const half4_t*>(a.bias + bn + second);
@@ -193,11 +197,12 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
       }
     }
   }
+  __builtin_amdgcn_sched_barrier(0);
   // x through the wave's LDS buffer into the operand layout, a chunk at a time (rows past 4 RP,
   // which are rows past T, read what is there: their columns of the result are not stored)
   half8_t xb[MAXC][4];
   {
-    unsigned char* xs = xstage[wave];
+    unsigned char* xs = slices[wave];
     const int xr = lane >> 4, xc = lane & 15;
 #pragma unroll
     for (int c = 0; c < MAXC; ++c) {
@@ -208,7 +213,7 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
       const int mr = r < 4 * RP ? r : 0;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        xb[c][i] = *reinterpret_cast<const half8_t*>(xs + mr * SMALL_XROW + (4 * kq + i) * 16);
+        xb[c][i] = *reinterpret_cast<const half8_t*>(xs + mr * SMALL_XROW + (8 * (i >> 1) + xcol + (i & 1)) * 16);
       __builtin_amdgcn_wave_barrier();
     }
   }
@@ -243,42 +248,69 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
         for (int i = 0; i < 4; ++i) {
           half8_t o;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] = (half_t)((float)xb[c][i][e] * rinv);   // fp32 product, one rounding
-          xb[c][i] = o * nw[c][i];                                                      // packed fp16 products
+          for (int e = 0; e < 8; ++e) {
+            // as fma with zero: v_fma_mix_f32 reads the fp16 operands, where a product converts them first
+            const float v = __builtin_fmaf((float)xb[c][i][e], rinv, 0.f);
+            o[e] = (half_t)__builtin_fmaf(v, (float)nw[c][i][e], 0.f);
+          }
+          xb[c][i] = o;
         }
       }
     }
   }
 
   // ---- the wave's part of the tile(s) ----
+  const half_t one = (half_t)1.f;
+  const half8_t ones = {one, one, one, one, one, one, one, one};
+  const float4_t zero = {0.f, 0.f, 0.f, 0.f};
   float4_t acc[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    acc[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; ++t) acc[t] = zero;
 #pragma unroll
-    for (int c = 0; c < MAXC; ++c) {
-      if (c < nch) {
-        // the pair of chunk c sits in lane (r, c); this lane's columns are in its half kq / 2
+  for (int c = 0; c < MAXC; ++c) {
+    if (c < nch) {
+      float4_t sx[2];
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        xb[c][2 * g] = sp_permute8(xb[c][2 * g]);
+        xb[c][2 * g + 1] = sp_permute8(xb[c][2 * g + 1]);
+        sx[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g], ones, zero, 0, 0, 0);
+        sx[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g + 1], ones, sx[g], 0, 0, 0);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        // the pair of chunk c sits in lane (r, c)
         const uint32_t s2 = __shfl(spair[t], r + 16 * c, 64), b2 = __shfl(bpair[t], r + 16 * c, 64);
-        const half_t sraw = __builtin_bit_cast(half_t, (unsigned short)(kq & 2 ? s2 >> 16 : s2 & 0xffffu));
-        const half_t bi = __builtin_bit_cast(half_t, (unsigned short)(kq & 2 ? b2 >> 16 : b2 & 0xffffu));
-        const half_t sc = (half_t)((float)sraw * 262144.f);
+        const auto w02 = __builtin_amdgcn_permlane32_swap(wv[t][c][0], wv[t][c][2], false, false);
+        const auto w13 = __builtin_amdgcn_permlane32_swap(wv[t][c][1], wv[t][c][3], false, false);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const half8_t av = sp_dequant(wv[t][c][i], half2_t{sc, sc}, half2_t{bi, bi});
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, sp_permute8(xb[c][i]), acc[t], 0, 0, 0);
+        for (int g = 0; g < 2; ++g) {
+          const float sc = (float)__builtin_bit_cast(half_t, (unsigned short)(g ? s2 >> 16 : s2 & 0xffffu));
+          const float bi = (float)__builtin_bit_cast(half_t, (unsigned short)(g ? b2 >> 16 : b2 & 0xffffu));
+          float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g], sp_expand(w02[g]), zero, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g + 1], sp_expand(w13[g]), d, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[t][i] = __builtin_fmaf(bi, sx[g][i], __builtin_fmaf(sc, d[i], acc[t][i]));
         }
       }
     }
-    *(sp_lds_float4*)&red[wave][t][lane] = acc[t];
+  }
+  // Into LDS so that a lane of the epilogue reads four weight rows of one x row with one load: x row m,
+  // weight row n at 4 m + 68 (n / 4) + n % 4 (68: the sixteen weight rows of a store in different banks).
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    float* red = reinterpret_cast<float*>(slices[wave]) + t * (4 * SMALL_RED);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[4 * (4 * kq + i) + SMALL_RED * (r >> 2) + (r & 3)] = acc[t][i];
   }
   __syncthreads();
   if (wave != 0) return;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    float4_t sum = red[0][t][lane];
+    const int at = t * (4 * SMALL_RED) + 4 * r + SMALL_RED * kq;
+    float4_t sum = zero;
 #pragma unroll
-    for (int w = 1; w < NW; ++w) sum += red[w][t][lane];
+    for (int w = 0; w < NW; ++w) sum += *(const sp_lds_float4*)(reinterpret_cast<const float*>(slices[w]) + at);
     acc[t] = sum;
   }
 
@@ -346,6 +378,7 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
     *reinterpret_cast<half4_t*>(a.out + (long)m * (a.N >> 1) + (row0 >> 1) + 4 * q4) = o;
   } else {
     const int n = row0 + 4 * q4;
+    if (n >= a.N) return;
     half4_t o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -360,40 +393,64 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
   }
 }
 
-constexpr int SMALL_K4 = 4 * SMALL_MAXC * 128;       // four waves, three chunks each
-constexpr int SMALL_K8 = 8 * SMALL_MAXC * 128;
-constexpr int SMALL_K16 = 16 * SMALL_MAXC * 128;
+constexpr int SMALL_K16 = 16 * SMALL_MAXC * 128;      // sixteen waves, three chunks each
+
+template <int NW, int MAXC, int MODE, bool NORM>
+void small_go(const SmallArgs& a, int grid, hipStream_t st) {
+  if (a.T > 8)
+    hipLaunchKernelGGL((qmm_small_kernel<NW, MAXC, 4, MODE, NORM>), dim3(grid), dim3(NW * 64), 0, st, a);
+  else
+    hipLaunchKernelGGL((qmm_small_kernel<NW, MAXC, 2, MODE, NORM>), dim3(grid), dim3(NW * 64), 0, st, a);
+}
 
 template <int MODE>
 void small_launch(const SmallArgs& a, int grid, hipStream_t st) {
-  const bool tall = a.T > 8;
-#define SMALL_GO(NW, NORM)                                                                                \
-  do {                                                                                                 \
-    if (tall)                                                                                          \
-      hipLaunchKernelGGL((qmm_small_kernel<NW, 4, MODE, NORM>), dim3(grid), dim3(NW * 64), 0, st, a);  \
-    else                                                                                               \
-      hipLaunchKernelGGL((qmm_small_kernel<NW, 2, MODE, NORM>), dim3(grid), dim3(NW * 64), 0, st, a);  \
-  } while (0)
+  // A load that a wave makes for a chunk it does not own costs what any other does, so the waves are chosen
+  // to own whole loads (8 rows, us): 7 x 1 against 4 x 2 for the 7 chunks of K = 896 (o 2.68 / 2.85, 8192 rows
+  // 3.28 / 3.51; the other way round for the many workgroups of gate|up, 9728 rows: 6.2 / 5.8), 4 x 2 against
+  // 4 x 3 (gate|up 5.8 / 6.3), 16 x 2 against 16 x 3 for K = 3584 (4.9 / 5.7), 13 x 3 against 16 x 3 for
+  // K = 4864 (5.08 / 5.18).  By N and K alone: a SwiGLU product gives the bits of the plain one.
+  const int chunks = a.K >> 7;
+  if (chunks <= 4) return small_go<4, 1, MODE, true>(a, grid, st);
+  if (chunks <= 7 && a.N <= 8192) return small_go<7, 1, MODE, true>(a, grid, st);
+  if (chunks <= 8) return small_go<4, 2, MODE, true>(a, grid, st);
+  if (chunks <= 12) return small_go<4, 3, MODE, true>(a, grid, st);
+  if (chunks <= 16) return small_go<8, 2, MODE, true>(a, grid, st);
+  if (chunks <= 24) return small_go<8, 3, MODE, true>(a, grid, st);
   // Sixteen waves leave a wave 128 registers: the norm weights of its chunks (48 of them) only
   // have room in a build of their own, so the products without a norm (o, down) get one that
   // does not hold them.
-  if (a.K <= SMALL_K4)
-    SMALL_GO(4, true);
-  else if (a.K <= SMALL_K8)
-    SMALL_GO(8, true);
-  else if (a.norm_w)
-    SMALL_GO(16, true);
-  else
-    SMALL_GO(16, false);
-#undef SMALL_GO
+  const bool norm = a.norm_w != nullptr;
+  if (chunks <= 32) return norm ? small_go<16, 2, MODE, true>(a, grid, st) : small_go<16, 2, MODE, false>(a, grid, st);
+  if (chunks <= 39) return norm ? small_go<13, 3, MODE, true>(a, grid, st) : small_go<13, 3, MODE, false>(a, grid, st);
+  return norm ? small_go<16, 3, MODE, true>(a, grid, st) : small_go<16, 3, MODE, false>(a, grid, st);
 }
 
 }  // namespace
 
 EAGLE_EXPORT int eagle_qmm_small_supported(int T, int N, int K, int norm, int swiglu) {
   (void)norm;
-  return T >= 1 && T <= 16 && N >= 16 && (N % (swiglu ? 32 : 16)) == 0 && K >= 128 && (K % 128) == 0 &&
+  return T >= 1 && T <= 16 && N >= (swiglu ? 32 : 8) && (N % (swiglu ? 32 : 8)) == 0 && K >= 128 && (K % 128) == 0 &&
          K <= SMALL_K16;
+}
+
+// Where this kernel beats the vector kernel and the streaming kernel for a plain (or SwiGLU) product:
+// measured over K 384 .. 6144, N 512 .. 18944, 1 .. 16 rows, launches back to back over rotating weights.
+// Its workgroups have no loop over N and share nothing, so it holds as long as they fit the compute units in
+// a few rounds: sixteen waves (K above 3072) are one workgroup per unit, eight two, four five.  Eight rows
+// against the streaming kernel: 3584 x 3584 4.9 / 8.6 us, 2048 -> 8192 5.5 / 7.5, 4864 -> 896 5.1 / 8.0;
+// just past the line, 4096 -> 12288 13.1 / 12.9.  One row where the vector kernel runs: only at K above
+// 3072 (3584 x 3584 4.7 / 5.4; 2048 -> 2048 3.7 / 3.7).
+EAGLE_EXPORT int eagle_qmm_small_preferred(int M, int N, int K) {
+  if (!eagle_qmm_small_supported(M, N, K, 0, 0)) return 0;
+  const int groups = (N + 15) / 16, cus = 256;
+  if (M == 1 && eagle_qmv_preferred(M, N, K)) return K > 3072 && groups <= cus;
+  const bool few = M <= 8;
+  if (K <= 1536) return groups <= 5 * cus;
+  if (K <= 2048) return groups <= (few ? 3 : 2) * cus;
+  if (K <= 3072) return groups <= 2 * cus;
+  if (K <= 4992) return groups <= (few ? 2 : 1) * cus;
+  return groups <= cus;
 }
 
 EAGLE_EXPORT int eagle_qmm_small_w4g64_f16(const void* x, const void* norm_w, float eps, const uint32_t* wq,
@@ -430,7 +487,7 @@ EAGLE_EXPORT int eagle_qmm_small_w4g64_f16(const void* x, const void* norm_w, fl
   if (swiglu)
     small_launch<SMALL_SWIGLU>(a, N / 32, st);
   else
-    small_launch<SMALL_PLAIN>(a, N / 16, st);
+    small_launch<SMALL_PLAIN>(a, (N + 15) / 16, st);
   return eagle_launch_status();
 }
 

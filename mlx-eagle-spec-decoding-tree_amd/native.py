@@ -108,7 +108,7 @@ def _build(model):
     if at0._inv_freqs.numel() != hd // 2 or not at0._inv_freqs.is_cuda or at0._inv_freqs.dtype != torch.float32:
         return None
 
-    form, small, derived, thead = _derive(model, layers, head_w, shapes, I, D, V, H, G, hd)
+    form, derived, thead = _derive(model, layers, head_w, shapes, I, D, V, H, G, hd)
     described = []
     for i, lins in enumerate(layers):
         layer = m.layers[i]
@@ -116,16 +116,16 @@ def _build(model):
                                          layer.self_attn.o_proj, layer.mlp.gate_proj, layer.mlp.up_proj, layer.mlp.down_proj)]
         described.append((*leaves, *derived[i], layer.input_layernorm.weight, layer.post_attention_layernorm.weight))
     return ops._native().decoder_new(
-        (D, I, H, G, hd, V, form, int(small)), (args.rms_norm_eps, float(at0._scaling_factor), float(at0.scale)), emb_w, head_w,
+        (D, I, H, G, hd, V, form), (args.rms_norm_eps, float(at0._scaling_factor), float(at0.scale)), emb_w, head_w,
         thead, m.norm.weight, at0._inv_freqs, described, m.layers, KVCache)
 
 
 def _derive(model, layers, head_w, shapes, I, D, V, H, G, hd):
-    """(form, scales small enough for the small-row products, per layer (qkv, gu, four tiled copies), tiled head)."""
+    """(form, per layer (qkv, gu, four tiled copies), tiled head)."""
     from . import eagle
     none = (None,) * 6
     if D < FUSE_HIDDEN:
-        return PLAIN, False, [none] * len(layers), None
+        return PLAIN, [none] * len(layers), None
     W = (H + 2 * G) * hd
     products = {"qkv": (W, D), "o": shapes["o"], "down": shapes["down"]}
     tiled = all(ops.slab_steps(32, n, k) and ops.tiled_supported(32, n, k) for n, k in products.values()) \
@@ -135,11 +135,8 @@ def _derive(model, layers, head_w, shapes, I, D, V, H, G, hd):
         sets = eagle.tile_model(model)
         derived = [(None, None, *((t.wt, t.sbt, t.N, t.K, t.small, b) for t, b in entry)) for entry in sets]
         th = eagle.tiled_head(model) if head_w[3] is None else None
-        return TILED, False, derived, None if th is None else (th.wt, th.sbt, th.N, th.K, th.small, None)
+        return TILED, derived, None if th is None else (th.wt, th.sbt, th.N, th.K, th.small, None)
     if not ops.swiglu_supported(32, I, D) or W % 16 or D % 16:
-        return PLAIN, False, [none] * len(layers), None
+        return PLAIN, [none] * len(layers), None
     qkv_w, gu_w = eagle.fuse_projections(model, True)
-    worst = torch.stack([t.abs().amax() for i, lins in enumerate(layers)
-                         for t in (qkv_w[i][1], lins["o"].scales, gu_w[i][1], lins["down"].scales)]).amax()
-    small = bool(worst.item() < ops.SMALL_SCALE_LIMIT)
-    return FUSED, small, [(qkv_w[i], gu_w[i], None, None, None, None) for i in range(len(layers))], None
+    return FUSED, [(qkv_w[i], gu_w[i], None, None, None, None) for i in range(len(layers))], None

@@ -75,7 +75,8 @@ def as_packed_u32(w_q):
 def quantized_matmul(x, w_q, scales, biases, transpose=True, group_size=64, bits=4, bias=None,
                      out=None, tuned=None, gemm=None):
     """`mx.quantized_matmul(x, w, scales, biases, transpose=True, group_size=64, bits=4)`
-    (any leading dims, flattened as qmm_kernel.py:99-100,136): the vector-ALU kernel for one row (or
+    (any leading dims, flattened as qmm_kernel.py:99-100,136): the small-row kernel for up to 16 rows
+    where the library prefers it (eagle_qmm_small_preferred), the vector-ALU kernel for one row (or
     two) where `qmv_preferred` says so, the streaming kernel for up to 32 rows of x, two passes of it
     for 33..64 rows (a tree above 32 tokens; faster there than the GEMM's few long-running workgroups:
     21 against 31 us for 40 x 4608 x 3584, 44 against 185 us for 40 x 3584 x 18944), a tiled GEMM above
@@ -300,7 +301,7 @@ def quantized_matmul_swiglu_slab(x, w_q, scales, biases, bias=None, out=None):
 def quantized_matmul_swiglu(x, w_q, scales, biases, bias=None, out=None, gemm=None, tiled=None):
     """silu(x @ Wg.T) * (x @ Wu.T) (mlx_llama.py:214-215) in one launch: w_q / scales / biases
     / bias hold the gate and up projections interleaved by `interleave_gate_up`.  With more than
-    one row on the streaming kernel the result equals `silu_mul(quantized_matmul(x, gate...),
+    one row on the streaming or the small-row kernel the result equals `silu_mul(quantized_matmul(x, gate...),
     quantized_matmul(x, up...))` bit for bit; the other forms agree with it to the tolerance of
     the product.  33..64 rows run on the slab kernel with 64-row tiles
     (`quantized_matmul_swiglu_slab`), more rows as the tiled GEMM form with the same epilogue
@@ -339,6 +340,8 @@ def quantized_matmul_swiglu(x, w_q, scales, biases, bias=None, out=None, gemm=No
     if out is None:
         out = torch.empty((*lead, N // 2), dtype=torch.float16, device=x.device)
     L = _lib.lib()
+    if not gemm and N % 32 == 0 and L.eagle_qmm_small_preferred(M, N, K):
+        return quantized_matmul_small(x, w_q, scales, biases, bias=bias, out=out, swiglu=True)
     if not gemm and L.eagle_qmm_slab_swiglu_preferred(M, N, K):
         # the slab kernel with one slab over all of K: above 32 rows one launch with 64-row tiles
         # (35 us against 48..56 us for two passes of the 32-row kernel at the 7B shape), and from
@@ -420,9 +423,6 @@ def tile_weights(w_q, scales, biases):
     return TiledWeights(wt, sbt, N, K, worst.item() < TILED_SMALL_SCALE)
 
 
-SMALL_SCALE_LIMIT = 0.2499       # |scale| * 2^18 has to stay a finite fp16 (the small-row kernels)
-
-
 def small_supported(T, N, K, norm=False, swiglu=False):
     """True when `quantized_matmul_small` takes this shape."""
     return bool(_lib.lib().eagle_qmm_small_supported(T, N, K, int(bool(norm)), int(bool(swiglu))))
@@ -432,8 +432,7 @@ def quantized_matmul_small(x, w_q, scales, biases, bias=None, out=None, norm_wei
                            residual=None, swiglu=False):
     """The product for at most 16 rows with its neighbours folded in (mlx_llama.py:195-196,
     214-215, 225-249): RMSNorm of x before it (norm_weight), the residual added to it (residual;
-    may be `out`), or SwiGLU over gate|up interleaved by `interleave_gate_up` (swiglu).  Every
-    scale must be below SMALL_SCALE_LIMIT in magnitude; the caller checks that once per matrix."""
+    may be `out`), or SwiGLU over gate|up interleaved by `interleave_gate_up` (swiglu)."""
     _need_cuda(x, w_q, scales, biases, bias, norm_weight, residual)
     x = _f16(x, "x")
     w_q = as_packed_u32(w_q)

@@ -20,6 +20,9 @@ from .eagle import slab_plan as eagle_slab_plan
 
 Y_LEN = 8
 MAX_CHUNK = 2048     # rows of one causal prompt pass (EAGLE_MAX_CHUNK)
+# A pass object folds its small-row products for weights below this scale only.  (The kernel takes any scale;
+# a model beyond keeps the launches, and so the results, that it always had.)
+FOLD_SCALE_LIMIT = 0.2499
 
 
 class DecoderPass:
@@ -56,7 +59,7 @@ class DecoderPass:
         W = (H + 2 * G) * hd
         can_fold = self.swiglu and ops.small_supported(T, W, D, norm=True) \
             and ops.small_supported(T, D, H * hd) and ops.small_supported(T, 2 * I, D, norm=True, swiglu=True) \
-            and ops.small_supported(T, D, I) and self._scales_within(ops.SMALL_SCALE_LIMIT)
+            and ops.small_supported(T, D, I) and self._scales_within(FOLD_SCALE_LIMIT)
         if folded and not can_fold:
             raise ValueError("the small-row form does not take these shapes or weights")
         self.folded = can_fold if folded is None else bool(folded)
