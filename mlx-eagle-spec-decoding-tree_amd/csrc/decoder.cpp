@@ -183,6 +183,8 @@ struct Pass {
     if (eagle_qmm_small_preferred(R, m.N, m.K) && eagle_qmm_small_supported(R, m.N, m.K, 0, 1) &&
         small_aligned(x, m.s, m.b, m.bias, out))
       return eagle_qmm_small_w4g64_f16(x, nullptr, 0.f, m.w, m.s, m.b, m.bias, nullptr, out, R, m.N, m.K, 64, 4, 1, st);
+    if (R <= EAGLE_MAX_M && m.N % 32 == 0 && rows_takes(R, m.N, m.K, x, m.s, m.b, out))
+      return rows(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);
     if (eagle_qmm_slab_swiglu_preferred(R, m.N, m.K))
       return eagle_qmm_slab_swiglu_w4g64_f16(x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, 64, 4, st);
     if (R > 2 * EAGLE_MAX_M) return gemm(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);

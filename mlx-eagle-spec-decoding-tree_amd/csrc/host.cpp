@@ -60,6 +60,20 @@ int gemm(const at::Tensor& like, const void* x, const void* w, const void* s, co
                                         need ? ws.data_ptr() : nullptr, need, st);
 }
 
+bool rows_takes(int M, int N, int K, const void* x, const void* s, const void* b, const void* out) {
+  return eagle_qmm_rows_preferred(M, N, K) && small_aligned(x, s, b, nullptr, out);
+}
+
+int rows(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out, int M,
+         int N, int K, bool swiglu, void* st) {
+  // the partial sums go back to torch's allocator with the launches in the stream
+  const size_t need = eagle_qmm_rows_workspace_bytes(M, N, K);
+  at::Tensor ws;
+  if (need) ws = empty({(int64_t)need}, at::kByte, like);
+  return eagle_qmm_rows_w4g64_f16(x, static_cast<const uint32_t*>(w), s, b, bias, out, M, N, K, 64, 4, swiglu,
+                                  need ? ws.data_ptr() : nullptr, need, st);
+}
+
 // what the small-row kernel asks of its operands beyond the other forms
 bool small_aligned(const void* x, const void* s, const void* b, const void* bias, const void* out) {
   auto low = [](const void* p, uintptr_t bits) { return reinterpret_cast<uintptr_t>(p) & bits; };
@@ -70,6 +84,7 @@ int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, 
            int M, int N, int K, void* st) {
   const uint32_t* wq = static_cast<const uint32_t*>(w);
   if (M > 2 * EAGLE_MAX_M) return gemm(like, x, w, s, b, bias, out, M, N, K, false, st);
+  if (M > EAGLE_MAX_M && rows_takes(M, N, K, x, s, b, out)) return rows(like, x, w, s, b, bias, out, M, N, K, false, st);
   for (int r0 = 0; r0 < M; r0 += EAGLE_MAX_M) {
     const int m = M - r0 < EAGLE_MAX_M ? M - r0 : EAGLE_MAX_M;
     const void* xr = static_cast<const char*>(x) + (size_t)r0 * K * 2;
@@ -79,6 +94,8 @@ int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, 
       rc = eagle_qmm_small_w4g64_f16(xr, nullptr, 0.f, wq, s, b, bias, nullptr, outr, m, N, K, 64, 4, 0, st);
     } else if (eagle_qmv_preferred(m, N, K)) {
       rc = eagle_qmv_rows_w4g64_f16(xr, wq, s, b, bias, outr, m, N, K, 64, 4, st);
+    } else if (rows_takes(m, N, K, xr, s, b, outr)) {
+      rc = rows(like, xr, w, s, b, bias, outr, m, N, K, false, st);
     } else {
       Slot ws;
       if (!qmm_workspace(like, eagle_qmm_workspace_bytes(m, N, K), &ws)) return -1;

@@ -43,6 +43,11 @@ bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out);
 // Whether the operands have the alignment that the small-row kernel asks for
 bool small_aligned(const void* x, const void* s, const void* b, const void* bias, const void* out);
 
+// The product of up to 64 rows on eagle_qmm_rows_w4g64_f16, and whether it is the form to take
+bool rows_takes(int M, int N, int K, const void* x, const void* s, const void* b, const void* out);
+int rows(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out, int M,
+         int N, int K, bool swiglu, void* st);
+
 // The product of M rows: which form runs is the rule of ops.quantized_matmul (its docstring).  A negative
 // result: a Python error is set.
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,

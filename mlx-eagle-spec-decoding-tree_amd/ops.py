@@ -77,10 +77,8 @@ def quantized_matmul(x, w_q, scales, biases, transpose=True, group_size=64, bits
     """`mx.quantized_matmul(x, w, scales, biases, transpose=True, group_size=64, bits=4)`
     (any leading dims, flattened as qmm_kernel.py:99-100,136): the small-row kernel for up to 16 rows
     where the library prefers it (eagle_qmm_small_preferred), the vector-ALU kernel for one row (or
-    two) where `qmv_preferred` says so, the streaming kernel for up to 32 rows of x, two passes of it
-    for 33..64 rows (a tree above 32 tokens; faster there than the GEMM's few long-running workgroups:
-    21 against 31 us for 40 x 4608 x 3584, 44 against 185 us for 40 x 3584 x 18944), a tiled GEMM above
-    that.  `bias` ([N] fp16) is added after rounding, as the patched linear layer does
+    two) where `qmv_preferred` says so, up to 64 rows the kernel of csrc/rows.hip where the library prefers
+    it (eagle_qmm_rows_preferred), else the streaming kernel in passes of 32 rows, a tiled GEMM above that.  `bias` ([N] fp16) is added after rounding, as the patched linear layer does
     (mlx_model_fwd_bench.py:70-71).  `tuned` forces a launch shape of the streaming kernel,
     `gemm=True` the tiled GEMM whatever the row count.  The default path is native code
     (csrc/host.cpp)."""
@@ -301,8 +299,7 @@ def quantized_matmul_swiglu_slab(x, w_q, scales, biases, bias=None, out=None):
 def quantized_matmul_swiglu(x, w_q, scales, biases, bias=None, out=None, gemm=None, tiled=None):
     """silu(x @ Wg.T) * (x @ Wu.T) (mlx_llama.py:214-215) in one launch: w_q / scales / biases
     / bias hold the gate and up projections interleaved by `interleave_gate_up`.  With more than
-    one row on the streaming or the small-row kernel the result equals `silu_mul(quantized_matmul(x, gate...),
-    quantized_matmul(x, up...))` bit for bit; the other forms agree with it to the tolerance of
+    one row, up to 32, the result equals `silu_mul` of the concatenated product bit for bit; the other forms agree with it to the tolerance of
     the product.  33..64 rows run on the slab kernel with 64-row tiles
     (`quantized_matmul_swiglu_slab`), more rows as the tiled GEMM form with the same epilogue
     (`gemm=True`: that form whatever the row count).
@@ -342,6 +339,14 @@ def quantized_matmul_swiglu(x, w_q, scales, biases, bias=None, out=None, gemm=No
     L = _lib.lib()
     if not gemm and N % 32 == 0 and L.eagle_qmm_small_preferred(M, N, K):
         return quantized_matmul_small(x, w_q, scales, biases, bias=bias, out=out, swiglu=True)
+    if not gemm and M <= ROW_PASS and N % 32 == 0 and L.eagle_qmm_rows_preferred(M, N, K) \
+            and (scales.data_ptr() | biases.data_ptr()) % 4 == 0:
+        need = L.eagle_qmm_rows_workspace_bytes(M, N, K)
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+        rc = L.eagle_qmm_rows_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(out), M, N, K,
+                                        64, 4, 1, _ptr(ws), need, _stream())
+        _lib.check(rc, "quantized_matmul_swiglu")
+        return out
     if not gemm and L.eagle_qmm_slab_swiglu_preferred(M, N, K):
         # the slab kernel with one slab over all of K: above 32 rows one launch with 64-row tiles
         # (35 us against 48..56 us for two passes of the 32-row kernel at the 7B shape), and from
