@@ -118,6 +118,14 @@ int eagle_qmm_rows_w4g64_f16(const void* x, const uint32_t* wq, const void* scal
                              const void* bias, void* out, int M, int N, int K, int group_size, int bits,
                              int swiglu, void* workspace, size_t workspace_bytes, eagle_stream_t stream);
 
+/* The same product left as fp32 partial sums for its consumer (eagle_rmsnorm_slabs_f16,
+ * eagle_rope_kv_append_slabs_f16): partial [splits][R][N] with splits = eagle_qmm_rows_partial_splits (0: shape not
+ * taken) and R = 32 up to 32 rows, 64 above. */
+int eagle_qmm_rows_partial_splits(int M, int N, int K);
+int eagle_qmm_rows_partial_w4g64(const void* x, const uint32_t* wq, const void* scales, const void* biases,
+                                 float* partial, size_t partial_bytes, int M, int N, int K, int group_size,
+                                 int bits, eagle_stream_t stream);
+
 /* q|k|v of a small pass with everything around it in one launch: RMSNorm of x (norm_w, or NULL for
  * none), the product with the fused q|k|v matrix [(H + 2 G) hd, D] (+ bias), the rotation of q and
  * k with the per-token (cos, sin) table of eagle_rope_table_f32, and the append of the new K / V

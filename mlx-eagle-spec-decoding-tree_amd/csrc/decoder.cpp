@@ -4,12 +4,11 @@
 // Bound by the host before: 30 operators x 28 layers at 10 us each, 14 ms for a 40-token tree on the 7B
 // shape, whose kernels take 3 ms.  A launch from here costs about 2 us, so the GPU is the bound again.
 //
-// Three forms of a layer, chosen per model when the decoder is built (native.py):
+// Two forms of a layer, chosen per model when the decoder is built (native.py):
 //   PLAIN   one launch per projection on the checkpoint's tensors, the launches of the module path;
-//   FUSED   q|k|v as one product and gate|up as one with SwiGLU in its epilogue; for at most 16 rows, where the
-//           shapes allow it, the small-row products with norm, residual, rope and cache append folded in;
-//   TILED   the products of up to 64 rows from tiled copies of the weights, as partial sums that the norm
-//           and rope launches add (the launches of eagle.TreeVerifier).
+//   FUSED   q|k|v as one product and gate|up as one with SwiGLU in its epilogue.  Up to 16 rows, where the shapes
+//           allow it, the small-row products with norm, residual, rope and cache append folded in; for 17..64 rows the
+//           products stay partial sums, which the norm and rope launches add.
 // More than 64 rows (a prompt) go through the GEMM and the causal attention in either form.
 #include "host.h"
 
@@ -20,30 +19,24 @@
 namespace eagle_host {
 namespace {
 
-enum Form { PLAIN = 0, FUSED = 1, TILED = 2 };
+enum Form { PLAIN = 0, FUSED = 1 };
 
 struct Mat {
   const uint32_t* w = nullptr;
   const void *s = nullptr, *b = nullptr, *bias = nullptr;
   int N = 0, K = 0;
 };
-struct Tiles {
-  const uint32_t* wt = nullptr;
-  const void *sbt = nullptr, *bias = nullptr;
-  int N = 0, K = 0, small = 0;
-};
 enum { Q, K_, V_, O, GATE, UP, DOWN, NPROJ };
 struct Layer {
   Mat p[NPROJ], qkv, gu;
-  Tiles tqkv, to, tgu, tdown;
   const void *norm1 = nullptr, *norm2 = nullptr;
 };
 
 struct Decoder {
   int D, I, H, G, hd, V, form;
+  bool linear_bias = false;                // an o or down projection with a bias
   float eps, rope_factor, scale;
   Mat emb, head;
-  Tiles thead;
   const void* norm = nullptr;
   const float* inv_freqs = nullptr;
   std::vector<Layer> layers;
@@ -89,20 +82,6 @@ Mat take_mat(Decoder* d, PyObject* o) {
   if (PyTuple_GET_ITEM(o, 3) != Py_None) m.bias = take(d, PyTuple_GET_ITEM(o, 3)).data_ptr();
   return m;
 }
-// (wt, sbt, N, K, small, bias or None)
-Tiles take_tiles(Decoder* d, PyObject* o) {
-  Tiles t;
-  if (o == Py_None) return t;
-  if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) != 6) throw Bad();
-  t.wt = static_cast<const uint32_t*>(take(d, PyTuple_GET_ITEM(o, 0)).data_ptr());
-  t.sbt = take(d, PyTuple_GET_ITEM(o, 1)).data_ptr();
-  t.N = (int)PyLong_AsLong(PyTuple_GET_ITEM(o, 2));
-  t.K = (int)PyLong_AsLong(PyTuple_GET_ITEM(o, 3));
-  t.small = PyObject_IsTrue(PyTuple_GET_ITEM(o, 4));
-  if (PyTuple_GET_ITEM(o, 5) != Py_None) t.bias = take(d, PyTuple_GET_ITEM(o, 5)).data_ptr();
-  return t;
-}
-
 // One allocation for a pass's buffers, handed out in order
 struct Arena {
   size_t size = 0;
@@ -131,8 +110,8 @@ struct Pass {
   Arena ar;
   size_t h, hn, qkv, q_rot, attn, o, act, gate, down, cs, pos, words, lens, pieces, partial, attn_ws;
   size_t attn_ws_bytes = 0, partial_bytes = 0;
-  int slab_qkv = 0, slab_o = 0, slab_down = 0;
-  bool chunk, folded, tiled, fused;
+  int splits_qkv = 0, splits_o = 0, splits_down = 0;
+  bool chunk, folded, summed, fused;
   const uint32_t* mask_words = nullptr;
   std::vector<void*> keys, values;
 
@@ -142,11 +121,19 @@ struct Pass {
   void plan() {
     const int W = (d.H + 2 * d.G) * d.hd;
     chunk = T > 2 * EAGLE_MAX_TREE;
-    tiled = d.form == TILED && !chunk;
     fused = d.form == FUSED;
     folded = fused && T <= 16 && eagle_qkv_rope_small_supported(T, d.D, d.H, d.G, d.hd) &&
              eagle_qmm_small_supported(T, d.D, d.H * d.hd, 0, 0) && eagle_qmm_small_supported(T, 2 * d.I, d.D, 1, 1) &&
              eagle_qmm_small_supported(T, d.D, d.I, 0, 0);
+    summed = false;
+    if (fused && !chunk && T > EAGLE_MAX_M / 2 && !d.linear_bias) {
+      splits_qkv = eagle_qmm_rows_partial_splits(T, W, d.D);
+      splits_o = eagle_qmm_rows_partial_splits(T, d.D, d.H * d.hd);
+      splits_down = eagle_qmm_rows_partial_splits(T, d.D, d.I);
+      summed = splits_qkv && splits_o && splits_down;
+      const size_t rows = T > EAGLE_MAX_M ? 2 * EAGLE_MAX_M : EAGLE_MAX_M;
+      partial_bytes = summed ? rows * sizeof(float) * std::max({(size_t)splits_qkv * W, (size_t)splits_o * d.D, (size_t)splits_down * d.D}) : 0;
+    }
     const size_t f16 = 2, rows = (size_t)R;
     h = ar.add(rows * d.D * f16);
     hn = ar.add(rows * d.D * f16);
@@ -155,20 +142,12 @@ struct Pass {
     attn = ar.add(rows * d.H * d.hd * f16);
     o = ar.add(rows * d.D * f16);
     act = ar.add(rows * d.I * f16);
-    gate = ar.add(d.form == FUSED || tiled ? 256 : rows * 2 * d.I * f16);
+    gate = ar.add(d.form == FUSED ? 256 : rows * 2 * d.I * f16);
     cs = ar.add(rows * (d.hd / 2) * 2 * 4);
     pos = ar.add(rows * 4);
     words = ar.add(rows * 2 * 4);
     lens = ar.add(8);
     pieces = ar.add((rows / 32 + 1) * 4);
-    if (tiled) {
-      slab_qkv = eagle_qmm_slab_steps(T, W, d.D);
-      slab_o = eagle_qmm_slab_steps(T, d.D, d.H * d.hd);
-      slab_down = eagle_qmm_slab_steps(T, d.D, d.I);
-      partial_bytes = std::max({eagle_qmm_slab_partial_bytes_rows(T, W, d.D, slab_qkv),
-                                eagle_qmm_slab_partial_bytes_rows(T, d.D, d.H * d.hd, slab_o),
-                                eagle_qmm_slab_partial_bytes_rows(T, d.D, d.I, slab_down)});
-    }
     partial = ar.add(partial_bytes);
     attn_ws_bytes = chunk ? eagle_causal_attention_workspace_bytes(R, d.H, d.hd, S)
                           : eagle_tree_attention_wide_workspace_bytes(T, d.H, d.hd, S);
@@ -183,10 +162,8 @@ struct Pass {
     if (eagle_qmm_small_preferred(R, m.N, m.K) && eagle_qmm_small_supported(R, m.N, m.K, 0, 1) &&
         small_aligned(x, m.s, m.b, m.bias, out))
       return eagle_qmm_small_w4g64_f16(x, nullptr, 0.f, m.w, m.s, m.b, m.bias, nullptr, out, R, m.N, m.K, 64, 4, 1, st);
-    if (R <= EAGLE_MAX_M && m.N % 32 == 0 && rows_takes(R, m.N, m.K, x, m.s, m.b, out))
+    if (m.N % 32 == 0 && rows_takes(R, m.N, m.K, x, m.s, m.b, out))
       return rows(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);
-    if (eagle_qmm_slab_swiglu_preferred(R, m.N, m.K))
-      return eagle_qmm_slab_swiglu_w4g64_f16(x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, 64, 4, st);
     if (R > 2 * EAGLE_MAX_M) return gemm(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);
     for (int r0 = 0; r0 < R; r0 += EAGLE_MAX_M) {
       const int rows = std::min(R - r0, EAGLE_MAX_M);
@@ -211,9 +188,8 @@ struct Pass {
                                      p(attn_ws), attn_ws_bytes, st);
   }
 
-  int slabs(const Tiles& t, const void* x, int steps) {
-    return eagle_qmm_slab_partial_tiled_w4g64(x, t.wt, t.sbt, static_cast<float*>(p(partial)), partial_bytes, T, t.N, t.K, steps,
-                                              t.small, st);
+  int partial_product(const Mat& m, const void* x) {
+    return eagle_qmm_rows_partial_w4g64(x, m.w, m.s, m.b, static_cast<float*>(p(partial)), partial_bytes, T, m.N, m.K, 64, 4, st);
   }
 
   int layer(int i, const void* next_norm) {
@@ -231,10 +207,10 @@ struct Pass {
                                           l.gu.K, 64, 4, 1, st));
       return eagle_qmm_small_w4g64_f16(p(act), nullptr, d.eps, md.w, md.s, md.b, md.bias, p(h), p(h), T, md.N, md.K, 64, 4, 0, st);
     }
-    if (tiled) {
-      EAGLE_TRY(slabs(l.tqkv, p(hn), slab_qkv));
-      EAGLE_TRY(eagle_rope_kv_append_slabs_f16(part, eagle_qmm_slab_count(d.D, slab_qkv), l.tqkv.bias, table, p(q_rot), keys[i],
-                                               values[i], len(0), T, d.H, d.G, d.hd, cap, st));
+    if (summed) {
+      EAGLE_TRY(partial_product(l.qkv, p(hn)));
+      EAGLE_TRY(eagle_rope_kv_append_slabs_f16(part, splits_qkv, l.qkv.bias, table, p(q_rot), keys[i], values[i], len(0), T, d.H, d.G,
+                                               d.hd, cap, st));
     } else if (fused) {
       EAGLE_TRY(product(l.qkv, p(hn), p(qkv)));
       const char* base = static_cast<const char*>(p(qkv));
@@ -255,14 +231,12 @@ struct Pass {
                                                  st));
     }
     EAGLE_TRY(attention(i));
-    if (tiled) {
-      EAGLE_TRY(slabs(l.to, p(attn), slab_o));
-      EAGLE_TRY(eagle_rmsnorm_slabs_f16(part, eagle_qmm_slab_count(d.H * d.hd, slab_o), p(h), l.norm2, d.eps, p(h), p(hn), T, d.D,
-                                        st));
-      EAGLE_TRY(eagle_qmm_slab_swiglu_tiled_w4g64_f16(p(hn), l.tgu.wt, l.tgu.sbt, l.tgu.bias, p(act), T, l.tgu.N, l.tgu.K,
-                                                      l.tgu.small, st));
-      EAGLE_TRY(slabs(l.tdown, p(act), slab_down));
-      return eagle_rmsnorm_slabs_f16(part, eagle_qmm_slab_count(d.I, slab_down), p(h), next_norm, d.eps, p(h), p(hn), T, d.D, st);
+    if (summed) {
+      EAGLE_TRY(partial_product(l.p[O], p(attn)));
+      EAGLE_TRY(eagle_rmsnorm_slabs_f16(part, splits_o, p(h), l.norm2, d.eps, p(h), p(hn), T, d.D, st));
+      EAGLE_TRY(swiglu(l.gu, p(hn), p(act)));
+      EAGLE_TRY(partial_product(l.p[DOWN], p(act)));
+      return eagle_rmsnorm_slabs_f16(part, splits_down, p(h), next_norm, d.eps, p(h), p(hn), T, d.D, st);
     }
     EAGLE_TRY(product(l.p[O], p(attn), p(o)));
     EAGLE_TRY(eagle_rmsnorm_f16(p(o), p(h), l.norm2, d.eps, p(h), p(hn), R, d.D, st));
@@ -281,13 +255,6 @@ struct Pass {
   // logits of `rows` rows from row0 on
   int head(int row0, int rows, void* out) {
     const char* x = static_cast<const char*>(p(hn)) + (size_t)row0 * d.D * 2;
-    if (d.thead.wt && rows <= 2 * EAGLE_MAX_M) {
-      for (int r0 = 0; r0 < rows; r0 += EAGLE_MAX_M)
-        EAGLE_TRY(eagle_qmm_rows_tiled_w4g64_f16(x + (size_t)r0 * d.D * 2, d.thead.wt, d.thead.sbt, nullptr,
-                                                 static_cast<char*>(out) + (size_t)r0 * d.V * 2, std::min(rows - r0, EAGLE_MAX_M),
-                                                 d.V, d.D, d.thead.small, st));
-      return EAGLE_OK;
-    }
     return matmul(like, x, d.head.w, d.head.s, d.head.b, d.head.bias, out, rows, d.V, d.D, st);
   }
 };
@@ -296,15 +263,15 @@ PyObject* str(const char* s) { return PyUnicode_InternFromString(s); }
 
 }  // namespace
 
-// decoder_new(ints, floats, emb, head, thead, norm, inv_freqs, layers, layer_list, cache_type) -> capsule
+// decoder_new(ints, floats, emb, head, norm, inv_freqs, layers, layer_list, cache_type) -> capsule
 //   ints: (D, I, H, G, hd, V, form); floats: (eps, rope_factor, scale); layers: per layer (seven projections, qkv, gu,
-//   four tiled copies, two norms)
+//   two norms)
 PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int v[7];
   float f[3];
-  if (n != 10 || !PyArg_ParseTuple(a[0], "iiiiiii", v, v + 1, v + 2, v + 3, v + 4, v + 5, v + 6) ||
-      !PyArg_ParseTuple(a[1], "fff", f, f + 1, f + 2) || !PyList_Check(a[7]) || !PyList_Check(a[8])) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "decoder_new takes ten arguments");
+  if (n != 9 || !PyArg_ParseTuple(a[0], "iiiiiii", v, v + 1, v + 2, v + 3, v + 4, v + 5, v + 6) ||
+      !PyArg_ParseTuple(a[1], "fff", f, f + 1, f + 2) || !PyList_Check(a[6]) || !PyList_Check(a[7])) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "decoder_new takes nine arguments");
     return nullptr;
   }
   std::unique_ptr<Decoder> d(new Decoder());
@@ -312,38 +279,34 @@ PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n) {
   d->eps = f[0]; d->rope_factor = f[1]; d->scale = f[2];
   d->emb = take_mat(d.get(), a[2]);
   d->head = take_mat(d.get(), a[3]);
-  d->norm = take(d.get(), a[5]).data_ptr();
-  const Py_ssize_t nl = PyList_GET_SIZE(a[7]);
+  d->norm = take(d.get(), a[4]).data_ptr();
+  const Py_ssize_t nl = PyList_GET_SIZE(a[6]);
   d->layers.resize(nl);
   for (Py_ssize_t i = 0; i < nl; ++i) {
-    PyObject* t = PyList_GET_ITEM(a[7], i);
-    if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != NPROJ + 8) throw Bad();
+    PyObject* t = PyList_GET_ITEM(a[6], i);
+    if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != NPROJ + 4) throw Bad();
     Layer& l = d->layers[i];
     for (int j = 0; j < NPROJ; ++j) l.p[j] = take_mat(d.get(), PyTuple_GET_ITEM(t, j));
-    l.norm1 = take(d.get(), PyTuple_GET_ITEM(t, NPROJ + 6)).data_ptr();
-    l.norm2 = take(d.get(), PyTuple_GET_ITEM(t, NPROJ + 7)).data_ptr();
+    l.norm1 = take(d.get(), PyTuple_GET_ITEM(t, NPROJ + 2)).data_ptr();
+    l.norm2 = take(d.get(), PyTuple_GET_ITEM(t, NPROJ + 3)).data_ptr();
   }
   d->n_source = d->kept.size();
   for (const at::Tensor& t : d->kept) d->versions.push_back(version_of(t));
-  d->thead = take_tiles(d.get(), a[4]);
-  d->inv_freqs = static_cast<const float*>(take(d.get(), a[6]).data_ptr());
+  d->inv_freqs = static_cast<const float*>(take(d.get(), a[5]).data_ptr());
   for (Py_ssize_t i = 0; i < nl; ++i) {
-    PyObject* t = PyList_GET_ITEM(a[7], i);
+    PyObject* t = PyList_GET_ITEM(a[6], i);
     Layer& l = d->layers[i];
     l.qkv = take_mat(d.get(), PyTuple_GET_ITEM(t, NPROJ));
     l.gu = take_mat(d.get(), PyTuple_GET_ITEM(t, NPROJ + 1));
-    l.tqkv = take_tiles(d.get(), PyTuple_GET_ITEM(t, NPROJ + 2));
-    l.to = take_tiles(d.get(), PyTuple_GET_ITEM(t, NPROJ + 3));
-    l.tgu = take_tiles(d.get(), PyTuple_GET_ITEM(t, NPROJ + 4));
-    l.tdown = take_tiles(d.get(), PyTuple_GET_ITEM(t, NPROJ + 5));
+    d->linear_bias |= l.p[O].bias || l.p[DOWN].bias;
   }
-  Py_INCREF(d->layer_list = a[8]);
-  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[8]); ++i) {
-    PyObject* o = PyList_GET_ITEM(a[8], i);
+  Py_INCREF(d->layer_list = a[7]);
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[7]); ++i) {
+    PyObject* o = PyList_GET_ITEM(a[7], i);
     Py_INCREF(o);
     d->layer_items.push_back(o);
   }
-  Py_INCREF(d->cache_type = a[9]);
+  Py_INCREF(d->cache_type = a[8]);
   PyObject* cap = PyCapsule_New(d.get(), "eagle.decoder", destroy);
   if (cap) d.release();
   return cap;

@@ -32,9 +32,10 @@ struct RowsArgs {
   const half_t* b;
   const half_t* bias;     // [N] or nullptr
   half_t* out;            // [M, N], [M, N / 2] with SwiGLU
-  float* partial;         // [gridDim.y, M, N] or nullptr
+  float* partial;         // [gridDim.y, pitch, N] or nullptr
   int M, N, K, swiglu;
   int both;               // scales and biases fit LDS together
+  int pitch;              // rows of x per split in `partial`
 };
 
 constexpr int ROWS_WAVES = 8;
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
     float v[8];
     sum8(m, at, v);
     if (a.partial) {
-      float* p = a.partial + ((long)blockIdx.y * M + m) * N + n;
+      float* p = a.partial + ((long)blockIdx.y * a.pitch + m) * N + n;
       *reinterpret_cast<float4_t*>(p) = float4_t{v[0], v[1], v[2], v[3]};
       *reinterpret_cast<float4_t*>(p + 4) = float4_t{v[4], v[5], v[6], v[7]};
       continue;
@@ -515,8 +516,10 @@ struct RowsPlan {
 // N 512 .. 152064, 8 .. 64 rows, every form, launches back to back over rotating weights.  A compute unit takes
 // its workgroups one after the other; each costs its start, its share of the weights and its x at the rates a
 // unit ingests them (40 and 72 GB/s), and 0.22 us per unit of four chunks, tile and 16 rows of x.  What the whole
-// grid reads counts a little, a split as much as its second launch and the partial sums.
-RowsPlan rows_find_plan(int M, int N, int K, bool may_split) {
+// grid reads counts a little, a split as much as its second launch and the partial sums (the sums alone where
+// the consumer of the product adds them).
+enum { ROWS_WHOLE = 0, ROWS_SPLIT = 1, ROWS_PARTIAL = 2 };
+RowsPlan rows_find_plan(int M, int N, int K, int mode) {
   const int units = ((K >> 7) + 3) / 4, mt = (M + 15) / 16;
   RowsPlan best = {-1, 1};
   double least = 1e30;
@@ -526,7 +529,7 @@ RowsPlan rows_find_plan(int M, int N, int K, bool may_split) {
     const int wrows = ROWS_WAVES / form.kp * form.rt * 16;
     const long blocks = (N + wrows - 1) / wrows;
     int last = 0;
-    for (int z = 1; z <= (may_split ? 32 : 1) && units / z >= form.kp; ++z) {
+    for (int z = 1; z <= (mode == ROWS_WHOLE ? 1 : 32) && units / z >= form.kp; ++z) {
       const int nu = ((units + z - 1) / z + form.kp - 1) / form.kp;
       if (nu == last) continue;                    // more workgroups, none of them shorter
       last = nu;
@@ -534,7 +537,7 @@ RowsPlan rows_find_plan(int M, int N, int K, bool may_split) {
       const double rounds = (double)((blocks * z + 255) / 256);
       const double w = wrows * (double)nu * form.kp * (512 * 0.5625 / 1e3), x = 16. * mt * nu * form.kp * (1024 / 1e3);
       double t = rounds * (1.03 + 0.0246 * w + 0.0138 * x + 0.221 * nu * form.rt * mt) + 0.0107 * (blocks * z / 256.) * (w + 0.5 * x);
-      if (z > 1) t += 2.93 + 0.49 * 4e-6 * z * M * N;
+      if (z > 1) t += (mode == ROWS_SPLIT ? 2.93 : 0.) + 0.49 * 4e-6 * z * M * N;
       if (t < least) {
         least = t;
         best = {f, z};
@@ -544,19 +547,19 @@ RowsPlan rows_find_plan(int M, int N, int K, bool may_split) {
   return best;
 }
 
-RowsPlan rows_plan(int M, int N, int K, bool may_split) {
+RowsPlan rows_plan(int M, int N, int K, int mode) {
   struct Known {
-    int M = 0, N = 0, K = 0, split = 0;
+    int M = 0, N = 0, K = 0, mode = 0;
     RowsPlan plan;
   };
   static thread_local Known known[64];
-  Known& k = known[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 9176u ^ (unsigned)may_split) >> 7 & 63];
-  if (k.M != M || k.N != N || k.K != K || k.split != (int)may_split) {
-    k.plan = rows_find_plan(M, N, K, may_split);
+  Known& k = known[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 9176u ^ (unsigned)mode << 9) >> 7 & 63];
+  if (k.M != M || k.N != N || k.K != K || k.mode != mode) {
+    k.plan = rows_find_plan(M, N, K, mode);
     k.M = M;
     k.N = N;
     k.K = K;
-    k.split = may_split;
+    k.mode = mode;
   }
   return k.plan;
 }
@@ -565,7 +568,7 @@ RowsPlan rows_plan(int M, int N, int K, bool may_split) {
 
 EAGLE_EXPORT int eagle_qmm_rows_supported(int M, int N, int K, int swiglu) {
   return M >= 1 && M <= 2 * EAGLE_MAX_M && N >= 16 && (N % (swiglu ? 32 : 8)) == 0 && K >= 128 && (K % 128) == 0 &&
-         (long)N * K < (1L << 33) && rows_plan(M, N, K, true).form >= 0;
+         (long)N * K < (1L << 33) && rows_plan(M, N, K, ROWS_SPLIT).form >= 0;
 }
 
 // Where it beats the other forms (us, against the streaming kernel unless noted).  33 rows on: everywhere (two
@@ -588,7 +591,7 @@ EAGLE_EXPORT int eagle_qmm_rows_preferred(int M, int N, int K) {
 
 EAGLE_EXPORT size_t eagle_qmm_rows_workspace_bytes(int M, int N, int K) {
   if (!eagle_qmm_rows_supported(M, N, K, 0)) return 0;
-  const RowsPlan p = rows_plan(M, N, K, true);
+  const RowsPlan p = rows_plan(M, N, K, ROWS_SPLIT);
   return p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
 }
 
@@ -603,7 +606,7 @@ EAGLE_EXPORT int eagle_qmm_rows_w4g64_f16(const void* x, const uint32_t* wq, con
     if (p && !eagle_aligned16(p)) return EAGLE_ERR_ALIGN;
   if ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 3u) return EAGLE_ERR_ALIGN;
   if (x == out) return EAGLE_ERR_UNSUPPORTED;          // other workgroups still read x
-  const RowsPlan p = rows_plan(M, N, K, workspace != nullptr);
+  const RowsPlan p = rows_plan(M, N, K, workspace ? ROWS_SPLIT : ROWS_WHOLE);
   if (p.form < 0) return EAGLE_ERR_SHAPE;
   if (p.splits > 1 && workspace_bytes < (size_t)p.splits * M * N * sizeof(float)) return EAGLE_ERR_WORKSPACE;
   RowsArgs a;
@@ -619,6 +622,7 @@ EAGLE_EXPORT int eagle_qmm_rows_w4g64_f16(const void* x, const uint32_t* wq, con
   a.K = K;
   a.swiglu = swiglu != 0;
   a.both = 0;
+  a.pitch = M;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int rc = rows_forms[p.form].launch(a, p.splits, st);
   if (rc != EAGLE_OK || p.splits == 1) return rc;
@@ -628,4 +632,31 @@ EAGLE_EXPORT int eagle_qmm_rows_w4g64_f16(const void* x, const uint32_t* wq, con
   else
     hipLaunchKernelGGL(rows_sum_kernel<false>, grid, dim3(256), 0, st, a.partial, p.splits, a.bias, a.out, M, N);
   return eagle_launch_status();
+}
+
+EAGLE_EXPORT int eagle_qmm_rows_partial_splits(int M, int N, int K) {
+  return eagle_qmm_rows_supported(M, N, K, 0) ? rows_plan(M, N, K, ROWS_PARTIAL).splits : 0;
+}
+
+EAGLE_EXPORT int eagle_qmm_rows_partial_w4g64(const void* x, const uint32_t* wq, const void* scales, const void* biases, float* partial,
+                                              size_t partial_bytes, int M, int N, int K, int group_size, int bits,
+                                              eagle_stream_t stream) {
+  if (!x || !wq || !scales || !biases || !partial) return EAGLE_ERR_NULL;
+  if (group_size != 64 || bits != 4) return EAGLE_ERR_UNSUPPORTED;
+  const int splits = eagle_qmm_rows_partial_splits(M, N, K);
+  if (splits < 1) return EAGLE_ERR_SHAPE;
+  if (!eagle_aligned16(x) || !eagle_aligned16(wq) || !eagle_aligned16(partial)) return EAGLE_ERR_ALIGN;
+  if ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 3u) return EAGLE_ERR_ALIGN;
+  RowsArgs a = {};
+  a.x = static_cast<const half_t*>(x);
+  a.w = wq;
+  a.s = static_cast<const half_t*>(scales);
+  a.b = static_cast<const half_t*>(biases);
+  a.partial = partial;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.pitch = eagle_slab_rows(M);
+  if (partial_bytes < (size_t)splits * a.pitch * N * sizeof(float)) return EAGLE_ERR_WORKSPACE;
+  return rows_forms[rows_plan(M, N, K, ROWS_PARTIAL).form].launch(a, splits, static_cast<hipStream_t>(stream));
 }

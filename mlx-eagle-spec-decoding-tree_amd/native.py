@@ -9,7 +9,7 @@ import torch
 from . import ops
 from .cache import KVCache
 
-PLAIN, FUSED, TILED = 0, 1, 2
+PLAIN, FUSED = 0, 1
 
 # Below this hidden size the layers keep one launch per projection on the checkpoint's own tensors: their
 # weights (under 4 MB per layer) are a few microseconds of reading either way, and no copy of them is made.
@@ -108,7 +108,7 @@ def _build(model):
     if at0._inv_freqs.numel() != hd // 2 or not at0._inv_freqs.is_cuda or at0._inv_freqs.dtype != torch.float32:
         return None
 
-    form, derived, thead = _derive(model, layers, head_w, shapes, I, D, V, H, G, hd)
+    form, derived = _derive(model, layers, shapes, I, D, H, G, hd)
     described = []
     for i, lins in enumerate(layers):
         layer = m.layers[i]
@@ -117,26 +117,47 @@ def _build(model):
         described.append((*leaves, *derived[i], layer.input_layernorm.weight, layer.post_attention_layernorm.weight))
     return ops._native().decoder_new(
         (D, I, H, G, hd, V, form), (args.rms_norm_eps, float(at0._scaling_factor), float(at0.scale)), emb_w, head_w,
-        thead, m.norm.weight, at0._inv_freqs, described, m.layers, KVCache)
+        m.norm.weight, at0._inv_freqs, described, m.layers, KVCache)
 
 
-def _derive(model, layers, head_w, shapes, I, D, V, H, G, hd):
-    """(form, per layer (qkv, gu, four tiled copies), tiled head)."""
-    from . import eagle
-    none = (None,) * 6
-    if D < FUSE_HIDDEN:
-        return PLAIN, [none] * len(layers), None
+def _derive(model, layers, shapes, I, D, H, G, hd):
+    """(form, per layer (q|k|v, gate|up))."""
+    none = (None, None)
     W = (H + 2 * G) * hd
-    products = {"qkv": (W, D), "o": shapes["o"], "down": shapes["down"]}
-    tiled = all(ops.slab_steps(32, n, k) and ops.tiled_supported(32, n, k) for n, k in products.values()) \
-        and ops.tiled_supported(32, 2 * I, D) and I % 16 == 0 \
-        and all(lins["o"].bias is None and lins["down"].bias is None for lins in layers)
-    if tiled:
-        sets = eagle.tile_model(model)
-        derived = [(None, None, *((t.wt, t.sbt, t.N, t.K, t.small, b) for t, b in entry)) for entry in sets]
-        th = eagle.tiled_head(model) if head_w[3] is None else None
-        return TILED, derived, None if th is None else (th.wt, th.sbt, th.N, th.K, th.small, None)
-    if not ops.swiglu_supported(32, I, D) or W % 16 or D % 16:
-        return PLAIN, [none] * len(layers), None
-    qkv_w, gu_w = eagle.fuse_projections(model, True)
-    return FUSED, [(qkv_w[i], gu_w[i], None, None, None, None) for i in range(len(layers))], None
+    if D < FUSE_HIDDEN or not ops.swiglu_supported(32, I, D) or W % 16 or D % 16:
+        return PLAIN, [none] * len(layers)
+    sources = [(t.data_ptr(), 0 if t.is_inference() else t._version) for lins in layers
+               for name in ("q", "k", "v", "gate", "up") for t in _leaf(lins[name]) if t is not None]
+    done = model.__dict__.get("_native_fused")
+    if done is None or done[0] != sources:
+        model.__dict__.pop("_native_fused", None)          # the old copies go before the new ones are made
+        done = (sources, [(_rows(lins["q"], lins["k"], lins["v"]), _gate_up(lins["gate"], lins["up"])) for lins in layers])
+        model.__dict__["_native_fused"] = done
+    return FUSED, done[1]
+
+
+def _biases(*lins):
+    if all(lin.bias is None for lin in lins):
+        return None
+    return [lin.bias if lin.bias is not None else torch.zeros(lin.weight.shape[0], dtype=torch.float16, device=lin.weight.device)
+            for lin in lins]
+
+
+def _rows(*lins):
+    """The matrices one below the other: a view where they already lie so, else a copy."""
+    def stack(parts):
+        first, at = parts[0], parts[0].data_ptr()
+        for t in parts:
+            if t.data_ptr() != at or t.untyped_storage().data_ptr() != first.untyped_storage().data_ptr():
+                return torch.cat(parts)
+            at += t.numel() * t.element_size()
+        return first.as_strided((sum(t.shape[0] for t in parts), *first.shape[1:]), first.stride())
+    biases = _biases(*lins)
+    return (*(stack([getattr(lin, k) for lin in lins]) for k in ("weight", "scales", "biases")),
+            None if biases is None else torch.cat(biases))
+
+
+def _gate_up(gate, up):
+    biases = _biases(gate, up)
+    return (*(ops.interleave_gate_up(getattr(gate, k), getattr(up, k)) for k in ("weight", "scales", "biases")),
+            None if biases is None else ops.interleave_gate_up(*biases))

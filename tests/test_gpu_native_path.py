@@ -42,10 +42,10 @@ def test_tree_layout_from_lists(dev, depth, total, root_dtype):
     assert got.is_contiguous() and np.array_equal(got.cpu().numpy(), want)
 
 
-FORMS = {       # one launch per projection; fused products (K not a multiple of 512); tiled copies
+FORMS = {       # one launch per projection; fused products, K not a multiple of 512; the same with it
     "plain": dict(hidden=256, inter=512, heads=4, kv_heads=2, head_dim=64),
     "fused": dict(hidden=896, inter=1152, heads=14, kv_heads=2, head_dim=64),
-    "tiled": dict(hidden=1024, inter=1536, heads=8, kv_heads=2, head_dim=128),
+    "wide": dict(hidden=1024, inter=1536, heads=8, kv_heads=2, head_dim=128),
 }
 
 
@@ -121,7 +121,7 @@ def test_native_causal_pass(dev, form, T, P):
 def test_native_decoder_follows_the_weights(dev):
     """Weights written to, exchanged layers and patched layers reach the next pass; arguments the native
     path does not take (no room for the padding of a chunk) still run."""
-    model, ids = small_model(dev, "tiled"), torch.arange(6, device=dev)[None]
+    model, ids = small_model(dev, "wide"), torch.arange(6, device=dev)[None]
     first = same_pass(model, ids, 3, 16)
     model.layers[1].mlp.down_proj.scales.mul_(0.5)
     second = same_pass(model, ids, 3, 16)
