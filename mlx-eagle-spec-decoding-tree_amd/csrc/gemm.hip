@@ -1,34 +1,31 @@
 // 4-bit group-64 quantised matmul for many rows (the prompt pass, mlx_eagle.py:522-533 through
 // the QuantizedLinear layers of mlx_llama.py): out[M,N] = fp16( x[M,K] . (s*q + b)[N,K]^T ).
 //
-// With hundreds of rows the product is bound by the matrix cores, not by the weight stream, so
-// this is a tiled GEMM: a workgroup of four waves side by side along the weight rows owns a
-// 64 x 128, 128 x 128 or 128 x 256 output block (x rows x weight rows), each wave all x rows of
-// the block as v_mfma_f32_32x32x16_f16 tiles (weights are the A operand: an accumulator lane
-// then holds one output row and four consecutive columns per register group).  Per 64-wide K
-// step (one quantisation group):
-//   * the x block goes through LDS (double buffered, one barrier per step), loaded one or two
-//     steps ahead into registers, a whole 128-byte row of the step per eight lanes;
-//   * every lane loads the 16 bytes (four packed words = 32 weights) of its weight row that its
-//     half of the MFMA K range needs, two steps ahead, and expands them in registers:
-//     a shift and v_and_or_b32 make the fp16 pair (16 + q_i, 16 + q_{i+4}); one packed fp16
-//     fma with (s, b - 16 s) gives the weights in fp16, as the reference kernels hold them.
-//     That yields the eight weights of a word in the order q0 q4 q1 q5 q2 q6 q3 q7; x is stored
-//     to LDS in the same order within every group of eight, so both MFMA operands agree on
-//     which K index sits where.  The expanded word j of a step is replaced by the next step's
-//     as soon as this step's matrix instructions have read it (one register set, which lets
-//     two workgroups share a compute unit with the 128 x 256 block);
+// With hundreds of rows the product is bound by the matrix cores, not by the weight stream, so this is a tiled
+// GEMM: a workgroup of four waves side by side along the weight rows owns a block of 64 x 128 to 256 x 256 (x rows x
+// weight rows), each wave all x rows of the block as v_mfma_f32_32x32x16_f16 tiles (weights are the A operand: an
+// accumulator lane then holds one output row and four consecutive columns per register group).  Per 64-wide K step
+// (one quantisation group):
+//   * the x block goes through LDS, loaded ahead into registers, a whole 128-byte row of the step per eight lanes;
+//   * every lane loads the 16 bytes (four packed words = 32 weights) of its weight row that its half of the MFMA K
+//     range needs, some steps ahead, and expands them in registers to the weights in fp16, as the reference kernels
+//     hold them; x is stored to LDS in the order in which the expansion leaves the eight weights of a word;
 //   * the output tile of a wave leaves through LDS as whole rows.
-// Measured for 512 x 28672 x 4096 (s_memtime / s_memrealtime inside the kernel): the core clock
-// is 1.55 - 1.85 GHz while this kernel runs (a loop of matrix instructions alone sustains 2.1 - 2.4
-// PFLOP/s on the same box), a workgroup alone on a compute unit needs 1900 clocks per step for
-// 1024 clocks of matrix instructions, two together 1330 each; 448 workgroups on 512 places leave
-// a quarter of the compute units with one workgroup, which ends 25 % before the others.  Blocks
-// of 128 x 512 and 256 x 256 (half the LDS reads, or half the expansions, per matrix instruction;
-// 512 registers, one workgroup per compute unit) were 3 - 5 % faster on that shape and half as
-// fast on the narrow ones, and are not built.  The narrow shapes (N = 4096: one 64 x 128 block per
-// compute unit) run two groups of four waves per workgroup, each over half of K (+5 %); loading
-// the packed weights by whole 128-byte lines (timing only, results wrong) is worth 0 - 7 %.
+//
+// The deep loop (DEEP, K a multiple of 256) has a compute unit's registers for one or two workgroups and hides
+// everything under the matrix instructions of one wave: three x buffers, so that the operands of the next word are
+// read across the barrier of a step; operands and expanded weights of the next word made while this word's matrix
+// instructions run, the mix pinned with scheduling groups; a third of the x of the step after next stored, and its
+// registers requested again, in each of the first three words.  Nibbles through the fp8 conversion, one rounding.
+// The shallow loop (other K) has two x buffers and leaves the mix to two workgroups per compute unit.
+//
+// What bounds it: the power budget.  The clock is 2.2 GHz for a short launch and falls to 1.4 - 1.6 GHz under
+// sustained load (counters: 51 % of the cycles in matrix instructions at 1.47 GHz for 2048 x 37888 x 3584 with the
+// shallow loop; a library's fp16 product 89 % at 1.33 GHz), so fewer expansions and LDS reads per matrix instruction
+// are worth more than their cycles: 256 x 256 blocks expand a weight once for 256 rows.  Shallow -> deep, us:
+// 2048 x 37888 x 3584 582 -> 498, 2048 x 3584 x 18944 302 -> 256, 512 x 14336 x 4096 69 -> 64; error against unrounded
+// weights 1.2e-3 -> 3e-4.  (x stored in one piece per step instead of three: 311 against 299 us for 2048 x 18944 x 3584;
+// 128 x 512 blocks, which halve the LDS reads instead: 307 against 277.)
 // fp32 accumulation, one fp16 rounding, optional fp16 bias added after the rounding.
 #include "common.h"
 
@@ -37,7 +34,6 @@
 namespace {
 
 constexpr int BK = 64;
-constexpr long GEMM_SPLIT_WGS = 384;        // two K groups per workgroup up to this many workgroups
 constexpr long NUM_CU = 256;
 constexpr int XS = BK + 8;                  // LDS row stride in halves (144 bytes: conflict-free 16-byte reads)
 
@@ -114,8 +110,26 @@ __device__ inline half8_t dequant_word_sub(uint32_t w, half2_t s20, half2_t b2) 
   return o;
 }
 
-// MT = 32-row x tiles per wave: 2 (128-row blocks) or 4 (256-row blocks: twice the matrix work
-// per expanded weight and per byte read from LDS).
+// Through the fp8 conversion: a byte that holds a nibble is q * 2^-9 exactly when read as OCP e4m3, so two
+// conversions per four nibbles give fp16 q, and one packed fma fp16(s*q + b) with a single rounding, any scale: as
+// many instructions as the forms above, no offset to prepare.  Order q0 q2 q4 q6 q1 q3 q5 q7.
+__device__ inline half8_t permute8_fp8(half8_t v) { return half8_t{v[0], v[2], v[4], v[6], v[1], v[3], v[5], v[7]}; }
+__device__ inline half8_t dequant_word_fp8(uint32_t w, half2_t s2, half2_t b2) {
+  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
+  const half2_t c[4] = {__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, false),
+                        __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, true),
+                        __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, false),
+                        __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, true)};
+  half8_t o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const half2_t v = __builtin_elementwise_fma(c[i], s2, b2);
+    o[2 * i] = v[0];
+    o[2 * i + 1] = v[1];
+  }
+  return o;
+}
+
 template <int E>
 struct StepIndex {
   static constexpr int value = E;
@@ -134,8 +148,8 @@ struct StepIndex {
 // result is silu(g) * u, [M, N / 2].
 // SPLITK: gridDim.z workgroups share an output block, each over its own part of K, and leave fp32 partial
 // sums in `partial` [z][M][N] for gemm_sum_kernel.
-template <int NTW, int MT, int SBW, int KGRP = 1, bool SWI = false, bool SPLITK = false>
-__global__ __launch_bounds__(256 * KGRP, (KGRP == 1 ? 2 : 1)) void qmm_gemm_w4g64_kernel(
+template <int NTW, int MT, int SBW, int KGRP = 1, bool SWI = false, bool SPLITK = false, bool DEEP = false>
+__global__ __launch_bounds__(256 * KGRP, (KGRP == 1 && !DEEP ? 2 : 1)) void qmm_gemm_w4g64_kernel(
     const half_t* __restrict__ x, const uint32_t* __restrict__ w, const half_t* __restrict__ s,
     const half_t* __restrict__ b, const half_t* __restrict__ bias, half_t* __restrict__ out, int M,
     int N, int K, float* __restrict__ partial) {
@@ -193,11 +207,11 @@ __global__ __launch_bounds__(256 * KGRP, (KGRP == 1 ? 2 : 1)) void qmm_gemm_w4g6
 
   // x is requested one step ahead, or two with the small blocks: their few matrix instructions
   // per step do not cover the latency of that load, and a step cannot be shorter than the lead
-  constexpr int XD = MT <= 2 ? 2 : 1;
+  constexpr int XD = DEEP || MT <= 2 ? 2 : 1;
   half8_t xreg[XD][PP];
   // packed weights: two steps in flight, four with the small blocks (where the unrolled loop
   // makes the register set of a step a constant), for the same reason
-  constexpr int WD = (MT <= 2 && SBW >= 4) ? 4 : 2;
+  constexpr int WD = ((DEEP ? MT <= 4 : MT <= 2) && SBW >= 4) ? 4 : 2;
   uint4_t wreg[WD][NTW];
   constexpr bool SBV = SBW > 1;
   typedef half_t sbvec_t __attribute__((ext_vector_type(SBV ? SBW : 2)));
@@ -252,6 +266,103 @@ __global__ __launch_bounds__(256 * KGRP, (KGRP == 1 ? 2 : 1)) void qmm_gemm_w4g6
       for (int i = 0; i < 16; ++i) acc[nt][mt][i] = 0.f;
 
   const int chunks = steps / SBW;
+  if constexpr (DEEP) {
+    constexpr int BUF = BMT * XS;            // halves per x buffer; three of them
+    half8_t bv[2][MT], av[2][NTW];           // operands of this word and of the next
+    auto read_x = [&](half8_t* to, const half_t* buf, int j) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) to[mt] = *reinterpret_cast<const half8_t*>(buf + (mt * 32 + ql) * XS + hb * 32 + j * 8);
+    };
+    auto write_x = [&](half_t* buf, int set, int from, int to) {
+#pragma unroll
+      for (int g = from; g < to; ++g) *reinterpret_cast<half8_t*>(buf + (xr + 32 * g) * XS + xc * 8) = permute8_fp8(xreg[set][g]);
+    };
+    auto load_x = [&](int ks, int set, int from, int to) {
+#pragma unroll
+      for (int g = from; g < to; ++g) xreg[set][g] = *reinterpret_cast<const half8_t*>(x + (xo[g] + (uint32_t)(ks * BK)));
+    };
+    auto expand_word = [&](half8_t* to, int j, int e) {
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt) {
+        const half_t sc = s8[e / SBW][nt][e % SBW], bi = b8[e / SBW][nt][e % SBW];
+        to[nt] = dequant_word_fp8(wreg[e % WD][nt][j], half2_t{sc, sc}, half2_t{bi, bi});
+      }
+    };
+    auto last = [&](int k) { return k < steps ? k : steps - 1; };
+    fetch_x(0, 0);
+    fetch_x(last(1), 1);
+    fetch_sb(0, 0);
+    fetch_sb(chunks > 1 ? 1 : 0, 1);
+#pragma unroll
+    for (int i = 0; i < WD; ++i) fetch_w(last(i), i);
+    write_x(xs_all, 0, 0, PP);
+    write_x(xs_all + BUF, 1, 0, PP);
+    fetch_x(last(2), 0);
+    fetch_x(last(3), 1);
+    __syncthreads();
+    half_t *cur = xs_all, *nxt = xs_all + BUF, *fut = xs_all + 2 * BUF;
+    read_x(bv[0], cur, 0);
+    expand_word(av[0], 0, 0);
+    auto step = [&](int ks, auto E) {
+      constexpr int e = decltype(E)::value;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (j == 3) fetch_w(last(ks + WD), e % WD);
+        read_x(bv[(j + 1) & 1], j < 3 ? cur : nxt, (j + 1) & 3);
+        // x of the step after next to LDS, a third in each of the first three words, and its registers
+        // requested again
+        constexpr int cut[5] = {0, (PP + 2) / 3, (2 * PP + 2) / 3, PP, PP};
+        write_x(fut, e & 1, cut[j], cut[j + 1]);
+        load_x(last(ks + 4), e & 1, cut[j], cut[j + 1]);
+        expand_word(av[(j + 1) & 1], (j + 1) & 3, j < 3 ? e : e + 1);
+#pragma unroll
+        for (int nt = 0; nt < NTW; ++nt)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+            acc[nt][mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[j & 1][nt], bv[j & 1][mt], acc[nt][mt], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < NTW * MT; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // a matrix instruction
+          if (i < MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, MT > 4 ? 2 : 3, 0);
+          if (i >= NTW * MT - 1 - (cut[j + 1] - cut[j]) && i < NTW * MT - 1) {
+            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (e == SBW - 1) {
+#pragma unroll
+        for (int nt = 0; nt < NTW; ++nt) {
+          s8[0][nt] = s8[1][nt];
+          b8[0][nt] = b8[1][nt];
+        }
+        const int c = ks / SBW + 2;
+        fetch_sb(c < chunks ? c : chunks - 1, 1);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      half_t* const t = cur;
+      cur = nxt;
+      nxt = fut;
+      fut = t;
+    };
+    for (int ks = 0; ks < steps; ks += SBW) {
+      step(ks, StepIndex<0>{});
+      step(ks + 1, StepIndex<1>{});
+      if constexpr (SBW >= 4) {
+        step(ks + 2, StepIndex<2>{});
+        step(ks + 3, StepIndex<3>{});
+      }
+      if constexpr (SBW == 8) {
+        step(ks + 4, StepIndex<4>{});
+        step(ks + 5, StepIndex<5>{});
+        step(ks + 6, StepIndex<6>{});
+        step(ks + 7, StepIndex<7>{});
+      }
+    }
+  } else {
   fetch_x(0, 0);
   if (XD == 2) fetch_x(steps > 1 ? 1 : 0, 1);
 #pragma unroll
@@ -335,6 +446,8 @@ __global__ __launch_bounds__(256 * KGRP, (KGRP == 1 ? 2 : 1)) void qmm_gemm_w4g6
       body(ks + 1, StepIndex<1>{});
     }
     if (ks < steps) body(ks, StepIndex<0>{});
+  }
+
   }
 
   // Accumulator register i of a lane: weight row (output column) 8*(i/4) + 4*hb + i%4 of the
@@ -504,13 +617,13 @@ __global__ __launch_bounds__(256) void gemm_sum_kernel(const float* __restrict__
   }
 }
 
-template <int NTW, int MT, int SBW, int KGRP = 1, bool SWI = false, bool SPLITK = false>
+template <int NTW, int MT, int SBW, int KGRP = 1, bool SWI = false, bool SPLITK = false, bool DEEP = false>
 int launch_gemm(const half_t* x, const uint32_t* w, const half_t* s, const half_t* b, const half_t* bias,
                 half_t* out, int M, int N, int K, hipStream_t st, int splits = 1, float* partial = nullptr) {
   constexpr int BMT = 32 * MT;
   constexpr int BN = 128 * NTW;
   static_assert(256 % BMT == 0 && BMT >= 32, "block load mapping");
-  const size_t lds_x = KGRP * 2 * (size_t)BMT * XS * sizeof(half_t);
+  const size_t lds_x = KGRP * (DEEP ? 3 : 2) * (size_t)BMT * XS * sizeof(half_t);
   const size_t lds_out = 4 * (size_t)BMT * (64 * NTW + 16);         // the output tiles of the four waves
   const size_t lds_red = KGRP > 1 ? 4 * (size_t)NTW * MT * 4 * 64 * sizeof(float4_t) : 0;
   size_t lds = lds_x > lds_out ? lds_x : lds_out;
@@ -519,13 +632,13 @@ int launch_gemm(const half_t* x, const uint32_t* w, const half_t* s, const half_
   lds = lds > lds_part ? lds : lds_part;
   static bool configured = false;
   if (!configured) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&qmm_gemm_w4g64_kernel<NTW, MT, SBW, KGRP, SWI, SPLITK>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&qmm_gemm_w4g64_kernel<NTW, MT, SBW, KGRP, SWI, SPLITK, DEEP>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return EAGLE_ERR_HIP;
     configured = true;
   }
   const dim3 grid((N + BN - 1) / BN, (M + BMT - 1) / BMT, splits);
-  hipLaunchKernelGGL((qmm_gemm_w4g64_kernel<NTW, MT, SBW, KGRP, SWI, SPLITK>), grid, dim3(256 * KGRP), lds, st, x, w, s, b,
+  hipLaunchKernelGGL((qmm_gemm_w4g64_kernel<NTW, MT, SBW, KGRP, SWI, SPLITK, DEEP>), grid, dim3(256 * KGRP), lds, st, x, w, s, b,
                      bias, out, M, N, K, partial);
   return eagle_launch_status();
 }
@@ -1279,7 +1392,7 @@ int launch_rows_tiled(const half_t* x, const uint32_t* w, const half_t* s, const
 // The tiled layout of a weight matrix (see TL above) from row-major parts: thread = one 16-byte
 // piece of the output.  The parts are stacked (q, k and v as one matrix) or, `interleave`, two of
 // them alternate in 16-row tiles (gate and up), so that the stacked or interleaved row-major matrix
-// is never written: 8 instead of 16 ms for the layers of a 7B model.  max_scale (or null): the largest |scale|
+// is never written (58 us per matrix of a 7B model on average, 1.3 TB/s).  max_scale (or null): the largest |scale|
 // met so far, as the bits of a non-negative float.
 struct TileParts {
   const uint32_t* w[EAGLE_MAX_TILE_PARTS];
@@ -1724,25 +1837,41 @@ EAGLE_EXPORT int eagle_qmm_rows_tiled_w4g64_f16(const void* x, const uint32_t* w
 
 // Block shape and K splits of the many-row product.
 //
-// Block: 64 x 128, 128 x 128 or 128 x 256 (x rows x weight rows).  The compute unit with the
-// most workgroups sets the time, and a workgroup's work goes with its block (bigger
-// blocks do a little less per output: 0.55 / 1 / 1.85); the estimate below reproduced the
-// faster choice for every projection shape of the 7B / 8B / 0.5B models at 512 and 2048 rows.
+// Splits: a grid of a few dozen workgroups walks a long K one step after the other whatever the grid, so several
+// workgroups share an output block, each over a part of K, and a second launch adds their fp32 sums.
 //
-// Splits: a grid of a few dozen workgroups walks a long K one step after the other (0.4 - 1.1 us a step
-// whatever the grid), so several workgroups share an output block, each over a part of K, and a second
-// launch adds their fp32 sums.  `gemm_cost` is fitted to 900 forced launches (65 .. 2048 rows, K 896 .. 18944,
-// N 896 .. 37888): us per K step of a workgroup alone on its compute unit and of two that share one, 3.5 us
-// and the traffic of the partial sums for the second launch.  A split is taken where it is estimated at least
-// a tenth faster.  Measured, us without and with: 65 x 3584 x 18944 104 / 32, 128 x 896 x 4864 27 / 13,
-// 512 x 2896 x 9344 71 / 52, 128 x 3584 x 3584 20 / 16; 512 x 14336 x 4096 stays whole (66).
+// K a multiple of 256: the deep loop in blocks of 64 x 128, 128 x 128, 128 x 256 or 256 x 256 (x rows x weight rows),
+// or the two K groups of the shallow loop where they fit.  The form and the splits with the least predicted time,
+// from a model fitted to 1300 forced launches (65 .. 2048 rows, K 1024 .. 18944, N 512 .. 37888): us per launch, per
+// round of workgroups, per K step of a workgroup alone on its compute unit and of two together (the two small
+// blocks; the large ones have a unit to themselves), per step as the units fill (they share a power budget: the
+// clock falls from 2.2 to 1.4 GHz); a split costs 3.3 us and 0.2 us per MB of sums.  Choosing by it instead of by trial
+// loses 1 % on average, at most 13 % (K = 8192 over 1024 rows).
+// Other K (scales in fetches of one or two groups): the shallow loop by the older model below.
 struct GemmPlan {
-  int block;      // 0: 64 x 128, 1: 128 x 128, 2: 128 x 256
+  int block;      // 0: 64 x 128, 1: 128 x 128, 2: 128 x 256, 3: 256 x 256
   int kgrp;       // K groups inside a workgroup
   int splits;     // workgroups along K
   int sbw;        // scale groups per fetch
 };
+constexpr int GEMM_NTW[4] = {1, 1, 2, 2}, GEMM_MT[4] = {2, 4, 4, 8};
 
+static double gemm_deep_cost(int block, long wgs, double steps) {
+  static const double launch[4] = {2.65, 0., 4.25, 7.98}, round[4] = {1.03, 4.66, 1.91, 1.54}, alone[4] = {0.274, 0.407, 0.513, 0.912},
+                      pair[2] = {0.603, 0.957}, fill[4] = {0.105, 0.165, 0.406, 0.682};
+  const double c = (double)wgs / NUM_CU;
+  if (c <= 1.) return launch[block] + round[block] + steps * (alone[block] + c * fill[block]);
+  if (block < 2) {
+    const long full = (long)c / 2;
+    const double rest = c - 2. * full;
+    const double pairs = full + (rest > 1. ? 1 : 0), single = rest > 0. && rest <= 1. ? 1 : 0;
+    return launch[block] + (pairs + single) * round[block] + steps * (single * alone[block] + pairs * pair[block]);
+  }
+  const double rounds = ceil(c), busy = block == 2 ? 0.455 : 0.822;
+  return launch[block] + rounds * round[block] + steps * (rounds * alone[block] + c * busy);
+}
+
+// us per K step of the shallow loop, a workgroup alone and two that share a compute unit (fitted likewise)
 static double gemm_cost(int block, long wgs, double steps) {
   static const double alone[3] = {0.40, 0.64, 1.08}, pair[3] = {0.68, 1.14, 2.05};
   const double c = (double)wgs / NUM_CU;
@@ -1753,14 +1882,7 @@ static double gemm_cost(int block, long wgs, double steps) {
 }
 
 static GemmPlan gemm_plan(int M, int N, int K, const void* scales, const void* biases, bool swiglu, bool may_split) {
-  auto most = [](long blocks) { return (double)((blocks + NUM_CU - 1) / NUM_CU); };
-  const long nb = (N + 127) / 128, wgs_of[3] = {nb * ((M + 63) / 64), nb * ((M + 127) / 128),
-                                                ((N + 255) / 256) * (long)((M + 127) / 128)};
-  const double cost_norm = most(wgs_of[1]);
-  const double cost_small = M > 64 && !swiglu ? 0.55 * most(wgs_of[0]) : 1e30;
-  const double cost_big = 1.85 * most(wgs_of[2]);
   GemmPlan p;
-  p.block = cost_small < cost_norm && cost_small <= cost_big ? 0 : cost_big < cost_norm ? 2 : 1;
   // scales and biases per fetch: as many groups as divide a row and as the base addresses are
   // aligned for
   const uintptr_t sb_addr = reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases);
@@ -1768,31 +1890,39 @@ static GemmPlan gemm_plan(int M, int N, int K, const void* scales, const void* b
           : (K % 256) == 0 && (sb_addr & 7u) == 0 ? 4
           : (K % 128) == 0 && (sb_addr & 3u) == 0 ? 2
                                                   : 1;
-  // (the SwiGLU epilogue of the 128 x 256 block is built for eight groups only)
-  if (swiglu && p.block == 2 && p.sbw != 8) p.block = 1;
-  // two K groups per workgroup where the grid would leave a compute unit with one workgroup
-  p.kgrp = !swiglu && p.sbw == 8 && (K % 1024) == 0 && p.block != 2 && wgs_of[p.block] <= GEMM_SPLIT_WGS ? 2 : 1;
-  p.splits = 1;
-  if (!may_split) return p;
+  static const int tried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
   const double steps = K / 64;
-  double best = p.kgrp == 2 ? 4. + steps / 2 * (p.block == 0 ? 0.70 : 1.15) * (wgs_of[p.block] > NUM_CU ? 2 : 1)
-                            : gemm_cost(p.block, wgs_of[p.block], steps);
-  best *= 0.9;
-  static const int tried[] = {2, 3, 4, 6, 8, 12, 16, 24};
-  for (int b = 0; b < 3; ++b)
-    for (int z : tried) {
-      const int unit = b == 2 && p.sbw == 8 ? 4 : p.sbw;     // steps are dealt in fetches of scales
-      const int units = K / 64 / unit;
-      if (z > units || wgs_of[b] * z > 6 * NUM_CU) continue;
-      const double c = gemm_cost(b, wgs_of[b] * z, (double)((units + z - 1) / z * unit)) + 3.5 +
-                       8e-6 / 4.5 * z * (double)M * N;
-      if (c < best) {
-        best = c;
-        p.block = b;
-        p.splits = z;
-        p.kgrp = 1;
-      }
+  const int units = K / 64 / p.sbw;                    // steps are dealt in fetches of scales
+  auto blocks_of = [&](int b) {
+    return (long)((N + 128 * GEMM_NTW[b] - 1) / (128 * GEMM_NTW[b])) * ((M + 32 * GEMM_MT[b] - 1) / (32 * GEMM_MT[b]));
+  };
+  double best = 1e30;
+  auto consider = [&](int block, int kgrp, int splits, double cost) {
+    if (splits > 1) cost += 3.3 + 0.2 * 4e-6 * splits * (double)M * N;
+    if (cost < best) {
+      best = cost;
+      p.block = block;
+      p.kgrp = kgrp;
+      p.splits = splits;
     }
+  };
+  const bool deep = p.sbw >= 4;
+  if (deep && p.sbw == 8 && (K % 1024) == 0 && !swiglu)
+    for (int b = 0; b < 2; ++b) {
+      const double c = (double)blocks_of(b) / NUM_CU;
+      const double fixed = b == 0 ? 2.68 : 2.99, round = b == 0 ? 1.79 : 2.13, alone = b == 0 ? 0.442 : 0.755;
+      const double fill = b == 0 ? (c <= 1. ? 0.233 : 0.243) : (c <= 1. ? 0.404 : 0.446);
+      consider(b, 2, 1, fixed + ceil(c) * round + steps / 2 * (ceil(c) * alone + c * fill));
+    }
+  for (int b = 0; b < (deep ? 4 : swiglu ? 2 : 3); ++b) {
+    if (!deep && swiglu && b == 0 && !may_split) continue;       // (the shallow SwiGLU epilogue: 128 x 128 blocks)
+    for (int z : tried) {
+      if (z > 1 && (!may_split || z > units || blocks_of(b) * z > 6 * NUM_CU)) break;
+      if (z == 1 && !deep && swiglu && b == 0) continue;
+      const double part = (double)((units + z - 1) / z * p.sbw);
+      consider(b, 1, z, deep ? gemm_deep_cost(b, blocks_of(b) * z, part) : gemm_cost(b, blocks_of(b) * z, part));
+    }
+  }
   return p;
 }
 
@@ -1829,18 +1959,28 @@ static int gemm_dispatch(const void* x, const uint32_t* wq, const void* scales, 
   half_t* oh = static_cast<half_t*>(out);
   GemmPlan p = gemm_plan(M, N, K, scales, biases, swiglu, workspace != nullptr);
   if (p.splits > 1 && workspace_bytes < (size_t)p.splits * M * N * sizeof(float)) return EAGLE_ERR_WORKSPACE;
-  if (p.splits > 1) {
-    float* part = static_cast<float*>(workspace);
-    int rc = EAGLE_ERR_UNSUPPORTED;
-#define EAGLE_GEMM_SPLIT(NTW, MT)                                                                                       \
-  switch (p.sbw) {                                                                                                      \
-    case 8: rc = launch_gemm<NTW, MT, (NTW == 2 ? 4 : 8), 1, false, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break; \
-    case 4: rc = launch_gemm<NTW, MT, 4, 1, false, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break;   \
-    case 2: rc = launch_gemm<NTW, MT, 2, 1, false, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break;   \
-    default: rc = launch_gemm<NTW, MT, 1, 1, false, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break;  \
+  float* part = static_cast<float*>(workspace);
+  int rc = EAGLE_ERR_UNSUPPORTED;
+#define EAGLE_GEMM_DEEP(SBW, SWI, SPLIT)                                                                                \
+  switch (p.block) {                                                                                                    \
+    case 0: rc = launch_gemm<1, 2, SBW, 1, SWI, SPLIT, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break; \
+    case 1: rc = launch_gemm<1, 4, SBW, 1, SWI, SPLIT, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break; \
+    case 2: rc = launch_gemm<2, 4, SBW, 1, SWI, SPLIT, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break; \
+    default: rc = launch_gemm<2, 8, SBW, 1, SWI, SPLIT, true>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break; \
   }
-    if (p.block == 0) { EAGLE_GEMM_SPLIT(1, 2) } else if (p.block == 1) { EAGLE_GEMM_SPLIT(1, 4) } else { EAGLE_GEMM_SPLIT(2, 4) }
-#undef EAGLE_GEMM_SPLIT
+#define EAGLE_GEMM_SHALLOW(SBW, SPLIT)                                                                                  \
+  switch (p.block) {                                                                                                    \
+    case 0: rc = launch_gemm<1, 2, SBW, 1, false, SPLIT>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break;  \
+    case 1: rc = launch_gemm<1, 4, SBW, 1, false, SPLIT>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break;  \
+    default: rc = launch_gemm<2, 4, SBW, 1, false, SPLIT>(xh, wq, sh, bh, bi, oh, M, N, K, st, p.splits, part); break; \
+  }
+  if (p.splits > 1) {
+    switch (p.sbw) {
+      case 8: EAGLE_GEMM_DEEP(8, false, true) break;
+      case 4: EAGLE_GEMM_DEEP(4, false, true) break;
+      case 2: EAGLE_GEMM_SHALLOW(2, true) break;
+      default: EAGLE_GEMM_SHALLOW(1, true) break;
+    }
     if (rc != EAGLE_OK) return rc;
     const long total = (long)M * ((swiglu ? N / 2 : N) / 8);
     const dim3 grid((unsigned)((total + 255) / 256));
@@ -1851,33 +1991,26 @@ static int gemm_dispatch(const void* x, const uint32_t* wq, const void* scales, 
     return eagle_launch_status();
   }
   if (swiglu) {
-    // the wide gate|up matrix: the 128 x 256 block where it pays, else 128 x 128
     switch (p.sbw) {
-      case 8: return p.block == 2 ? launch_gemm<2, 4, 4, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st)
-                                  : launch_gemm<1, 4, 8, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st);
-      case 4: return launch_gemm<1, 4, 4, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st);
+      case 8: EAGLE_GEMM_DEEP(8, true, false) break;
+      case 4: EAGLE_GEMM_DEEP(4, true, false) break;
       case 2: return launch_gemm<1, 4, 2, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st);
       default: return launch_gemm<1, 4, 1, 1, true>(xh, wq, sh, bh, bi, oh, M, N, K, st);
     }
-  }
-#define EAGLE_GEMM_SHAPE(NTW, MT)                                                              \
-  switch (p.sbw) {                                                                             \
-    case 8: return launch_gemm<NTW, MT, 8>(xh, wq, sh, bh, bi, oh, M, N, K, st);               \
-    case 4: return launch_gemm<NTW, MT, 4>(xh, wq, sh, bh, bi, oh, M, N, K, st);               \
-    case 2: return launch_gemm<NTW, MT, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st);               \
-    default: return launch_gemm<NTW, MT, 1>(xh, wq, sh, bh, bi, oh, M, N, K, st);              \
+    return rc;
   }
   if (p.kgrp == 2)
     return p.block == 0 ? launch_gemm<1, 2, 8, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st)
                         : launch_gemm<1, 4, 8, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st);
-  if (p.block == 0) { EAGLE_GEMM_SHAPE(1, 2) }
-  if (p.block == 1) { EAGLE_GEMM_SHAPE(1, 4) }
-  // (the 128 x 256 block takes its scales four groups per fetch at most: with eight it spills
-  // twenty registers and is no faster, 149-153 us against 143-152 us for 512 x 28672 x 4096)
-  if (p.sbw >= 4) return launch_gemm<2, 4, 4>(xh, wq, sh, bh, bi, oh, M, N, K, st);
-  return p.sbw == 2 ? launch_gemm<2, 4, 2>(xh, wq, sh, bh, bi, oh, M, N, K, st)
-                    : launch_gemm<2, 4, 1>(xh, wq, sh, bh, bi, oh, M, N, K, st);
-#undef EAGLE_GEMM_SHAPE
+  switch (p.sbw) {
+    case 8: EAGLE_GEMM_DEEP(8, false, false) break;
+    case 4: EAGLE_GEMM_DEEP(4, false, false) break;
+    case 2: EAGLE_GEMM_SHALLOW(2, false) break;
+    default: EAGLE_GEMM_SHALLOW(1, false) break;
+  }
+  return rc;
+#undef EAGLE_GEMM_DEEP
+#undef EAGLE_GEMM_SHALLOW
 }
 
 EAGLE_EXPORT int eagle_qmm_gemm_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
