@@ -14,34 +14,63 @@ constexpr int TOPK_MAX = 8;          // k of the expansion (candidates per node)
 constexpr int CHUNK = 4096;          // logits per workgroup
 constexpr int THREADS = 256;
 
-struct Cand {
-  float v;
-  int i;
-};
-__device__ inline Cand better(Cand a, Cand b) {
-  return (b.v > a.v || (b.v == a.v && b.i < a.i)) ? b : a;
+// Reductions over a wave without the LDS shuffles: halves and rows of sixteen lanes by half-wave swaps, then rotations
+// within a row.  Every lane gets the result; sums are formed in the order of a butterfly from 32 lanes down.
+template <int ROR>
+__device__ inline int row_ror(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x120 + ROR, 0xf, 0xf, false); }
+template <typename Op>
+__device__ inline uint32_t wave_reduce(uint32_t v, Op op) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  v = op(a[0], a[1]);
+  const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = op(b[0], b[1]);
+  v = op(v, (uint32_t)row_ror<8>((int)v));
+  v = op(v, (uint32_t)row_ror<4>((int)v));
+  v = op(v, (uint32_t)row_ror<2>((int)v));
+  return op(v, (uint32_t)row_ror<1>((int)v));
 }
-__device__ inline Cand wave_best(Cand a) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    Cand b;
-    b.v = __shfl_xor(a.v, o, 64);
-    b.i = __shfl_xor(a.i, o, 64);
-    a = better(a, b);
-  }
-  return a;
+__device__ inline float f32(uint32_t v) { return __builtin_bit_cast(float, v); }
+__device__ inline uint32_t u32(float v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ inline float sum64(float v) {
+  return f32(wave_reduce(u32(v), [](uint32_t a, uint32_t b) { return u32(f32(a) + f32(b)); }));
+}
+__device__ inline float max64(float v) {
+  return f32(wave_reduce(u32(v), [](uint32_t a, uint32_t b) { return u32(fmaxf(f32(a), f32(b))); }));
+}
+__device__ inline uint32_t max64(uint32_t v) {
+  return wave_reduce(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
 }
 
-// Best candidate of the block; every thread gets it.  red: THREADS / 64 entries.
-__device__ inline Cand block_best(Cand c, Cand* red) {
-  c = wave_best(c);
-  __syncthreads();                   // red is free again
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
-  __syncthreads();
-  Cand b = red[0];
+// A candidate as one integer: its value (fp16, exactly) as an ordered integer, then its place from the back, so that
+// the larger integer is the better candidate ("larger score first, equal scores lowest index first").  0: none
+// (also a NaN, which is never picked).
+__device__ inline uint32_t key_of(float v, int place) {
+  uint32_t h = __builtin_bit_cast(unsigned short, (half_t)v);
+  if (h == 0x8000u) h = 0u;
+  const uint32_t key = (h & 0x8000u ? ~h & 0xffffu : h | 0x8000u) << 16 | (0xffffu - (uint32_t)place);
+  return v != v ? 0u : key;
+}
+__device__ inline float key_value(uint32_t key) {
+  const uint32_t o = key >> 16;
+  return (float)__builtin_bit_cast(half_t, (unsigned short)(o & 0x8000u ? o & 0x7fffu : ~o & 0xffffu));
+}
+__device__ inline int key_place(uint32_t key) { return (int)(0xffffu - (key & 0xffffu)); }
+
+// The k best of the keys that the lanes of a wave hold (N each, distinct apart from 0); lane n gets the n-th.
+template <int N>
+__device__ inline uint32_t wave_topk(uint32_t (&key)[N], int k) {
+  const int lane = threadIdx.x & 63;
+  uint32_t mine = 0;
+  for (int n = 0; n < k; ++n) {
+    uint32_t best = key[0];
 #pragma unroll
-  for (int w = 1; w < THREADS / 64; ++w) b = better(b, red[w]);
-  return b;
+    for (int j = 1; j < N; ++j) best = key[j] > best ? key[j] : best;
+    best = max64(best);
+#pragma unroll
+    for (int j = 0; j < N; ++j) key[j] = key[j] == best ? 0u : key[j];
+    if (lane == n) mine = best;
+  }
+  return mine;
 }
 
 __device__ inline const half_t* row_ptr(const half_t* logits, const int32_t* row_index, int row,
@@ -66,14 +95,14 @@ __global__ __launch_bounds__(THREADS) void lse_partial_kernel(
     x[j] = i < V ? (float)r[i] : -INFINITY;
     m = fmaxf(m, x[j]);
   }
-  m = wave_max(m);
+  m = max64(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   float s = 0.f;
 #pragma unroll
   for (int j = 0; j < CHUNK / THREADS; ++j) s += x[j] == -INFINITY ? 0.f : expf(x[j] - m);
-  s = wave_sum(s);
+  s = sum64(s);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
@@ -83,15 +112,36 @@ __global__ __launch_bounds__(THREADS) void lse_partial_kernel(
   }
 }
 
-// Row statistics from the partials, the same arithmetic in every workgroup that needs them.
-__device__ inline void row_stats(const float* pm, const float* ps, int row, int nch, float* M,
-                                 float* S) {
-  float m = -INFINITY;
-  for (int c = 0; c < nch; ++c) m = fmaxf(m, pm[row * nch + c]);
-  float s = 0.f;
-  for (int c = 0; c < nch; ++c) {
-    const float pmc = pm[row * nch + c];
-    if (pmc != -INFINITY) s += ps[row * nch + c] * expf(pmc - m);
+// Row statistics from the partials, the same arithmetic in every workgroup that needs them: the terms of the sum in
+// parallel, the sum itself over the chunks in order.  shared: STATS floats.
+constexpr int STATS = 256;
+__device__ inline void row_stats(const float* pm, const float* ps, int row, int nch, float* shared, float* M, float* S) {
+  const float *rm = pm + row * nch, *rs = ps + row * nch;
+  float m = -INFINITY, s = 0.f;
+  if (nch > STATS) {
+    for (int c = 0; c < nch; ++c) m = fmaxf(m, rm[c]);
+    for (int c = 0; c < nch; ++c)
+      if (rm[c] != -INFINITY) s += rs[c] * expf(rm[c] - m);
+  } else {
+    const int lane = threadIdx.x & 63;
+    float v[STATS / 64], t[STATS / 64];
+#pragma unroll
+    for (int j = 0; j < STATS / 64; ++j) {
+      const int c = lane + 64 * j;
+      v[j] = c < nch ? rm[c] : -INFINITY;
+      t[j] = c < nch ? rs[c] : 0.f;
+      m = fmaxf(m, v[j]);
+    }
+    m = max64(m);
+#pragma unroll
+    for (int j = 0; j < STATS / 64; ++j)             // (every wave writes the same values)
+      shared[lane + 64 * j] = v[j] == -INFINITY ? 0.f : t[j] * expf(v[j] - m);
+    __syncthreads();
+    for (int c = 0; c < nch; c += 4) {
+      const float4_t t4 = *reinterpret_cast<const float4_t*>(shared + c);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s += t4[e];        // (zeros past the last chunk)
+    }
   }
   *M = m;
   *S = s;
@@ -108,79 +158,91 @@ __device__ inline float score_of(float x, float M, float S, float lse16) {
 }
 
 // Pass 2: per chunk the k best entries by the ordering key (MODE 0: the logit; MODE 1: the
-// fp16 log-probability, in which distinct logits can tie).  Grid (chunks, rows).
+// fp16 log-probability, in which distinct logits can tie).  Grid (chunks, rows).  Bound by the chain of its
+// phases; each wave picks the k best of its entries with integer maxima over registers and lanes, one wave the k best
+// of those (with shuffles through LDS and a barrier per pick the three passes took 40 us for 8 rows of 152064; now 16.5).
 template <int MODE>
 __global__ __launch_bounds__(THREADS) void topk_partial_kernel(
     const half_t* __restrict__ logits, const int32_t* __restrict__ row_index, long V, int k,
     const float* __restrict__ pm, const float* __restrict__ ps, float* __restrict__ pv,
     int32_t* __restrict__ pi) {
-  __shared__ Cand red[THREADS / 64];
+  static_assert(CHUNK <= 0x10000, "the place of a candidate takes sixteen bits");
+  __shared__ __attribute__((aligned(16))) float stats[STATS];
+  __shared__ uint32_t best[THREADS / 64 * TOPK_MAX];
   const int row = blockIdx.y, ch = blockIdx.x, nch = gridDim.x;
   const half_t* r = row_ptr(logits, row_index, row, V);
-  float M = 0.f, S = 1.f;
-  if (MODE == 1) row_stats(pm, ps, row, nch, &M, &S);
   const long beg = (long)ch * CHUNK;
-  float key[CHUNK / THREADS];
+  float x[CHUNK / THREADS];
 #pragma unroll
   for (int j = 0; j < CHUNK / THREADS; ++j) {
     const long i = beg + threadIdx.x + (long)j * THREADS;
-    key[j] = -INFINITY;
-    if (i < V) key[j] = MODE == 0 ? (float)r[i] : score_of<1>((float)r[i], M, S, 0.f);
+    x[j] = (float)r[i < V ? i : V - 1];
   }
-  unsigned taken = 0;                 // bit j: key[j] has been handed out
-  for (int n = 0; n < k; ++n) {
-    Cand c{-INFINITY, 0x7fffffff};
+  float M = 0.f, S = 1.f;
+  if (MODE == 1) row_stats(pm, ps, row, nch, stats, &M, &S);
+  uint32_t key[CHUNK / THREADS];
 #pragma unroll
-    for (int j = 0; j < CHUNK / THREADS; ++j) {
-      const long i = beg + threadIdx.x + (long)j * THREADS;
-      if (!((taken >> j) & 1u) && i < V) c = better(c, Cand{key[j], (int)i});
-    }
-    const Cand b = block_best(c, red);
-#pragma unroll
-    for (int j = 0; j < CHUNK / THREADS; ++j)
-      if ((int)(beg + threadIdx.x + (long)j * THREADS) == b.i) taken |= 1u << j;
-    if (threadIdx.x == 0) {
-      pv[((long)row * nch + ch) * TOPK_MAX + n] = b.v;
-      pi[((long)row * nch + ch) * TOPK_MAX + n] = b.i;     // 0x7fffffff: chunk exhausted
-    }
+  for (int j = 0; j < CHUNK / THREADS; ++j) {
+    const int place = threadIdx.x + j * THREADS;
+    key[j] = beg + place < V ? key_of(MODE == 0 ? x[j] : score_of<1>(x[j], M, S, 0.f), place) : 0u;
+  }
+  const uint32_t mine = wave_topk(key, k);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (lane < TOPK_MAX) best[wave * TOPK_MAX + lane] = mine;
+  __syncthreads();
+  if (wave) return;
+  uint32_t last[1] = {lane < THREADS / 64 * TOPK_MAX ? best[lane] : 0u};
+  const uint32_t pick = wave_topk(last, k);
+  if (lane < k) {
+    const long at = ((long)row * nch + ch) * TOPK_MAX + lane;
+    pv[at] = pick ? key_value(pick) : -INFINITY;
+    pi[at] = pick ? (int)beg + key_place(pick) : 0x7fffffff;     // 0x7fffffff: chunk exhausted
   }
 }
 
-// Pass 3: one workgroup per row merges the chunk candidates and writes indices and fp16 scores.
+// Pass 3: one wave per row merges the chunk candidates and writes indices and fp16 scores.  The candidates stand in the
+// order of their indexes wherever scores are equal (chunks in order, picks of a chunk in order), so a candidate's
+// place breaks ties as its index would.
+constexpr int MERGE = 8;               // candidates per lane at a time
 template <int MODE>
-__global__ __launch_bounds__(THREADS) void topk_merge_kernel(
+__global__ __launch_bounds__(64) void topk_merge_kernel(
     const half_t* __restrict__ logits, const int32_t* __restrict__ row_index, long V, int k,
     int nch, const float* __restrict__ pm, const float* __restrict__ ps,
     const float* __restrict__ pv, const int32_t* __restrict__ pi, int32_t* __restrict__ out_index,
     half_t* __restrict__ out_score) {
-  __shared__ Cand red[THREADS / 64];
-  const int row = blockIdx.x;
+  __shared__ __attribute__((aligned(16))) float stats[STATS];
+  const int row = blockIdx.x, lane = threadIdx.x;
   const int ncand = nch * TOPK_MAX;
-  float M, S;
-  row_stats(pm, ps, row, nch, &M, &S);
-  const float lse16 = (float)(half_t)(M + logf(S));
+  uint32_t mine = 0;
+  for (int from = 0; from < ncand; from += 64 * MERGE) {
+    uint32_t key[MERGE + 1];
+    float v[MERGE];
+    int32_t ix[MERGE];
+#pragma unroll
+    for (int j = 0; j < MERGE; ++j) {
+      const int c = from + j * 64 + lane;
+      const long at = (long)row * ncand + (c < ncand ? c : ncand - 1);
+      v[j] = pv[at];
+      ix[j] = pi[at];
+    }
+#pragma unroll
+    for (int j = 0; j < MERGE; ++j) {
+      const int c = from + j * 64 + lane;
+      key[j] = c < ncand && c % TOPK_MAX < k && ix[j] != 0x7fffffff ? key_of(v[j], c) : 0u;
+    }
+    key[MERGE] = mine;
+    mine = wave_topk(key, k);
+  }
+  float M = 0.f, S = 1.f, lse16 = 0.f;
+  if (MODE == 0) {
+    row_stats(pm, ps, row, nch, stats, &M, &S);
+    lse16 = (float)(half_t)(M + logf(S));
+  }
   const half_t* r = row_ptr(logits, row_index, row, V);
-  int last = -1;
-  float last_v = INFINITY;
-  for (int n = 0; n < k; ++n) {
-    // best candidate that comes after the previous pick in the ordering
-    Cand c{-INFINITY, 0x7fffffff};
-    for (int j = threadIdx.x; j < ncand; j += THREADS) {
-      const int slot = j % TOPK_MAX;
-      if (slot >= k) continue;
-      const Cand e{pv[(long)row * ncand + j], pi[(long)row * ncand + j]};
-      if (e.i == 0x7fffffff) continue;
-      const bool after = e.v < last_v || (e.v == last_v && e.i > last);
-      if (after) c = better(c, e);
-    }
-    const Cand b = block_best(c, red);
-    last = b.i;
-    last_v = b.v;
-    if (threadIdx.x == 0) {
-      const int idx = b.i == 0x7fffffff ? 0 : b.i;
-      out_index[row * k + n] = idx;
-      out_score[row * k + n] = MODE == 0 ? (half_t)score_of<0>((float)r[idx], M, S, lse16) : (half_t)b.v;
-    }
+  if (lane < k) {
+    const int idx = mine ? pi[(long)row * ncand + key_place(mine)] : 0;
+    out_index[row * k + lane] = idx;
+    out_score[row * k + lane] = MODE == 0 ? (half_t)score_of<0>((float)r[idx], M, S, lse16) : (half_t)(mine ? key_value(mine) : -INFINITY);
   }
 }
 
@@ -303,6 +365,7 @@ EAGLE_EXPORT int eagle_logsoftmax_topk_f16(const void* logits, const int32_t* ro
                                            eagle_stream_t stream) {
   if (!logits || !out_index || !out_score) return EAGLE_ERR_NULL;
   if (R < 1 || R > EAGLE_MAX_TREE || V < 1 || k < 1 || k > TOPK_MAX || k > V) return EAGLE_ERR_SHAPE;
+  if (chunks_for(V) * TOPK_MAX > 0x10000) return EAGLE_ERR_SHAPE;
   if (mode != 0 && mode != 1) return EAGLE_ERR_UNSUPPORTED;
   if (!workspace || !eagle_aligned16(workspace) ||
       workspace_bytes < eagle_logsoftmax_topk_workspace_bytes(R, V))
@@ -319,12 +382,12 @@ EAGLE_EXPORT int eagle_logsoftmax_topk_f16(const void* logits, const int32_t* ro
   if (mode == 0) {
     hipLaunchKernelGGL(topk_partial_kernel<0>, dim3(nch, R), dim3(THREADS), 0, st, lg, row_index, V, k,
                        pm, ps, pv, pi);
-    hipLaunchKernelGGL(topk_merge_kernel<0>, dim3(R), dim3(THREADS), 0, st, lg, row_index, V, k, nch, pm,
+    hipLaunchKernelGGL(topk_merge_kernel<0>, dim3(R), dim3(64), 0, st, lg, row_index, V, k, nch, pm,
                        ps, pv, pi, out_index, os);
   } else {
     hipLaunchKernelGGL(topk_partial_kernel<1>, dim3(nch, R), dim3(THREADS), 0, st, lg, row_index, V, k,
                        pm, ps, pv, pi);
-    hipLaunchKernelGGL(topk_merge_kernel<1>, dim3(R), dim3(THREADS), 0, st, lg, row_index, V, k, nch, pm,
+    hipLaunchKernelGGL(topk_merge_kernel<1>, dim3(R), dim3(64), 0, st, lg, row_index, V, k, nch, pm,
                        ps, pv, pi, out_index, os);
   }
   return eagle_launch_status();

@@ -22,64 +22,92 @@ struct TreeLists {
   int n, pn, root64;
 };
 
+// Element i of a list.  The pieces are compared in turn with constant indexes: their ends and addresses are scalar
+// loads at the kernel's start, where a search per lane would wait for memory at every piece.
 template <typename T>
 __device__ inline T list_at(const T* const (&ptr)[EAGLE_MAX_SEGMENTS], const int (&end)[EAGLE_MAX_SEGMENTS], int n, int i) {
-  int s = 0;
-  while (s + 1 < n && i >= end[s]) ++s;
-  return ptr[s][s ? i - end[s - 1] : i];
+  const T* p = ptr[0];
+  int base = 0;
+#pragma unroll
+  for (int s = 1; s < EAGLE_MAX_SEGMENTS; ++s)
+    if (s < n && i >= end[s - 1]) {
+      p = ptr[s];
+      base = end[s - 1];
+    }
+  return p[i - base];
 }
 
-constexpr int TREE_THREADS = 512;
+constexpr int TREE_THREADS = 1024;
+constexpr int TREE_HALF = TREE_THREADS / 2;
 
-// mlx_eagle.py:217-250 (with topk :24-58 and search_sorted :61-93).  One workgroup; bound by the
-// chain of its phases, so none of them is a loop of one thread: the picked candidates are counted
-// with ballots and every token walks up to the root by itself (one thread that ORed the rows in
-// order took longer than the rest of the kernel: 18 -> 7 us for 39 of 328 candidates).
+// mlx_eagle.py:217-250 (with topk :24-58 and search_sorted :61-93).  One workgroup; bound by the chain of its
+// phases (two dependent loads, the ranks, the walk), so none of them is a loop of one thread: each candidate is ranked
+// by two threads, on one integer comparison per pair; the picked ones are counted with ballots; every token walks up
+// to the root by itself.  24.4 -> 8.2 us for 39 of 328 candidates in six pieces.
 __global__ __launch_bounds__(TREE_THREADS) void process_draft_tree_kernel(
     TreeLists in, int C, int k, int total, int32_t* __restrict__ pos_ids, int32_t* __restrict__ mask_index,
     int32_t* __restrict__ draft_tokens, uint32_t* __restrict__ bits_out, uint16_t* __restrict__ mask_out) {
-  __shared__ __attribute__((aligned(16))) float sc[MAXC];
+  __shared__ __attribute__((aligned(16))) uint32_t keys[MAXC];
+  __shared__ int upper[MAXC];          // ranks among the second half of the candidates
   __shared__ int wave_picked[MAXC / 64];
   __shared__ int sel[MAXT];
   __shared__ int midx[MAXT];
   __shared__ unsigned long long bits[MAXT];
   const int tid = threadIdx.x;
-  // a NaN score ranks as -inf: with the index tie rule the order below is then total, so
-  // exactly `total` candidates are picked whatever the scores hold
-  const int C4 = (C + 3) / 4 * 4;
-  for (int i = tid; i < C4; i += TREE_THREADS) {
-    const float v = i < C ? (float)list_at(in.scores, in.end, in.n, i) : -INFINITY;
-    sc[i] = v != v ? -INFINITY : v;
+  // Key of a candidate: its fp16 score as an ordered integer, then its index from the back, so that a larger key is
+  // ahead in the stable descending order.  A NaN score ranks as -inf and -0 as 0: the order is total and exactly
+  // `total` candidates are picked whatever the scores hold.
+  const int C8 = (C + 7) / 8 * 8;
+  if (tid < C8) {
+    uint32_t key = 0;
+    if (tid < C) {
+      uint32_t h = __builtin_bit_cast(unsigned short, list_at(in.scores, in.end, in.n, tid));
+      if ((h & 0x7fffu) > 0x7c00u) h = 0xfc00u;
+      if (h == 0x8000u) h = 0u;
+      key = (h & 0x8000u ? ~h & 0xffffu : h | 0x8000u) << 16 | (0xffffu - (uint32_t)tid);
+    }
+    keys[tid] = key;
   }
   __syncthreads();
-  // rank in the stable descending order: candidates ahead of i are those with a larger
-  // score, or an equal score and a lower flat index
-  bool picked[MAXC / TREE_THREADS];
+  // rank: candidates ahead, counted over half of them by each of two threads
+  const int half = tid / TREE_HALF, c0 = tid % TREE_HALF;
+  int rank[MAXC / TREE_HALF];
 #pragma unroll
-  for (int r = 0; r < MAXC / TREE_THREADS; ++r) {
-    const int i = tid + r * TREE_THREADS;
-    const float si = sc[i < C ? i : 0];
-    int rank = 0;
-    if (r * TREE_THREADS < C) {
-      for (int j = 0; j < C4; j += 4) {
-        const float4_t s4 = *reinterpret_cast<const float4_t*>(sc + j);
+  for (int r = 0; r < MAXC / TREE_HALF; ++r) {
+    const int i = c0 + r * TREE_HALF;
+    rank[r] = 0;
+    if (r * TREE_HALF < C) {
+      const uint32_t key = keys[i < C ? i : 0];
+      const int from = half * (C8 / 2), to = from + C8 / 2;
+#pragma unroll 4
+      for (int j = from; j < to; j += 4) {
+        const uint4_t k4 = *reinterpret_cast<const uint4_t*>(keys + j);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) rank += (s4[e] > si) || (s4[e] == si && j + e < i);
+        for (int e = 0; e < 4; ++e) rank[r] += k4[e] > key;
       }
+      if (half) upper[i] = rank[r];
     }
-    picked[r] = i < C && rank < total;
+  }
+  __syncthreads();
+  bool picked[MAXC / TREE_HALF];
+#pragma unroll
+  for (int r = 0; r < MAXC / TREE_HALF; ++r) {
+    const int i = c0 + r * TREE_HALF;
+    picked[r] = !half && i < C && rank[r] + upper[i] < total;
     const unsigned long long m = __ballot(picked[r]);
-    if ((tid & 63) == 0) wave_picked[i >> 6] = __popcll(m);
+    if (!half && (tid & 63) == 0) wave_picked[i >> 6] = __popcll(m);
   }
   __syncthreads();
   // the picked candidates in ascending flat index
 #pragma unroll
-  for (int r = 0; r < MAXC / TREE_THREADS; ++r) {
-    const int i = tid + r * TREE_THREADS;
+  for (int r = 0; r < MAXC / TREE_HALF; ++r) {
+    const int i = c0 + r * TREE_HALF;
     const unsigned long long m = __ballot(picked[r]);
-    int before = __popcll(m & ((1ull << (tid & 63)) - 1ull));
-    for (int w = 0; w < (i >> 6); ++w) before += wave_picked[w];
-    if (picked[r] && before < total) sel[before] = i;
+    if (picked[r]) {
+      int before = __popcll(m & ((1ull << (tid & 63)) - 1ull));
+      for (int w = 0; w < (i >> 6); ++w) before += wave_picked[w];
+      if (before < total) sel[before] = i;
+    }
   }
   __syncthreads();
   if (tid < total) {
