@@ -32,6 +32,25 @@ struct Layer {
   const void *norm1 = nullptr, *norm2 = nullptr;
 };
 
+// A tensor that a decoder reads, as it was when the decoder was built.  The storage is held beside it: memory that
+// `tensor.data = other` takes away stays valid until the decoder goes, and its address is not given out again.
+struct Source {
+  at::Tensor tensor;
+  c10::Storage storage;
+  const void* ptr;
+  int64_t version;                         // (of an inference tensor: none, its writes are not counted)
+  at::ScalarType type;
+  at::DimVector sizes;
+
+  static int64_t version_of(const at::Tensor& t) { return t.is_inference() ? 0 : (int64_t)t._version(); }
+  explicit Source(const at::Tensor& t)
+      : tensor(t), storage(t.storage()), ptr(t.data_ptr()), version(version_of(t)), type(t.scalar_type()), sizes(t.sizes()) {}
+  bool same() const {
+    return tensor.has_storage() && tensor.data_ptr() == ptr && version_of(tensor) == version && tensor.scalar_type() == type &&
+           tensor.sizes() == sizes && tensor.is_contiguous();
+  }
+};
+
 struct Decoder {
   int D, I, H, G, hd, V, form;
   bool linear_bias = false;                // an o or down projection with a bias
@@ -40,14 +59,10 @@ struct Decoder {
   const void* norm = nullptr;
   const float* inv_freqs = nullptr;
   std::vector<Layer> layers;
-  std::vector<at::Tensor> kept;            // every tensor whose address is held
-  std::vector<int64_t> versions;           // of the checkpoint's tensors, which the derived copies came from
-  size_t n_source = 0;
+  std::vector<Source> kept;                // every tensor whose address is held
   PyObject *layer_list = nullptr, *cache_type = nullptr;
   std::vector<PyObject*> layer_items;
 };
-
-int64_t version_of(const at::Tensor& t) { return t.is_inference() ? 0 : (int64_t)t._version(); }
 
 void destroy(PyObject* cap) {
   Decoder* d = static_cast<Decoder*>(PyCapsule_GetPointer(cap, "eagle.decoder"));
@@ -64,9 +79,9 @@ struct Bad : std::exception {
 
 const at::Tensor& take(Decoder* d, PyObject* o) {
   const at::Tensor* t = tensor(o);
-  if (!t || !t->is_cuda() || !t->is_contiguous()) throw Bad();
-  d->kept.push_back(*t);
-  return d->kept.back();
+  if (!t || !t->has_storage() || !t->is_contiguous() || (!d->kept.empty() && t->device() != d->kept[0].tensor.device())) throw Bad();
+  d->kept.emplace_back(*t);
+  return *t;
 }
 // (weight, scales, biases, bias or None)
 Mat take_mat(Decoder* d, PyObject* o) {
@@ -290,8 +305,6 @@ PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n) {
     l.norm1 = take(d.get(), PyTuple_GET_ITEM(t, NPROJ + 2)).data_ptr();
     l.norm2 = take(d.get(), PyTuple_GET_ITEM(t, NPROJ + 3)).data_ptr();
   }
-  d->n_source = d->kept.size();
-  for (const at::Tensor& t : d->kept) d->versions.push_back(version_of(t));
   d->inv_freqs = static_cast<const float*>(take(d.get(), a[5]).data_ptr());
   for (Py_ssize_t i = 0; i < nl; ++i) {
     PyObject* t = PyList_GET_ITEM(a[6], i);
@@ -312,15 +325,16 @@ PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return cap;
 }
 
-// decoder_current(capsule): the layers are the ones the decoder was built from, and nobody wrote to their tensors
+// decoder_current(capsule): the layers are the ones the decoder was built from, their tensors lie where they lay, and no
+// write to them was counted
 PyObject* py_decoder_current(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Decoder* d = n == 1 ? static_cast<Decoder*>(PyCapsule_GetPointer(a[0], "eagle.decoder")) : nullptr;
   if (!d) return nullptr;
   if (PyList_GET_SIZE(d->layer_list) != (Py_ssize_t)d->layer_items.size()) Py_RETURN_FALSE;
   for (size_t i = 0; i < d->layer_items.size(); ++i)
     if (PyList_GET_ITEM(d->layer_list, i) != d->layer_items[i]) Py_RETURN_FALSE;
-  for (size_t i = 0; i < d->n_source; ++i)
-    if (version_of(d->kept[i]) != d->versions[i]) Py_RETURN_FALSE;
+  for (const Source& s : d->kept)
+    if (!s.same()) Py_RETURN_FALSE;
   Py_RETURN_TRUE;
 }
 
@@ -339,7 +353,7 @@ PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   const at::Tensor *ids = tensor(a[1]), *mask = tensor(a[3]), *words = tensor(a[4]), *pos = tensor(a[6]);
   if (!ids || !ids->is_cuda() || !ids->is_contiguous() || ids->dim() != 2 || ids->size(0) != 1 || ids->size(1) < 1 ||
-      (ids->scalar_type() != at::kInt && ids->scalar_type() != at::kLong) || ids->device() != d->kept[0].device())
+      (ids->scalar_type() != at::kInt && ids->scalar_type() != at::kLong) || ids->device() != d->kept[0].tensor.device())
     Py_RETURN_NONE;
   const int64_t T = ids->size(1);
   const bool causal = a[3] == Py_None && a[4] == Py_None;

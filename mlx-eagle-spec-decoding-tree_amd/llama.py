@@ -258,6 +258,14 @@ class Model(Module):
     def layers(self):
         return self.model.layers
 
+    def weights_written(self):
+        """To be called after weights were written in a way that torch does not count (`t.data.copy_(...)`, a kernel
+        or another library on the same memory): every laid-out copy of them is dropped and made again when it is next
+        needed.  Pass objects built before (`TreeVerifier`, `SpeculativeDecoder`, ...) keep theirs and are built anew."""
+        native.forget(self)
+        for key in ("_fused_projections", "_tiled_model", "_tiled_projections", "_tiled_head"):
+            self.__dict__.pop(key, None)
+
 
 def _qtuple(tensors, prefix):
     return (tensors[f"{prefix}.weight"], tensors[f"{prefix}.scales"], tensors[f"{prefix}.biases"],

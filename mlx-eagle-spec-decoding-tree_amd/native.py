@@ -1,9 +1,12 @@
 """The native form of a decoder (csrc/decoder.cpp): built once per model from its layers, used by
 `Model.__call__`, `tree_decoding` and the draft expansion for every pass that it takes.
 
-A decoder is rebuilt when an attribute of a module changed, a layer was exchanged, or somebody wrote
-to a weight tensor.  Models it does not take (a patched layer, another group size, CPU tensors) run
-the Python operators of the module path."""
+A decoder is rebuilt when an attribute of a module changed, a layer was exchanged, a tensor's memory was
+(`t.data = other`), or torch counted a write to a weight tensor.  A write that is not counted
+(`t.data.copy_(...)`, another library on the same memory) reaches what is read in place, but not the fused
+copies: after one, call `Model.weights_written()`.  Writes to inference tensors are never counted, so layers
+made of them keep one launch per projection on their own tensors.  Models it does not take (a patched layer,
+another group size, CPU tensors) run the Python operators of the module path."""
 import torch
 
 from . import ops
@@ -28,10 +31,18 @@ def decoder(model):
     if st is not None:
         if st.epoch == Module.epoch and (st.handle is None or ops._native().decoder_current(st.handle)):
             return st.handle
+    model.__dict__.pop("_native", None)          # the old decoder goes before the new one is made
+    del st
     epoch = Module.epoch
     handle = _build(model)
     model.__dict__["_native"] = _State(epoch if Module.epoch == epoch else Module.epoch, handle)
     return handle
+
+
+def forget(model):
+    """Drop the decoder and its copies of the weights; the next pass builds them again."""
+    for key in ("_native", "_native_fused"):
+        model.__dict__.pop(key, None)
 
 
 def forward(model, ids, cache, mask=None, words=None, Tk=0, positions=None, pos_add=0, pos_step=0, head=2):
@@ -59,7 +70,8 @@ def _plain_leaf(lin, n, k, device):
             and (lin.bias is None or tuple(lin.bias.shape) == (n,)))
 
 
-def _build(model):
+def _build(model, kind="cuda"):
+    """The handle of a decoder on the model's tensors, which have to be on a device of this kind, or None."""
     from .llama import Attention, LlamaModel, MLP, QuantizedEmbedding, RMSNorm, TransformerBlock
     args, m = model.args, model.model
     if type(m) is not LlamaModel or not isinstance(m.layers, list) or not m.layers or type(m.norm) is not RMSNorm:
@@ -67,7 +79,7 @@ def _build(model):
     D, I, V = args.hidden_size, args.intermediate_size, args.vocab_size
     H, G, hd = args.num_attention_heads, args.num_key_value_heads, args.head_dim
     emb = m.embed_tokens
-    if type(emb) is not QuantizedEmbedding or emb.group_size != 64 or emb.bits != 4 or not emb.weight.is_cuda:
+    if type(emb) is not QuantizedEmbedding or emb.group_size != 64 or emb.bits != 4 or emb.weight.device.type != kind:
         return None
     dev = emb.weight.device
     # what the kernels of every form take
@@ -105,7 +117,7 @@ def _build(model):
     if any(l.self_attn._inv_freqs is not at0._inv_freqs and not torch.equal(l.self_attn._inv_freqs, at0._inv_freqs)
            or l.self_attn._scaling_factor != at0._scaling_factor or l.self_attn.scale != at0.scale for l in m.layers):
         return None
-    if at0._inv_freqs.numel() != hd // 2 or not at0._inv_freqs.is_cuda or at0._inv_freqs.dtype != torch.float32:
+    if at0._inv_freqs.numel() != hd // 2 or at0._inv_freqs.device != dev or at0._inv_freqs.dtype != torch.float32:
         return None
 
     form, derived = _derive(model, layers, shapes, I, D, H, G, hd)
@@ -126,14 +138,18 @@ def _derive(model, layers, shapes, I, D, H, G, hd):
     W = (H + 2 * G) * hd
     if D < FUSE_HIDDEN or not ops.swiglu_supported(32, I, D) or W % 16 or D % 16:
         return PLAIN, [none] * len(layers)
-    sources = [(t.data_ptr(), 0 if t.is_inference() else t._version) for lins in layers
-               for name in ("q", "k", "v", "gate", "up") for t in _leaf(lins[name]) if t is not None]
+    leaves = [t for lins in layers for name in ("q", "k", "v", "gate", "up") for t in _leaf(lins[name]) if t is not None]
+    if any(t.is_inference() for t in leaves):              # a write to one could not be seen
+        return PLAIN, [none] * len(layers)
+    sources = [(t.data_ptr(), t._version) for t in leaves]
     done = model.__dict__.get("_native_fused")
     if done is None or done[0] != sources:
         model.__dict__.pop("_native_fused", None)          # the old copies go before the new ones are made
-        done = (sources, [(_rows(lins["q"], lins["k"], lins["v"]), _gate_up(lins["gate"], lins["up"])) for lins in layers])
+        # (the sources' memory is held beside them, so that an address stands for one content)
+        done = (sources, [t.detach() for t in leaves],
+                [(_rows(lins["q"], lins["k"], lins["v"]), _gate_up(lins["gate"], lins["up"])) for lins in layers])
         model.__dict__["_native_fused"] = done
-    return FUSED, done[1]
+    return FUSED, done[2]
 
 
 def _biases(*lins):

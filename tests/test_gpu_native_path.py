@@ -138,3 +138,28 @@ def test_native_decoder_follows_the_weights(dev):
     assert model(long, cache).shape == (1, 97, 1000) and cache[0].offset == 100
     llama.patch_model(model, lambda *a: ops.matmul(*a)[0])
     assert native.decoder(model) is None
+
+
+def test_native_decoder_follows_memory_that_no_counter_shows(dev):
+    """`t.data = other`, an uncounted write announced by weights_written(), writes to inference tensors: each reaches
+    the next pass, as it does operator by operator."""
+    model, ids = small_model(dev, "wide"), torch.arange(6, device=dev)[None]
+    seen = [same_pass(model, ids, 3, 16)]
+    for lin, key in ((model.layers[1].mlp.down_proj, "scales"), (model.layers[0].mlp.gate_proj, "weight"),
+                     (model.layers[1].self_attn.q_proj, "weight"), (model.model.embed_tokens, "weight")):
+        getattr(lin, key).data = getattr(lin, key).data.flip(0).contiguous()
+        filler = [torch.full_like(getattr(lin, key), 0) for _ in range(4)]       # takes the old memory if it was given back
+        seen.append(same_pass(model, ids, 3, 16))
+        del filler
+    gate = model.layers[1].mlp.gate_proj.weight
+    gate.data.copy_(gate.data.flip(0))
+    model.weights_written()
+    seen.append(same_pass(model, ids, 3, 16))
+    with torch.inference_mode():
+        for layer in model.layers:
+            layer.mlp.up_proj.weight = layer.mlp.up_proj.weight.clone()
+        seen.append(same_pass(model, ids, 3, 16))
+        up = model.layers[0].mlp.up_proj.weight
+        up.copy_(up.flip(0))
+        seen.append(same_pass(model, ids, 3, 16))
+    assert all(not torch.equal(a, b) for i, a in enumerate(seen) for b in seen[:i] if not (i == 6 and b is seen[5]))

@@ -1,0 +1,88 @@
+"""When a native decoder (native.py, csrc/decoder.cpp) is still the one of its model: built here on CPU tensors, which
+it can be checked on but runs no pass for."""
+import pytest
+import torch
+
+from mlx_eagle_spec_decoding_tree_amd import llama, native, ops, synth
+
+CPU = torch.device("cpu")
+FUSED = dict(hidden=1024, inter=256, heads=8, kv_heads=2, head_dim=128)
+PLAIN = dict(hidden=256, inter=512, heads=4, kv_heads=2, head_dim=64)
+
+
+def model_of(shape, seed=3, **kw):
+    args = synth.tiny(layers=2, vocab=64, attention_bias=True, **{**shape, **kw})
+    return llama.Model.from_numpy(args, synth.make_model_weights(args, seed=seed), CPU)
+
+
+def current(handle):
+    return ops._native().decoder_current(handle)
+
+
+def exchange_memory(t):
+    t.data = t.data.clone()
+
+
+TENSORS = {
+    "gate": lambda m: m.layers[1].mlp.gate_proj.weight, "down": lambda m: m.layers[0].mlp.down_proj.scales,
+    "q": lambda m: m.layers[1].self_attn.q_proj.biases, "q bias": lambda m: m.layers[0].self_attn.q_proj.bias,
+    "norm": lambda m: m.layers[1].input_layernorm.weight, "last norm": lambda m: m.model.norm.weight,
+    "embedding": lambda m: m.model.embed_tokens.weight, "frequencies": lambda m: m.layers[0].self_attn._inv_freqs,
+}
+
+
+@pytest.mark.parametrize("name", list(TENSORS))
+@pytest.mark.parametrize("change", [exchange_memory, lambda t: t.mul_(1), lambda t: t.resize_(1)],
+                         ids=["other memory", "counted write", "other size"])
+@pytest.mark.parametrize("shape", [FUSED, PLAIN], ids=["fused", "plain"])
+def test_a_decoder_is_current_until_a_tensor_changes(shape, change, name):
+    model = model_of(shape)
+    handle = native._build(model, "cpu")
+    assert handle is not None and current(handle)
+    change(TENSORS[name](model))
+    assert not current(handle)
+
+
+def test_exchanged_memory_stays_valid_and_its_address_is_not_taken_for_the_old_content():
+    """`t.data = other` twice between two passes: the second memory cannot lie where the first lay."""
+    model = model_of(FUSED)
+    handle = native._build(model, "cpu")
+    w = model.layers[0].mlp.gate_proj.weight
+    old = w.data_ptr()
+    exchange_memory(w)
+    for _ in range(8):
+        w.data = torch.zeros_like(w)
+        assert w.data_ptr() != old
+    copies = native._derive(model, *derive_args(model))
+    assert copies[0] == native.FUSED and int(copies[1][0][1][0][:16].abs().max()) == 0     # layer 0, gate rows of gate|up
+    assert not current(handle)
+
+
+def derive_args(model):
+    a = model.args
+    layers = [dict(q=l.self_attn.q_proj, k=l.self_attn.k_proj, v=l.self_attn.v_proj, o=l.self_attn.o_proj,
+                   gate=l.mlp.gate_proj, up=l.mlp.up_proj, down=l.mlp.down_proj) for l in model.layers]
+    return layers, None, a.intermediate_size, a.hidden_size, a.num_attention_heads, a.num_key_value_heads, a.head_dim
+
+
+def test_layers_of_inference_tensors_are_read_in_place():
+    with torch.inference_mode():
+        model = model_of(FUSED)
+        for layer in model.layers:
+            layer.mlp.up_proj.weight = layer.mlp.up_proj.weight.clone()
+    assert native._derive(model, *derive_args(model)) == (native.PLAIN, [(None, None)] * 2)
+    assert native._build(model, "cpu") is not None
+
+
+def test_uncounted_writes_reach_the_copies_after_the_call_for_them():
+    model = model_of(FUSED)
+    form, copies = native._derive(model, *derive_args(model))
+    assert form == native.FUSED
+    gate = model.layers[1].mlp.gate_proj
+    gate.weight.data.zero_()
+    again = native._derive(model, *derive_args(model))[1]
+    assert again is copies and int(again[1][1][0][:16].abs().max()) != 0
+    model.weights_written()
+    again = native._derive(model, *derive_args(model))[1]
+    assert int(again[1][1][0][:16].abs().max()) == 0
+    assert torch.equal(again[1][1][0], ops.interleave_gate_up(gate.weight, model.layers[1].mlp.up_proj.weight))
