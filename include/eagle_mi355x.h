@@ -104,11 +104,12 @@ int eagle_qmm_small_w4g64_f16(const void* x, const void* norm_w, float eps, cons
                               const void* residual, void* out, int T, int N, int K,
                               int group_size, int bits, int swiglu, eagle_stream_t stream);
 
-/* The product of 1..64 rows on the checkpoint's own layout without rounding a weight: out [M, N], or with swiglu
+/* The product of 1..EAGLE_MAX_CHUNK rows on the checkpoint's own layout without rounding a weight: out [M, N], or with swiglu
  * out [M, N / 2] = silu(g) * u of gate and up rows interleaved in 16-row tiles.  Where the library splits K over
  * workgroups it needs eagle_qmm_rows_workspace_bytes bytes for fp32 partial sums (no initialisation, free after the
  * call in stream order); with workspace NULL it does not split (EAGLE_ERR_SHAPE for a K that only fits split).  eagle_qmm_rows_preferred: whether it is the fastest
- * form (after eagle_qmm_small_preferred and eagle_qmv_preferred).
+ * form of up to 64 rows (after eagle_qmm_small_preferred and eagle_qmv_preferred); above them eagle_qmm_gemm_split_w4g64_f16
+ * is, which rounds the weights to fp16.
  * Constraints (eagle_qmm_rows_supported): K % 128 == 0; N % 8 == 0 (32 with swiglu), N >= 16; x must not alias out; x,
  * wq, out, workspace 16-byte, scales and biases 4-byte aligned. */
 int eagle_qmm_rows_supported(int M, int N, int K, int swiglu);

@@ -50,13 +50,14 @@ bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out) {
   return true;
 }
 
-int gemm(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out, int M,
-         int N, int K, bool swiglu, void* st) {
+// the many-row product, split over K where the library says so
+static int gemm(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out, int M,
+                int N, int K, void* st) {
   // the partial sums go back to torch's allocator with the launches in the stream
-  const size_t need = eagle_qmm_gemm_workspace_bytes(M, N, K, swiglu);
+  const size_t need = eagle_qmm_gemm_workspace_bytes(M, N, K, 0);
   at::Tensor ws;
   if (need) ws = empty({(int64_t)need}, at::kByte, like);
-  return eagle_qmm_gemm_split_w4g64_f16(x, static_cast<const uint32_t*>(w), s, b, bias, out, M, N, K, 64, 4, swiglu,
+  return eagle_qmm_gemm_split_w4g64_f16(x, static_cast<const uint32_t*>(w), s, b, bias, out, M, N, K, 64, 4, 0,
                                         need ? ws.data_ptr() : nullptr, need, st);
 }
 
@@ -83,7 +84,7 @@ bool small_aligned(const void* x, const void* s, const void* b, const void* bias
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
            int M, int N, int K, void* st) {
   const uint32_t* wq = static_cast<const uint32_t*>(w);
-  if (M > 2 * EAGLE_MAX_M) return gemm(like, x, w, s, b, bias, out, M, N, K, false, st);
+  if (M > 2 * EAGLE_MAX_M) return gemm(like, x, w, s, b, bias, out, M, N, K, st);
   if (M > EAGLE_MAX_M && rows_takes(M, N, K, x, s, b, out)) return rows(like, x, w, s, b, bias, out, M, N, K, false, st);
   for (int r0 = 0; r0 < M; r0 += EAGLE_MAX_M) {
     const int m = M - r0 < EAGLE_MAX_M ? M - r0 : EAGLE_MAX_M;

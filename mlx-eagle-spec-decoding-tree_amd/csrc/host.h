@@ -43,7 +43,7 @@ bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out);
 // Whether the operands have the alignment that the small-row kernel asks for
 bool small_aligned(const void* x, const void* s, const void* b, const void* bias, const void* out);
 
-// The product of up to 64 rows on eagle_qmm_rows_w4g64_f16, and whether it is the form to take
+// The product on eagle_qmm_rows_w4g64_f16, and whether it is the form to take for up to 64 rows
 bool rows_takes(int M, int N, int K, const void* x, const void* s, const void* b, const void* out);
 int rows(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out, int M,
          int N, int K, bool swiglu, void* st);
@@ -52,10 +52,6 @@ int rows(const at::Tensor& like, const void* x, const void* w, const void* s, co
 // result: a Python error is set.
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
            int M, int N, int K, void* st);
-
-// The many-row product, split over K where the library says so (SwiGLU: interleaved gate|up rows)
-int gemm(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out, int M,
-         int N, int K, bool swiglu, void* st);
 
 PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* py_decoder_current(PyObject*, PyObject* const* a, Py_ssize_t n);

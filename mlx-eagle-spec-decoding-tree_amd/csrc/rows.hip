@@ -1,4 +1,4 @@
-// 4-bit group-64 quantised product for 2..64 rows of x on the weights in the MLX layout:
+// 4-bit group-64 quantised product for 2..2048 rows of x on the weights in the MLX layout, no weight rounded:
 // out[m][n] = fp16( sum_k x[m][k] (s[n,k/64] q[n,k] + b[n,k/64]) ) (+ bias[n]), or silu(g) * u of gate and up
 // rows interleaved in 16-row tiles.  (Reference: mx.quantized_matmul, mlx_model_fwd_bench.py:65-73; the
 // factorisation of kernels/qmv/1b.metal:121-147.)
@@ -17,10 +17,15 @@
 //     instead, 16 bytes of a row at a time, every line came from memory as often as it has blocks: 32 x 3584 x 152064
 //     90 us, 71 us so; without reading any 67.
 //
+//   * More than 64 rows (a prompt of the module path) are blocks of 48 or 64 rows of the same kernel, the blocks of one
+//     group of weight rows next to each other in the grid, so that an XCD's L2 gives the weights to several of them.
+//
 // What bounds it: the bytes a compute unit takes in, its weights and all of its x (the loads and the x path alone
 // 58 .. 65 of those 71 us), then the vector instructions of the expansion.  Against the streaming kernel (us, launches
 // back to back over rotating weights): 32 x 3584 x 152064 71 / 80, 27 x 18944 x 3584 18 / 23, 32 x 2048 x 8192 8.2 / 11.0,
-// 64 x 8192 x 8192 24 / 40.
+// 64 x 8192 x 8192 24 / 40.  With many rows the vector instructions (expansion per block, a multiply-add per group and
+// output) about equal the matrix instructions: 2048 x 37888 x 3584 675 us = 0.82 PFLOP/s, 512 x 3584 x 18944 114 us; the
+// GEMM, which rounds the weights to fp16 and expands them once per 256 rows, takes 580 and 93.
 #include "common.h"
 
 namespace {
@@ -36,6 +41,7 @@ struct RowsArgs {
   int M, N, K, swiglu;
   int both;               // scales and biases fit LDS together
   int pitch;              // rows of x per split in `partial`
+  int zb;                 // blocks of 16 MT rows of x
 };
 
 constexpr int ROWS_WAVES = 8;
@@ -100,7 +106,9 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r = lane & 15, kq = lane >> 4;
   const int kp = wave % KP, rg = wave / KP;
-  const int K = a.K, M = a.M, N = a.N;
+  const int nb = a.zb == 1 ? blockIdx.x : blockIdx.x / a.zb;            // weight rows, then block of x
+  const int m0 = (blockIdx.x - nb * a.zb) * ROWS;
+  const int K = a.K, M = a.M - m0 < ROWS ? a.M - m0 : ROWS, N = a.N;
   const int all = K >> 7;
   // K in units of four chunks (512 columns), dealt over the workgroups along y and then over the K parts
   const int units = (all + 3) >> 2;
@@ -118,12 +126,12 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
   unsigned char* const sbl = rows_lds + 2 * BUF + KP * XC * ROWS * 8 + wave * (RT * 16) * stride * (a.both ? 2 : 1);
 
   // ---- addresses: buffer loads, a uniform offset per tile and chunk beside one 32-bit lane offset ----
-  const int row0 = blockIdx.x * WROWS + rg * (RT * 16);
+  const int row0 = nb * WROWS + rg * (RT * 16);
   const int G = K >> 6;
   const auto wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.w), 0, (int)((long)N * K >> 1), ROWS_RSRC);
   const auto sbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.s), 0, N * G * 2, ROWS_RSRC);
   const auto bbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.b), 0, N * G * 2, ROWS_RSRC);
-  const auto xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.x), 0, M * K * 2, ROWS_RSRC);
+  const auto xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.x) + (long)m0 * K, 0, M * K * 2, ROWS_RSRC);
   const uint32_t wlane = (uint32_t)r * (K >> 1) + kq * 16;
   uint32_t wbase[RT];
 #pragma unroll
@@ -388,7 +396,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
       for (int i = 0; i < 4; ++i)
         red[(long)(kp * ROWS + mt * 16 + 4 * kq + i) * OROW + rg * (RT * 16) + t * 16 + r] = acc[t][mt][i];
   rows_barrier();
-  const int base = blockIdx.x * WROWS;
+  const int base = nb * WROWS;
   auto sum8 = [&](int m, int at, float* v) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = 0.f;
@@ -414,7 +422,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
     float v[8];
     sum8(m, at, v);
     if (a.partial) {
-      float* p = a.partial + ((long)blockIdx.y * a.pitch + m) * N + n;
+      float* p = a.partial + ((long)blockIdx.y * a.pitch + m0 + m) * N + n;
       *reinterpret_cast<float4_t*>(p) = float4_t{v[0], v[1], v[2], v[3]};
       *reinterpret_cast<float4_t*>(p + 4) = float4_t{v[4], v[5], v[6], v[7]};
       continue;
@@ -436,9 +444,9 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
         const half_t act = (half_t)(gf / (1.0f + expf(-gf)));
         h[e] = (half_t)((float)act * (float)u);
       }
-      *reinterpret_cast<half8_t*>(a.out + (long)m * (N >> 1) + ((n >> 5) << 4) + (n & 15)) = h;
+      *reinterpret_cast<half8_t*>(a.out + (long)(m0 + m) * (N >> 1) + ((n >> 5) << 4) + (n & 15)) = h;
     } else {
-      *reinterpret_cast<half8_t*>(a.out + (long)m * N + n) = h;
+      *reinterpret_cast<half8_t*>(a.out + (long)(m0 + m) * N + n) = h;
     }
   }
 }
@@ -448,6 +456,7 @@ int rows_launch(const RowsArgs& a, int splits, hipStream_t st) {
   constexpr int WROWS = ROWS_WAVES / KP * RT * 16;
   const int units = ((a.K >> 7) + 3) / 4, most = (units + splits - 1) / splits, nu = (most + KP - 1) / KP;
   RowsArgs b = a;
+  b.zb = (a.M + 16 * MT - 1) / (16 * MT);
   b.both = rows_lds_bytes(RT, MT, KP, nu, true) <= ROWS_LDS;
   const size_t lds = rows_lds_bytes(RT, MT, KP, nu, b.both);
   if (lds > ROWS_LDS) return EAGLE_ERR_SHAPE;
@@ -458,7 +467,7 @@ int rows_launch(const RowsArgs& a, int splits, hipStream_t st) {
       return EAGLE_ERR_HIP;
     ready = true;
   }
-  hipLaunchKernelGGL((qmm_rows_kernel<RT, MT, KP, AH>), dim3((a.N + WROWS - 1) / WROWS, splits), dim3(ROWS_WAVES * 64), lds, st, b);
+  hipLaunchKernelGGL((qmm_rows_kernel<RT, MT, KP, AH>), dim3((a.N + WROWS - 1) / WROWS * b.zb, splits), dim3(ROWS_WAVES * 64), lds, st, b);
   return eagle_launch_status();
 }
 
@@ -517,17 +526,20 @@ struct RowsPlan {
 // its workgroups one after the other; each costs its start, its share of the weights and its x at the rates a
 // unit ingests them (40 and 72 GB/s), and 0.22 us per unit of four chunks, tile and 16 rows of x.  What the whole
 // grid reads counts a little, a split as much as its second launch and the partial sums (the sums alone where
-// the consumer of the product adds them).
+// the consumer of the product adds them).  For 65 .. 2048 rows the same formula over the blocks of x: over 12600 random
+// products, each in every form and split, its choice took 1.2 % longer than the best on average, 7.5 % at the 95th
+// percentile, 25 % at most.
 enum { ROWS_WHOLE = 0, ROWS_SPLIT = 1, ROWS_PARTIAL = 2 };
 RowsPlan rows_find_plan(int M, int N, int K, int mode) {
-  const int units = ((K >> 7) + 3) / 4, mt = (M + 15) / 16;
+  const int units = ((K >> 7) + 3) / 4;
+  const int least_zb = (M + 63) / 64, mt = (M + 16 * least_zb - 1) / (16 * least_zb), zb = (M + 16 * mt - 1) / (16 * mt);
   RowsPlan best = {-1, 1};
   double least = 1e30;
   for (int f = 0; f < ROWS_FORMS; ++f) {
     const RowsForm& form = rows_forms[f];
     if (form.mt != mt) continue;
     const int wrows = ROWS_WAVES / form.kp * form.rt * 16;
-    const long blocks = (N + wrows - 1) / wrows;
+    const long blocks = (long)((N + wrows - 1) / wrows) * zb;
     int last = 0;
     for (int z = 1; z <= (mode == ROWS_WHOLE ? 1 : 32) && units / z >= form.kp; ++z) {
       const int nu = ((units + z - 1) / z + form.kp - 1) / form.kp;
@@ -537,7 +549,7 @@ RowsPlan rows_find_plan(int M, int N, int K, int mode) {
       const double rounds = (double)((blocks * z + 255) / 256);
       const double w = wrows * (double)nu * form.kp * (512 * 0.5625 / 1e3), x = 16. * mt * nu * form.kp * (1024 / 1e3);
       double t = rounds * (1.03 + 0.0246 * w + 0.0138 * x + 0.221 * nu * form.rt * mt) + 0.0107 * (blocks * z / 256.) * (w + 0.5 * x);
-      if (z > 1) t += (mode == ROWS_SPLIT ? 2.93 : 0.) + 0.49 * 4e-6 * z * M * N;
+      if (z > 1) t += (mode == ROWS_SPLIT ? 2.93 : 0.) + 0.49 * 4e-6 * z * (double)M * N;
       if (t < least) {
         least = t;
         best = {f, z};
@@ -567,7 +579,7 @@ RowsPlan rows_plan(int M, int N, int K, int mode) {
 }  // namespace
 
 EAGLE_EXPORT int eagle_qmm_rows_supported(int M, int N, int K, int swiglu) {
-  return M >= 1 && M <= 2 * EAGLE_MAX_M && N >= 16 && (N % (swiglu ? 32 : 8)) == 0 && K >= 128 && (K % 128) == 0 &&
+  return M >= 1 && M <= EAGLE_MAX_CHUNK && N >= 16 && (N % (swiglu ? 32 : 8)) == 0 && K >= 128 && (K % 128) == 0 &&
          (long)N * K < (1L << 33) && rows_plan(M, N, K, ROWS_SPLIT).form >= 0;
 }
 
@@ -577,7 +589,8 @@ EAGLE_EXPORT int eagle_qmm_rows_supported(int M, int N, int K, int swiglu) {
 // 1152 7.7 / 7.5).  Up to 16 rows the streaming kernel's waves hold all of x and its weights come in whole lines:
 // even at K up to 2048 and in a middle range (3584 -> 37888 24.2 / 23.3, 4864 -> 18944 21.0 / 20.3), behind below
 // (3584 -> 18944 15.6 / 16.7) and above it (8192 -> 37888 42 / 50, 3584 -> 152064 61 / 66, 18944 -> 3584 16 / 20).
-// The forms for one or a few rows come first where they apply (the caller asks them before).
+// The forms for one or a few rows come first where they apply (the caller asks them before).  Above 64 rows the GEMM is
+// faster; who must not round a weight asks for this kernel.
 EAGLE_EXPORT int eagle_qmm_rows_preferred(int M, int N, int K) {
   if (M < 1 || M > 2 * EAGLE_MAX_M) return 0;
   const double size = (double)N * K;
@@ -635,7 +648,7 @@ EAGLE_EXPORT int eagle_qmm_rows_w4g64_f16(const void* x, const uint32_t* wq, con
 }
 
 EAGLE_EXPORT int eagle_qmm_rows_partial_splits(int M, int N, int K) {
-  return eagle_qmm_rows_supported(M, N, K, 0) ? rows_plan(M, N, K, ROWS_PARTIAL).splits : 0;
+  return M <= 2 * EAGLE_MAX_M && eagle_qmm_rows_supported(M, N, K, 0) ? rows_plan(M, N, K, ROWS_PARTIAL).splits : 0;
 }
 
 EAGLE_EXPORT int eagle_qmm_rows_partial_w4g64(const void* x, const uint32_t* wq, const void* scales, const void* biases, float* partial,

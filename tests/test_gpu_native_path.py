@@ -6,7 +6,7 @@ import torch
 from mlx_eagle_spec_decoding_tree_amd import eagle, llama, native, ops, synth
 from mlx_eagle_spec_decoding_tree_amd.cache import make_prompt_cache
 from oracle import tree_oracle as to
-from util import MODEL_TOL, rel_err, to_dev
+from util import MODEL_TOL, TOL, rel_err, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -163,3 +163,33 @@ def test_native_decoder_follows_memory_that_no_counter_shows(dev):
         up.copy_(up.flip(0))
         seen.append(same_pass(model, ids, 3, 16))
     assert all(not torch.equal(a, b) for i, a in enumerate(seen) for b in seen[:i] if not (i == 6 and b is seen[5]))
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("T", [64, 65, 130, 512])
+def test_a_prompt_rounds_no_weight(dev, form, T):
+    """Layers that add nothing, embedding rows whose groups sum to zero, and a head of weights 64 + s q: rounded to fp16
+    (multiples of 1/16) they would lose most of q, and what is left of the product is the sum of s q x."""
+    args = synth.tiny(layers=1, vocab=1000, **FORMS[form])
+    assert not args.tie_word_embeddings
+    D, rng = args.hidden_size, np.random.default_rng(T)
+    w = synth.make_model_weights(args, seed=3)
+    for name in ("self_attn.o_proj", "mlp.down_proj"):
+        for key in ("scales", "biases"):
+            w[f"model.layers.0.{name}.{key}"][:] = 0
+    q = rng.integers(0, 16, (1000, D // 2))
+    nibbles = np.stack([q, 15 - q], axis=-1).reshape(1000, D // 8, 8).astype(np.uint32)
+    w["model.embed_tokens.weight"] = (nibbles << (4 * np.arange(8, dtype=np.uint32))).sum(-1).astype(np.uint32)
+    w["model.embed_tokens.scales"][:] = 0.25
+    w["model.embed_tokens.biases"][:] = -7.5 * 0.25
+    w["model.norm.weight"][:] = 1
+    w["lm_head.biases"][:] = 64
+    model = llama.Model.from_numpy(args, w, dev)
+    ids = rng.integers(0, 1000, (1, T))
+    got = model(to_dev(ids, dev), make_prompt_cache(model, capacity=T + 31))[0].cpu().numpy()
+    h = (np.stack([q, 15 - q], axis=-1).reshape(1000, D) - 7.5)[ids[0]] * 0.25
+    x = (h / np.sqrt((h * h).mean(1, keepdims=True) + args.rms_norm_eps)).astype(np.float16).astype(np.float64)
+    words = w["lm_head.weight"]
+    sq = ((words[..., None] >> (4 * np.arange(8, dtype=np.uint32))) & 15).reshape(1000, D).astype(np.float64) \
+        * np.repeat(w["lm_head.scales"].astype(np.float64), 64, axis=1)
+    assert rel_err(got, x @ sq.T) <= TOL

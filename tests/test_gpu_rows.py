@@ -72,3 +72,48 @@ def test_large_head(dev):
     rows = np.concatenate([np.arange(64), rng.choice(N, 400, replace=False), np.arange(N - 700, N)])
     want = oracle.qmm(x, layer["weight"][rows], layer["scales"][rows], layer["biases"][rows])
     assert rel_err(got[:, rows], want) <= TOL
+
+
+def cancelling(rng, N, K, M):
+    """Weights b + s q with b so much larger than s that fp16 would lose q, and rows of x that sum to zero in every group:
+    the product is the sum of s q x, which only unrounded weights give."""
+    layer = synth.make_qlinear(rng, N, K)
+    layer["scales"] = rng.uniform(0.005, 0.02, (N, K // 64)).astype(np.float16)
+    layer["biases"] = rng.uniform(50, 100, (N, K // 64)).astype(np.float16)
+    x = rng.standard_normal((M, K // 2, 2)).astype(np.float16)
+    x[..., 1] = -x[..., 0]
+    return layer, x.reshape(M, K)
+
+
+# rows: two blocks of 48, of 64 and less, many; N: less than a workgroup to several; K: one unit, a remainder, splits
+@pytest.mark.parametrize("M,N,K", [(65, 24, 512), (96, 1160, 896), (97, 136, 18944), (130, 904, 5248), (300, 40, 3712),
+                                   (1000, 264, 1536), (2047, 96, 1024), (2048, 16, 128), (129, 37888, 3584)])
+def test_more_rows(dev, M, N, K):
+    print(f"rows M={M} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    for layer, x in (cancelling(rng, N, K, M), (synth.make_qlinear(rng, N, K, bias=N % 16 == 8), synth.make_x(rng, M, K))):
+        d, xd = layer_to_dev(layer, dev), to_dev(x, dev)
+        pick = np.unique(np.concatenate([[0, M - 1], rng.choice(M, 22)]))
+        want = oracle.qmm(x[pick], layer["weight"], layer["scales"], layer["biases"], layer.get("bias"))
+        for split in (False, True):
+            out = torch.full((M + 1, N), float("nan"), dtype=torch.float16, device=dev)
+            rc = call(xd, d, out, False, split)
+            if rc == 2 and not split and K == 18944:
+                continue
+            assert rc == 0
+            got = out.cpu().numpy()
+            assert np.isnan(got[M].astype(np.float32)).all() and rel_err(got[pick], want) <= TOL, split
+
+
+@pytest.mark.parametrize("M,I,K", [(65, 16, 896), (100, 464, 3584), (2000, 48, 7168)])
+def test_more_rows_with_swiglu(dev, M, I, K):
+    rng = np.random.default_rng(M + I + K)
+    d = layer_to_dev(synth.make_qlinear(rng, 2 * I, K, bias=True, gain=1.0), dev)
+    x = to_dev(synth.make_x(rng, M, K), dev)
+    order = ops.interleave_gate_up(torch.arange(I, device=dev), torch.arange(I, 2 * I, device=dev)).long()
+    inter = {k: v[order].contiguous() for k, v in d.items()}
+    for split in (False, True):
+        flat = torch.empty((M, 2 * I), dtype=torch.float16, device=dev)
+        got = torch.empty((M, I), dtype=torch.float16, device=dev)
+        assert call(x, d, flat, False, split) == 0 and call(x, inter, got, True, split) == 0
+        assert torch.equal(got, ops.silu_mul(flat)), split
