@@ -18,7 +18,7 @@
  * eagle_qkv_rope_small_* (a drafter's passes), eagle_qmm_gemm_* (prompt chunks), every rope, norm,
  * attention, embedding, argmax, tree and loop-state entry point.  ON REQUEST: complete and tested,
  * but picked by a caller only: eagle_qmm_plan / eagle_qmm_w4g64_f16_tuned (a launch shape chosen by
- * hand), eagle_slab_sum_f16 (partial sums written out as a plain product),
+ * hand), eagle_qmm_gemm_plan (what the many-row product would do), eagle_slab_sum_f16 (partial sums written out as a plain product),
  * eagle_qmv_rows_w4g64_f16 at three to eight rows, eagle_qmm_w4g64_f16_noalloc (callers that cannot
  * allocate).  There are no experimental entry points.
  */
@@ -223,8 +223,11 @@ int eagle_qmm_gemm_swiglu_w4g64_f16(const void* x, const uint32_t* wq, const voi
 /* Either of the two with a workspace for products whose grid would leave most of the GPU idle (few rows, few
  * weight rows, a long K): several workgroups then share an output block, each over a part of K, and a second
  * launch adds their fp32 sums in order.  The library decides; workspace bytes 0: no split.  Same
- * roundings; workspace 16-byte aligned. */
+ * roundings; workspace 16-byte aligned.  The bytes serve any alignment of scales and biases; eagle_qmm_gemm_plan tells
+ * what is chosen for one (a power of two, in bytes): plan4 = {block (0..3: 64 x 128, 128 x 128, 128 x 256, 256 x 256 rows
+ * of x by weight rows), K groups inside a workgroup, workgroups along K, scales per fetch}. */
 size_t eagle_qmm_gemm_workspace_bytes(int M, int N, int K, int swiglu);
+int eagle_qmm_gemm_plan(int M, int N, int K, int swiglu, int sb_align, int may_split, int* plan4);
 int eagle_qmm_gemm_split_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
                                    const void* biases, const void* bias, void* out, int M, int N,
                                    int K, int group_size, int bits, int swiglu, void* workspace,

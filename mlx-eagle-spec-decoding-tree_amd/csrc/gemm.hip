@@ -1881,11 +1881,11 @@ static double gemm_cost(int block, long wgs, double steps) {
   return 4. + steps * (pair[block] * full + (rest > 1. ? pair[block] : rest > 0. ? alone[block] : 0.));
 }
 
-static GemmPlan gemm_plan(int M, int N, int K, const void* scales, const void* biases, bool swiglu, bool may_split) {
+// `sb_addr`: the addresses of scales and biases, or'ed
+static GemmPlan gemm_plan(int M, int N, int K, uintptr_t sb_addr, bool swiglu, bool may_split) {
   GemmPlan p;
   // scales and biases per fetch: as many groups as divide a row and as the base addresses are
   // aligned for
-  const uintptr_t sb_addr = reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases);
   p.sbw = (K % 512) == 0 && (sb_addr & 15u) == 0 ? 8
           : (K % 256) == 0 && (sb_addr & 7u) == 0 ? 4
           : (K % 128) == 0 && (sb_addr & 3u) == 0 ? 2
@@ -1928,15 +1928,25 @@ static GemmPlan gemm_plan(int M, int N, int K, const void* scales, const void* b
 
 EAGLE_EXPORT size_t eagle_qmm_gemm_workspace_bytes(int M, int N, int K, int swiglu) {
   if (M < 1 || N < 8 || K < 64 || (K % 64) != 0) return 0;
-  // (the fetch width, which depends on the addresses, only moves the split: the largest of the two)
+  // The alignment of scales and biases sets the fetch width and with it the split: the largest of the four.
   size_t need = 0;
-  for (uintptr_t addr = 0; addr <= 2; addr += 2) {
-    const void* a = reinterpret_cast<const void*>(addr);
-    const GemmPlan p = gemm_plan(M, N, K, a, a, swiglu != 0, true);
+  for (uintptr_t addr = 2; addr <= 16; addr *= 2) {
+    const GemmPlan p = gemm_plan(M, N, K, addr, swiglu != 0, true);
     const size_t bytes = p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
     need = bytes > need ? bytes : need;
   }
   return need;
+}
+
+EAGLE_EXPORT int eagle_qmm_gemm_plan(int M, int N, int K, int swiglu, int sb_align, int may_split, int* plan4) {
+  if (!plan4) return EAGLE_ERR_NULL;
+  if (M < 1 || N < 8 || K < 64 || (K % 64) != 0 || sb_align < 2 || (sb_align & (sb_align - 1)) != 0) return EAGLE_ERR_SHAPE;
+  const GemmPlan p = gemm_plan(M, N, K, (uintptr_t)sb_align, swiglu != 0, may_split != 0);
+  plan4[0] = p.block;
+  plan4[1] = p.kgrp;
+  plan4[2] = p.splits;
+  plan4[3] = p.sbw;
+  return EAGLE_OK;
 }
 
 static int gemm_dispatch(const void* x, const uint32_t* wq, const void* scales, const void* biases,
@@ -1957,7 +1967,8 @@ static int gemm_dispatch(const void* x, const uint32_t* wq, const void* scales, 
   const half_t* bh = static_cast<const half_t*>(biases);
   const half_t* bi = static_cast<const half_t*>(bias);
   half_t* oh = static_cast<half_t*>(out);
-  GemmPlan p = gemm_plan(M, N, K, scales, biases, swiglu, workspace != nullptr);
+  const GemmPlan p = gemm_plan(M, N, K, reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases), swiglu,
+                               workspace != nullptr);
   if (p.splits > 1 && workspace_bytes < (size_t)p.splits * M * N * sizeof(float)) return EAGLE_ERR_WORKSPACE;
   float* part = static_cast<float*>(workspace);
   int rc = EAGLE_ERR_UNSUPPORTED;

@@ -42,3 +42,26 @@ def test_split_product_with_swiglu(dev, M, I, K, bias):
     got = ops.quantized_matmul_swiglu(*args, bias=d.get("bias"))
     whole = ops.quantized_matmul_swiglu(*args, bias=d.get("bias"), gemm=True)
     close_fp16(got.cpu().numpy(), whole.cpu().numpy(), "split and whole")
+
+
+@pytest.mark.parametrize("M,N,K,align,swiglu", [(513, 3584, 18944, 8, False), (129, 3584, 3584, 4, False), (81, 2304, 3584, 4, True),
+                                                (130, 896, 4864, 2, False), (130, 264, 9344, 8, False)])
+def test_scales_off_the_widest_alignment(dev, M, N, K, align, swiglu):
+    """Scales and biases at an address that moves the split: accepted, and the product of the aligned operands."""
+    print(f"M={M} N={N} K={K} align={align}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 8), dtype=torch.int32, device=dev, generator=g)
+    s = (torch.rand((N, K // 64), device=dev, generator=g) * 0.004 + 0.001).half()
+    b = (-7.5 * s.float()).half()
+    x = torch.randn((M, K), device=dev, generator=g).half()
+
+    def moved(t):
+        room = torch.zeros(t.numel() + 8, dtype=torch.float16, device=dev)
+        off = room[align // 2:align // 2 + t.numel()].view(t.shape)
+        off.copy_(t)
+        assert off.data_ptr() % (2 * align) == align
+        return off
+
+    op = ops.quantized_matmul_swiglu if swiglu else ops.quantized_matmul
+    want = op(x, w, s, b).cpu().numpy()
+    close_fp16(op(x, w, moved(s), moved(b)).cpu().numpy(), want, "moved scales")
