@@ -224,7 +224,9 @@ def evaluate_posterior_greedy(logits, candidates):
 def tree_decoding(token_ids, tree_mask, tree_position_ids, base_model, cache):
     """mlx_eagle.py:329-346."""
     offset = cache[0].offset
-    if isinstance(base_model, Model) and isinstance(tree_mask, torch.Tensor) and tree_mask.dim() == 2:
+    # (a model with a pass of its own runs that one)
+    if getattr(type(base_model), "__call__", None) is Model.__call__ and isinstance(tree_mask, torch.Tensor) \
+            and tree_mask.dim() == 2:
         # the mask covers the tree's own rows, everything before them is visible: no [T, S] mask is built
         out = native.forward(base_model, token_ids, cache, mask=tree_mask, Tk=tree_mask.shape[1],
                              positions=tree_position_ids, pos_add=offset)

@@ -3,7 +3,7 @@ it can be checked on but runs no pass for."""
 import pytest
 import torch
 
-from mlx_eagle_spec_decoding_tree_amd import llama, native, ops, synth
+from mlx_eagle_spec_decoding_tree_amd import eagle, llama, native, ops, synth
 
 CPU = torch.device("cpu")
 FUSED = dict(hidden=1024, inter=256, heads=8, kv_heads=2, head_dim=128)
@@ -86,3 +86,26 @@ def test_uncounted_writes_reach_the_copies_after_the_call_for_them():
     again = native._derive(model, *derive_args(model))[1]
     assert int(again[1][1][0][:16].abs().max()) == 0
     assert torch.equal(again[1][1][0], ops.interleave_gate_up(gate.weight, model.layers[1].mlp.up_proj.weight))
+
+
+def test_tree_decoding_calls_a_subclass_of_the_model(monkeypatch):
+    """Its own __call__, with the mask over the whole cache; a subclass without one may take the native pass."""
+    class Own(llama.Model):
+        def __call__(self, inputs, cache=None, mask=None, position_ids=None, flat_rope=False):
+            return inputs, mask, position_ids
+
+    class Plain(llama.Model):
+        pass
+
+    class Cache:
+        offset = 5
+
+    model, ids = model_of(PLAIN), torch.arange(3)[None]
+    tree, depth = torch.zeros(3, 3), torch.arange(3)
+    monkeypatch.setattr(native, "forward", lambda *a, **k: "native")
+    model.__class__ = Own
+    got = eagle.tree_decoding(ids, tree, depth, model, [Cache()])
+    assert got[0] is ids and tuple(got[1].shape) == (1, 1, 3, 8) and got[2].tolist() == [[5, 6, 7]]
+    for cls in (Plain, llama.Model):
+        model.__class__ = cls
+        assert eagle.tree_decoding(ids, tree, depth, model, [Cache()]) == "native"
