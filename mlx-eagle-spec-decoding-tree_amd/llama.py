@@ -36,6 +36,10 @@ class Module:
         Module.epoch += 1
         object.__delattr__(self, name)
 
+    def __getstate__(self):
+        """What a copy or a file of the module holds: its native decoder belongs to these tensors and stays here."""
+        return {k: v for k, v in vars(self).items() if k not in native.KEPT}
+
     def children(self):
         for name, value in vars(self).items():
             if isinstance(value, Module):

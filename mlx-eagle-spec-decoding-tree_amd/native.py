@@ -39,9 +39,12 @@ def decoder(model):
     return handle
 
 
+KEPT = ("_native", "_native_fused")          # what is kept with a model, and made again where it is missing
+
+
 def forget(model):
     """Drop the decoder and its copies of the weights; the next pass builds them again."""
-    for key in ("_native", "_native_fused"):
+    for key in KEPT:
         model.__dict__.pop(key, None)
 
 

@@ -1,5 +1,8 @@
 """When a native decoder (native.py, csrc/decoder.cpp) is still the one of its model: built here on CPU tensors, which
 it can be checked on but runs no pass for."""
+import copy
+import pickle
+
 import pytest
 import torch
 
@@ -109,3 +112,24 @@ def test_tree_decoding_calls_a_subclass_of_the_model(monkeypatch):
     for cls in (Plain, llama.Model):
         model.__class__ = cls
         assert eagle.tree_decoding(ids, tree, depth, model, [Cache()]) == "native"
+
+
+@pytest.mark.parametrize("how", ["deepcopy", "copy", "pickle", "torch.save"])
+def test_a_model_is_copied_and_stored_after_its_first_pass(how, tmp_path):
+    """Without its decoder; the copy's next pass builds one on the copy's tensors."""
+    model = model_of(FUSED)
+    model.__dict__["_native"] = native._State(llama.Module.epoch, native._build(model, "cpu"))
+    assert "_native_fused" in vars(model)
+    if how == "deepcopy":
+        other = copy.deepcopy(model)
+    elif how == "copy":
+        other = copy.copy(model)
+    elif how == "pickle":
+        other = pickle.loads(pickle.dumps(model))
+    else:
+        torch.save(model, tmp_path / "model.pt")
+        other = torch.load(tmp_path / "model.pt", weights_only=False)          # written just above
+    assert not any(key in vars(other) for key in native.KEPT) and all(key in vars(model) for key in native.KEPT)
+    a, b = model.layers[1].mlp.up_proj.weight, other.layers[1].mlp.up_proj.weight
+    assert torch.equal(a, b) and (a.data_ptr() == b.data_ptr()) == (how == "copy")
+    assert current(native._build(other, "cpu")) and current(model.__dict__["_native"].handle)
