@@ -61,16 +61,18 @@ def _leaf(lin):
     return lin.weight, lin.scales, lin.biases, lin.bias
 
 
+def _plain(w, n, k, device):
+    """Whether (weight, scales, biases, bias or None) is a matrix [n, k] as the kernels read it."""
+    ts = [t for t in w if t is not None]
+    return (all(isinstance(t, torch.Tensor) and t.device == device and t.is_contiguous() for t in ts)
+            and w[0].dtype in (torch.int32, torch.uint32) and tuple(w[0].shape) == (n, k // 8)
+            and all(t.dtype == torch.float16 for t in ts[1:]) and all(t.data_ptr() % 16 == 0 for t in ts)
+            and tuple(w[1].shape) == tuple(w[2].shape) == (n, k // 64) and (w[3] is None or tuple(w[3].shape) == (n,)))
+
+
 def _plain_leaf(lin, n, k, device):
     from .llama import QuantizedLinear
-    if type(lin) is not QuantizedLinear or lin.group_size != 64 or lin.bits != 4:
-        return False
-    ts = [t for t in _leaf(lin) if t is not None]
-    return (all(isinstance(t, torch.Tensor) and t.device == device and t.is_contiguous() for t in ts)
-            and lin.weight.dtype in (torch.int32, torch.uint32) and tuple(lin.weight.shape) == (n, k // 8)
-            and all(t.dtype == torch.float16 for t in ts[1:]) and all(t.data_ptr() % 16 == 0 for t in ts)
-            and tuple(lin.scales.shape) == tuple(lin.biases.shape) == (n, k // 64)
-            and (lin.bias is None or tuple(lin.bias.shape) == (n,)))
+    return type(lin) is QuantizedLinear and lin.group_size == 64 and lin.bits == 4 and _plain(_leaf(lin), n, k, device)
 
 
 def _build(model, kind="cuda"):
@@ -107,15 +109,10 @@ def _build(model, kind="cuda"):
     if not all(type(n) is RMSNorm and n.eps == args.rms_norm_eps and n.weight.device == dev and n.weight.dtype == torch.float16
                and n.weight.is_contiguous() and tuple(n.weight.shape) == (D,) and n.weight.data_ptr() % 16 == 0 for n in norms):
         return None
-    head = emb if args.tie_word_embeddings else model.lm_head
-    head_w = (head.weight, head.scales, head.biases, None if head is emb else head.bias)
     emb_w = (emb.weight, emb.scales, emb.biases, None)
-    for w in (emb_w, head_w):
-        if w[0].dtype not in (torch.int32, torch.uint32) or tuple(w[0].shape) != (V, D // 8) \
-                or not all(t is None or (t.device == dev and t.is_contiguous()) for t in w):
-            return None
-    if head is not emb and not _plain_leaf(head, V, D, dev):
+    if not _plain(emb_w, V, D, dev) or not (args.tie_word_embeddings or _plain_leaf(model.lm_head, V, D, dev)):
         return None
+    head_w = emb_w if args.tie_word_embeddings else _leaf(model.lm_head)
     at0 = m.layers[0].self_attn
     if any(l.self_attn._inv_freqs is not at0._inv_freqs and not torch.equal(l.self_attn._inv_freqs, at0._inv_freqs)
            or l.self_attn._scaling_factor != at0._scaling_factor or l.self_attn.scale != at0.scale for l in m.layers):

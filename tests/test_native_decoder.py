@@ -133,3 +133,18 @@ def test_a_model_is_copied_and_stored_after_its_first_pass(how, tmp_path):
     a, b = model.layers[1].mlp.up_proj.weight, other.layers[1].mlp.up_proj.weight
     assert torch.equal(a, b) and (a.data_ptr() == b.data_ptr()) == (how == "copy")
     assert current(native._build(other, "cpu")) and current(model.__dict__["_native"].handle)
+
+
+@pytest.mark.parametrize("key,change", [("scales", lambda t: t.float()), ("biases", lambda t: t.float()), ("scales", lambda t: t.bfloat16()),
+                                        ("scales", lambda t: t[:, :-1].contiguous()), ("biases", lambda t: t[:-1].contiguous()),
+                                        ("biases", lambda t: torch.cat([t, t], 1)[:, ::2]), ("weight", lambda t: t[:-1].contiguous()),
+                                        ("scales", lambda t: torch.zeros(t.numel() + 1).half()[1:].view(t.shape))])
+@pytest.mark.parametrize("where", ["embedding", "head"])
+@pytest.mark.parametrize("tied", [False, True], ids=["own head", "tied"])
+def test_operands_of_embedding_and_head_are_checked(tied, where, key, change):
+    """Types, shapes and strides that the kernels would misread leave the pass to the operators, which convert or refuse."""
+    model = model_of(PLAIN, tie=tied)
+    assert native._build(model, "cpu") is not None
+    layer = model.model.embed_tokens if where == "embedding" or tied else model.lm_head
+    setattr(layer, key, change(getattr(layer, key)))
+    assert native._build(model, "cpu") is None
