@@ -44,11 +44,16 @@ struct Source {
   at::ScalarType type;
   at::DimVector sizes;
 
-  static int64_t version_of(const at::Tensor& t) { return t.is_inference() ? 0 : (int64_t)t._version(); }
+  // (at the implementation: seven hundred tensors are compared before a pass)
+  static int64_t version_of(const at::Tensor& t) {
+    const c10::VariableVersion& v = t.unsafeGetTensorImpl()->version_counter();
+    return v.enabled() ? (int64_t)v.current_version() : 0;
+  }
   explicit Source(const at::Tensor& t)
       : tensor(t), storage(t.storage()), ptr(t.data_ptr()), version(version_of(t)), type(t.scalar_type()), sizes(t.sizes()) {}
   bool same() const {
-    return tensor.has_storage() && tensor.data_ptr() == ptr && version_of(tensor) == version && tensor.scalar_type() == type &&
+    const c10::TensorImpl* t = tensor.unsafeGetTensorImpl();
+    return t->has_storage() && t->data() == ptr && version_of(tensor) == version && tensor.scalar_type() == type &&
            tensor.sizes() == sizes && tensor.is_contiguous();
   }
 };

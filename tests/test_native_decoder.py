@@ -148,3 +148,26 @@ def test_operands_of_embedding_and_head_are_checked(tied, where, key, change):
     layer = model.model.embed_tokens if where == "embedding" or tied else model.lm_head
     setattr(layer, key, change(getattr(layer, key)))
     assert native._build(model, "cpu") is None
+
+
+def test_assignments_elsewhere_do_not_rebuild_a_decoder(monkeypatch):
+    """Only one that changes what the model consists of does."""
+    build, built = native._build, []
+    monkeypatch.setattr(native, "_build", lambda m: built.append(m) or build(m, "cpu"))
+    model, other = model_of(FUSED), model_of(PLAIN)
+    handle = native.decoder(model)
+    assert native.decoder(model) is handle and native.decoder(other) is not None and built == [model, other]
+    other.note = 1                                                 # another model, a new module, the model's own note,
+    llama.RMSNorm(torch.ones(4), 1e-5)
+    model.note = 2
+    model.layers[0].mlp = model.layers[0].mlp                      # the same object again
+    assert native.decoder(model) is handle and native.decoder(model) is handle and len(built) == 2
+    up = model.layers[1].mlp.up_proj
+    for change in (lambda: setattr(up, "scales", up.scales.clone()), lambda: setattr(up, "group_size", 32),
+                   lambda: setattr(up, "group_size", 64), lambda: setattr(model.layers[0], "mlp", model.layers[1].mlp),
+                   lambda: model.layers.reverse(), lambda: model.weights_written(),
+                   lambda: setattr(model, "lm_head", llama.QuantizedLinear(up.weight, up.scales, up.biases))):
+        before = len(built)
+        change()
+        native.decoder(model)
+        assert len(built) == before + 1 and native.decoder(model) is native.decoder(model) and len(built) == before + 1
