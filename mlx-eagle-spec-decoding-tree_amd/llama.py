@@ -9,7 +9,8 @@ mlx_model_fwd_bench.py:43-86.
 A pass runs as one native call where `native` takes the model and the arguments; the modules below
 are the same pass operator by operator (patched layers, other caches).  There the kernels serve at
 most 32 rows per linear layer.  Passes without a mask are causal (mlx_llama.py:275-276); longer ones
-(the prompt) run as consecutive 32-token passes.
+(the prompt) run as consecutive passes of as many rows as one takes.  No product of this path rounds a
+weight, whatever its rows.
 """
 from functools import reduce
 
@@ -20,7 +21,8 @@ from . import native, ops
 from .synth import ModelArgs, inv_freqs
 
 
-CAUSAL_CHUNK = 32
+CAUSAL_CHUNK = 32              # rows of a causal pass operator by operator
+NATIVE_CHUNKS = (2048, 64)     # and of a native one: with (EAGLE_MAX_CHUNK) and without room for padding
 
 
 class Module:
@@ -246,12 +248,15 @@ class Model(Module):
         if out is not None:
             return out
         if mask is None and inputs.shape[1] > CAUSAL_CHUNK:
-            # a long causal pass (prompt prefill, mlx_eagle.py:522-533) as consecutive passes of
-            # at most 32 tokens: the kernels of this path take at most 32 rows
+            # a long causal pass (prompt prefill, mlx_eagle.py:522-533) as consecutive passes of as many tokens as
+            # one takes: natively 2048, 64 where the caches have no room for whole tiles behind them; 32 operator by
+            # operator, whose kernels take at most 32 rows
             if position_ids is not None or flat_rope:
                 raise NotImplementedError("chunked causal passes take their positions from the cache")
-            parts = [self(inputs[:, s:s + CAUSAL_CHUNK], cache)
-                     for s in range(0, inputs.shape[1], CAUSAL_CHUNK)]
+            L = inputs.shape[1]
+            steps = NATIVE_CHUNKS if native.decoder(self) is not None else ()
+            step = next((n for n in steps if L > n), CAUSAL_CHUNK)
+            parts = [self(inputs[:, s:s + step], cache) for s in range(0, L, step)]
             return torch.cat(parts, dim=1)
         out = self.model(inputs, cache, mask=mask, position_ids=position_ids, flat_rope=flat_rope)
         if self.args.tie_word_embeddings:

@@ -193,3 +193,28 @@ def test_a_prompt_rounds_no_weight(dev, form, T):
     sq = ((words[..., None] >> (4 * np.arange(8, dtype=np.uint32))) & 15).reshape(1000, D).astype(np.float64) \
         * np.repeat(w["lm_head.scales"].astype(np.float64), 64, axis=1)
     assert rel_err(got, x @ sq.T) <= TOL
+
+
+@pytest.mark.parametrize("form", ["plain", "wide"])
+@pytest.mark.parametrize("T,P,spare,parts", [(2100, 3, 30, [2048, 52]), (2048 + 97, 3, 0, [2048, 64, 33]), (2049, 0, 31, [2048, 1]),
+                                             (97, 3, 0, [64, 33]), (130, 0, 0, [64, 64, 2]), (96, 0, 0, [96])])
+def test_long_prompts_go_in_the_largest_passes(dev, form, T, P, spare, parts, monkeypatch):
+    """A prompt longer than a pass, or without room for the padding of its last one: few native calls, the bits of its parts."""
+    model = small_model(dev, form)
+    ids = to_dev(np.random.default_rng(T).integers(0, 1000, (1, T)), dev)
+    a, b = filled_cache(model, P, P + T + spare), filled_cache(model, P, P + T + 64)
+    run, taken = native.forward, []
+
+    def counted(m, ids, *args, **kw):
+        out = run(m, ids, *args, **kw)
+        if out is not None:
+            taken.append(ids.shape[1])
+        return out
+
+    monkeypatch.setattr(native, "forward", counted)
+    got = model(ids, a)
+    assert taken == parts and a[0].offset == P + T
+    ends = np.cumsum(parts)
+    want = torch.cat([model(ids[:, e - n:e], b) for n, e in zip(parts, ends)], dim=1)
+    assert torch.equal(got, want)
+    assert all(torch.equal(x.keys[:, :, :P + T], y.keys[:, :, :P + T]) for x, y in zip(a, b))
