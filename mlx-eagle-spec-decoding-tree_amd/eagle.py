@@ -356,7 +356,8 @@ def generate_step(prompt, base_model, draft_model, prefill_step_size=512, k=8, d
 def fuse_projections(model, swiglu):
     """Lay q/k/v and gate/up of every layer out as one matrix each (rows concatenated) and
     re-point the layers' tensors at row blocks of it, so that one matmul launch serves
-    the three (two) projections; memory use is unchanged."""
+    the three (two) projections; memory use is unchanged.  With swiglu, gate/up are a copy instead
+    (`native.gate_up_rows`, which the native decoder reads too)."""
     # one fused layout per model, shared by every pass object built on it
     done = getattr(model, "_fused_projections", None)
     if done is None:
@@ -364,17 +365,6 @@ def fuse_projections(model, swiglu):
     if swiglu in done:
         return done[swiglu]
     qkv_w, gu_w = [], []
-
-    def interleave(lins):
-        g, u = lins
-        fused = [ops.interleave_gate_up(getattr(g, k), getattr(u, k))
-                 for k in ("weight", "scales", "biases")]
-        bias = None
-        if g.bias is not None or u.bias is not None:
-            z = torch.zeros(g.weight.shape[0], dtype=torch.float16, device=g.weight.device)
-            bias = ops.interleave_gate_up(g.bias if g.bias is not None else z,
-                                          u.bias if u.bias is not None else z)
-        return (*fused, bias)
 
     def fuse(lins):
         parts = [[l.weight, l.scales, l.biases] for l in lins]
@@ -398,13 +388,15 @@ def fuse_projections(model, swiglu):
         at, mlp = layer.self_attn, layer.mlp
         if other is None:
             qkv_w.append(fuse([at.q_proj, at.k_proj, at.v_proj]))
-        if swiglu:
-            # a tile-interleaved copy: the layers keep their own tensors for the module path
-            gu_w.append(interleave([mlp.gate_proj, mlp.up_proj]))
-        else:
+        if not swiglu:
             gu_w.append(fuse([mlp.gate_proj, mlp.up_proj]))
+    if swiglu:
+        # a tile-interleaved copy: the layers keep their own tensors for the module path
+        gu_w = native.gate_up_rows(model)
     if other is not None:
         qkv_w = other[0]
+    else:
+        native.forget(model, "qkv")          # (a native decoder reads the layers' tensors where they now lie)
     done[swiglu] = (qkv_w, gu_w)
     return qkv_w, gu_w
 

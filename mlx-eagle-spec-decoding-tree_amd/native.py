@@ -64,13 +64,17 @@ def _parts(model):
     return found
 
 
-KEPT = ("_native", "_native_fused")          # what is kept with a model, and made again where it is missing
+KEPT = ("_native", "_laid_out")          # what is kept with a model, and made again where it is missing
 
 
-def forget(model):
-    """Drop the decoder and its copies of the weights; the next pass builds them again."""
-    for key in KEPT:
-        model.__dict__.pop(key, None)
+def forget(model, name=None):
+    """Drop the decoder and the laid-out copies of the weights (of one name: only those); whoever needs them makes
+    them again."""
+    model.__dict__.pop("_native", None)
+    if name is None:
+        model.__dict__.pop("_laid_out", None)
+    else:
+        model.__dict__.get("_laid_out", {}).pop(name, None)
 
 
 def forward(model, ids, cache, mask=None, words=None, Tk=0, positions=None, pos_add=0, pos_step=0, head=2):
@@ -163,18 +167,30 @@ def _derive(model, layers, shapes, I, D, H, G, hd):
     W = (H + 2 * G) * hd
     if D < FUSE_HIDDEN or not ops.swiglu_supported(32, I, D) or W % 16 or D % 16:
         return PLAIN, [none] * len(layers)
-    leaves = [t for lins in layers for name in ("q", "k", "v", "gate", "up") for t in _leaf(lins[name]) if t is not None]
-    if any(t.is_inference() for t in leaves):              # a write to one could not be seen
-        return PLAIN, [none] * len(layers)
-    sources = [(t.data_ptr(), t._version) for t in leaves]
-    done = model.__dict__.get("_native_fused")
+    if any(t.is_inference() for lins in layers for name in ("q", "k", "v", "gate", "up") for t in _leaf(lins[name]) if t is not None):
+        return PLAIN, [none] * len(layers)                 # a write to one could not be seen
+    qkv = _lay_out(model, "qkv", _rows, [(lins["q"], lins["k"], lins["v"]) for lins in layers])
+    return FUSED, list(zip(qkv, gate_up_rows(model)))
+
+
+def gate_up_rows(model):
+    """Per layer gate|up as `ops.interleave_gate_up` lays them out, (weight, scales, biases, bias or None): one set per
+    model, for its native decoder and its pass objects."""
+    return _lay_out(model, "gate_up", _gate_up, [(layer.mlp.gate_proj, layer.mlp.up_proj) for layer in model.model.layers])
+
+
+def _lay_out(model, name, make, groups):
+    """[make(*linears) for linears in groups], made again when a source was exchanged or torch counted a write to it."""
+    leaves = [t for linears in groups for lin in linears for t in _leaf(lin) if t is not None]
+    sources = [(t.data_ptr(), 0 if t.is_inference() else t._version) for t in leaves]
+    kept = model.__dict__.setdefault("_laid_out", {})
+    done = kept.get(name)
     if done is None or done[0] != sources:
-        model.__dict__.pop("_native_fused", None)          # the old copies go before the new ones are made
+        done = None
+        kept.pop(name, None)                               # the old copies go before the new ones are made
         # (the sources' memory is held beside them, so that an address stands for one content)
-        done = (sources, [t.detach() for t in leaves],
-                [(_rows(lins["q"], lins["k"], lins["v"]), _gate_up(lins["gate"], lins["up"])) for lins in layers])
-        model.__dict__["_native_fused"] = done
-    return FUSED, done[2]
+        done = kept[name] = sources, [t.detach() for t in leaves], [make(*linears) for linears in groups]
+    return done[2]
 
 
 def _biases(*lins):

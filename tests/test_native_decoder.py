@@ -84,7 +84,7 @@ def test_uncounted_writes_reach_the_copies_after_the_call_for_them():
     gate = model.layers[1].mlp.gate_proj
     gate.weight.data.zero_()
     again = native._derive(model, *derive_args(model))[1]
-    assert again is copies and int(again[1][1][0][:16].abs().max()) != 0
+    assert again[1][1] is copies[1][1] and int(again[1][1][0][:16].abs().max()) != 0
     model.weights_written()
     again = native._derive(model, *derive_args(model))[1]
     assert int(again[1][1][0][:16].abs().max()) == 0
@@ -119,7 +119,7 @@ def test_a_model_is_copied_and_stored_after_its_first_pass(how, tmp_path):
     """Without its decoder; the copy's next pass builds one on the copy's tensors."""
     model = model_of(FUSED)
     model.__dict__["_native"] = native._State(llama.Module.epoch, native._build(model, "cpu"))
-    assert "_native_fused" in vars(model)
+    assert "_laid_out" in vars(model)
     if how == "deepcopy":
         other = copy.deepcopy(model)
     elif how == "copy":
@@ -171,3 +171,18 @@ def test_assignments_elsewhere_do_not_rebuild_a_decoder(monkeypatch):
         change()
         native.decoder(model)
         assert len(built) == before + 1 and native.decoder(model) is native.decoder(model) and len(built) == before + 1
+
+
+@pytest.mark.parametrize("first", ["decoder", "pass object"])
+def test_decoder_and_pass_objects_share_the_laid_out_weights(first):
+    """gate|up is interleaved once, and q|k|v of a pass object are row blocks that the decoder reads in place."""
+    model = model_of(FUSED)
+    if first == "decoder":
+        assert native._build(model, "cpu") is not None
+    qkv_w, gu_w = eagle.fuse_projections(model, True)
+    assert "qkv" not in model.__dict__["_laid_out"]
+    form, copies = native._derive(model, *derive_args(model))
+    for layer, mine, (qkv, gu), fused in zip(model.layers, gu_w, copies, qkv_w):
+        assert all(a.data_ptr() == b.data_ptr() for a, b in zip(gu[:3] + qkv[:3], mine[:3] + fused[:3]))
+        assert qkv[0].data_ptr() == layer.self_attn.q_proj.weight.data_ptr()
+        assert torch.equal(gu[0], ops.interleave_gate_up(layer.mlp.gate_proj.weight, layer.mlp.up_proj.weight))
