@@ -186,10 +186,16 @@ def _lay_out(model, name, make, groups):
     kept = model.__dict__.setdefault("_laid_out", {})
     done = kept.get(name)
     if done is None or done[0] != sources:
+        dev = leaves[0].device
+        if done is not None and dev.type == "cuda":
+            torch.cuda.synchronize(dev)                    # (a pass on another stream may still read the old ones)
         done = None
         kept.pop(name, None)                               # the old copies go before the new ones are made
         # (the sources' memory is held beside them, so that an address stands for one content)
-        done = kept[name] = sources, [t.detach() for t in leaves], [make(*linears) for linears in groups]
+        done = sources, [t.detach() for t in leaves], [make(*linears) for linears in groups]
+        if dev.type == "cuda":
+            torch.cuda.current_stream(dev).synchronize()   # whichever stream reads them first, they are written
+        kept[name] = done
     return done[2]
 
 

@@ -218,3 +218,20 @@ def test_long_prompts_go_in_the_largest_passes(dev, form, T, P, spare, parts, mo
     want = torch.cat([model(ids[:, e - n:e], b) for n, e in zip(parts, ends)], dim=1)
     assert torch.equal(got, want)
     assert all(torch.equal(x.keys[:, :, :P + T], y.keys[:, :, :P + T]) for x, y in zip(a, b))
+
+
+def test_the_first_pass_on_another_stream_reads_finished_copies(dev):
+    """Copies laid out on a stream that is busy, then a pass on another one."""
+    want = same_pass(small_model(dev, "wide"), torch.arange(6, device=dev)[None], 3, 16)
+    for lay_out in (native.decoder, lambda m: eagle.fuse_projections(m, True)):
+        model = small_model(dev, "wide")
+        cache, ids = filled_cache(model, 3, 16), torch.arange(6, device=dev)[None]
+        torch.cuda.synchronize()
+        busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+        with torch.cuda.stream(busy):
+            torch.cuda._sleep(50_000_000)
+            lay_out(model)
+        with torch.cuda.stream(other):
+            got = model(ids, cache)
+        other.synchronize()
+        assert torch.equal(got, want)
