@@ -193,22 +193,13 @@ struct Pass {
   }
   int product(const Mat& m, const void* x, void* out) { return product(m, x, out, R); }
 
-  int swiglu(const Mat& m, const void* x, void* out) {
-    if (R > 2 * EAGLE_MAX_M && blocks_take(m, x, out, R, true))
-      return rows(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);
-    if (eagle_qmm_small_preferred(R, m.N, m.K) && eagle_qmm_small_supported(R, m.N, m.K, 0, 1) &&
-        small_aligned(x, m.s, m.b, m.bias, out))
-      return eagle_qmm_small_w4g64_f16(x, nullptr, 0.f, m.w, m.s, m.b, m.bias, nullptr, out, R, m.N, m.K, 64, 4, 1, st);
-    if (m.N % 32 == 0 && rows_takes(R, m.N, m.K, x, m.s, m.b, out))
-      return rows(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);
-    for (int r0 = 0; r0 < R; r0 += EAGLE_MAX_M) {
-      const int rows = std::min(R - r0, EAGLE_MAX_M);
-      Slot ws;
-      if (!qmm_workspace(like, eagle_qmm_workspace_bytes(rows, m.N, m.K), &ws)) return -1;
-      EAGLE_TRY(eagle_qmm_swiglu_w4g64_f16(static_cast<const char*>(x) + (size_t)r0 * m.K * 2, m.w, m.s, m.b, m.bias,
-                                           static_cast<char*>(out) + (size_t)r0 * m.N, rows, m.N, m.K, 64, 4, ws.ptr, ws.bytes,
-                                           st));
-    }
+  int gate_up(const Mat& m, const void* x, void* out) {
+    constexpr int PASS = 2 * EAGLE_MAX_M;
+    if (R <= PASS) return swiglu(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, st);
+    if (blocks_take(m, x, out, R, true)) return rows(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);
+    for (int r0 = 0; r0 < R; r0 += PASS)
+      EAGLE_TRY(swiglu(like, static_cast<const char*>(x) + (size_t)r0 * m.K * 2, m.w, m.s, m.b, m.bias,
+                       static_cast<char*>(out) + (size_t)r0 * m.N, std::min(R - r0, PASS), m.N, m.K, st));
     return EAGLE_OK;
   }
 
@@ -270,14 +261,14 @@ struct Pass {
     if (summed) {
       EAGLE_TRY(partial_product(l.p[O], p(attn)));
       EAGLE_TRY(eagle_rmsnorm_slabs_f16(part, splits_o, p(h), l.norm2, d.eps, p(h), p(hn), T, d.D, st));
-      EAGLE_TRY(swiglu(l.gu, p(hn), p(act)));
+      EAGLE_TRY(gate_up(l.gu, p(hn), p(act)));
       EAGLE_TRY(partial_product(l.p[DOWN], p(act)));
       return eagle_rmsnorm_slabs_f16(part, splits_down, p(h), next_norm, d.eps, p(h), p(hn), T, d.D, st);
     }
     EAGLE_TRY(product(l.p[O], p(attn), p(o)));
     EAGLE_TRY(eagle_rmsnorm_f16(p(o), p(h), l.norm2, d.eps, p(h), p(hn), R, d.D, st));
     if (fused) {
-      EAGLE_TRY(swiglu(l.gu, p(hn), p(act)));
+      EAGLE_TRY(gate_up(l.gu, p(hn), p(act)));
     } else {
       char* up = static_cast<char*>(p(gate)) + (size_t)R * d.I * 2;
       EAGLE_TRY(product(l.p[GATE], p(hn), p(gate)));

@@ -52,12 +52,12 @@ bool qmm_workspace(const at::Tensor& like, size_t need, Slot* out) {
 
 // the many-row product, split over K where the library says so
 static int gemm(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out, int M,
-                int N, int K, void* st) {
+                int N, int K, bool swiglu, void* st) {
   // the partial sums go back to torch's allocator with the launches in the stream
-  const size_t need = eagle_qmm_gemm_workspace_bytes(M, N, K, 0);
+  const size_t need = eagle_qmm_gemm_workspace_bytes(M, N, K, swiglu);
   at::Tensor ws;
   if (need) ws = empty({(int64_t)need}, at::kByte, like);
-  return eagle_qmm_gemm_split_w4g64_f16(x, static_cast<const uint32_t*>(w), s, b, bias, out, M, N, K, 64, 4, 0,
+  return eagle_qmm_gemm_split_w4g64_f16(x, static_cast<const uint32_t*>(w), s, b, bias, out, M, N, K, 64, 4, swiglu,
                                         need ? ws.data_ptr() : nullptr, need, st);
 }
 
@@ -84,7 +84,7 @@ bool small_aligned(const void* x, const void* s, const void* b, const void* bias
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
            int M, int N, int K, void* st) {
   const uint32_t* wq = static_cast<const uint32_t*>(w);
-  if (M > 2 * EAGLE_MAX_M) return gemm(like, x, w, s, b, bias, out, M, N, K, st);
+  if (M > 2 * EAGLE_MAX_M) return gemm(like, x, w, s, b, bias, out, M, N, K, false, st);
   if (M > EAGLE_MAX_M && rows_takes(M, N, K, x, s, b, out)) return rows(like, x, w, s, b, bias, out, M, N, K, false, st);
   for (int r0 = 0; r0 < M; r0 += EAGLE_MAX_M) {
     const int m = M - r0 < EAGLE_MAX_M ? M - r0 : EAGLE_MAX_M;
@@ -107,14 +107,32 @@ int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, 
   return EAGLE_OK;
 }
 
+int swiglu(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
+           int M, int N, int K, void* st) {
+  const uint32_t* wq = static_cast<const uint32_t*>(w);
+  if (M > 2 * EAGLE_MAX_M) return gemm(like, x, w, s, b, bias, out, M, N, K, true, st);
+  if (eagle_qmm_small_preferred(M, N, K) && eagle_qmm_small_supported(M, N, K, 0, 1) && small_aligned(x, s, b, bias, out))
+    return eagle_qmm_small_w4g64_f16(x, nullptr, 0.f, wq, s, b, bias, nullptr, out, M, N, K, 64, 4, 1, st);
+  if (N % 32 == 0 && rows_takes(M, N, K, x, s, b, out)) return rows(like, x, w, s, b, bias, out, M, N, K, true, st);
+  for (int r0 = 0; r0 < M; r0 += EAGLE_MAX_M) {
+    const int m = M - r0 < EAGLE_MAX_M ? M - r0 : EAGLE_MAX_M;
+    Slot ws;
+    if (!qmm_workspace(like, eagle_qmm_workspace_bytes(m, N, K), &ws)) return -1;
+    const int rc = eagle_qmm_swiglu_w4g64_f16(static_cast<const char*>(x) + (size_t)r0 * K * 2, wq, s, b, bias,
+                                              static_cast<char*>(out) + (size_t)r0 * N, m, N, K, 64, 4, ws.ptr, ws.bytes, st);
+    if (rc != EAGLE_OK) return rc;
+  }
+  return EAGLE_OK;
+}
+
 }  // namespace eagle_host
 
 namespace {
 
-// quantized_matmul(x, w_q, scales, biases, bias, out)
-PyObject* py_quantized_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
+// (x, w_q, scales, biases, bias, out) of a plain product, or of gate|up with SwiGLU
+PyObject* product(PyObject* const* a, Py_ssize_t n, bool swi, const char* name) {
   if (n != 6) {
-    PyErr_SetString(PyExc_TypeError, "quantized_matmul takes six arguments");
+    PyErr_Format(PyExc_TypeError, "%s takes six arguments", name);
     return nullptr;
   }
   const at::Tensor *x = tensor(a[0]), *w = tensor(a[1]), *s = tensor(a[2]), *b = tensor(a[3]), *bias = tensor(a[4]),
@@ -127,21 +145,27 @@ PyObject* py_quantized_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (a[4] != Py_None && !(plain(bias, at::kHalf) && bias->dim() == 1 && bias->size(0) == N)) Py_RETURN_NONE;
   const int64_t M = x->numel() / K;
   if (M < 1 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) Py_RETURN_NONE;
+  const int64_t cols = swi ? N / 2 : N;
   at::Tensor made;
   if (a[5] == Py_None) {
     at::DimVector sizes(x->sizes());
-    sizes.back() = N;
+    sizes.back() = cols;
     made = empty(sizes, at::kHalf, *x);
-  } else if (!plain(out, at::kHalf) || out->numel() != M * N) {
+  } else if (!plain(out, at::kHalf) || out->numel() != M * cols) {
     Py_RETURN_NONE;
   }
   const at::Tensor& o = a[5] == Py_None ? made : *out;
-  const int rc = matmul(*x, x->data_ptr(), w->data_ptr(), s->data_ptr(), b->data_ptr(), bias ? bias->data_ptr() : nullptr,
-                        o.data_ptr(), (int)M, (int)N, (int)K, stream_of(*x));
-  if (rc != EAGLE_OK) return fail(rc, "quantized_matmul");
+  const int rc = (swi ? swiglu : matmul)(*x, x->data_ptr(), w->data_ptr(), s->data_ptr(), b->data_ptr(),
+                                         bias ? bias->data_ptr() : nullptr, o.data_ptr(), (int)M, (int)N, (int)K, stream_of(*x));
+  if (rc != EAGLE_OK) return fail(rc, name);
   if (a[5] == Py_None) return THPVariable_Wrap(std::move(made));
   Py_INCREF(a[5]);
   return a[5];
+}
+
+PyObject* py_quantized_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) { return product(a, n, false, "quantized_matmul"); }
+PyObject* py_quantized_matmul_swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return product(a, n, true, "quantized_matmul_swiglu");
 }
 
 // rope_kv_append(q_lin, k_lin, v_lin, positions, inv_freqs, scaling_factor, q_out, k_cache, v_cache, len_dev, H, G,
@@ -365,6 +389,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 #define EAGLE_PY(name) {#name, reinterpret_cast<PyCFunction>(&guarded<py_##name>), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {EAGLE_PY(init),
                          EAGLE_PY(quantized_matmul),
+                         EAGLE_PY(quantized_matmul_swiglu),
                          EAGLE_PY(rope_kv_append),
                          EAGLE_PY(tree_attention),
                          EAGLE_PY(process_draft_tree),

@@ -53,6 +53,10 @@ int rows(const at::Tensor& like, const void* x, const void* w, const void* s, co
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
            int M, int N, int K, void* st);
 
+// silu(g) * u of interleaved gate|up rows: the rule of ops.quantized_matmul_swiglu
+int swiglu(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
+           int M, int N, int K, void* st);
+
 PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* py_decoder_current(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n);

@@ -61,9 +61,6 @@ def workspace(tag, nbytes, device):
     return buf
 
 
-ROW_PASS = 32        # rows of x the streaming kernel takes per launch
-
-
 def as_packed_u32(w_q):
     """MLX packs into uint32; torch has weak uint32 support, so int32 storage of
     the same bits is accepted too."""
@@ -300,11 +297,16 @@ def quantized_matmul_swiglu(x, w_q, scales, biases, bias=None, out=None, gemm=No
     """silu(x @ Wg.T) * (x @ Wu.T) (mlx_llama.py:214-215) in one launch: w_q / scales / biases
     / bias hold the gate and up projections interleaved by `interleave_gate_up`.  With more than
     one row, up to 32, the result equals `silu_mul` of the concatenated product bit for bit; the other forms agree with it to the tolerance of
-    the product.  33..64 rows run on the slab kernel with 64-row tiles
-    (`quantized_matmul_swiglu_slab`), more rows as the tiled GEMM form with the same epilogue
-    (`gemm=True`: that form whatever the row count).
+    the product.  Up to 64 rows no weight is rounded: the small-row kernel and that of csrc/rows.hip where the library
+    prefers them, else the streaming kernel in passes of 32 rows.  More rows run as the tiled GEMM form with the same
+    epilogue, split over K where that fills the GPU better (`gemm=True`: that form, unsplit, whatever the row count).  The
+    default path is native code (csrc/host.cpp), which the native decoder shares.
     tiled: the interleaved matrix as `TiledWeights`; up to 64 rows then run the slab kernel on
     that copy."""
+    if tiled is None and not gemm:
+        r = _native().quantized_matmul_swiglu(x, w_q, scales, biases, bias, out)
+        if r is not None:
+            return r
     _need_cuda(x, w_q, scales, biases, bias)
     x = _f16(x, "x")
     if tiled is not None and not gemm and x.numel() // x.shape[-1] <= 64:
@@ -334,45 +336,15 @@ def quantized_matmul_swiglu(x, w_q, scales, biases, bias=None, out=None, gemm=No
         bias = _f16(bias, "bias")
         if tuple(bias.shape) != (N,):
             raise ValueError("bias must have shape [N]")
+    if not gemm:                     # the arguments in plain form now
+        r = _native().quantized_matmul_swiglu(x, w_q, scales, biases, bias, out)
+        if r is None:
+            raise ValueError(f"out must be a contiguous float16 tensor of {M} x {N // 2} elements" if M > 0 else "x is empty")
+        return r
     if out is None:
         out = torch.empty((*lead, N // 2), dtype=torch.float16, device=x.device)
-    L = _lib.lib()
-    if not gemm and N % 32 == 0 and L.eagle_qmm_small_preferred(M, N, K):
-        return quantized_matmul_small(x, w_q, scales, biases, bias=bias, out=out, swiglu=True)
-    if not gemm and M <= ROW_PASS and N % 32 == 0 and L.eagle_qmm_rows_preferred(M, N, K) \
-            and (scales.data_ptr() | biases.data_ptr()) % 4 == 0:
-        need = L.eagle_qmm_rows_workspace_bytes(M, N, K)
-        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
-        rc = L.eagle_qmm_rows_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(out), M, N, K,
-                                        64, 4, 1, _ptr(ws), need, _stream())
-        _lib.check(rc, "quantized_matmul_swiglu")
-        return out
-    if not gemm and L.eagle_qmm_slab_swiglu_preferred(M, N, K):
-        # the slab kernel with one slab over all of K: above 32 rows one launch with 64-row tiles
-        # (35 us against 48..56 us for two passes of the 32-row kernel at the 7B shape), and from
-        # 24 rows where its workgroups fill the GPU in one round (the 8B shape: 24 against 27 us)
-        rc = L.eagle_qmm_slab_swiglu_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias),
-                                               _ptr(out), M, N, K, 64, 4, _stream())
-        _lib.check(rc, "quantized_matmul_swiglu")
-        return out
-    if ROW_PASS < M <= 2 * ROW_PASS and not gemm:
-        x2, out2 = x.reshape(M, K), out.view(M, N // 2)
-        for r0 in range(0, M, ROW_PASS):
-            quantized_matmul_swiglu(x2[r0:r0 + ROW_PASS], w_q, scales, biases, bias=bias,
-                                    out=out2[r0:r0 + ROW_PASS])
-        return out
-    if M > 32 or gemm:
-        # many rows (a prompt chunk): the tiled GEMM with the same epilogue, split over K where that fills
-        # the GPU better
-        need = L.eagle_qmm_gemm_workspace_bytes(M, N, K, 1) if not gemm else 0
-        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
-        rc = L.eagle_qmm_gemm_split_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias),
-                                              _ptr(out), M, N, K, 64, 4, 1, _ptr(ws), need, _stream())
-        _lib.check(rc, "quantized_matmul_swiglu")
-        return out
-    ws = workspace("qmm", L.eagle_qmm_workspace_bytes(M, N, K), x.device)
-    rc = L.eagle_qmm_swiglu_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias),
-                                      _ptr(out), M, N, K, 64, 4, _ptr(ws), ws.numel(), _stream())
+    rc = _lib.lib().eagle_qmm_gemm_swiglu_w4g64_f16(_ptr(x), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias),
+                                                    _ptr(out), M, N, K, 64, 4, _stream())
     _lib.check(rc, "quantized_matmul_swiglu")
     return out
 

@@ -5,7 +5,7 @@ import torch
 
 from mlx_eagle_spec_decoding_tree_amd import _lib, ops, synth
 from oracle import oracle
-from util import TOL, layer_to_dev, rel_err, to_dev
+from util import TOL, close_fp16, layer_to_dev, rel_err, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -117,3 +117,23 @@ def test_more_rows_with_swiglu(dev, M, I, K):
         got = torch.empty((M, I), dtype=torch.float16, device=dev)
         assert call(x, d, flat, False, split) == 0 and call(x, inter, got, True, split) == 0
         assert torch.equal(got, ops.silu_mul(flat)), split
+
+
+@pytest.mark.parametrize("M", [1, 2, 17, 32, 33, 49, 64])
+@pytest.mark.parametrize("I,K", [(464, 3584), (48, 896), (32, 192), (4096, 512)])
+def test_swiglu_of_up_to_64_rows_rounds_no_weight(dev, M, I, K):
+    """The rule of ops.quantized_matmul_swiglu, with operands at its narrowest alignment too."""
+    rng = np.random.default_rng(M + I + K)
+    layer, x = cancelling(rng, 2 * I, K, M)
+    g, u = (oracle.qmm(x, *(layer[k][h] for k in ("weight", "scales", "biases"))).astype(np.float64)
+            for h in (slice(0, I), slice(I, 2 * I)))
+    want = g / (1 + np.exp(-g)) * u
+    d, xd = layer_to_dev(layer, dev), to_dev(x, dev)
+    order = ops.interleave_gate_up(torch.arange(I, device=dev), torch.arange(I, 2 * I, device=dev)).long()
+    inter = [d[k][order].contiguous() for k in ("weight", "scales", "biases")]
+    for shift in (0, 1):
+        sb = []
+        for t in inter[1:]:
+            room = torch.zeros(t.numel() + 8, dtype=torch.float16, device=dev)
+            sb.append(room[shift:shift + t.numel()].view(t.shape).copy_(t))
+        close_fp16(ops.quantized_matmul_swiglu(xd, inter[0], *sb).cpu().numpy(), want, f"shift {shift}", rms_frac=0.2)
