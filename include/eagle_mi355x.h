@@ -19,7 +19,6 @@
  * attention, embedding, argmax, tree and loop-state entry point.  ON REQUEST: complete and tested,
  * but picked by a caller only: eagle_qmm_plan / eagle_qmm_w4g64_f16_tuned (a launch shape chosen by
  * hand), eagle_qmm_gemm_plan (what the many-row product would do), eagle_slab_sum_f16 (partial sums written out as a plain product),
- * eagle_qmm_slab_swiglu_w4g64_f16 / _preferred (row-major gate|up on the slab kernel),
  * eagle_qmv_rows_w4g64_f16 at three to eight rows, eagle_qmm_w4g64_f16_noalloc (callers that cannot
  * allocate).  There are no experimental entry points.
  */
@@ -263,8 +262,8 @@ int eagle_qmm_slab_partial_w4g64(const void* x, const uint32_t* wq, const void* 
  * [N] interleaved likewise or NULL), out [M, N/2] fp16 = silu(g) * u with the same roundings.
  * For 33..64 rows (a tree above 32 tokens) one launch in place of two of the 32-row kernel. */
 int eagle_qmm_slab_swiglu_supported(int M, int N, int K);
-/* 1 where this form measured faster than eagle_qmm_swiglu_w4g64_f16 (always above 32 rows).  The framework's own rule
- * takes eagle_qmm_rows_w4g64_f16 there, which rounds no weight. */
+/* 1 where this form measured faster than eagle_qmm_swiglu_w4g64_f16 (always above 32 rows).  It rounds the weights to
+ * fp16; eagle_qmm_rows_w4g64_f16 does not. */
 int eagle_qmm_slab_swiglu_preferred(int M, int N, int K);
 int eagle_qmm_slab_swiglu_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
                                     const void* biases, const void* bias, void* out, int M, int N, int K,

@@ -178,30 +178,17 @@ struct Pass {
 
   // more than 64 rows without rounding a weight: in blocks by one launch, or where that kernel does not take the operands
   // in passes of 64
-  bool blocks_take(const Mat& m, const void* x, const void* out, int M, bool swi) {
-    return eagle_qmm_rows_supported(M, m.N, m.K, swi) && small_aligned(x, m.s, m.b, nullptr, out);
-  }
-
   int product(const Mat& m, const void* x, void* out, int M) {
     constexpr int PASS = 2 * EAGLE_MAX_M;
     if (M <= PASS) return matmul(like, x, m.w, m.s, m.b, m.bias, out, M, m.N, m.K, st);
-    if (blocks_take(m, x, out, M, false)) return rows(like, x, m.w, m.s, m.b, m.bias, out, M, m.N, m.K, false, st);
+    if (eagle_qmm_rows_supported(M, m.N, m.K, 0) && small_aligned(x, m.s, m.b, nullptr, out))
+      return rows(like, x, m.w, m.s, m.b, m.bias, out, M, m.N, m.K, false, st);
     for (int r0 = 0; r0 < M; r0 += PASS)
       EAGLE_TRY(product(m, static_cast<const char*>(x) + (size_t)r0 * m.K * 2, static_cast<char*>(out) + (size_t)r0 * m.N * 2,
                         std::min(M - r0, PASS)));
     return EAGLE_OK;
   }
   int product(const Mat& m, const void* x, void* out) { return product(m, x, out, R); }
-
-  int gate_up(const Mat& m, const void* x, void* out) {
-    constexpr int PASS = 2 * EAGLE_MAX_M;
-    if (R <= PASS) return swiglu(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, st);
-    if (blocks_take(m, x, out, R, true)) return rows(like, x, m.w, m.s, m.b, m.bias, out, R, m.N, m.K, true, st);
-    for (int r0 = 0; r0 < R; r0 += PASS)
-      EAGLE_TRY(swiglu(like, static_cast<const char*>(x) + (size_t)r0 * m.K * 2, m.w, m.s, m.b, m.bias,
-                       static_cast<char*>(out) + (size_t)r0 * m.N, std::min(R - r0, PASS), m.N, m.K, st));
-    return EAGLE_OK;
-  }
 
   int attention(int i) {
     if (chunk)
@@ -261,14 +248,14 @@ struct Pass {
     if (summed) {
       EAGLE_TRY(partial_product(l.p[O], p(attn)));
       EAGLE_TRY(eagle_rmsnorm_slabs_f16(part, splits_o, p(h), l.norm2, d.eps, p(h), p(hn), T, d.D, st));
-      EAGLE_TRY(gate_up(l.gu, p(hn), p(act)));
+      EAGLE_TRY(swiglu(like, p(hn), l.gu.w, l.gu.s, l.gu.b, l.gu.bias, p(act), R, l.gu.N, l.gu.K, true, st));
       EAGLE_TRY(partial_product(l.p[DOWN], p(act)));
       return eagle_rmsnorm_slabs_f16(part, splits_down, p(h), next_norm, d.eps, p(h), p(hn), T, d.D, st);
     }
     EAGLE_TRY(product(l.p[O], p(attn), p(o)));
     EAGLE_TRY(eagle_rmsnorm_f16(p(o), p(h), l.norm2, d.eps, p(h), p(hn), R, d.D, st));
     if (fused) {
-      EAGLE_TRY(gate_up(l.gu, p(hn), p(act)));
+      EAGLE_TRY(swiglu(like, p(hn), l.gu.w, l.gu.s, l.gu.b, l.gu.bias, p(act), R, l.gu.N, l.gu.K, true, st));
     } else {
       char* up = static_cast<char*>(p(gate)) + (size_t)R * d.I * 2;
       EAGLE_TRY(product(l.p[GATE], p(hn), p(gate)));

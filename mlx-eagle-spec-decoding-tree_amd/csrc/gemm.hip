@@ -1551,7 +1551,8 @@ EAGLE_EXPORT int eagle_qmm_slab_swiglu_preferred(int M, int N, int K) {
   //   7B stream  23.5   22.7   27.6   28.7   48.5   56.1      (40, 64: two launches)
   //   8B slab    23.5   24.1   24.8   24.3   30.7   31.3      (224 workgroups of four waves)
   //   8B stream  20.8   21.2   26.1   27.0   45.5   52.8
-  // (eagle_qmm_rows_w4g64_f16, which the framework's own rule takes: 7B 28.3 and 36.1 at 32 and 40 rows, 42.4 at 64)
+  // (eagle_qmm_rows_w4g64_f16, graph-timed as 29.7, 37.8 and 39.1 are for the 7B slab form at 32, 40 and 64 rows: 28.3,
+  // 36.1 and 42.4.  Up to 32 rows the operator's rule asks for that one first.)
   // so: always above 32 rows; from 24 rows where workgroups of four waves fill at least half of
   // the compute units and at most all of them.
   if (!eagle_qmm_slab_swiglu_supported(M, N, K)) return 0;

@@ -107,13 +107,24 @@ int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, 
   return EAGLE_OK;
 }
 
+// what the slab kernel's SwiGLU form asks of the scales: whole fetches of eight groups, or of two for a ragged K
+static bool slab_aligned(const void* x, const void* s, const void* b, const void* bias, const void* out, int K) {
+  auto low = [](const void* p, uintptr_t bits) { return reinterpret_cast<uintptr_t>(p) & bits; };
+  const uintptr_t bits = K % 512 ? 3 : 15;
+  return !low(x, 15) && !low(out, 15) && !low(s, bits) && !low(b, bits) && !low(bias, 1);
+}
+
 int swiglu(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
-           int M, int N, int K, void* st) {
+           int M, int N, int K, bool exact, void* st) {
   const uint32_t* wq = static_cast<const uint32_t*>(w);
-  if (M > 2 * EAGLE_MAX_M) return gemm(like, x, w, s, b, bias, out, M, N, K, true, st);
+  if (M > 2 * EAGLE_MAX_M && !exact) return gemm(like, x, w, s, b, bias, out, M, N, K, true, st);
   if (eagle_qmm_small_preferred(M, N, K) && eagle_qmm_small_supported(M, N, K, 0, 1) && small_aligned(x, s, b, bias, out))
     return eagle_qmm_small_w4g64_f16(x, nullptr, 0.f, wq, s, b, bias, nullptr, out, M, N, K, 64, 4, 1, st);
-  if (N % 32 == 0 && rows_takes(M, N, K, x, s, b, out)) return rows(like, x, w, s, b, bias, out, M, N, K, true, st);
+  if (M > EAGLE_MAX_M && !exact && eagle_qmm_slab_swiglu_preferred(M, N, K) && slab_aligned(x, s, b, bias, out, K))
+    return eagle_qmm_slab_swiglu_w4g64_f16(x, wq, s, b, bias, out, M, N, K, 64, 4, st);
+  if (N % 32 == 0 && (M > 2 * EAGLE_MAX_M ? eagle_qmm_rows_supported(M, N, K, 1) && small_aligned(x, s, b, nullptr, out)
+                                          : rows_takes(M, N, K, x, s, b, out)))
+    return rows(like, x, w, s, b, bias, out, M, N, K, true, st);
   for (int r0 = 0; r0 < M; r0 += EAGLE_MAX_M) {
     const int m = M - r0 < EAGLE_MAX_M ? M - r0 : EAGLE_MAX_M;
     Slot ws;
@@ -155,8 +166,12 @@ PyObject* product(PyObject* const* a, Py_ssize_t n, bool swi, const char* name) 
     Py_RETURN_NONE;
   }
   const at::Tensor& o = a[5] == Py_None ? made : *out;
-  const int rc = (swi ? swiglu : matmul)(*x, x->data_ptr(), w->data_ptr(), s->data_ptr(), b->data_ptr(),
-                                         bias ? bias->data_ptr() : nullptr, o.data_ptr(), (int)M, (int)N, (int)K, stream_of(*x));
+  const void* bp = bias ? bias->data_ptr() : nullptr;
+  void* st = stream_of(*x);
+  const int rc = swi ? swiglu(*x, x->data_ptr(), w->data_ptr(), s->data_ptr(), b->data_ptr(), bp, o.data_ptr(), (int)M, (int)N, (int)K,
+                              false, st)
+                     : matmul(*x, x->data_ptr(), w->data_ptr(), s->data_ptr(), b->data_ptr(), bp, o.data_ptr(), (int)M, (int)N, (int)K,
+                              st);
   if (rc != EAGLE_OK) return fail(rc, name);
   if (a[5] == Py_None) return THPVariable_Wrap(std::move(made));
   Py_INCREF(a[5]);

@@ -53,9 +53,10 @@ int rows(const at::Tensor& like, const void* x, const void* w, const void* s, co
 int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
            int M, int N, int K, void* st);
 
-// silu(g) * u of interleaved gate|up rows: the rule of ops.quantized_matmul_swiglu
+// silu(g) * u of interleaved gate|up rows: the rule of ops.quantized_matmul_swiglu, or with `exact` the one of the native
+// decoder, which leaves out the forms that round the weights (the slab kernel for 33..64 rows, the GEMM above)
 int swiglu(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
-           int M, int N, int K, void* st);
+           int M, int N, int K, bool exact, void* st);
 
 PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* py_decoder_current(PyObject*, PyObject* const* a, Py_ssize_t n);

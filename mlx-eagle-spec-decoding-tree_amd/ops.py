@@ -297,10 +297,11 @@ def quantized_matmul_swiglu(x, w_q, scales, biases, bias=None, out=None, gemm=No
     """silu(x @ Wg.T) * (x @ Wu.T) (mlx_llama.py:214-215) in one launch: w_q / scales / biases
     / bias hold the gate and up projections interleaved by `interleave_gate_up`.  With more than
     one row, up to 32, the result equals `silu_mul` of the concatenated product bit for bit; the other forms agree with it to the tolerance of
-    the product.  Up to 64 rows no weight is rounded: the small-row kernel and that of csrc/rows.hip where the library
-    prefers them, else the streaming kernel in passes of 32 rows.  More rows run as the tiled GEMM form with the same
-    epilogue, split over K where that fills the GPU better (`gemm=True`: that form, unsplit, whatever the row count).  The
-    default path is native code (csrc/host.cpp), which the native decoder shares.
+    the product.  Up to 32 rows the small-row kernel and that of csrc/rows.hip where the library prefers them, else the
+    streaming kernel; 33..64 rows the slab kernel with 64-row tiles (`quantized_matmul_swiglu_slab`), which like the GEMM
+    rounds the weights to fp16, or those kernels where it does not take the operands.  More rows run as the tiled GEMM form
+    with the same epilogue, split over K where that fills the GPU better (`gemm=True`: that form, unsplit, whatever the row
+    count).  The default path is native code (csrc/host.cpp), whose function the native decoder shares.
     tiled: the interleaved matrix as `TiledWeights`; up to 64 rows then run the slab kernel on
     that copy."""
     if tiled is None and not gemm:
