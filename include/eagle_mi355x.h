@@ -338,7 +338,6 @@ typedef struct eagle_pass_begin {
   const void* norm_w;          /* [D] */
   void *h, *hn;                /* [R, D]; hn may be NULL (no norm) */
   const void* positions;       /* [T] int32 or (pos64) int64, or NULL: 0 for every row */
-  const int32_t* base_len;     /* device scalar added to every position, or NULL */
   const float* inv_freqs;      /* [half] */
   int32_t* positions_out;      /* [R] or NULL */
   float* rope_cs;              /* [R, half, 2] or NULL */
@@ -350,7 +349,7 @@ typedef struct eagle_pass_begin {
   float eps, scaling_factor;
   int ids64, pos64, mask_bits; /* mask_bits: 16 (any 16-bit float) or 32 */
   int T, R, D, V, half, Tk;
-  int pos_add, pos_step;       /* position of row t = positions[t] + *base_len + pos_add + pos_step * t */
+  int pos_add, pos_step;       /* position of row t = positions[t] + pos_add + pos_step * t */
   int write_len, attn_len;
 } eagle_pass_begin;
 int eagle_pass_begin_f16(const eagle_pass_begin* args, eagle_stream_t stream);

@@ -134,7 +134,6 @@ struct Pass {
   size_t attn_ws_bytes = 0, partial_bytes = 0;
   int splits_qkv = 0, splits_o = 0, splits_down = 0;
   bool chunk, folded, summed, fused;
-  const uint32_t* mask_words = nullptr;
   std::vector<void*> keys, values;
 
   void* p(size_t off) const { return ar.at(off); }
@@ -194,7 +193,7 @@ struct Pass {
     if (chunk)
       return eagle_causal_attention_f16(p(q_rot), keys[i], values[i], static_cast<const int32_t*>(p(pieces)), p(attn), R, d.H,
                                         d.G, d.hd, cap, S, d.scale, p(attn_ws), attn_ws_bytes, st);
-    const uint32_t* m = mask_words;
+    const uint32_t* m = static_cast<const uint32_t*>(p(words));
     if (T > EAGLE_MAX_TREE)
       return eagle_tree_attention_wide_f16(p(q_rot), keys[i], values[i], m, len(1), p(attn), T, Tk, d.H, d.G, d.hd, cap, S,
                                            d.scale, p(attn_ws), attn_ws_bytes, st);
@@ -265,12 +264,6 @@ struct Pass {
     EAGLE_TRY(product(l.p[DOWN], p(act), p(o)));
     return eagle_rmsnorm_f16(p(o), p(h), next_norm, d.eps, p(h), p(hn), R, d.D, st);
   }
-
-  // logits of `rows` rows from row0 on
-  int head(int row0, int rows, void* out) {
-    const char* x = static_cast<const char*>(p(hn)) + (size_t)row0 * d.D * 2;
-    return product(d.head, x, out, rows);
-  }
 };
 
 PyObject* str(const char* s) { return PyUnicode_InternFromString(s); }
@@ -337,31 +330,29 @@ PyObject* py_decoder_current(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Py_RETURN_TRUE;
 }
 
-// decoder_forward(capsule, ids, caches, mask, words, Tk, positions, pos_add, pos_step, head)
+// decoder_forward(capsule, ids, caches, mask, Tk, positions, pos_add, pos_step)
 //   mask: additive tensor [.., T, Tk] over the last Tk rows, or with Tk = 0 [.., T, S] (its last min(S, 64) columns are
-//   read), or None: causal, or with words given those ([T, 2] int32 mask words over the last Tk rows).  positions: int tensor [T] or None, plus pos_add + pos_step * row.
-//   head: 0 no logits, 1 of the last row, 2 of every row.
-//   Returns [1, rows, V] (True with head 0) and advances the caches' offsets; None, nothing done, where the arguments are
-//   not what this path takes.
+//   read), or None: causal.  positions: int tensor [T] or None, plus pos_add + pos_step * row.
+//   Returns the logits [1, T, V] and advances the caches' offsets; None, nothing done, where the arguments are not what
+//   this path takes.
 PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   static PyObject *s_keys = str("keys"), *s_values = str("values"), *s_offset = str("_offset");
-  Decoder* d = n == 10 ? static_cast<Decoder*>(PyCapsule_GetPointer(a[0], "eagle.decoder")) : nullptr;
+  Decoder* d = n == 8 ? static_cast<Decoder*>(PyCapsule_GetPointer(a[0], "eagle.decoder")) : nullptr;
   if (!d) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "decoder_forward takes ten arguments");
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "decoder_forward takes eight arguments");
     return nullptr;
   }
-  const at::Tensor *ids = tensor(a[1]), *mask = tensor(a[3]), *words = tensor(a[4]), *pos = tensor(a[6]);
+  const at::Tensor *ids = tensor(a[1]), *mask = tensor(a[3]), *pos = tensor(a[5]);
   if (!ids || !ids->is_cuda() || !ids->is_contiguous() || ids->dim() != 2 || ids->size(0) != 1 || ids->size(1) < 1 ||
       (ids->scalar_type() != at::kInt && ids->scalar_type() != at::kLong) || ids->device() != d->kept[0].tensor.device())
     Py_RETURN_NONE;
   const int64_t T = ids->size(1);
-  const bool causal = a[3] == Py_None && a[4] == Py_None;
-  if (T > (causal ? EAGLE_MAX_CHUNK : EAGLE_MAX_TREE_SLOTS) || (a[3] != Py_None && !mask) || (a[4] != Py_None && !words)) Py_RETURN_NONE;
-  if (a[6] != Py_None &&
+  if (T > (a[3] == Py_None ? EAGLE_MAX_CHUNK : EAGLE_MAX_TREE_SLOTS) || (a[3] != Py_None && !mask)) Py_RETURN_NONE;
+  if (a[5] != Py_None &&
       !(pos && pos->is_cuda() && pos->is_contiguous() && pos->numel() == T && (pos->scalar_type() == at::kInt || pos->scalar_type() == at::kLong)))
     Py_RETURN_NONE;
-  long Tk = PyLong_AsLong(a[5]);
-  const long pos_add = PyLong_AsLong(a[7]), pos_step = PyLong_AsLong(a[8]), head = PyLong_AsLong(a[9]);
+  long Tk = PyLong_AsLong(a[4]);
+  const long pos_add = PyLong_AsLong(a[6]), pos_step = PyLong_AsLong(a[7]);
   if (PyErr_Occurred()) return nullptr;
 
   // the caches: of this framework's class, all at one length
@@ -406,8 +397,6 @@ PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     b.mask_bits = mt == at::kFloat ? 32 : 16;
     b.mask_ld = mask->stride(-2);
     b.mask = static_cast<const char*>(mask->data_ptr()) + (cols - Tk) * (b.mask_bits / 8);
-  } else if (words) {
-    if (!plain(words, at::kInt) || words->numel() != 2 * T || Tk < 1 || Tk > 64 || Tk > S) Py_RETURN_NONE;
   } else {
     Tk = chunk ? 32 : (S < 64 ? S : 64);
   }
@@ -420,9 +409,7 @@ PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (chunk && (ps.S < 32 || d->D > 8192)) Py_RETURN_NONE;
   const at::Tensor buffers = empty({(int64_t)ps.ar.size}, at::kByte, *ids);
   ps.ar.base = static_cast<char*>(buffers.data_ptr());
-  const int64_t rows = head == 2 ? T : head == 1 ? 1 : 0;
-  at::Tensor logits;
-  if (rows) logits = empty({1, rows, d->V}, at::kHalf, *ids);
+  at::Tensor logits = empty({1, T, d->V}, at::kHalf, *ids);
 
   b.ids = ids->data_ptr();
   b.ids64 = ids->scalar_type() == at::kLong;
@@ -454,16 +441,14 @@ PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   b.attn_len = (int)(S - Tk);
   if (chunk)
     b.piece_len = static_cast<int32_t*>(ps.p(ps.pieces));
-  else if (!words)
+  else
     b.words = static_cast<uint32_t*>(ps.p(ps.words));
-  ps.mask_words = words ? static_cast<const uint32_t*>(words->data_ptr()) : b.words;
   int rc = eagle_pass_begin_f16(&b, ps.st);
   const int nl = (int)d->layers.size();
   for (int i = 0; rc == EAGLE_OK && i < nl; ++i) rc = ps.layer(i, i + 1 < nl ? d->layers[i + 1].norm1 : d->norm);
-  if (rc == EAGLE_OK && rows) {
-    if (ps.folded) rc = eagle_rmsnorm_f16(ps.p(ps.h), nullptr, d->norm, d->eps, nullptr, ps.p(ps.hn), (int)T, d->D, ps.st);
-    if (rc == EAGLE_OK) rc = ps.head((int)(T - rows), (int)rows, logits.data_ptr());
-  }
+  if (rc == EAGLE_OK && ps.folded)
+    rc = eagle_rmsnorm_f16(ps.p(ps.h), nullptr, d->norm, d->eps, nullptr, ps.p(ps.hn), (int)T, d->D, ps.st);
+  if (rc == EAGLE_OK) rc = ps.product(d->head, ps.p(ps.hn), logits.data_ptr(), (int)T);
   if (rc != EAGLE_OK) return fail(rc, "decoder pass");
   PyObject* end = PyLong_FromLong(S);
   for (Py_ssize_t i = 0; end && i < PyList_GET_SIZE(a[2]); ++i)
@@ -472,7 +457,6 @@ PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return nullptr;
     }
   Py_XDECREF(end);
-  if (!rows) Py_RETURN_TRUE;
   return THPVariable_Wrap(std::move(logits));
 }
 

@@ -361,7 +361,6 @@ __global__ __launch_bounds__(BLOCK) void pass_begin_kernel(eagle_pass_begin a) {
   int pos = a.pos_add + a.pos_step * r;
   if (a.positions)
     pos += a.pos64 ? (int)static_cast<const int64_t*>(a.positions)[src] : static_cast<const int32_t*>(a.positions)[src];
-  if (a.base_len) pos += *a.base_len;
 
   // embedding row and its norm, vector c of the row in thread c % BLOCK as in rmsnorm_kernel
   const int nvec = a.D >> 3;

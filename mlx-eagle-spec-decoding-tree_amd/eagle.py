@@ -404,43 +404,26 @@ def fuse_projections(model, swiglu):
 
 
 def tile_model(model):
-    """The q|k|v, o, gate|up (interleaved) and down matrices of every layer as `ops.TiledWeights`, with the
-    bias of the product (q|k|v, gate|up) or None: one [(tiled, bias) x 4] per layer.  One set per model,
-    rebuilt when a source tensor was exchanged or written to; the copies are slices of two allocations."""
-    sources, layers = [], []
+    """The q|k|v, o, gate|up (interleaved) and down matrices of every layer as `ops.TiledWeights`: one list of four per
+    layer, slices of two allocations."""
+    groups = []
     for layer in model.model.layers:
         at, mlp = layer.self_attn, layer.mlp
-        groups = ([at.q_proj, at.k_proj, at.v_proj], [at.o_proj], [mlp.gate_proj, mlp.up_proj], [mlp.down_proj])
-        layers.append(groups)
-        sources += [(t.data_ptr(), 0 if t.is_inference() else t._version) for g in groups for lin in g
-                    for t in (lin.weight, lin.scales, lin.biases, lin.bias) if t is not None]
-    done = model.__dict__.get("_tiled_model")
-    if done is not None and done[0] == sources:
-        return done[1]
-    dev = model.model.layers[0].self_attn.q_proj.weight.device
-    sizes = [(sum(lin.weight.shape[0] for lin in g), g[0].weight.shape[1] * 8) for groups in layers for g in groups]
+        groups += [[at.q_proj, at.k_proj, at.v_proj], [at.o_proj], [mlp.gate_proj, mlp.up_proj], [mlp.down_proj]]
+    dev = groups[0][0].weight.device
+    sizes = [(sum(lin.weight.shape[0] for lin in g), g[0].weight.shape[1] * 8) for g in groups]
     wt = torch.empty(sum(n * k // 8 for n, k in sizes), dtype=torch.int32, device=dev)
     sbt = torch.empty(sum(n * k // 32 for n, k in sizes), dtype=torch.float16, device=dev)
     worst = torch.zeros(len(sizes), dtype=torch.float32, device=dev)
     made, w0, s0 = [], 0, 0
-    for i, (g, (n, k)) in enumerate(zip((g for groups in layers for g in groups), sizes)):
+    for i, (g, (n, k)) in enumerate(zip(groups, sizes)):
         w1, s1 = w0 + n * k // 8, s0 + n * k // 32
         made.append(ops.tile_parts(g, len(g) == 2, wt[w0:w1].view(n // 32, k // 64, 64, 4),
                                    sbt[s0:s1].view(n // 32, k // 512, 64, 8), worst[i:i + 1]))
         w0, s0 = w1, s1
     for t, m in zip(made, worst.tolist()):
         t.small = m < ops.TILED_SMALL_SCALE
-
-    def bias_of(g):
-        if all(lin.bias is None for lin in g):
-            return None
-        parts = [lin.bias if lin.bias is not None else torch.zeros(lin.weight.shape[0], dtype=torch.float16, device=dev)
-                 for lin in g]
-        return ops.interleave_gate_up(*parts) if len(g) == 2 else torch.cat(parts)
-
-    out = [[(t, bias_of(g)) for t, g in zip(made[4 * i:4 * i + 4], groups)] for i, groups in enumerate(layers)]
-    model.__dict__["_tiled_model"] = (sources, out)
-    return out
+    return [made[i:i + 4] for i in range(0, len(made), 4)]
 
 
 def tiled_projections(model, qkv_w, gu_w, plan, swiglu):
@@ -463,7 +446,7 @@ def tiled_projections(model, qkv_w, gu_w, plan, swiglu):
             qkv_w[0], gu_w[0], (model.model.layers[0].self_attn.o_proj.weight,),
             (model.model.layers[0].mlp.down_proj.weight,))):
         sets = tile_model(model)
-        done[key] = {name: [entry[j][0] for entry in sets] for j, name in enumerate(("qkv", "o", "gu", "down"))}
+        done[key] = {name: [entry[j] for entry in sets] for j, name in enumerate(("qkv", "o", "gu", "down"))}
         return done[key]
     out = {"qkv": [], "o": [], "down": [], "gu": []}
     for i, layer in enumerate(model.model.layers):

@@ -272,7 +272,7 @@ class Model(Module):
         or another library on the same memory): every laid-out copy of them is dropped and made again when it is next
         needed.  Pass objects built before (`TreeVerifier`, `SpeculativeDecoder`, ...) keep theirs and are built anew."""
         native.forget(self)
-        for key in ("_fused_projections", "_tiled_model", "_tiled_projections", "_tiled_head"):
+        for key in ("_fused_projections", "_tiled_projections", "_tiled_head"):
             self.__dict__.pop(key, None)
 
 

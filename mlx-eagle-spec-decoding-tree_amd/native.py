@@ -77,13 +77,13 @@ def forget(model, name=None):
         model.__dict__.get("_laid_out", {}).pop(name, None)
 
 
-def forward(model, ids, cache, mask=None, words=None, Tk=0, positions=None, pos_add=0, pos_step=0, head=2):
-    """One pass (see decoder_forward in csrc/decoder.cpp): logits [1, rows, V], True with head=0, or None
-    where this path does not take the arguments (nothing has been done then)."""
+def forward(model, ids, cache, mask=None, Tk=0, positions=None, pos_add=0, pos_step=0):
+    """One pass (see decoder_forward in csrc/decoder.cpp): logits [1, T, V], or None where this path does not take
+    the arguments (nothing has been done then)."""
     handle = decoder(model)
     if handle is None:
         return None
-    return ops._native().decoder_forward(handle, ids, cache, mask, words, Tk, positions, pos_add, pos_step, head)
+    return ops._native().decoder_forward(handle, ids, cache, mask, Tk, positions, pos_add, pos_step)
 
 
 def _leaf(lin):
