@@ -136,7 +136,7 @@ int eagle_qmm_rows_partial_w4g64(const void* x, const uint32_t* wq, const void* 
  *   x [T, D] fp16; rope_cs [T, hd / 2, 2] fp32; q_out [H, T, hd] fp16; k_cache, v_cache
  *   [G, capacity, hd] fp16 (rows *cache_len_dev + t are written; rows at or past capacity are not).
  * Constraints (eagle_qkv_rope_small_supported): T <= 16, D a multiple of 128 up to 6144, hd a
- * multiple of 32. */
+ * multiple of 32; alignment as for eagle_qmm_small_w4g64_f16. */
 int eagle_qkv_rope_small_supported(int T, int D, int H, int G, int hd);
 int eagle_qkv_rope_small_w4g64_f16(const void* x, const void* norm_w, float eps, const uint32_t* wq,
                                    const void* scales, const void* biases, const void* bias,

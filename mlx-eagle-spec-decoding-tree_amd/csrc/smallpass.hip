@@ -426,6 +426,12 @@ void small_launch(const SmallArgs& a, int grid, hipStream_t st) {
   return norm ? small_go<16, 3, MODE, true>(a, grid, st) : small_go<16, 3, MODE, false>(a, grid, st);
 }
 
+// two scales or biases of a row are one load, four values of the bias another
+bool small_vectors_aligned(const void* scales, const void* biases, const void* bias) {
+  return ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 3u) == 0 &&
+         (reinterpret_cast<uintptr_t>(bias) & 7u) == 0;
+}
+
 }  // namespace
 
 EAGLE_EXPORT int eagle_qmm_small_supported(int T, int N, int K, int norm, int swiglu) {
@@ -464,6 +470,7 @@ EAGLE_EXPORT int eagle_qmm_small_w4g64_f16(const void* x, const void* norm_w, fl
   const void* aligned[] = {x, norm_w, wq, residual, out};
   for (const void* p : aligned)
     if (p && !eagle_aligned16(p)) return EAGLE_ERR_ALIGN;
+  if (!small_vectors_aligned(scales, biases, bias)) return EAGLE_ERR_ALIGN;
   if (x == out) return EAGLE_ERR_UNSUPPORTED;          // other workgroups still read x
   SmallArgs a;
   a.x = static_cast<const half_t*>(x);
@@ -509,6 +516,7 @@ EAGLE_EXPORT int eagle_qkv_rope_small_w4g64_f16(const void* x, const void* norm_
   const void* aligned[] = {x, norm_w, wq, rope_cs, q_out, k_cache, v_cache};
   for (const void* p : aligned)
     if (p && !eagle_aligned16(p)) return EAGLE_ERR_ALIGN;
+  if (!small_vectors_aligned(scales, biases, bias)) return EAGLE_ERR_ALIGN;
   SmallArgs a;
   a.x = static_cast<const half_t*>(x);
   a.norm_w = static_cast<const half_t*>(norm_w);

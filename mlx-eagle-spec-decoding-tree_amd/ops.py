@@ -43,6 +43,11 @@ def _f16(t, name):
     return t.contiguous()
 
 
+def _at(t, nbytes):
+    """t, or a copy of it where its address is not a multiple of nbytes (a kernel loads vectors of that size from it)."""
+    return t if t.data_ptr() % nbytes == 0 else t.clone()
+
+
 def workspace(tag, nbytes, device):
     """A zero-initialised device buffer that persists between calls (and across
     HIP-graph replays).  It only grows; growing is not graph-capture safe, so
@@ -421,9 +426,12 @@ def quantized_matmul_small(x, w_q, scales, biases, bias=None, out=None, norm_wei
     if w_q.shape[1] * 8 != K or tuple(scales.shape) != (N, K // 64) or tuple(biases.shape) != (N, K // 64):
         raise ValueError(f"shape mismatch: x {tuple(x.shape)}, w {tuple(w_q.shape)}, "
                          f"scales {tuple(scales.shape)}, biases {tuple(biases.shape)}")
+    scales, biases = _at(scales, 4), _at(biases, 4)
     n_out = N // 2 if swiglu else N
-    if bias is not None and tuple(_f16(bias, "bias").shape) != (N,):
-        raise ValueError("bias must have shape [N]")
+    if bias is not None:
+        bias = _at(_f16(bias, "bias"), 8)
+        if tuple(bias.shape) != (N,):
+            raise ValueError("bias must have shape [N]")
     if norm_weight is not None and tuple(_f16(norm_weight, "norm_weight").shape) != (K,):
         raise ValueError("norm_weight must have shape [K]")
     if out is None:
@@ -456,9 +464,10 @@ def qkv_rope_small(x, w_q, scales, biases, bias, rope_cs, q_rot, k_cache, v_cach
     for t in (q_rot, k_cache, v_cache, rope_cs):
         if not t.is_contiguous():
             raise ValueError("non-contiguous buffer")
+    scales, biases = _at(_f16(scales, "scales"), 4), _at(_f16(biases, "biases"), 4)
+    bias = bias if bias is None else _at(bias, 8)
     rc = _lib.lib().eagle_qkv_rope_small_w4g64_f16(
-        _ptr(x), _ptr(norm_weight), float(eps), _ptr(w_q), _ptr(_f16(scales, "scales")), _ptr(_f16(biases, "biases")),
-        _ptr(bias), _ptr(rope_cs), _ptr(q_rot), _ptr(k_cache), _ptr(v_cache), _ptr(cache_len_dev), T, D, H, G, hd,
+        _ptr(x), _ptr(norm_weight), float(eps), _ptr(w_q), _ptr(scales), _ptr(biases), _ptr(bias), _ptr(rope_cs), _ptr(q_rot), _ptr(k_cache), _ptr(v_cache), _ptr(cache_len_dev), T, D, H, G, hd,
         k_cache.shape[-2], 64, 4, _stream())
     _lib.check(rc, "qkv_rope_small")
     return q_rot

@@ -53,3 +53,29 @@ def test_operands_it_does_not_take(dev):
         e = dict(d, **{key: off})
         out = ops.quantized_matmul(x, e["weight"], e["scales"], e["biases"], bias=e["bias"])
         assert rel_err(out.cpu().numpy(), got.astype(np.float64)) <= TOL
+
+
+def test_small_row_forms_take_any_alignment(dev):
+    """The forms that a caller asks for by name: operands off the kernel's alignment are copied, same bits."""
+    T, D, H, G, hd = 5, 256, 4, 2, 64
+    W, rng = (H + 2 * G) * hd, np.random.default_rng(1)
+    d = layer_to_dev(synth.make_qlinear(rng, W, D, bias=True), dev)
+    x = to_dev(synth.make_x(rng, T, D), dev)
+
+    def moved(t):
+        room = torch.zeros(t.numel() + 1, dtype=torch.float16, device=dev)
+        return room[1:].view(t.shape).copy_(t)
+
+    def qkv(scales, biases, bias):
+        q = torch.zeros((H, T, hd), dtype=torch.float16, device=dev)
+        k, v = (torch.zeros((G, 16, hd), dtype=torch.float16, device=dev) for _ in range(2))
+        ops.qkv_rope_small(x, d["weight"], scales, biases, bias, cs, q, k, v, torch.zeros(1, dtype=torch.int32, device=dev), H, G, hd)
+        return torch.cat([q.flatten(), k.flatten(), v.flatten()])
+
+    cs = ops.rope_table(torch.arange(T, dtype=torch.int32, device=dev), ops.default_inv_freqs(hd, device=dev))
+    plain = [d["scales"], d["biases"], d["bias"]]
+    want = ops.quantized_matmul_small(x, d["weight"], *plain[:2], bias=plain[2]), qkv(*plain)
+    for i in range(3):
+        e = [moved(t) if i == j else t for j, t in enumerate(plain)]
+        assert torch.equal(ops.quantized_matmul_small(x, d["weight"], *e[:2], bias=e[2]), want[0])
+        assert torch.equal(qkv(*e), want[1])

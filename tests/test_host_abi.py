@@ -270,3 +270,17 @@ def test_gemm_refuses_an_x_beyond_32_bit_indexing():
     p = (ctypes.addressof(buf) + 15) & ~15
     assert L.eagle_qmm_gemm_w4g64_f16(p, p, p, p, None, p, 1 << 20, 64, 2048, 64, 4, None) == 2
     assert L.eagle_qmm_gemm_w4g64_f16(None, p, p, p, None, p, 64, 64, 2048, 64, 4, None) == 1
+
+
+def test_small_row_products_check_the_alignment_of_their_vectors():
+    """Scales and biases are loaded four bytes at a time, the bias eight: refused on the host off these."""
+    L = _lib.lib()
+    buf = (ctypes.c_char * 4096)()
+    p = (ctypes.addressof(buf) + 15) & ~15
+    q = p + 512
+    small = lambda s, b, bias: L.eagle_qmm_small_w4g64_f16(p, None, 1e-6, p, s, b, bias, None, q, 4, 64, 128, 64, 4, 0, None)
+    rope = lambda s, b, bias: L.eagle_qkv_rope_small_w4g64_f16(p, None, 1e-6, p, s, b, bias, p, q, q, q, p, 4, 128, 2, 1, 64, 64,
+                                                               64, 4, None)
+    for call in (small, rope):
+        for operands in ((p + 2, p, None), (p, p + 2, None), (p, p, p + 2), (p, p, p + 4)):
+            assert call(*operands) == 3
