@@ -35,6 +35,21 @@ __device__ inline float wave_max(float v) {
   return v;
 }
 
+// Eight nibbles -> fp16 q, exact, in the order q0 q2 q4 q6 q1 q3 q5 q7.  A byte that holds a nibble is, read as OCP e4m3,
+// q * 2^-9 (subnormals up to 7, the first exponents up to 15), so the fp8 conversion gives the fp16 values of q two at a
+// time: seven instructions per packed word.
+__device__ inline half8_t eagle_expand8(uint32_t w) {
+  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
+  union { half2_t h2[4]; half8_t h8; } o;
+  o.h2[0] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, false);
+  o.h2[1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, true);
+  o.h2[2] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, false);
+  o.h2[3] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, true);
+  return o.h8;
+}
+// eight values of x in that order
+__device__ inline half8_t eagle_permute8(half8_t v) { return half8_t{v[0], v[2], v[4], v[6], v[1], v[3], v[5], v[7]}; }
+
 // Rows of a partial tile of the slab form: 32 for up to 32 rows of x, 64 for 33..64.
 __host__ __device__ inline int eagle_slab_rows(int M) { return M > 32 ? 64 : 32; }
 

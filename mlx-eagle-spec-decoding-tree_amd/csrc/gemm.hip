@@ -110,20 +110,14 @@ __device__ inline half8_t dequant_word_sub(uint32_t w, half2_t s20, half2_t b2) 
   return o;
 }
 
-// Through the fp8 conversion: a byte that holds a nibble is q * 2^-9 exactly when read as OCP e4m3, so two
-// conversions per four nibbles give fp16 q, and one packed fma fp16(s*q + b) with a single rounding, any scale: as
-// many instructions as the forms above, no offset to prepare.  Order q0 q2 q4 q6 q1 q3 q5 q7.
-__device__ inline half8_t permute8_fp8(half8_t v) { return half8_t{v[0], v[2], v[4], v[6], v[1], v[3], v[5], v[7]}; }
+// Through the fp8 conversion (eagle_expand8): one packed fma fp16(s*q + b) with a single rounding, any scale: as many
+// instructions as the forms above, no offset to prepare.
 __device__ inline half8_t dequant_word_fp8(uint32_t w, half2_t s2, half2_t b2) {
-  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
-  const half2_t c[4] = {__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, false),
-                        __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, true),
-                        __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, false),
-                        __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, true)};
+  const half8_t q = eagle_expand8(w);
   half8_t o;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const half2_t v = __builtin_elementwise_fma(c[i], s2, b2);
+    const half2_t v = __builtin_elementwise_fma(half2_t{q[2 * i], q[2 * i + 1]}, s2, b2);
     o[2 * i] = v[0];
     o[2 * i + 1] = v[1];
   }
@@ -275,7 +269,7 @@ __global__ __launch_bounds__(256 * KGRP, (KGRP == 1 && !DEEP ? 2 : 1)) void qmm_
     };
     auto write_x = [&](half_t* buf, int set, int from, int to) {
 #pragma unroll
-      for (int g = from; g < to; ++g) *reinterpret_cast<half8_t*>(buf + (xr + 32 * g) * XS + xc * 8) = permute8_fp8(xreg[set][g]);
+      for (int g = from; g < to; ++g) *reinterpret_cast<half8_t*>(buf + (xr + 32 * g) * XS + xc * 8) = eagle_permute8(xreg[set][g]);
     };
     auto load_x = [&](int ks, int set, int from, int to) {
 #pragma unroll

@@ -49,20 +49,6 @@ constexpr int ROWS_LDS = 160 * 1024;
 constexpr int ROWS_RSRC = 0x00020000;      // buffer descriptor: untyped bytes
 constexpr int ROWS_XROW = 256 + 16;        // bytes of a staged x row: a chunk of 128 columns, padded against bank conflicts
 
-__device__ inline half8_t rows_permute8(half8_t v) { return half8_t{v[0], v[2], v[4], v[6], v[1], v[3], v[5], v[7]}; }
-
-// eight nibbles -> fp16 q, in the order q0 q2 q4 q6 q1 q3 q5 q7: a byte that holds a nibble is q * 2^-9 as OCP
-// e4m3, so the fp8 conversion gives fp16 q exactly, two at a time
-__device__ inline half8_t rows_expand(uint32_t w) {
-  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
-  union { half2_t h2[4]; half8_t h8; } o;
-  o.h2[0] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, false);
-  o.h2[1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, true);
-  o.h2[2] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, false);
-  o.h2[3] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, true);
-  return o.h8;
-}
-
 // a barrier that leaves the loads from memory in flight
 __device__ inline void rows_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -162,7 +148,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
     for (int i = 0; i < NP; ++i) {
       const int at = i * ROWS_WAVES + wave, slot = at / QUADS, row = at % QUADS * 4 + xr4;
       const half8_t v = __builtin_bit_cast(half8_t, xr[i]);
-      *reinterpret_cast<half8_t*>(buf + slot * SLOT + row * ROWS_XROW + xpc * 16) = rows_permute8(v);
+      *reinterpret_cast<half8_t*>(buf + slot * SLOT + row * ROWS_XROW + xpc * 16) = eagle_permute8(v);
       const half2_t one = {(half_t)1.f, (half_t)1.f};
       float sum = 0.f;
 #pragma unroll
@@ -304,7 +290,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
         reload(t);
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-          const half8_t q0 = rows_expand(v[2 * g]), q1 = rows_expand(v[2 * g + 1]);
+          const half8_t q0 = eagle_expand8(v[2 * g]), q1 = eagle_expand8(v[2 * g + 1]);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) d[t & 1][g][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[mt][g][0], q0, zero, 0, 0, 0);
 #pragma unroll
@@ -325,7 +311,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
           if (g == 0) regroup(ring[u % AH][t]);
-          const half8_t q0 = rows_expand(ring[u % AH][t][2 * g]), q1 = rows_expand(ring[u % AH][t][2 * g + 1]);
+          const half8_t q0 = eagle_expand8(ring[u % AH][t][2 * g]), q1 = eagle_expand8(ring[u % AH][t][2 * g + 1]);
           if (g == 1) reload(t);
           float4_t d[MT];
 #pragma unroll

@@ -41,24 +41,6 @@ namespace {
 
 typedef __attribute__((address_space(3))) float4_t sp_lds_float4;
 
-// x in the order of the expanded weights below
-__device__ inline half8_t sp_permute8(half8_t v) {
-  return half8_t{v[0], v[2], v[4], v[6], v[1], v[3], v[5], v[7]};
-}
-
-// eight nibbles -> fp16 q, in the order q0 q2 q4 q6 q1 q3 q5 q7.  A byte that holds a nibble is, read as OCP
-// e4m3, q * 2^-9 exactly (subnormals up to 7, the first exponent up to 15), so the fp8 conversion gives the
-// fp16 values of q two at a time: seven instructions.
-__device__ inline half8_t sp_expand(uint32_t w) {
-  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
-  union { half2_t h2[4]; half8_t h8; } o;
-  o.h2[0] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, false);
-  o.h2[1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, true);
-  o.h2[2] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, false);
-  o.h2[3] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, true);
-  return o.h8;
-}
-
 struct SmallArgs {
   const half_t* x;          // [T, K]
   const half_t* norm_w;     // [K] or nullptr
@@ -272,8 +254,8 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
       float4_t sx[2];
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
-        xb[c][2 * g] = sp_permute8(xb[c][2 * g]);
-        xb[c][2 * g + 1] = sp_permute8(xb[c][2 * g + 1]);
+        xb[c][2 * g] = eagle_permute8(xb[c][2 * g]);
+        xb[c][2 * g + 1] = eagle_permute8(xb[c][2 * g + 1]);
         sx[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g], ones, zero, 0, 0, 0);
         sx[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g + 1], ones, sx[g], 0, 0, 0);
       }
@@ -287,8 +269,8 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
         for (int g = 0; g < 2; ++g) {
           const float sc = (float)__builtin_bit_cast(half_t, (unsigned short)(g ? s2 >> 16 : s2 & 0xffffu));
           const float bi = (float)__builtin_bit_cast(half_t, (unsigned short)(g ? b2 >> 16 : b2 & 0xffffu));
-          float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g], sp_expand(w02[g]), zero, 0, 0, 0);
-          d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g + 1], sp_expand(w13[g]), d, 0, 0, 0);
+          float4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g], eagle_expand8(w02[g]), zero, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g + 1], eagle_expand8(w13[g]), d, 0, 0, 0);
 #pragma unroll
           for (int i = 0; i < 4; ++i) acc[t][i] = __builtin_fmaf(bi, sx[g][i], __builtin_fmaf(sc, d[i], acc[t][i]));
         }
