@@ -13,6 +13,7 @@
  *
  * Two groups.  DEFAULT: what the library's own verification step, draft loop and prompt pass
  * call when nothing is chosen by hand: eagle_qmm_w4g64_f16 (+ _workspace_bytes), eagle_qmm_swiglu_*,
+ * eagle_qmm_rows_* (17 rows up, and every product of a prompt of the module path), eagle_pass_begin_f16,
  * eagle_qmm_slab_* (partial sums, SwiGLU, their tiled forms and eagle_qmm_tile_w4g64),
  * eagle_qmv_w4g64_f16 / eagle_qmv_rows_w4g64_f16 (one and two rows), eagle_qmm_small_* and
  * eagle_qkv_rope_small_* (a drafter's passes), eagle_qmm_gemm_* (prompt chunks), every rope, norm,
@@ -204,8 +205,8 @@ int eagle_qmm_swiglu_w4g64_f16(const void* x, const uint32_t* wq, const void* sc
                                int M, int N, int K, int group_size, int bits,
                                void* workspace, size_t workspace_bytes, eagle_stream_t stream);
 
-/* The same product for any number of rows M, as a tiled MFMA GEMM (128 x 128 output blocks,
- * weights expanded to fp16 in registers): the form for the prompt pass (mlx_eagle.py:522-533,
+/* The same product for any number of rows M, as a tiled MFMA GEMM (output blocks of 64 x 128 to
+ * 256 x 256, weights expanded and rounded to fp16 in registers): the form for the prompt pass (mlx_eagle.py:522-533,
  * where mlx_model_fwd_bench.py:65-73 falls back to mx.quantized_matmul because the row count is
  * not 8..32).  Bound by the matrix cores, not by the weight stream, from a few hundred rows on.
  * No workspace.  N % 8 == 0, K % 64 == 0; bias (may be NULL) 8-byte aligned. */

@@ -260,8 +260,8 @@ def accept_candidate(cache, accept_indices, accept_length, offset):
 
 def _check_tree_size(verify_num_tokens):
     """The tree kernels lay a tree out in 64 slots (root + 63 nodes), which covers the reference's
-    default of 39 nodes (mlx_eagle.py:390,510): above 32 tokens the matmuls run as two passes of
-    32 rows and attention over two mask words per query in pieces of 32 queries."""
+    default of 39 nodes (mlx_eagle.py:390,510): above 32 tokens the products run with 64-row tiles
+    and attention over two mask words per query in pieces of 32 queries."""
     if verify_num_tokens + 1 > TREE_SLOTS:
         raise NotImplementedError(
             f"verify_num_tokens={verify_num_tokens}: this build verifies at most {TREE_SLOTS - 1} draft nodes "
@@ -535,7 +535,7 @@ class TreeVerifier:
     into `tokens`, `tree_position_ids`, `mask_index` and `mask_bits`; results appear in
     `logits`, `node_argmax`, `result` (best, accept_length, bonus_node, next_token,
     accept_indices...) and `accepted_tokens`; the cache length advances on the device.
-    Same kernels and operator order as Model.__call__ + the host functions above."""
+    Same operator order as Model.__call__ + the host functions above."""
 
     def __init__(self, model, cache, total_tokens=31, max_len=None, compact=True, fuse=True,
                  swiglu=True, slab_plan=None, tiled=None):
@@ -552,9 +552,9 @@ class TreeVerifier:
                                       f"(total_tokens <= {TREE_SLOTS - 1})")
         self.V = total_tokens
         self.T = T = total_tokens + 1
-        # above 32 tree tokens: q|k|v, o and down in the slab form with 64-row partial tiles, the
-        # other matmuls in two passes of the 32-row streaming kernel, two mask words per token and
-        # attention in pieces of 32 query rows (one launch pair)
+        # above 32 tree tokens: q|k|v, o, down and gate|up in the slab form with 64-row tiles where the shapes
+        # allow it, the tiled head in two passes, other products on the kernels of `ops.quantized_matmul`; two
+        # mask words per token and attention in pieces of 32 query rows (one launch pair)
         self.wide = T > MAXT
         if self.wide and not fuse:
             raise ValueError(f"a tree of more than {MAXT} tokens runs with the fused projections only")
@@ -621,7 +621,7 @@ class TreeVerifier:
         # size every workspace before any capture
         L = _lib.lib()
         head = model.lm_head if not args.tie_word_embeddings else model.model.embed_tokens
-        # (a tree above 32 tokens goes through the 32-row matmul kernel in two passes)
+        # (what the streaming kernel needs of it: a tree above 32 tokens takes that in two passes)
         need = max(L.eagle_qmm_workspace_bytes(rows, n, k) for n, k in
                    ((H * hd, D), (G * hd, D), ((H + 2 * G) * hd, D), (D, H * hd), (I, D), (2 * I, D),
                     (D, I), (head.weight.shape[0], D))
@@ -727,8 +727,8 @@ class TreeVerifier:
                                               c0.capacity, st), "kv_compact")
 
     def _layer_one_launch_per_projection(self, i, layer):
-        """fuse=False: the kernels and launch shapes of the module path (one launch per
-        projection), on the static buffers."""
+        """fuse=False: one launch per projection, as the layers operator by operator, on the
+        static buffers."""
         m, args, T = self.model, self.args, self.T
         H, G, hd = args.num_attention_heads, args.num_key_value_heads, args.head_dim
         layers = m.model.layers

@@ -1,14 +1,13 @@
 """Llama / Qwen2 decoder with the tree-decoding arguments of the reference model
 (mlx_llama.py:21-323): `Model(inputs, cache, mask, position_ids, flat_rope)`.
 
-Same module tree and the same operator boundaries as the reference, so that the
-fp16 roundings fall in the same places; every operator runs as a HIP kernel
-behind the C ABI.  `patch_model(model, kernel)` is the plug-in seam of
-mlx_model_fwd_bench.py:43-86.
+Same module tree and the same operator boundaries as the reference; every operator runs as a HIP kernel
+behind the C ABI.  `patch_model(model, kernel)` is the plug-in seam of mlx_model_fwd_bench.py:43-86.
 
-A pass runs as one native call where `native` takes the model and the arguments; the modules below
-are the same pass operator by operator (patched layers, other caches).  There the kernels serve at
-most 32 rows per linear layer.  Passes without a mask are causal (mlx_llama.py:275-276); longer ones
+A pass runs as one native call where `native` takes the model and the arguments: the same values, with fewer
+fp16 roundings between operators than the reference has where its products are fused (partial sums, folded norms).  The
+modules below are the pass operator by operator (patched layers, other caches), with the roundings where the
+reference has them.  There the kernels serve at most 32 rows per linear layer.  Passes without a mask are causal (mlx_llama.py:275-276); longer ones
 (the prompt) run as consecutive passes of as many rows as one takes.  No product of this path rounds a
 weight, whatever its rows.
 """

@@ -136,7 +136,8 @@ class DecoderPass:
 
 class ChunkPass:
     """A causal pass of R rows (a multiple of 32, at most 2048) through a decoder: the linear
-    layers see all R rows at once (the tiled GEMM form of the matmul above 32 rows), so do rope
+    layers see all R rows at once (the tiled GEMM form of the matmul above 64 rows, which rounds the weights to
+    fp16; `Model.__call__` has prompt passes that do not), so do rope
     and the cache append; attention runs per piece of 32 rows (all pieces in one launch), every
     piece seeing the cache rows before it and its own rows causally.  Rows are appended at the cache length, which advances by R."""
 
@@ -154,7 +155,7 @@ class ChunkPass:
         H, G, hd = args.num_attention_heads, args.num_key_value_heads, args.head_dim
         self.max_len = max_len or cache[0].capacity
         self.T = R
-        # above 32 rows: the tiled GEMM form everywhere, gate|up with the SwiGLU epilogue
+        # above 64 rows: the tiled GEMM form everywhere, gate|up with the SwiGLU epilogue
         self.swiglu = bool(ops.swiglu_supported(R, args.intermediate_size, args.hidden_size))
         self.qkv_w, self.gu_w = fuse_projections(model, self.swiglu)
         self.slab = {"qkv": 0, "o": 0, "down": 0}

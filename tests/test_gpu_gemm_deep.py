@@ -1,5 +1,5 @@
 """The many-row product (blocks of 64 x 128 to 256 x 256, K a multiple of 256): edges of the blocks, the shortest loops,
-against the same product in passes of up to 64 rows."""
+against the product in 64 bits and the same product in passes of up to 64 rows."""
 import pytest
 import torch
 
@@ -18,6 +18,18 @@ def layer_on(dev, N, K, bias):
     return w, s, b, torch.randn(N, device=dev, generator=g).half() if bias else None
 
 
+# Every weight is rounded to fp16 once and so is the result: each error is at most 2^-11 of its value, and errors of
+# different weights do not line up, so the two together stay below sqrt(2) 2^-11 = 6.9e-4 of the result's norm.
+ROUNDED = 7e-4
+
+
+def product64(x, w, s, b, bias):
+    q = (w[..., None] >> (4 * torch.arange(8, device=w.device, dtype=torch.int32))) & 15
+    wide = lambda t: t.double().repeat_interleave(64, dim=1)  # noqa: E731
+    y = x.double() @ (q.reshape(w.shape[0], -1).double() * wide(s) + wide(b)).T
+    return y if bias is None else y + bias.double()
+
+
 @pytest.mark.parametrize("M,N,K,bias", [(65, 8, 256, True), (129, 264, 512, False), (257, 136, 768, True), (300, 1000, 2304, False),
                                         (513, 4616, 1024, True), (2048, 4608, 512, False), (700, 18944, 256, True),
                                         (1100, 9000, 1536, False), (2047, 3592, 1280, True)])
@@ -33,6 +45,9 @@ def test_products(dev, M, N, K, bias):
     assert err <= 1e-3 and (out[:M].float() - want).abs().amax() <= TOL * want.square().mean().sqrt()
     whole = ops.quantized_matmul(x, w, s, b, bias=bi, gemm=True).float()      # never split over K
     assert (whole - want).norm() / want.norm() <= 1e-3
+    exact = product64(x, w, s, b, bi)
+    for y in (out[:M], whole):
+        assert (y.double() - exact).norm() / exact.norm() <= ROUNDED
 
 
 @pytest.mark.parametrize("M,I,K", [(65, 16, 256), (130, 208, 512), (300, 9472, 768), (1030, 4624, 1024), (2048, 2320, 512)])
@@ -46,3 +61,8 @@ def test_swiglu(dev, M, I, K):
     for gemm in (None, True):
         got = ops.quantized_matmul_swiglu(x, *inter[:3], bias=inter[3], gemm=gemm).float()
         assert tuple(got.shape) == (M, I) and (got - want).norm() / want.norm() <= 2e-3
+    # gate and up each within ROUNDED of their norm, silu's slope at most 1.1, and two more fp16 roundings
+    g, u = product64(x, w, s, b, bi).split(I, dim=1)
+    exact = torch.nn.functional.silu(g) * u
+    bound = ROUNDED * (1.1 * g.norm() * u.square().mean().sqrt() + u.norm() * torch.nn.functional.silu(g).square().mean().sqrt())
+    assert (got.double() - exact).norm() <= bound + 2 ** -10 * exact.norm()
