@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <unordered_set>
 #include <vector>
 
 namespace eagle_host {
@@ -51,11 +52,12 @@ struct Source {
   }
   explicit Source(const at::Tensor& t)
       : tensor(t), storage(t.storage()), ptr(t.data_ptr()), version(version_of(t)), type(t.scalar_type()), sizes(t.sizes()) {}
-  bool same() const {
-    const c10::TensorImpl* t = tensor.unsafeGetTensorImpl();
-    return t->has_storage() && t->data() == ptr && version_of(tensor) == version && tensor.scalar_type() == type &&
-           tensor.sizes() == sizes && tensor.is_contiguous();
+  bool same(const at::Tensor& now) const {
+    const c10::TensorImpl* t = now.unsafeGetTensorImpl();
+    return t->has_storage() && t->data() == ptr && version_of(now) == version && now.scalar_type() == type &&
+           now.sizes() == sizes && now.is_contiguous();
   }
+  bool same() const { return same(tensor); }
 };
 
 struct Decoder {
@@ -270,6 +272,83 @@ PyObject* str(const char* s) { return PyUnicode_InternFromString(s); }
 
 }  // namespace
 
+// The tensors of a list as they are now
+static bool list_sources(PyObject* list, std::vector<const at::Tensor*>* out) {
+  if (!PyList_Check(list)) return false;
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); ++i) {
+    out->push_back(tensor(PyList_GET_ITEM(list, i)));
+    if (!out->back() || !out->back()->has_storage()) return false;
+  }
+  return true;
+}
+
+// module_parts(roots, Module) -> every attribute of the modules among `roots` and of those they hold, in order (a few
+// thousand objects, 30 us; a walk in Python takes ten times that)
+PyObject* py_module_parts(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 2 || !PyList_Check(a[0]) || !PyType_Check(a[1])) {
+    PyErr_SetString(PyExc_TypeError, "module_parts takes a list and a type");
+    return nullptr;
+  }
+  PyTypeObject* type = reinterpret_cast<PyTypeObject*>(a[1]);
+  PyObject* found = PyList_GetSlice(a[0], 0, PyList_GET_SIZE(a[0]));
+  std::vector<PyObject*> todo;                       // (all held by `found` or by the roots)
+  std::unordered_set<PyObject*> seen;
+  auto look = [&](PyObject* o) {
+    if (PyObject_TypeCheck(o, type)) todo.push_back(o);
+  };
+  for (Py_ssize_t i = 0; found && i < PyList_GET_SIZE(found); ++i) look(PyList_GET_ITEM(found, i));
+  while (found && !todo.empty()) {
+    PyObject* m = todo.back();
+    todo.pop_back();
+    if (!seen.insert(m).second) continue;
+    PyObject* dict = PyObject_GenericGetDict(m, nullptr);
+    PyObject *key, *value;
+    Py_ssize_t at = 0;
+    bool ok = dict != nullptr;
+    while (ok && PyDict_Next(dict, &at, &key, &value)) {
+      ok = PyList_Append(found, value) == 0;
+      look(value);
+      for (Py_ssize_t i = 0; ok && PyList_Check(value) && i < PyList_GET_SIZE(value); ++i) {
+        ok = PyList_Append(found, PyList_GET_ITEM(value, i)) == 0;
+        look(PyList_GET_ITEM(value, i));
+      }
+    }
+    Py_XDECREF(dict);
+    if (!ok) Py_CLEAR(found);
+  }
+  return found;
+}
+
+// sources_new(tensors) -> capsule: their addresses, sizes and versions, their memory held with it
+PyObject* py_sources_new(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  std::vector<const at::Tensor*> ts;
+  if (n != 1 || !list_sources(a[0], &ts)) {
+    PyErr_SetString(PyExc_TypeError, "sources_new takes a list of tensors");
+    return nullptr;
+  }
+  std::unique_ptr<std::vector<Source>> made(new std::vector<Source>());
+  for (const at::Tensor* t : ts) made->emplace_back(*t);
+  PyObject* cap = PyCapsule_New(made.get(), "eagle.sources", [](PyObject* c) {
+    delete static_cast<std::vector<Source>*>(PyCapsule_GetPointer(c, "eagle.sources"));
+  });
+  if (cap) made.release();
+  return cap;
+}
+
+// sources_current(capsule, tensors): these tensors lie where those lay, and no write to them was counted
+PyObject* py_sources_current(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  auto* of = n == 2 ? static_cast<std::vector<Source>*>(PyCapsule_GetPointer(a[0], "eagle.sources")) : nullptr;
+  std::vector<const at::Tensor*> ts;
+  if (!of || !list_sources(a[1], &ts)) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "sources_current takes a capsule and a list of tensors");
+    return nullptr;
+  }
+  if (ts.size() != of->size()) Py_RETURN_FALSE;
+  for (size_t i = 0; i < ts.size(); ++i)
+    if (!(*of)[i].same(*ts[i])) Py_RETURN_FALSE;
+  Py_RETURN_TRUE;
+}
+
 // decoder_new(ints, floats, emb, head, norm, inv_freqs, layers, layer_list, cache_type) -> capsule
 //   ints: (D, I, H, G, hd, V, form); floats: (eps, rope_factor, scale); layers: per layer (seven projections, qkv, gu,
 //   two norms)
@@ -282,6 +361,7 @@ PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return nullptr;
   }
   std::unique_ptr<Decoder> d(new Decoder());
+  d->kept.reserve(PyList_GET_SIZE(a[6]) * 40 + 16);
   d->D = v[0]; d->I = v[1]; d->H = v[2]; d->G = v[3]; d->hd = v[4]; d->V = v[5]; d->form = v[6];
   d->eps = f[0]; d->rope_factor = f[1]; d->scale = f[2];
   d->emb = take_mat(d.get(), a[2]);

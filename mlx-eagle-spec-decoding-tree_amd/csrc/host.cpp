@@ -410,6 +410,9 @@ PyMethodDef methods[] = {EAGLE_PY(init),
                          EAGLE_PY(process_draft_tree),
                          EAGLE_PY(post_process_draft_tree),
                          EAGLE_PY(tile_parts),
+                         EAGLE_PY(module_parts),
+                         EAGLE_PY(sources_new),
+                         EAGLE_PY(sources_current),
                          EAGLE_PY(decoder_new),
                          EAGLE_PY(decoder_current),
                          EAGLE_PY(decoder_forward),

@@ -58,6 +58,9 @@ int matmul(const at::Tensor& like, const void* x, const void* w, const void* s, 
 int swiglu(const at::Tensor& like, const void* x, const void* w, const void* s, const void* b, const void* bias, void* out,
            int M, int N, int K, bool exact, void* st);
 
+PyObject* py_module_parts(PyObject*, PyObject* const* a, Py_ssize_t n);
+PyObject* py_sources_new(PyObject*, PyObject* const* a, Py_ssize_t n);
+PyObject* py_sources_current(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* py_decoder_new(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* py_decoder_current(PyObject*, PyObject* const* a, Py_ssize_t n);
 PyObject* py_decoder_forward(PyObject*, PyObject* const* a, Py_ssize_t n);

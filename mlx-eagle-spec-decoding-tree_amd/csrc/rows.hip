@@ -78,7 +78,8 @@ size_t rows_lds_bytes(int RT, int MT, int KP, int nu, bool both) {
   return stage > epi ? stage : epi;
 }
 
-template <int RT, int MT, int KP, int AH>
+// MANY: more than one block of x rows
+template <int RT, int MT, int KP, int AH, bool MANY>
 __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
   constexpr int B = rows_block(MT, KP);            // chunks per K part and block of staged x
   constexpr int ROWS = 16 * MT;                    // rows of x
@@ -92,9 +93,9 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r = lane & 15, kq = lane >> 4;
   const int kp = wave % KP, rg = wave / KP;
-  const int nb = a.zb == 1 ? blockIdx.x : blockIdx.x / a.zb;            // weight rows, then block of x
-  const int m0 = (blockIdx.x - nb * a.zb) * ROWS;
-  const int K = a.K, M = a.M - m0 < ROWS ? a.M - m0 : ROWS, N = a.N;
+  const int nb = MANY ? blockIdx.x / a.zb : blockIdx.x;                  // weight rows, then block of x
+  const int m0 = MANY ? (blockIdx.x - nb * a.zb) * ROWS : 0;
+  const int K = a.K, M = MANY && a.M - m0 > ROWS ? ROWS : a.M - m0, N = a.N;
   const int all = K >> 7;
   // K in units of four chunks (512 columns), dealt over the workgroups along y and then over the K parts
   const int units = (all + 3) >> 2;
@@ -437,7 +438,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
   }
 }
 
-template <int RT, int MT, int KP, int AH>
+template <int RT, int MT, int KP, int AH, bool MANY>
 int rows_launch(const RowsArgs& a, int splits, hipStream_t st) {
   constexpr int WROWS = ROWS_WAVES / KP * RT * 16;
   const int units = ((a.K >> 7) + 3) / 4, most = (units + splits - 1) / splits, nu = (most + KP - 1) / KP;
@@ -448,12 +449,12 @@ int rows_launch(const RowsArgs& a, int splits, hipStream_t st) {
   if (lds > ROWS_LDS) return EAGLE_ERR_SHAPE;
   static bool ready = false;             // (set twice by two first calls at once: the same value)
   if (!ready) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&qmm_rows_kernel<RT, MT, KP, AH>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&qmm_rows_kernel<RT, MT, KP, AH, MANY>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, ROWS_LDS) != hipSuccess)
       return EAGLE_ERR_HIP;
     ready = true;
   }
-  hipLaunchKernelGGL((qmm_rows_kernel<RT, MT, KP, AH>), dim3((a.N + WROWS - 1) / WROWS * b.zb, splits), dim3(ROWS_WAVES * 64), lds, st, b);
+  hipLaunchKernelGGL((qmm_rows_kernel<RT, MT, KP, AH, MANY>), dim3((a.N + WROWS - 1) / WROWS * b.zb, splits), dim3(ROWS_WAVES * 64), lds, st, b);
   return eagle_launch_status();
 }
 
@@ -488,9 +489,17 @@ __global__ __launch_bounds__(256) void rows_sum_kernel(const float* __restrict__
 struct RowsForm {
   int rt, mt, kp;
   int (*launch)(const RowsArgs&, int, hipStream_t);
+  int (*launch_many)(const RowsArgs&, int, hipStream_t);      // more than 64 rows (blocks of 48 or 64), or nullptr
 };
+template <int RT, int MT, int KP, int AH>
+constexpr RowsForm rows_form() {
+  if constexpr (MT >= 3)
+    return {RT, MT, KP, rows_launch<RT, MT, KP, AH, false>, rows_launch<RT, MT, KP, AH, true>};
+  else
+    return {RT, MT, KP, rows_launch<RT, MT, KP, AH, false>, nullptr};
+}
 const RowsForm rows_forms[] = {
-#define ROWS_FORM(RT, MT, KP, AH) {RT, MT, KP, rows_launch<RT, MT, KP, AH>}
+#define ROWS_FORM(RT, MT, KP, AH) rows_form<RT, MT, KP, AH>()
     ROWS_FORM(1, 1, 1, 4), ROWS_FORM(1, 1, 2, 4), ROWS_FORM(1, 1, 4, 4), ROWS_FORM(2, 1, 1, 4), ROWS_FORM(3, 1, 1, 4),
     ROWS_FORM(3, 1, 4, 2), ROWS_FORM(5, 1, 1, 2), ROWS_FORM(5, 1, 4, 2),
     ROWS_FORM(1, 2, 1, 4), ROWS_FORM(1, 2, 2, 4), ROWS_FORM(1, 2, 4, 4), ROWS_FORM(2, 2, 1, 4), ROWS_FORM(2, 2, 2, 4),
@@ -623,7 +632,8 @@ EAGLE_EXPORT int eagle_qmm_rows_w4g64_f16(const void* x, const uint32_t* wq, con
   a.both = 0;
   a.pitch = M;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int rc = rows_forms[p.form].launch(a, p.splits, st);
+  const RowsForm& form = rows_forms[p.form];
+  const int rc = (M > 2 * EAGLE_MAX_M ? form.launch_many : form.launch)(a, p.splits, st);
   if (rc != EAGLE_OK || p.splits == 1) return rc;
   const dim3 grid((unsigned)(((long)M * ((swiglu ? N / 2 : N) / 8) + 255) / 256));
   if (swiglu)

@@ -398,7 +398,7 @@ def fuse_projections(model, swiglu):
     else:
         native.forget(model, "qkv")          # (a native decoder reads the layers' tensors where they now lie)
     if qkv_w[0][0].is_cuda:
-        torch.cuda.current_stream(qkv_w[0][0].device).synchronize()    # (a pass on another stream may read them first)
+        torch.cuda.synchronize(qkv_w[0][0].device)    # (a pass on another stream may read them first)
     done[swiglu] = (qkv_w, gu_w)
     return qkv_w, gu_w
 
