@@ -25,7 +25,8 @@
 // back to back over rotating weights): 32 x 3584 x 152064 71 / 80, 27 x 18944 x 3584 18 / 23, 32 x 2048 x 8192 8.2 / 11.0,
 // 64 x 8192 x 8192 24 / 40.  With many rows the vector instructions (expansion per block, a multiply-add per group and
 // output) about equal the matrix instructions: 2048 x 37888 x 3584 675 us = 0.82 PFLOP/s, 512 x 3584 x 18944 114 us; the
-// GEMM, which rounds the weights to fp16 and expands them once per 256 rows, takes 580 and 93.
+// GEMM, which rounds the weights to fp16 and expands them once per 256 rows, takes 580 and 93.  In a prompt pass, weights
+// not in a cache: 732 and (2048 x 3584 x 18944) 372 us against 553 and 263; counters in profiles/products_sq_counters.md.
 #include "common.h"
 
 namespace {
@@ -516,14 +517,14 @@ struct RowsPlan {
   int form, splits;
 };
 
-// The division of the work with the least predicted time (us).  Fitted to 1600 timings (7 % rms): K 896 .. 18944,
-// N 512 .. 152064, 8 .. 64 rows, every form, launches back to back over rotating weights.  A compute unit takes
+// The division of the work with the least predicted time (us), from a model fitted to timings of every form, launches
+// back to back over rotating weights.  A compute unit takes
 // its workgroups one after the other; each costs its start, its share of the weights and its x at the rates a
 // unit ingests them (40 and 72 GB/s), and 0.22 us per unit of four chunks, tile and 16 rows of x.  What the whole
 // grid reads counts a little, a split as much as its second launch and the partial sums (the sums alone where
-// the consumer of the product adds them).  For 65 .. 2048 rows the same formula over the blocks of x: over 12600 random
-// products, each in every form and split, its choice took 1.2 % longer than the best on average, 7.5 % at the 95th
-// percentile, 25 % at most.
+// the consumer of the product adds them).  For 65 .. 2048 rows the same formula over the blocks of x.  Its choice against
+// the best of all forms and splits of random products (profiles/form_choice_sweeps.md): 17 .. 64 rows 1.4 % longer on
+// average, 8 % at the 95th percentile (up to 16 rows, most of which other kernels serve, 4 and 16); 65 .. 2048 rows 1.2 and 7.5.
 enum { ROWS_WHOLE = 0, ROWS_SPLIT = 1, ROWS_PARTIAL = 2 };
 RowsPlan rows_find_plan(int M, int N, int K, int mode) {
   const int units = ((K >> 7) + 3) / 4;
