@@ -708,7 +708,9 @@ def small_m_bench(opt):
                 t_v = float(np.median(graph_time_ms(torch, valu, reps=7)[0])) * 1e3 / iters
                 rec["valu_us"] = round(t_v, 2)
                 rec["valu_frac"] = round(byts / t_v / 1e3 / HBM_PEAK_GBS, 4)
-            rec["dispatched_to"] = "valu" if ops.qmv_preferred(N, K, M) else "mfma"
+            # the order in which quantized_matmul asks; "mfma" is the streaming kernel
+            rec["dispatched_to"] = ("small" if L.eagle_qmm_small_preferred(M, N, K) else "valu" if ops.qmv_preferred(N, K, M)
+                                    else "rows" if L.eagle_qmm_rows_preferred(M, N, K) else "mfma")
             rows.append(rec)
             print(f"[small-m] {rec}", file=sys.stderr, flush=True)
         del ws, ss, bs
