@@ -50,6 +50,8 @@ def decoder(model):
     del st
     parts = _parts(model)
     handle = _build(model)
+    if handle is None:
+        forget(model)                            # (pass objects hold the copies that they use)
     model.__dict__["_native"] = _State(epoch, handle, parts, list(model.__dict__.get("_laid_out", {}).values()))
     return handle
 
@@ -67,10 +69,11 @@ def forget(model, name=None):
     """Drop the decoder and the laid-out copies of the weights (of one name: only those); whoever needs them makes
     them again."""
     model.__dict__.pop("_native", None)
-    if name is None:
-        model.__dict__.pop("_laid_out", None)
-    else:
-        model.__dict__.get("_laid_out", {}).pop(name, None)
+    kept = model.__dict__.get("_laid_out", {})
+    for key in list(kept) if name is None else [name]:
+        if key in kept:
+            kept[key].unused()
+            del kept[key]
 
 
 def forward(model, ids, cache, mask=None, Tk=0, positions=None, pos_add=0, pos_step=0):
@@ -181,12 +184,9 @@ def _lay_out(model, name, make, groups):
     kept = model.__dict__.setdefault("_laid_out", {})
     done = kept.get(name)
     if done is None or not ops._native().sources_current(done.sources, leaves):
-        dev = leaves[0].device
-        if done is not None and dev.type == "cuda":
-            torch.cuda.synchronize(dev)                    # (a pass on another stream may still read the old ones)
         done = None
-        kept.pop(name, None)                               # the old copies go before the new ones are made
-        done = kept[name] = _LaidOut(ops._native().sources_new(leaves), [make(*linears) for linears in groups], dev)
+        forget(model, name)                                # the old copies go before the new ones are made
+        done = kept[name] = _LaidOut(ops._native().sources_new(leaves), [make(*linears) for linears in groups], leaves[0].device)
     done.wait()
     return done.copies
 
@@ -198,6 +198,11 @@ class _LaidOut:
     def __init__(self, sources, copies, dev):
         self.sources, self.copies, self.dev = sources, copies, dev
         self.ready = torch.cuda.current_stream(dev).record_event() if dev.type == "cuda" else None
+
+    def unused(self):
+        """Returns when no stream reads the copies any more."""
+        if self.dev.type == "cuda":
+            torch.cuda.synchronize(self.dev)
 
     def wait(self):
         """Whatever the current stream enqueues from here on finds the copies written."""

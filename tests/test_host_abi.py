@@ -284,3 +284,13 @@ def test_small_row_products_check_the_alignment_of_their_vectors():
     for call in (small, rope):
         for operands in ((p + 2, p, None), (p, p + 2, None), (p, p, p + 2), (p, p, p + 4)):
             assert call(*operands) == 3
+
+
+def test_rows_form_takes_a_prompt_but_leaves_partial_sums_for_64_rows():
+    L = _lib.lib()
+    assert L.eagle_qmm_rows_supported(2048, 64, 128, 0) == 1 and L.eagle_qmm_rows_supported(2049, 64, 128, 0) == 0
+    assert L.eagle_qmm_rows_preferred(64, 3584, 3584) == 1 and L.eagle_qmm_rows_preferred(65, 3584, 3584) == 0
+    assert L.eagle_qmm_rows_partial_splits(64, 3584, 3584) > 0 and L.eagle_qmm_rows_partial_splits(65, 3584, 3584) == 0
+    for M in (65, 512, 2048):                   # room for every split that the plan can take, without overflow
+        for N, K in ((512, 18944), (3584, 3584), (152064, 3584), (16, 128)):
+            assert L.eagle_qmm_rows_workspace_bytes(M, N, K) % (4 * M * N) == 0

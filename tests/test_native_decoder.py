@@ -186,3 +186,23 @@ def test_decoder_and_pass_objects_share_the_laid_out_weights(first):
         assert all(a.data_ptr() == b.data_ptr() for a, b in zip(gu[:3] + qkv[:3], mine[:3] + fused[:3]))
         assert qkv[0].data_ptr() == layer.self_attn.q_proj.weight.data_ptr()
         assert torch.equal(gu[0], ops.interleave_gate_up(layer.mlp.gate_proj.weight, layer.mlp.up_proj.weight))
+
+
+def test_copies_go_with_the_decoder(monkeypatch):
+    """Each after a wait for whoever still reads them: weights_written(), an exchanged source, a model no longer taken."""
+    build, waited = native._build, []
+    monkeypatch.setattr(native, "_build", lambda m: build(m, "cpu"))
+    monkeypatch.setattr(native._LaidOut, "unused", lambda self: waited.append(self))
+    model = model_of(FUSED)
+    assert native.decoder(model) is not None
+    first = dict(model.__dict__["_laid_out"])
+    assert set(first) == {"qkv", "gate_up"} and not waited
+    model.weights_written()
+    assert sorted(map(id, waited)) == sorted(map(id, first.values())) and not model.__dict__["_laid_out"]
+    assert native.decoder(model) is not None
+    second = dict(model.__dict__["_laid_out"])
+    exchange_memory(model.layers[0].mlp.up_proj.scales)
+    native.decoder(model)
+    assert waited[2:] == [second["gate_up"]] and model.__dict__["_laid_out"]["qkv"] is second["qkv"]
+    model.layers[1].mlp.up_proj.group_size = 32
+    assert native.decoder(model) is None and len(waited) == 5 and not model.__dict__["_laid_out"]
