@@ -21,7 +21,7 @@
 //
 // What bounds it: the matrix pipes and the power budget.  256 x 256 blocks keep the pipes 69 .. 74 % busy and the clock
 // falls to 1.74 .. 1.84 GHz (2048 x 37888 x 3584 514 us, 2048 x 3584 x 18944 254; 128 x 256 blocks at 512 x 14336 x 4096 60 % at
-// 2.1 GHz, 65 us; counters in profiles/products_sq_counters.md), so fewer expansions and LDS reads per matrix instruction
+// 2.1 GHz, 65 us), so fewer expansions and LDS reads per matrix instruction
 // are worth more than their cycles: 256 x 256 blocks expand a weight once for 256 rows.  Shallow -> deep, us:
 // 2048 x 37888 x 3584 582 -> 498, 2048 x 3584 x 18944 302 -> 256, 512 x 14336 x 4096 69 -> 64; error against unrounded
 // weights 1.2e-3 -> 3e-4.  (x stored in one piece per step instead of three: 311 against 299 us for 2048 x 18944 x 3584;
@@ -1842,7 +1842,7 @@ EAGLE_EXPORT int eagle_qmm_rows_tiled_w4g64_f16(const void* x, const uint32_t* w
 // round of workgroups, per K step of a workgroup alone on its compute unit and of two together (the two small
 // blocks; the large ones have a unit to themselves), per step as the units fill (they share a power budget: the
 // clock falls); a split costs 3.3 us and 0.2 us per MB of sums.  Choosing by it instead of by trial loses 1.5 % on
-// average over 8592 random products, 9 % at the 95th percentile, 40 % at worst (profiles/form_choice_sweeps.md).
+// average over 8592 random products, 9 % at the 95th percentile, 40 % at worst.
 // Other K (scales in fetches of one or two groups): the shallow loop by the older model below.
 struct GemmPlan {
   int block;      // 0: 64 x 128, 1: 128 x 128, 2: 128 x 256, 3: 256 x 256

@@ -26,7 +26,7 @@
 // 64 x 8192 x 8192 24 / 40.  With many rows the vector instructions (expansion per block, a multiply-add per group and
 // output) about equal the matrix instructions: 2048 x 37888 x 3584 675 us = 0.82 PFLOP/s, 512 x 3584 x 18944 114 us; the
 // GEMM, which rounds the weights to fp16 and expands them once per 256 rows, takes 580 and 93.  In a prompt pass, weights
-// not in a cache: 732 and (2048 x 3584 x 18944) 372 us against 553 and 263; counters in profiles/products_sq_counters.md.
+// not in a cache: 732 and (2048 x 3584 x 18944) 372 us against 553 and 263; matrix pipes 37 % busy at 2.05 GHz.
 #include "common.h"
 
 namespace {
@@ -523,7 +523,7 @@ struct RowsPlan {
 // unit ingests them (40 and 72 GB/s), and 0.22 us per unit of four chunks, tile and 16 rows of x.  What the whole
 // grid reads counts a little, a split as much as its second launch and the partial sums (the sums alone where
 // the consumer of the product adds them).  For 65 .. 2048 rows the same formula over the blocks of x.  Its choice against
-// the best of all forms and splits of random products (profiles/form_choice_sweeps.md): 17 .. 64 rows 1.4 % longer on
+// the best of all forms and splits of 4600 and 12600 random products: 17 .. 64 rows 1.4 % longer on
 // average, 8 % at the 95th percentile (up to 16 rows, most of which other kernels serve, 4 and 16); 65 .. 2048 rows 1.2 and 7.5.
 enum { ROWS_WHOLE = 0, ROWS_SPLIT = 1, ROWS_PARTIAL = 2 };
 RowsPlan rows_find_plan(int M, int N, int K, int mode) {
