@@ -162,8 +162,8 @@ PyObject* product(PyObject* const* a, Py_ssize_t n, bool swi, const char* name) 
     at::DimVector sizes(x->sizes());
     sizes.back() = cols;
     made = empty(sizes, at::kHalf, *x);
-  } else if (!plain(out, at::kHalf) || out->numel() != M * cols) {
-    Py_RETURN_NONE;
+  } else if (!plain(out, at::kHalf) || (swi ? out->numel() < M * cols : out->numel() != M * cols)) {
+    Py_RETURN_NONE;                        // (the SwiGLU form has always taken a buffer with room to spare)
   }
   const at::Tensor& o = a[5] == Py_None ? made : *out;
   const void* bp = bias ? bias->data_ptr() : nullptr;

@@ -345,7 +345,7 @@ def quantized_matmul_swiglu(x, w_q, scales, biases, bias=None, out=None, gemm=No
     if not gemm:                     # the arguments in plain form now
         r = _native().quantized_matmul_swiglu(x, w_q, scales, biases, bias, out)
         if r is None:
-            raise ValueError(f"out must be a contiguous float16 tensor of {M} x {N // 2} elements" if M > 0 else "x is empty")
+            raise ValueError(f"out must be a contiguous float16 tensor with room for {M} x {N // 2} elements" if M > 0 else "x is empty")
         return r
     if out is None:
         out = torch.empty((*lead, N // 2), dtype=torch.float16, device=x.device)

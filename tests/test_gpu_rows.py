@@ -147,6 +147,11 @@ def test_swiglu_of_more_rows_takes_any_alignment(dev, M, K):
     d = layer_to_dev(synth.make_qlinear(rng, 2 * I, K, bias=True, gain=1.0), dev)
     x = to_dev(synth.make_x(rng, M, K), dev)
     want = ops.quantized_matmul_swiglu(x, *(d[k] for k in ("weight", "scales", "biases")), bias=d["bias"]).cpu().numpy()
+    room = torch.full((M + 3, I), float("nan"), dtype=torch.float16, device=dev)
+    ops.quantized_matmul_swiglu(x, *(d[k] for k in ("weight", "scales", "biases")), bias=d["bias"], out=room)
+    assert np.array_equal(room[:M].cpu().numpy(), want) and bool(torch.isnan(room[M:]).all())
+    with pytest.raises(ValueError):
+        ops.quantized_matmul_swiglu(x, *(d[k] for k in ("weight", "scales", "biases")), out=room[:M - 1])
     for shift in (1, 2, 4):
         sb = []
         for key in ("scales", "biases"):
