@@ -31,10 +31,7 @@
 //     scales 16 per 2-byte load), 7.8 us for the down projection; shaped as below: 5.7 us;
 //   - a whole layer as ONE resident grid with grid-wide barriers between the products: a barrier
 //     plus the first load behind it costs what a launch costs (56 us per layer against 33 us for
-//     the launches it replaced);
-//   - attention of such a pass in one launch (a workgroup per query head, keys over its sixteen
-//     waves, merge through LDS): 14.7 to 30.8 us against 9.9 to 13.4 us for the split and merge
-//     launches over 64 to 2048 keys.
+//     the launches it replaced).
 #include "common.h"
 
 namespace {

@@ -261,7 +261,7 @@ def accept_candidate(cache, accept_indices, accept_length, offset):
 def _check_tree_size(verify_num_tokens):
     """The tree kernels lay a tree out in 64 slots (root + 63 nodes), which covers the reference's
     default of 39 nodes (mlx_eagle.py:390,510): above 32 tokens the products run with 64-row tiles
-    and attention over two mask words per query in pieces of 32 queries."""
+    and attention over two mask words per query."""
     if verify_num_tokens + 1 > TREE_SLOTS:
         raise NotImplementedError(
             f"verify_num_tokens={verify_num_tokens}: this build verifies at most {TREE_SLOTS - 1} draft nodes "
@@ -554,7 +554,7 @@ class TreeVerifier:
         self.T = T = total_tokens + 1
         # above 32 tree tokens: q|k|v, o, down and gate|up in the slab form with 64-row tiles where the shapes
         # allow it, the tiled head in two passes, other products on the kernels of `ops.quantized_matmul`; two
-        # mask words per token and attention in pieces of 32 query rows (one launch pair)
+        # mask words per token
         self.wide = T > MAXT
         if self.wide and not fuse:
             raise ValueError(f"a tree of more than {MAXT} tokens runs with the fused projections only")

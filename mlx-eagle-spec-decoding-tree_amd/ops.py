@@ -623,7 +623,7 @@ def mask_to_words(mask):
 def draft_attention(q, k_cache, v_cache, mask_words, cache_len_dev, Tk, scale, max_len=None, out=None):
     """q [H,T,hd]; k_cache, v_cache [G,capacity,hd] holding *cache_len_dev prefix rows followed
     by Tk <= 64 rows that query t sees according to mask_words [T,2].  Returns [T, H*hd].
-    More than 32 (up to 64) queries go in pieces of 32 rows through one launch pair."""
+    Up to 64 queries."""
     _need_cuda(q, k_cache, v_cache, mask_words, cache_len_dev)
     H, T, hd = q.shape
     G, cap, _ = k_cache.shape
@@ -676,8 +676,6 @@ def scaled_dot_product_attention(queries, keys, values, cache=None, scale=None, 
     q = _f16(queries[0], "q")
     if T > 64:
         raise ValueError("at most 64 query rows")
-    # more than 32 queries (a tree of up to 64 tokens) go in pieces of 32 query rows, each with
-    # its own mask rows over the same keys, inside the one launch pair
     out = draft_attention(q, k_buf, v_buf, words, len_dev, Tk, scale, max_len=S)
     return out.reshape(T, H, hd).permute(1, 0, 2).unsqueeze(0).contiguous()
 
