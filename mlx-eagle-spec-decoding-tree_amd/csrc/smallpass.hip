@@ -15,9 +15,11 @@
 //     chunks of K among themselves (at most three each) and add their tiles in LDS.  Every request
 //     of a wave (weights, scales, its columns of x as the B operand of v_mfma_f32_16x16x32_f16) is
 //     in flight together; there is no loop over K.
-//   * The norm is folded into the load of x: each wave sums the squares of its columns, the row
+//   * The norm is folded into x as it was loaded (whole rows, every lane columns of its own; in the operand layout
+//     half the lanes hold nothing when T <= 8): each wave sums the squares of its columns, the row
 //     sums are added across the waves in LDS; no launch and no pass over memory for it.  Every
-//     workgroup repeats it, so it is kept short: v_dot2 for the sums, mixed-precision products.
+//     workgroup repeats it, so it is kept short: v_dot2 for the sums, one square root and division per lane,
+//     mixed-precision products (8 rows, K 896: gate|up 5.8 -> 5.3 us, 4.5 without a norm; q|k|v 4.1 -> 3.9).
 //   * The weights are never rounded: the matrix instructions multiply x with the integers q (exact in
 //     fp16, through the fp8 conversion) a quantisation group at a time, and with ones for the group's
 //     sum of x; scale and bias are applied to the two sums in fp32.
@@ -64,7 +66,7 @@ enum { SMALL_PLAIN = 0, SMALL_SWIGLU = 1, SMALL_ROPE = 2 };
 
 // NW waves per workgroup, at most MAXC chunks of 128 columns per wave (a wave requests MAXC whatever it owns:
 // the smallest number that serves K), RP passes of four x rows
-// (2: T <= 8, 4: T <= 16).  MODE: one tile per workgroup (plain / residual), a (gate, up) tile pair
+// (1: T <= 4, 2: T <= 8, 4: T <= 16).  MODE: one tile per workgroup (plain / residual), a (gate, up) tile pair
 // 16 rows apart with the SwiGLU epilogue, or two tiles of one head half a head apart (the two
 // halves a rotation pairs) with the rope epilogue.  Lane (r = lane % 16, kq = lane / 16) of a wave
 // loads, per chunk, weight row r columns 32 kq .. + 32 (one 16-byte load, four packed words): two lanes
@@ -83,12 +85,25 @@ constexpr int SMALL_MAXC = 3;
 constexpr int SMALL_RED = 64 + 4;          // floats per four weight rows of a wave's tile
 constexpr int SMALL_XROW = 256 + 16;       // bytes per staged x row: 128 columns, padded against bank conflicts
 
+// the sum over sixteen neighbouring lanes, in all of them
+__device__ inline float row16_sum(float v) {
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true));   // row_ror:8
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x124, 0xf, 0xf, true));
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x122, 0xf, 0xf, true));
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xf, 0xf, true));
+  return v;
+}
+
 template <int NW, int MAXC, int RP, int MODE, bool NORM>
 __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
   constexpr int NT = MODE == SMALL_PLAIN ? 1 : 2;
-  // a slice per wave: first its x, then (written by the same wave) its tiles
-  constexpr int SLICE = RP * 4 * SMALL_XROW;
-  static_assert(NT * 16 * SMALL_RED <= SLICE, "a wave's tiles do not fit over its x");
+  // a slice per wave: first its x, then (written by the same wave) its weights, then its tiles
+  // Whether weights are loaded by whole 64-byte pieces (four lanes of a row next to each other, a quarter of the cache
+  // lines per load) and dealt to the lanes through LDS: where a wave has several loads in flight and one tile (8 rows, us
+  // without / with: 2048 -> 8192 5.6 / 5.3, 3072 -> 4096 4.9 / 4.7; gate|up with two tiles a wave 5.4 / 5.5, one chunk 2.4 / 2.5)
+  constexpr bool WHOLE = MAXC > 1 && NT == 1;
+  constexpr int XB = RP * 4 * SMALL_XROW, WB = WHOLE ? MAXC * 1024 : 0, TB = NT * 16 * SMALL_RED;
+  constexpr int XW = XB > WB ? XB : WB, SLICE = XW > TB ? XW : TB;
   __shared__ __attribute__((aligned(16))) unsigned char slices[NW][SLICE];
   __shared__ float ssq[NORM ? NW : 1][16];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -128,13 +143,11 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
       for (int c = 0; c < MAXC; ++c) xg[c][p] = *reinterpret_cast<const uint4_t*>(xp + (c < nch ? c : 0) * 128);
     }
   }
-  half8_t nw[MAXC][4];
+  half8_t nw[MAXC];
   if (NORM && a.norm_w) {
-    const half_t* np = a.norm_w + kb + xcol * 8;
+    const half_t* np = a.norm_w + kb + (lane & 15) * 8;
 #pragma unroll
-    for (int c = 0; c < MAXC; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) nw[c][i] = *reinterpret_cast<const half8_t*>(np + (c < nch ? c : 0) * 128 + (i >> 1) * 64 + (i & 1) * 8);
+    for (int c = 0; c < MAXC; ++c) nw[c] = *reinterpret_cast<const half8_t*>(np + (c < nch ? c : 0) * 128);
   }
   __builtin_amdgcn_sched_barrier(0);
   uint4_t wv[NT][MAXC];
@@ -143,10 +156,12 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
   for (int t = 0; t < NT; ++t) {
     long row = row0 + second * t + r;
     if (MODE == SMALL_PLAIN && row > a.N - 1) row = a.N - 1;         // (N a multiple of 8: never stored)
-    const uint32_t* wp = a.w + row * KW + (kb >> 3) + kq * 4;
+    long wrow = WHOLE ? row0 + second * t + (lane >> 2) : row;
+    if (WHOLE && wrow > a.N - 1) wrow = a.N - 1;
+    const uint32_t* wp = a.w + wrow * KW + (kb >> 3) + (WHOLE ? lane & 3 : kq) * 4;
 #pragma unroll
     for (int c = 0; c < MAXC; ++c) wv[t][c] = *reinterpret_cast<const uint4_t*>(wp + (c < nch ? c : 0) * 16);
-    const int cpair = kq < nch ? kq : 0;
+    const int cpair = MAXC > 1 && kq < nch ? kq : 0;
     spair[t] = *reinterpret_cast<const uint32_t*>(a.s + row * G + (kb >> 6) + cpair * 2);
     bpair[t] = *reinterpret_cast<const uint32_t*>(a.b + row * G + (kb >> 6) + cpair * 2);
   }
@@ -177,6 +192,51 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
     }
   }
   __builtin_amdgcn_sched_barrier(0);
+  // ---- RMSNorm folded into x, as it was loaded: lane l holds columns 8 (l % 16) .. + 8 of rows 4 p + l / 16 ----
+  if (NORM && a.norm_w) {
+    float ss[RP];
+#pragma unroll
+    for (int p = 0; p < RP; ++p) {
+      ss[p] = 0.f;
+#pragma unroll
+      for (int c = 0; c < MAXC; ++c) {
+        if (c < nch) {
+          const half8_t v = __builtin_bit_cast(half8_t, xg[c][p]);
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            const half2_t p2 = half2_t{v[e], v[e + 1]};
+            ss[p] = __builtin_amdgcn_fdot2(p2, p2, ss[p], false);      // exact products, fp32 sum
+          }
+        }
+      }
+      ss[p] = row16_sum(ss[p]);
+      if ((lane & 15) == 0) ssq[wave][4 * p + (lane >> 4)] = ss[p];
+    }
+    __syncthreads();
+    const int mr = r < 4 * RP ? r : 0;
+    float tot = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) tot += ssq[w][mr];
+    const float rinv_r = 1.0f / sqrtf(tot / (float)K + a.eps);         // of row r: one square root and division per lane
+#pragma unroll
+    for (int p = 0; p < RP; ++p) {
+      const float rinv = __shfl(rinv_r, 4 * p + (lane >> 4), 64);
+#pragma unroll
+      for (int c = 0; c < MAXC; ++c) {
+        if (c < nch) {
+          const half8_t v = __builtin_bit_cast(half8_t, xg[c][p]);
+          half8_t o;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            // as fma with zero: v_fma_mix_f32 reads the fp16 operands, where a product converts them first
+            const float n = __builtin_fmaf((float)v[e], rinv, 0.f);
+            o[e] = (half_t)__builtin_fmaf(n, (float)nw[c][e], 0.f);
+          }
+          xg[c][p] = __builtin_bit_cast(uint4_t, o);
+        }
+      }
+    }
+  }
   // x through the wave's LDS buffer into the operand layout, a chunk at a time (rows past 4 RP,
   // which are rows past T, read what is there: their columns of the result are not stored)
   half8_t xb[MAXC][4];
@@ -187,7 +247,7 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
     for (int c = 0; c < MAXC; ++c) {
 #pragma unroll
       for (int p = 0; p < RP; ++p)
-        *reinterpret_cast<uint4_t*>(xs + (4 * p + xr) * SMALL_XROW + xc * 16) = xg[c][p];
+        *reinterpret_cast<half8_t*>(xs + (4 * p + xr) * SMALL_XROW + xc * 16) = eagle_permute8(__builtin_bit_cast(half8_t, xg[c][p]));
       __builtin_amdgcn_wave_barrier();
       const int mr = r < 4 * RP ? r : 0;
 #pragma unroll
@@ -197,48 +257,16 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
     }
   }
 
-  // ---- RMSNorm folded into x ----
-  if (NORM && a.norm_w) {
-    float ss = 0.f;
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) {
-      if (c < nch) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int e = 0; e < 8; e += 2) {
-            const half2_t p2 = half2_t{xb[c][i][e], xb[c][i][e + 1]};
-            ss = __builtin_amdgcn_fdot2(p2, p2, ss, false);      // exact products, fp32 sum
-          }
-      }
-    }
-    ss += __shfl_xor(ss, 16, 64);
-    ss += __shfl_xor(ss, 32, 64);
-    if (kq == 0) ssq[wave][r] = ss;
-    __syncthreads();
-    float tot = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) tot += ssq[w][r];
-    const float rinv = 1.0f / sqrtf(tot / (float)K + a.eps);
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) {
-      if (c < nch) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          half8_t o;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            // as fma with zero: v_fma_mix_f32 reads the fp16 operands, where a product converts them first
-            const float v = __builtin_fmaf((float)xb[c][i][e], rinv, 0.f);
-            o[e] = (half_t)__builtin_fmaf(v, (float)nw[c][i][e], 0.f);
-          }
-          xb[c][i] = o;
-        }
-      }
-    }
-  }
-
   // ---- the wave's part of the tile(s) ----
+  // quarter q of row wr at 16 q + (wr + 4 q) % 16, in units of 16 bytes: neither the stores nor the loads meet in a bank
+  uint4_t* ws = reinterpret_cast<uint4_t*>(slices[wave]);
+  if (WHOLE) {
+    __builtin_amdgcn_wave_barrier();
+    const int wr = lane >> 2, q = lane & 3;
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) ws[c * 64 + 16 * q + ((wr + 4 * q) & 15)] = wv[0][c];
+    __builtin_amdgcn_wave_barrier();
+  }
   const half_t one = (half_t)1.f;
   const half8_t ones = {one, one, one, one, one, one, one, one};
   const float4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -251,17 +279,32 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
       float4_t sx[2];
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
-        xb[c][2 * g] = eagle_permute8(xb[c][2 * g]);
-        xb[c][2 * g + 1] = eagle_permute8(xb[c][2 * g + 1]);
         sx[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g], ones, zero, 0, 0, 0);
         sx[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[c][2 * g + 1], ones, sx[g], 0, 0, 0);
       }
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         // the pair of chunk c sits in lane (r, c)
-        const uint32_t s2 = __shfl(spair[t], r + 16 * c, 64), b2 = __shfl(bpair[t], r + 16 * c, 64);
-        const auto w02 = __builtin_amdgcn_permlane32_swap(wv[t][c][0], wv[t][c][2], false, false);
-        const auto w13 = __builtin_amdgcn_permlane32_swap(wv[t][c][1], wv[t][c][3], false, false);
+        const uint32_t s2 = MAXC > 1 ? __shfl(spair[t], r + 16 * c, 64) : spair[t], b2 = MAXC > 1 ? __shfl(bpair[t], r + 16 * c, 64) : bpair[t];
+        uint32_t w02[2], w13[2];
+        if (WHOLE) {
+#pragma unroll
+          for (int g = 0; g < 2; ++g) {
+            const int q = 2 * g + (kq & 1);
+            const uint2_t* p = reinterpret_cast<const uint2_t*>(ws + c * 64 + 16 * q + ((r + 4 * q) & 15));
+            const uint2_t v = p[kq >> 1];
+            w02[g] = v[0];
+            w13[g] = v[1];
+          }
+        } else {
+          const auto s02 = __builtin_amdgcn_permlane32_swap(wv[t][c][0], wv[t][c][2], false, false);
+          const auto s13 = __builtin_amdgcn_permlane32_swap(wv[t][c][1], wv[t][c][3], false, false);
+#pragma unroll
+          for (int g = 0; g < 2; ++g) {
+            w02[g] = s02[g];
+            w13[g] = s13[g];
+          }
+        }
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
           const float sc = (float)__builtin_bit_cast(half_t, (unsigned short)(g ? s2 >> 16 : s2 & 0xffffu));
@@ -274,6 +317,7 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
       }
     }
   }
+  __builtin_amdgcn_wave_barrier();
   // Into LDS so that a lane of the epilogue reads four weight rows of one x row with one load: x row m,
   // weight row n at 4 m + 68 (n / 4) + n % 4 (68: the sixteen weight rows of a store in different banks).
 #pragma unroll
@@ -376,7 +420,10 @@ constexpr int SMALL_K16 = 16 * SMALL_MAXC * 128;      // sixteen waves, three ch
 
 template <int NW, int MAXC, int MODE, bool NORM>
 void small_go(const SmallArgs& a, int grid, hipStream_t st) {
-  if (a.T > 8)
+  // (up to four rows in one pass: 1 x 3584 -> 3584 4.5 -> 4.3 us)
+  if (MODE == SMALL_PLAIN && a.T <= 4)
+    hipLaunchKernelGGL((qmm_small_kernel<NW, MAXC, 1, MODE, NORM>), dim3(grid), dim3(NW * 64), 0, st, a);
+  else if (a.T > 8)
     hipLaunchKernelGGL((qmm_small_kernel<NW, MAXC, 4, MODE, NORM>), dim3(grid), dim3(NW * 64), 0, st, a);
   else
     hipLaunchKernelGGL((qmm_small_kernel<NW, MAXC, 2, MODE, NORM>), dim3(grid), dim3(NW * 64), 0, st, a);
