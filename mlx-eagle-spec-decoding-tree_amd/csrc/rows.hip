@@ -25,7 +25,8 @@
 // back to back over rotating weights): 32 x 3584 x 152064 71 / 80, 27 x 18944 x 3584 18 / 23, 32 x 2048 x 8192 8.2 / 11.0,
 // 64 x 8192 x 8192 24 / 40.  With many rows the vector instructions (expansion per block, a multiply-add per group and
 // output) about equal the matrix instructions: 2048 x 37888 x 3584 675 us = 0.82 PFLOP/s, 512 x 3584 x 18944 114 us; the
-// GEMM, which rounds the weights to fp16 and expands them once per 256 rows, takes 580 and 93.  In a prompt pass, weights
+// GEMM, which rounds the weights to fp16 and expands them once per 256 rows, takes 580 and 93 (128 x 3584 x 37888 58 us
+// with the sums of a tile added behind its matrix instructions, 55 under the next tile's).  In a prompt pass, weights
 // not in a cache: 732 and (2048 x 3584 x 18944) 372 us against 553 and 263; matrix pipes 37 % busy at 2.05 GHz.
 #include "common.h"
 
@@ -267,8 +268,10 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
       for (int i = 0; i < 2; ++i)
         xv[i] = *reinterpret_cast<const half8_t*>(xa + mt * (16 * ROWS_XROW) + (8 * g + i) * 16);
     };
-    if (MT <= 2) {
-      // the matrix instructions of a tile run while the sums of the one before enter the accumulators
+    // The matrix instructions of a tile run while the sums of the one before enter the accumulators, both groups of a chunk
+    // at once where the registers hold that and it is faster (40 x 3584 x 37888 on three tiles and two parts: tile after tile
+    // 34.7 us, group by group with the overlap 33.3, both groups 31.7; one tile: 19.1 by both, 18.7 group by group)
+    if (MT <= 2 || (MT == 3 && (RT == 3 ? KP <= 2 : RT == 2 && KP > 1))) {
       half8_t xv[MT][2][2];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
@@ -304,29 +307,33 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
       }
       add(RT - 1);
     } else {
-      // more rows: a tile has enough matrix instructions by itself, and the registers are short; group by group
+      // group by group (64 x 3584 x 37888 39.8 us without the overlap, 37.3 with it)
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
         half8_t xv[MT][2];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) load_x(xv[mt], mt, g);
+        float4_t d[2][MT];
+        auto add = [&](int t) {
+          const float sg = scale(t, g);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[t][mt][i] = __builtin_fmaf(sg, d[t & 1][mt][i], acc[t][mt][i]);
+        };
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
           if (g == 0) regroup(ring[u % AH][t]);
           const half8_t q0 = eagle_expand8(ring[u % AH][t][2 * g]), q1 = eagle_expand8(ring[u % AH][t][2 * g + 1]);
           if (g == 1) reload(t);
-          float4_t d[MT];
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) d[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[mt][0], q0, zero, 0, 0, 0);
+          for (int mt = 0; mt < MT; ++mt) d[t & 1][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[mt][0], q0, zero, 0, 0, 0);
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) d[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[mt][1], q1, d[mt], 0, 0, 0);
-          const float sg = scale(t, g);
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[t][mt][i] = __builtin_fmaf(sg, d[mt][i], acc[t][mt][i]);
+          for (int mt = 0; mt < MT; ++mt) d[t & 1][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[mt][1], q1, d[t & 1][mt], 0, 0, 0);
+          if (t > 0) add(t - 1);
           __builtin_amdgcn_sched_barrier(0);
         }
+        add(RT - 1);
       }
     }
   };
