@@ -55,22 +55,22 @@ __host__ __device__ inline int eagle_slab_rows(int M) { return M > 32 ? 64 : 32;
 
 // Eight consecutive values of a matmul result that is held as fp32 partial sums of K slabs
 // (eagle_qmm_slab_partial_w4g64): fp16 of the sum in slab order, then the fp16 bias.  `at` is
-// the element offset inside a slab, `stride` the elements per slab.  All loads are issued
-// before the first add.
+// the element offset inside a slab, `stride` the elements per slab.  Up to twelve slabs are requested before
+// the first add, and none twice (a norm over 32 x 3584 with ten slabs: 5.1 us with eight at a time, 4.7 so; seven 4.3, 4.2).
 __device__ inline half8_t eagle_slab_sum8(const float* __restrict__ partial, int nslab, size_t stride,
                                           size_t at, const half_t* __restrict__ bias8) {
   float4_t lo = float4_t{0.f, 0.f, 0.f, 0.f}, hi = lo;
   const float* p = partial + at;
-  for (int z = 0; z < nslab; z += 8) {
-    float4_t a[8], c[8];
+  for (int z = 0; z < nslab; z += 12) {
+    float4_t a[12], c[12];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int zz = z + k < nslab ? z + k : nslab - 1;
-      a[k] = *reinterpret_cast<const float4_t*>(p + (size_t)zz * stride);
-      c[k] = *reinterpret_cast<const float4_t*>(p + (size_t)zz * stride + 4);
-    }
+    for (int k = 0; k < 12; ++k)
+      if (z + k < nslab) {
+        a[k] = *reinterpret_cast<const float4_t*>(p + (size_t)(z + k) * stride);
+        c[k] = *reinterpret_cast<const float4_t*>(p + (size_t)(z + k) * stride + 4);
+      }
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
+    for (int k = 0; k < 12; ++k)
       if (z + k < nslab) {
         lo += a[k];
         hi += c[k];

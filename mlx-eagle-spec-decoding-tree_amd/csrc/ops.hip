@@ -174,16 +174,16 @@ __global__ void rope_kv_append_slabs_kernel(const float* __restrict__ partial, i
     bhi = *reinterpret_cast<const half4_t*>(bias + (size_t)hh * hd + half + c);
   }
   float4_t lo = float4_t{0.f, 0.f, 0.f, 0.f}, hi = lo;
-  for (int z = 0; z < nslab; z += 8) {
-    float4_t a[8], b[8];
+  for (int z = 0; z < nslab; z += 12) {
+    float4_t a[12], b[12];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int zz = z + k < nslab ? z + k : nslab - 1;
-      a[k] = *reinterpret_cast<const float4_t*>(p + (size_t)zz * stride);
-      b[k] = *reinterpret_cast<const float4_t*>(p + (size_t)zz * stride + half);
-    }
+    for (int k = 0; k < 12; ++k)
+      if (z + k < nslab) {
+        a[k] = *reinterpret_cast<const float4_t*>(p + (size_t)(z + k) * stride);
+        b[k] = *reinterpret_cast<const float4_t*>(p + (size_t)(z + k) * stride + half);
+      }
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
+    for (int k = 0; k < 12; ++k)
       if (z + k < nslab) {
         lo += a[k];
         hi += b[k];
