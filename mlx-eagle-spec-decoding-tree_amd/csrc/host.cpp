@@ -15,6 +15,7 @@ using namespace eagle_host;
 namespace {
 PyObject* g_workspace = nullptr;     // ops.workspace(tag, nbytes, device)
 constexpr int MAX_DEVICES = 64;
+constexpr int POST_SPINS = 4000;     // about 50 us of pauses
 Slot g_qmm_ws[MAX_DEVICES];
 }  // namespace
 
@@ -316,8 +317,11 @@ PyObject* py_process_draft_tree(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // post_process_draft_tree(tree_position_ids, mask_index, total) -> retrieve_indices [leaves, depth + 1].  The result's
-// shape is data, so the host waits for the kernel; the rows are written without padding, so that what the wait
-// is for is two numbers, which the kernel puts into pinned host memory.
+// shape is data, so the host waits for it; the rows are written without padding, so that what the wait
+// is for is two numbers, which the kernel puts into pinned host memory with one store.  The host watches that
+// word for a while before it waits for the stream: the end of a stream is seen 5 us later than the store (39
+// nodes with the layout before it: 25.6 us without watching, 20.0 with).  A word that stays zero (a kernel that waits behind other work, a stream
+// in capture, an error) ends in the wait.
 PyObject* py_post_process_draft_tree(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 3) {
     PyErr_SetString(PyExc_TypeError, "post_process_draft_tree takes three arguments");
@@ -330,17 +334,20 @@ PyObject* py_post_process_draft_tree(PyObject*, PyObject* const* a, Py_ssize_t n
   const c10::hip::HIPStream st = c10::hip::getCurrentHIPStream(pos->device().index());
   at::Tensor full = empty({EAGLE_MAX_TREE_SLOTS * EAGLE_MAX_TREE_SLOTS}, at::kInt, *pos);
   at::Tensor shape = at::empty({2}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  volatile uint64_t* word = static_cast<volatile uint64_t*>(shape.data_ptr());
+  *word = 0;                               // (there is at least one leaf)
   const int rc = eagle_post_process_draft_tree_packed(
       static_cast<const int32_t*>(pos->data_ptr()), static_cast<const int32_t*>(idx->data_ptr()), (int)total,
       static_cast<int32_t*>(full.data_ptr()), static_cast<int32_t*>(shape.data_ptr()), static_cast<void*>(st.stream()));
   if (rc != EAGLE_OK) return fail(rc, "post_process_draft_tree");
-  hipError_t err;
+  hipError_t err = hipSuccess;
   Py_BEGIN_ALLOW_THREADS
-  err = hipStreamSynchronize(st.stream());
+  for (int i = 0; i < POST_SPINS && *word == 0; ++i) __builtin_ia32_pause();
+  if (*word == 0) err = hipStreamSynchronize(st.stream());
   Py_END_ALLOW_THREADS
   if (err != hipSuccess) return fail(EAGLE_ERR_HIP, "post_process_draft_tree");
-  const int32_t* s = static_cast<const int32_t*>(shape.data_ptr());
-  const int64_t leaves = s[0], cols = s[1];
+  const uint64_t seen = *word;
+  const int64_t leaves = (int32_t)(uint32_t)seen, cols = (int32_t)(seen >> 32);
   if (leaves < 1 || leaves > EAGLE_MAX_TREE_SLOTS || cols < 1 || cols > EAGLE_MAX_TREE_SLOTS) Py_RETURN_NONE;
   return THPVariable_Wrap(full.narrow(0, 0, leaves * cols).view({leaves, cols}));
 }

@@ -38,17 +38,44 @@ __device__ inline T list_at(const T* const (&ptr)[EAGLE_MAX_SEGMENTS], const int
 }
 
 constexpr int TREE_THREADS = 1024;
-constexpr int TREE_HALF = TREE_THREADS / 2;
+constexpr int RANK_PARTS = 8;                              // threads that share the ranking of a candidate
+constexpr int RANK_BASE = TREE_THREADS / RANK_PARTS;       // candidates c, c + RANK_BASE, ... to a thread
+
+// Adds to the ranks of candidates c0 + r RANK_BASE (r < N) how many of keys[from .. to) are ahead of each
+template <int N>
+__device__ inline void count_ahead(const uint32_t* keys, int* ranks, int c0, int C, int from, int to) {
+  uint32_t key[N];
+  int ahead[N];
+#pragma unroll
+  for (int r = 0; r < N; ++r) {
+    const int i = c0 + r * RANK_BASE;
+    key[r] = keys[i < C ? i : 0];
+    ahead[r] = 0;
+  }
+#pragma unroll 2
+  for (int j = from; j < to; j += 4) {
+    const uint4_t k4 = *reinterpret_cast<const uint4_t*>(keys + j);
+#pragma unroll
+    for (int r = 0; r < N; ++r)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ahead[r] += k4[e] > key[r];
+  }
+#pragma unroll
+  for (int r = 0; r < N; ++r)
+    if (c0 + r * RANK_BASE < C) atomicAdd(ranks + c0 + r * RANK_BASE, ahead[r]);
+}
 
 // mlx_eagle.py:217-250 (with topk :24-58 and search_sorted :61-93).  One workgroup; bound by the chain of its
-// phases (two dependent loads, the ranks, the walk), so none of them is a loop of one thread: each candidate is ranked
-// by two threads, on one integer comparison per pair; the picked ones are counted with ballots; every token walks up
-// to the root by itself.  24.4 -> 8.2 us for 39 of 328 candidates in six pieces.
+// phases (two dependent loads, the ranks, the walk), so none of them is a loop of one thread: a candidate is ranked by eight
+// threads, on one integer comparison per pair, and a thread ranks several, so that a read of four keys from LDS serves
+// several comparisons; the picked ones are counted with ballots; every token walks up to the root by itself.  39 of 328 candidates,
+// us in a graph: 7.0 (7.7 with a candidate to two threads and a read for every four comparisons), of 200 5.4 (6.4), 7 of 72 4.4 (4.9);
+// the comparisons themselves are what is left above that.
 __global__ __launch_bounds__(TREE_THREADS) void process_draft_tree_kernel(
     TreeLists in, int C, int k, int total, int32_t* __restrict__ pos_ids, int32_t* __restrict__ mask_index,
     int32_t* __restrict__ draft_tokens, uint32_t* __restrict__ bits_out, uint16_t* __restrict__ mask_out) {
   __shared__ __attribute__((aligned(16))) uint32_t keys[MAXC];
-  __shared__ int upper[MAXC];          // ranks among the second half of the candidates
+  __shared__ int ranks[MAXC];
   __shared__ int wave_picked[MAXC / 64];
   __shared__ int sel[MAXT];
   __shared__ int midx[MAXT];
@@ -57,8 +84,11 @@ __global__ __launch_bounds__(TREE_THREADS) void process_draft_tree_kernel(
   // Key of a candidate: its fp16 score as an ordered integer, then its index from the back, so that a larger key is
   // ahead in the stable descending order.  A NaN score ranks as -inf and -0 as 0: the order is total and exactly
   // `total` candidates are picked whatever the scores hold.
-  const int C8 = (C + 7) / 8 * 8;
-  if (tid < C8) {
+  static_assert(TREE_THREADS == MAXC, "a thread per candidate");
+  constexpr int ROUND = 4 * RANK_PARTS;
+  const int CR = (C + ROUND - 1) / ROUND * ROUND;        // every part whole reads of four keys (keys of 0 are never ahead)
+  ranks[tid] = 0;
+  if (tid < CR) {
     uint32_t key = 0;
     if (tid < C) {
       uint32_t h = __builtin_bit_cast(unsigned short, list_at(in.scores, in.end, in.n, tid));
@@ -69,45 +99,24 @@ __global__ __launch_bounds__(TREE_THREADS) void process_draft_tree_kernel(
     keys[tid] = key;
   }
   __syncthreads();
-  // rank: candidates ahead, counted over half of them by each of two threads
-  const int half = tid / TREE_HALF, c0 = tid % TREE_HALF;
-  int rank[MAXC / TREE_HALF];
-#pragma unroll
-  for (int r = 0; r < MAXC / TREE_HALF; ++r) {
-    const int i = c0 + r * TREE_HALF;
-    rank[r] = 0;
-    if (r * TREE_HALF < C) {
-      const uint32_t key = keys[i < C ? i : 0];
-      const int from = half * (C8 / 2), to = from + C8 / 2;
-#pragma unroll 4
-      for (int j = from; j < to; j += 4) {
-        const uint4_t k4 = *reinterpret_cast<const uint4_t*>(keys + j);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) rank[r] += k4[e] > key;
-      }
-      if (half) upper[i] = rank[r];
-    }
-  }
-  __syncthreads();
-  bool picked[MAXC / TREE_HALF];
-#pragma unroll
-  for (int r = 0; r < MAXC / TREE_HALF; ++r) {
-    const int i = c0 + r * TREE_HALF;
-    picked[r] = !half && i < C && rank[r] + upper[i] < total;
-    const unsigned long long m = __ballot(picked[r]);
-    if (!half && (tid & 63) == 0) wave_picked[i >> 6] = __popcll(m);
+  {
+    const int c0 = tid % RANK_BASE, from = tid / RANK_BASE * (CR / RANK_PARTS), to = from + CR / RANK_PARTS;
+    if (C <= RANK_BASE) count_ahead<1>(keys, ranks, c0, C, from, to);
+    else if (C <= 2 * RANK_BASE) count_ahead<2>(keys, ranks, c0, C, from, to);
+    else if (C <= 3 * RANK_BASE) count_ahead<3>(keys, ranks, c0, C, from, to);
+    else if (C <= 4 * RANK_BASE) count_ahead<4>(keys, ranks, c0, C, from, to);
+    else count_ahead<MAXC / RANK_BASE>(keys, ranks, c0, C, from, to);
   }
   __syncthreads();
   // the picked candidates in ascending flat index
-#pragma unroll
-  for (int r = 0; r < MAXC / TREE_HALF; ++r) {
-    const int i = c0 + r * TREE_HALF;
-    const unsigned long long m = __ballot(picked[r]);
-    if (picked[r]) {
-      int before = __popcll(m & ((1ull << (tid & 63)) - 1ull));
-      for (int w = 0; w < (i >> 6); ++w) before += wave_picked[w];
-      if (before < total) sel[before] = i;
-    }
+  const bool picked = tid < C && ranks[tid] < total;
+  const unsigned long long m = __ballot(picked);
+  if ((tid & 63) == 0) wave_picked[tid >> 6] = __popcll(m);
+  __syncthreads();
+  if (picked) {
+    int before = __popcll(m & ((1ull << (tid & 63)) - 1ull));
+    for (int w = 0; w < (tid >> 6); ++w) before += wave_picked[w];
+    if (before < total) sel[before] = tid;
   }
   __syncthreads();
   if (tid < total) {
@@ -167,7 +176,8 @@ __global__ __launch_bounds__(TREE_THREADS) void process_draft_tree_kernel(
 }
 
 // mlx_eagle.py:254-295 in one wave (a lane per token, T <= 64).  retrieve [64][64], shape {leaf_num,
-// max_depth + 1}; PACKED: rows of max_depth + 1 entries, leaf_num of them, without padding.
+// max_depth + 1}; PACKED: rows of max_depth + 1 entries, leaf_num of them, without padding, and the shape last, as one 8-byte
+// store to memory that the host may be watching: who sees it may use the rows, on any stream, as after a wait for this one.
 template <bool PACKED>
 __global__ __launch_bounds__(64) void post_process_kernel(const int32_t* __restrict__ pos_ids,
                                                          const int32_t* __restrict__ mask_index,
@@ -196,7 +206,7 @@ __global__ __launch_bounds__(64) void post_process_kernel(const int32_t* __restr
     md = other > md ? other : md;
   }
   const int leaves = total - (n_inner - 1), cols = md + 1;
-  if (tid == 0) {
+  if (!PACKED && tid == 0) {
     shape[0] = leaves;
     shape[1] = cols;
   }
@@ -212,6 +222,12 @@ __global__ __launch_bounds__(64) void post_process_kernel(const int32_t* __restr
       cur = (cur == 0) ? par[total - 1] : par[cur - 1];
       cur = cur < 0 ? 0 : (cur > total ? total : cur);
     }
+  }
+  if (PACKED) {
+    __syncthreads();
+    if (tid == 0)
+      __hip_atomic_store(reinterpret_cast<unsigned long long*>(shape),
+                         (unsigned long long)(uint32_t)cols << 32 | (uint32_t)leaves, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -389,6 +405,7 @@ static int post_process(const int32_t* tree_position_ids, const int32_t* mask_in
                         int32_t* retrieve_indices, int32_t* shape_out, bool packed, eagle_stream_t stream) {
   if (!tree_position_ids || !mask_index || !retrieve_indices || !shape_out) return EAGLE_ERR_NULL;
   if (total < 1 || total >= MAXT) return EAGLE_ERR_SHAPE;
+  if (packed && (reinterpret_cast<uintptr_t>(shape_out) & 7u)) return EAGLE_ERR_ALIGN;     // one 8-byte store
   if (packed)
     hipLaunchKernelGGL(post_process_kernel<true>, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream),
                        tree_position_ids, mask_index, total, retrieve_indices, shape_out);
