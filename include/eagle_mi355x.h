@@ -475,7 +475,7 @@ int eagle_tree_attention_wide_f16(const void* q, const void* k_cache, const void
  * mlx_llama.py:275-276; mlx_eagle.py:522-533): R query rows (a multiple of 32, at most
  * EAGLE_MAX_CHUNK) in pieces of 32.  Piece j has its rows at cache rows piece_len_dev[j] ..
  * piece_len_dev[j] + 31 (already appended), sees every cache row before them and its own rows
- * causally.  q [H,R,hd] (rotated), out [R, H*hd].  One launch pair for all pieces. */
+ * causally.  q [H,R,hd] (rotated), out [R, H*hd].  One launch for all pieces, two where the keys are split. */
 size_t eagle_causal_attention_workspace_bytes(int R, int H, int hd, int max_len);
 int eagle_causal_attention_f16(const void* q, const void* k_cache, const void* v_cache,
                                const int32_t* piece_len_dev, void* out, int R, int H, int G, int hd,

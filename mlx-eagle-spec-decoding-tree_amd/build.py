@@ -40,8 +40,6 @@ SCRATCH_ALLOWED = [
     # (SwiGLU, rope) or with the norm weights of three chunks; the drafter's K is 896 there
     (r"qmm_small_kernelILi1[346]ELi[23]ELi\dELi[12]E", "small-row kernel, sixteen waves, two tiles"),
     (r"qmm_small_kernelILi1[36]ELi3ELi\dELi0ELb1E", "small-row kernel, sixteen waves, norm folded in"),
-    # one query head per KV group at head dimension 128
-    (r"causal_split_kernelILi128ELi8ELi1ELi1E", "attention of a prompt chunk, eight vectors per thread"),
 ]
 
 _NAME = re.compile(r"Function Name: (\S+)")

@@ -8,15 +8,14 @@
 // Tk <= 64 rows of the earlier expansion levels and this one).  Call site replaced: mlx_llama.py:185-195.
 //
 // tree_attn_kernel: 1..64 query rows, one launch, or two where the keys are split over workgroups.
-// causal_split_kernel, causal_merge_kernel: a prompt chunk (mlx_llama.py:275-276) in pieces of 32 rows on blockIdx.z, each
-// with its own cache length, the mask generated in the kernel, one launch pair for all pieces.
+// causal_attn_kernel: a prompt chunk (mlx_llama.py:275-276) in pieces of 32 rows, each with its own cache length, the mask
+// generated in the kernel, one launch for all pieces (two where the keys are split).
 #include "common.h"
 
 #include <math.h>
 
 namespace {
 
-constexpr int KT = 32;   // keys per block
 constexpr float M_FLOOR = -3.0e38f;   // running maximum of a row that has seen no key yet
 
 // ds_read_b64_tr_b16: 16 lanes x 4 halves, transposed (lane i of a group of 16 receives element
@@ -345,217 +344,185 @@ int launch_tree(const void* q, const void* kc, const void* vc, const uint32_t* b
 
 // ---- a prompt chunk in pieces of 32 rows ----
 //
-// Split-KV: grid (kv head g, key split s, piece); one wave per query head of the group, so a K/V tile is read from memory
-// once per group and shared through LDS.  Per block of 32 keys (a tile holds one or two) a wave computes S^T = K Q^T with
-// v_mfma_f32_32x32x16_f16 (rows = keys, columns = the 32 rows of the piece), runs the online softmax on its accumulator
-// (a lane owns one row, its partner lane+32 the other half of the keys), and feeds exp(S^T) straight back as the B operand of
-// O^T += V^T P^T; only V needs a transposed read from LDS (ds_read_b64_tr_b16).  Partial (m, l, O) per split go to a
-// workspace and a second kernel merges them.  The key tiles of the live length are dealt evenly to as many splits as give each at
-// least two tiles and the launch at most as many workgroups as the GPU holds at once; the busiest workgroup sets the time.
+// A workgroup of eight waves owns up to four (query head, piece) pairs of a KV group: four heads of one piece, or with fewer
+// heads per group several pieces.  K and V go through LDS in tiles of 128 keys; four waves take the first 64 keys of a tile, the other
+// four the second, so that two waves of a SIMD work on the same rows, and the halves' (m, l, O) meet in LDS at the end.
+// Per block of 32 keys a wave computes S^T = K Q^T with v_mfma_f32_32x32x16_f16 (rows = keys, columns = the 32 rows of its piece),
+// runs the online softmax on its accumulator (a lane owns one row, its partner lane + 32 the other half of the keys) and feeds
+// exp(S^T) straight back as the B operand of O^T += V^T P^T; only V needs a transposed read from LDS (ds_read_b64_tr_b16).
+//
+// A chunk has hundreds of pairs, so the keys are split over workgroups only where a few pairs would leave most of the GPU idle (fp16
+// partial results, added by a second kernel).  What bounds it: 2.5 us per tile of a workgroup, of which the matrix instructions are 0.9,
+// and the last workgroups of a causal triangle.  Before, a workgroup held all heads of a group (seven waves) on tiles of 64 keys, one
+// per compute unit, the longest twice the average, and every result went through partials and a merge; us per chunk
+// (28 heads of 128 in 4 groups; before / now): 2048 rows 101 / 52, 512 rows 24.8 / 15.7, 128 rows 13.4 / 8.1, 512 rows behind 1536
+// 41 / 36; 14 heads of 64 in 2 groups, 2048 rows 37 / 27.
+constexpr int CAUSAL_TILE = 128;
 
-// splits that get work when `ntiles` key tiles are dealt to a grid of `nsplit` splits
-// `lanes` = KV groups x pieces of query rows, the (group, piece) pairs that share the GPU: with
-// many of them (a prompt chunk) the keys are split less, so that the launch has about as many
-// workgroups as the GPU holds at once (`slots`) and each covers more tiles per partial result
-// it writes (8B shape, 512-row chunk, us per launch pair with 2 / 4 / 8 / 16 tiles at least: 33 /
-// 29 / 33 / 44 on an empty cache, 94 / 78 / 70 / 66 behind 1536 rows).
-__host__ __device__ inline int active_splits(int ntiles, int nsplit, int lanes, int slots, int floor_tiles) {
+// cached rows before piece p (never past the cache, whatever the counter says: a graph replayed beyond the capacity
+// would otherwise read beyond the last head's buffer), and rows that pieces p .. p + n - 1 see
+__device__ inline int causal_length(const int32_t* len_dev, int p, long cap) {
+  int P = len_dev[p];
+  if (P > cap - 32) P = (int)(cap - 32);
+  return P < 0 ? 0 : P;
+}
+__device__ inline int causal_rows(const int32_t* len_dev, int p, int n, int pieces, long cap) {
+  int most = 0;
+  for (int i = p; i < p + n && i < pieces; ++i) {
+    const int rows = causal_length(len_dev, i, cap) + 32;
+    most = rows > most ? rows : most;
+  }
+  return most;
+}
+
+// Splits in use for `ntiles` tiles in a grid of `nsplit`, `units` workgroups beside each other: as many as fill the GPU, with
+// at least four tiles each (two where there are few units): a split costs its partial results and the second launch (28
+// heads of 128, us with no split / at least 4 / 2 / 1 tiles: 512 rows 15.7 / 15.7 / 19.1 / 21.1, 256 rows behind 1792 41.6 / 25.3 / 25.9 /
+// 26.2, 64 rows behind 2000 46 / 21.4 / 17.7 / 17.5).
+__host__ __device__ inline int causal_splits(int ntiles, int nsplit, int units) {
   int tpw = (ntiles + nsplit - 1) / nsplit;
-  int min_tiles = (lanes * ntiles + slots - 1) / slots;
-  if (min_tiles < floor_tiles) min_tiles = floor_tiles;
-  if (tpw < min_tiles) tpw = min_tiles;
+  const int fill = (units * ntiles + 255) / 256, least = units <= 32 ? 2 : 4;
+  tpw = tpw > fill ? tpw : fill;
+  tpw = tpw > least ? tpw : least;
   return (ntiles + tpw - 1) / tpw;
 }
 
-// Workgroups of `rep` waves that the 256 compute units hold at once: the split kernel's registers
-// allow two waves per SIMD at head dimension 128 and three at 64.  One workgroup more than that
-// costs a second round (264 workgroups of seven waves 20.6 us; 176, one round, 10.4).
-__host__ __device__ inline int split_slots(int rep, int hd) {
-  const int waves_per_cu = hd > 64 ? 8 : 12;
-  const int per_cu = waves_per_cu / rep;
-  return 256 * (per_cu < 1 ? 1 : per_cu);
-}
+constexpr int MAX_CAUSAL_SPLITS = 64;     // what the workspace holds
 
-// q [H,T,hd] is rotated already and the cache holds the tree rows.
-// NVU: 16-byte vectors of a K (or V) tile per thread, a power of two with NVU * blockDim.x >= the
-// vectors of a tile.  DEPTH: tiles requested ahead, each in registers of its own (a tile's way
-// from the L2 into LDS takes longer than its arithmetic: with one tile ahead the loop runs at one
-// load latency per tile).
 template <int V>
 struct Stage { static constexpr int value = V; };
 
-// SUB: 32-key blocks per tile (1 or 2).  With two, the S products, the exponentials and the O
-// products of 64 keys each form one phase of a tile instead of two: the phases of a tile depend on
-// each other inside a wave, so a tile of 64 keys takes little longer than one of 32.
-template <int HD, int NVU, int DEPTH, int SUB>
-__global__ __launch_bounds__(512) void causal_split_kernel(
+template <int HD, int DEPTH>
+__global__ __launch_bounds__(512, 2) void causal_attn_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ kc, const half_t* __restrict__ vc,
-    const int32_t* __restrict__ len_dev, half_t* __restrict__ part_o, float* __restrict__ part_ml, int H, int G, long cap,
-    float scale_log2e, int q_rows) {
+    const int32_t* __restrict__ len_dev, half_t* __restrict__ out, half_t* __restrict__ part_o, float* __restrict__ part_ml, int H,
+    int G, long cap, float scale_log2e, int pieces, int hp, int pp) {
   constexpr int KSTEPS = HD / 16;       // MFMA steps over the head dimension for S
   constexpr int DB = HD / 32;           // 32-wide blocks of the head dimension for O
   constexpr int STR = HD * 2 + 16;      // LDS row stride in bytes (pad: conflict-free reads)
   constexpr int VEC_ROW = HD / 8;       // 16-byte vectors per K/V row
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  constexpr int KTT = KT * SUB;         // keys per tile
+  constexpr int KTT = CAUSAL_TILE;
+  constexpr int NVU = KTT * VEC_ROW / 512;        // vectors of K (or V) per thread
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * KTT * STR];
+  __shared__ float2_t ml_half[4][32];
   unsigned char* ldsK = lds;
   unsigned char* ldsV = lds + KTT * STR;
-
-  const int g = blockIdx.x;
-  const int split = blockIdx.y;
-  const int nsplit = gridDim.y;
-  const int rep = H / G;
+  const int rep = H / G, quads = (rep + hp - 1) / hp;
+  const int g = blockIdx.x / quads, hq = blockIdx.x % quads;
+  const int split = blockIdx.y, nsplit = gridDim.y;
+  const int group = gridDim.z - 1 - blockIdx.z;   // (the last pieces see the most keys: dispatched first)
   const int tid = threadIdx.x;
-  const int nthr = blockDim.x;          // rep * 64
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
-  const int ql = lane & 31;             // tree token (column of S^T / O^T)
-  const int hb = lane >> 5;             // which half of the k / key index this lane holds
-  const int head = g * rep + wave;
-
-  // blockIdx.z: piece of 32 query rows, queries at rows 32 * piece of q [H, q_rows, hd], with a cache length of its own
-  // (the last piece sees the most keys: dispatched first)
-  const int piece = gridDim.z - 1 - blockIdx.z;
-  const int qrow = piece * 32 + ql;
-  int P = len_dev[piece];
-  // never index past the cache, whatever the counter says (a graph replayed beyond the
-  // capacity would otherwise read beyond the last head's buffer)
-  if (P > cap - 32) P = (int)(cap - 32);
-  if (P < 0) P = 0;
-  const int Ltot = P + 32;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wave = wid & 3, khalf = wid >> 2;
+  const int ql = lane & 31, hb = lane >> 5;
+  // this wave's head of the group and piece; a wave that has none carries keys and values like the others
+  int hin = hq * hp + wave % hp, piece = group * pp + wave / hp;
+  const bool live = hin < rep && piece < pieces && wave < hp * pp;
+  if (!live) {
+    hin = 0;
+    piece = group * pp;
+  }
+  const int head = g * rep + hin;
+  const int P = causal_length(len_dev, piece, cap);
+  const int Ltot = causal_rows(len_dev, group * pp, pp, pieces, cap);
   const int ntiles = (Ltot + KTT - 1) / KTT;
-  // Splits in use for this length: every workgroup gets at most `tpw` key tiles, two at
-  // least (with one, writing and merging the partials costs more than reading the keys).
-  // The tile count of the busiest workgroup sets the time, so the tiles are spread evenly
-  // over exactly as many workgroups as that takes; the rest of the grid leaves at once.
-  const int nactive = active_splits(ntiles, nsplit, gridDim.x * gridDim.z, split_slots(rep, HD), 3 - SUB);
+  const int own = live ? P + 32 : 0;       // keys up to here concern this wave's rows
+  const int nactive = causal_splits(ntiles, nsplit, gridDim.x * gridDim.z);
   if (split >= nactive) return;
   half8_t qreg[KSTEPS];
-  const half_t* qp = q + ((long)head * q_rows + qrow) * HD;
+  const half_t* qp = q + ((long)head * pieces * 32 + piece * 32 + ql) * HD;
 #pragma unroll
   for (int kk = 0; kk < KSTEPS; ++kk) qreg[kk] = *reinterpret_cast<const half8_t*>(qp + kk * 16 + hb * 8);
 
   float m_run = M_FLOOR, l_run = 0.f;
-  // this lane's address for the transposing loads of V (see the O^T step below)
+  // this lane's address for the transposing loads of V: within 16 lanes, lane s asks for key row s / 4 at the four d
+  // columns 4 (s % 4) .. + 3 of the group's 16 and gets four keys of its own d
   const unsigned char* vt_base =
-      ldsV + (4 * hb + ((lane & 15) >> 2)) * STR + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+      ldsV + (64 * khalf + 4 * hb + ((lane & 15) >> 2)) * STR + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   float16_t o_acc[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o_acc[db][i] = 0.f;
-
   const half_t* kbase_ptr = kc + (long)g * cap * HD;
   const half_t* vbase_ptr = vc + (long)g * cap * HD;
-
-  // This workgroup's tiles are split, split + nactive, ...: all workgroups share the live part
-  // of the cache however short it is.  The next DEPTH tiles are in flight into registers while
-  // the current one is being used.
-  constexpr int NVEC = KTT * VEC_ROW;                // 16-byte vectors per K (or V) tile
   half8_t kreg[DEPTH][NVU], vreg[DEPTH][NVU];
   auto fetch = [&](auto S, int tile) {
     constexpr int st = decltype(S)::value;
     const int kb = tile * KTT;
 #pragma unroll
     for (int it = 0; it < NVU; ++it) {
-      int v = tid + it * nthr;
-      if (v > NVEC - 1) v = NVEC - 1;
-      const int row = v / VEC_ROW;
-      const int c = v % VEC_ROW;
-      int kidx = kb + row;
-      if (kidx > Ltot - 1) kidx = Ltot - 1;          // rows past the end are masked out below
-      const half_t* kp = kbase_ptr + (long)kidx * HD;
-      const half_t* vp = vbase_ptr + (long)kidx * HD;
-      kreg[st][it] = *reinterpret_cast<const half8_t*>(kp + c * 8);
-      vreg[st][it] = *reinterpret_cast<const half8_t*>(vp + c * 8);
+      const int v = tid + it * 512;
+      int kidx = kb + v / VEC_ROW;
+      if (kidx > Ltot - 1) kidx = Ltot - 1;
+      kreg[st][it] = *reinterpret_cast<const half8_t*>(kbase_ptr + (long)kidx * HD + v % VEC_ROW * 8);
+      vreg[st][it] = *reinterpret_cast<const half8_t*>(vbase_ptr + (long)kidx * HD + v % VEC_ROW * 8);
     }
   };
   auto stash = [&](auto S) {
     constexpr int st = decltype(S)::value;
 #pragma unroll
     for (int it = 0; it < NVU; ++it) {
-      const int v = tid + it * nthr;
-      if (v < NVEC) {
-        const int row = v / VEC_ROW;
-        const int c = v % VEC_ROW;
-        *reinterpret_cast<half8_t*>(ldsK + row * STR + c * 16) = kreg[st][it];
-        *reinterpret_cast<half8_t*>(ldsV + row * STR + c * 16) = vreg[st][it];
-      }
+      const int v = tid + it * 512;
+      *reinterpret_cast<half8_t*>(ldsK + v / VEC_ROW * STR + v % VEC_ROW * 16) = kreg[st][it];
+      *reinterpret_cast<half8_t*>(ldsV + v / VEC_ROW * STR + v % VEC_ROW * 16) = vreg[st][it];
     }
   };
-
-  // Every fetch is issued whether or not its tile exists (the index is clamped to the last
-  // tile, whose rows are in the cache): with a fetch under a condition the compiler no longer
-  // knows how many loads are outstanding where a stage is waited for, and waits for all of them.
+  // every fetch is issued whether or not its tile exists (the last one again), so that what is in flight is known at every wait
   auto tile_at = [&](int t) { return t < ntiles ? t : ntiles - 1; };
-  // (and the stages are requested in the order in which they are waited for, here as in the loop)
   __builtin_amdgcn_sched_barrier(0);
   fetch(Stage<0>{}, split);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (DEPTH > 1) fetch(Stage<1>{}, tile_at(split + nactive));
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (DEPTH > 2) fetch(Stage<2>{}, tile_at(split + 2 * nactive));
-  __builtin_amdgcn_sched_barrier(0);
-  // one tile: its registers (stage S) into LDS, the tile DEPTH ahead requested into the same
-  // registers, then the arithmetic on LDS
   auto do_tile = [&](auto S, int tile) {
-    constexpr int st = decltype(S)::value;
-    const int kb = tile * KTT;
-    __syncthreads();   // every wave is done with the previous tile
+    const int kb = tile * KTT + 64 * khalf;
+    __syncthreads();
     stash(S);
     fetch(S, tile_at(tile + DEPTH * nactive));
     __syncthreads();
-
-    // S^T[key][token] = sum_d K[key][d] Q[token][d], one accumulator per block of 32 keys
-    float16_t sacc[SUB];
+    if (kb >= own) return;                        // (a wave)
+    float16_t sacc[2];
 #pragma unroll
-    for (int h = 0; h < SUB; ++h)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 16; ++i) sacc[h][i] = 0.f;
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk)
 #pragma unroll
-      for (int h = 0; h < SUB; ++h) {
-        const half8_t a = *reinterpret_cast<const half8_t*>(ldsK + (32 * h + ql) * STR + kk * 32 + hb * 16);
+      for (int h = 0; h < 2; ++h) {
+        const half8_t a = *reinterpret_cast<const half8_t*>(ldsK + (64 * khalf + 32 * h + ql) * STR + kk * 32 + hb * 16);
         sacc[h] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qreg[kk], sacc[h], 0, 0, 0);
       }
-
-    // accumulator register i of this lane is key 8*(i/4) + 4*hb + i%4 of its block.  The scores
-    // stay unscaled: the scale (> 0) goes into the exponent's fused multiply-add, and the running
-    // maximum starts at a finite floor instead of -inf, so that no case needs a select.
+    // accumulator register i of this lane is key 8*(i/4) + 4*hb + i%4 of its block of 32; unscaled, as in the kernel above
     float bm = M_FLOOR;
-    if (kb + KTT <= P) {
-      // a tile of prefix rows: visible to every row, no mask arithmetic
+    if (kb + 64 > P) {
 #pragma unroll
-      for (int h = 0; h < SUB; ++h)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) bm = fmaxf(bm, sacc[h][i]);
-    } else {
-#pragma unroll
-      for (int h = 0; h < SUB; ++h)
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int key = kb + 32 * h + 8 * (i >> 2) + 4 * hb + (i & 3);
           sacc[h][i] = key - P <= ql ? sacc[h][i] : -INFINITY;
-          bm = fmaxf(bm, sacc[h][i]);
         }
     }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) bm = fmaxf(bm, sacc[h][i]);
     bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
     const float m_new = fmaxf(m_run, bm * scale_log2e);
-    // arguments are <= 0: the bare hardware exp2 (results below 2^-126 flush to zero, -inf gives 0)
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     float psum = 0.f;
-    half8_t bp[SUB][2];     // exp(S^T) as the B operand of the O products: step u = registers 8u..8u+7
+    half8_t bp[2][2];       // exp(S^T) as the B operand of the O products: step u = registers 8u..8u+7
 #pragma unroll
-    for (int h = 0; h < SUB; ++h)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float pv = __builtin_amdgcn_exp2f(fmaf(sacc[h][i], scale_log2e, -m_new));
         psum += pv;
         bp[h][i >> 3][i & 7] = (half_t)pv;
       }
-    psum += __shfl_xor(psum, 32, 64);
-    l_run = l_run * alpha + psum;
+    l_run = l_run * alpha + psum;                 // this lane's keys; its partner's are added at the end
     m_run = m_new;
     if (alpha != 1.f) {
 #pragma unroll
@@ -563,14 +530,8 @@ __global__ __launch_bounds__(512) void causal_split_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) o_acc[db][i] *= alpha;
     }
-
-    // O^T[d][token] += sum_key V[key][d] P[token][key]; step u of block h covers accumulator
-    // registers 8u..8u+7, i.e. keys 32h + 8*(2u + j/4) + 4*hb + j%4, j = 0..7.  The V^T operand
-    // comes from the row-major tile through the transposing LDS load: within 16 lanes, lane i
-    // receives element i % 4 of the four lanes 4 jj + i / 4, so lane s of a group asks for key row
-    // s / 4 at the four d columns 4 (s % 4) .. + 3 of the group's 16 and gets four keys of its own d.
 #pragma unroll
-    for (int h = 0; h < SUB; ++h)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -581,179 +542,152 @@ __global__ __launch_bounds__(512) void causal_split_kernel(
           o_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bp[h][u], o_acc[db], 0, 0, 0);
         }
   };
-  // whole rounds of DEPTH tiles (no condition between the stages of a round, so that the loads
-  // outstanding at every wait are known), then the last DEPTH - 1 tiles at most
   int t0 = split;
   for (; t0 + (DEPTH - 1) * nactive < ntiles; t0 += DEPTH * nactive) {
     do_tile(Stage<0>{}, t0);
     if constexpr (DEPTH > 1) do_tile(Stage<1>{}, t0 + nactive);
-    if constexpr (DEPTH > 2) do_tile(Stage<2>{}, t0 + 2 * nactive);
   }
-  if constexpr (DEPTH > 1) {
-    if (t0 < ntiles) {
-      do_tile(Stage<0>{}, t0);
-      if constexpr (DEPTH > 2)
-        if (t0 + nactive < ntiles) do_tile(Stage<1>{}, t0 + nactive);
+  if constexpr (DEPTH > 1)
+    if (t0 < ntiles) do_tile(Stage<0>{}, t0);
+  l_run += __shfl_xor(l_run, 32, 64);
+  // the second half of the waves hands its (m, l, O) to the first through LDS
+  __syncthreads();
+  constexpr int OS = HD + 4;
+  static_assert(4 * 32 * OS * 4 <= 2 * KTT * STR, "the halves' tiles do not fit over K and V");
+  float* half_o = reinterpret_cast<float*>(lds) + wave * (32 * OS) + ql * OS + 4 * hb;
+  if (khalf) {
+    if (hb == 0) ml_half[wave][ql] = float2_t{m_run, l_run};
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4)
+        *reinterpret_cast<float4_t*>(half_o + db * 32 + 8 * i4) =
+            float4_t{o_acc[db][4 * i4], o_acc[db][4 * i4 + 1], o_acc[db][4 * i4 + 2], o_acc[db][4 * i4 + 3]};
+  }
+  __syncthreads();
+  if (khalf) return;
+  {
+    const float2_t other = ml_half[wave][ql];
+    const float m_new = fmaxf(m_run, other[0]);
+    const float fa = __builtin_amdgcn_exp2f(m_run - m_new), fb = __builtin_amdgcn_exp2f(other[0] - m_new);
+    l_run = l_run * fa + other[1] * fb;
+    m_run = m_new;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const float4_t o = *reinterpret_cast<const float4_t*>(half_o + db * 32 + 8 * i4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o_acc[db][4 * i4 + e] = o_acc[db][4 * i4 + e] * fa + o[e] * fb;
+      }
+  }
+  if (nactive > 1) {
+    if (!live) return;
+    const long slot = (((long)piece * H + head) * nsplit + split) * 32 + ql;
+    if (hb == 0) {
+      part_ml[slot * 2 + 0] = m_run;
+      part_ml[slot * 2 + 1] = l_run;
     }
+    half_t* po = part_o + slot * HD;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4)
+        *reinterpret_cast<half4_t*>(po + db * 32 + 8 * i4 + 4 * hb) =
+            half4_t{(half_t)o_acc[db][4 * i4 + 0], (half_t)o_acc[db][4 * i4 + 1], (half_t)o_acc[db][4 * i4 + 2], (half_t)o_acc[db][4 * i4 + 3]};
+    return;
   }
-
-  // partials: part_ml [H][nsplit][32][2], part_o [H][nsplit][32][HD]
-  const long slot = (((long)piece * H + head) * nsplit + split) * 32 + ql;
-  if (hb == 0) {
-    part_ml[slot * 2 + 0] = m_run;
-    part_ml[slot * 2 + 1] = l_run;
-  }
-  half_t* po = part_o + slot * HD;     // fp16: |O| <= keys per split, relative error 2^-11
+  // one split: the rows as they lie in memory, through the wave's part of LDS
+  unsigned char* mine = lds + wave * (32 * OS * 4);
+  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const int d0 = db * 32 + 8 * i4 + 4 * hb;
-      half4_t v = half4_t{(half_t)o_acc[db][4 * i4 + 0], (half_t)o_acc[db][4 * i4 + 1],
-                          (half_t)o_acc[db][4 * i4 + 2], (half_t)o_acc[db][4 * i4 + 3]};
-      *reinterpret_cast<half4_t*>(po + d0) = v;
-    }
+    for (int i4 = 0; i4 < 4; ++i4)
+      *reinterpret_cast<half4_t*>(mine + ql * STR + (db * 32 + 8 * i4 + 4 * hb) * 2) =
+          half4_t{(half_t)(o_acc[db][4 * i4 + 0] * inv), (half_t)(o_acc[db][4 * i4 + 1] * inv), (half_t)(o_acc[db][4 * i4 + 2] * inv),
+                  (half_t)(o_acc[db][4 * i4 + 3] * inv)};
+  __builtin_amdgcn_wave_barrier();
+  if (!live) return;
+#pragma unroll
+  for (int it = 0; it < 32 * VEC_ROW / 64; ++it) {
+    const int v = lane + it * 64, row = v / VEC_ROW, c = v % VEC_ROW;
+    *reinterpret_cast<half8_t*>(out + ((long)(piece * 32 + row) * H + head) * HD + c * 8) =
+        *reinterpret_cast<const half8_t*>(mine + row * STR + c * 16);
+  }
 }
 
-// Merge the splits.  Grid (H, 8, piece): a workgroup owns four rows of one head; one
-// thread per four output elements.  The softmax weights of the splits are computed once per
-// row with one split per lane, then every thread adds its slice of the partial outputs.
-constexpr int MERGE_TOK = 4;
-
+// Adds the splits of a piece: a thread per eight output elements, every split in use requested at once.
 template <int HD>
-__global__ void causal_merge_kernel(const half_t* __restrict__ part_o,
-                                    const float* __restrict__ part_ml,
-                                    half_t* __restrict__ out, int H, int nsplit,
-                                    const int32_t* __restrict__ len_dev, long cap, int groups, int sub) {
-  const int piece = blockIdx.z;                     // as in the split kernel
-  part_o += (long)piece * H * nsplit * 32 * HD;
-  part_ml += (long)piece * H * nsplit * 32 * 2;
-  out += (long)piece * 32 * H * HD;
-  constexpr int QW = HD / 4;                       // threads per token
-  constexpr int TPW = 256 / HD;                    // tokens per wave: MERGE_TOK tokens on HD / 64 waves
-  constexpr int PRE = 32;                          // partial outputs requested before anything is waited for
-  __shared__ float wts[MERGE_TOK][64];
-  const int head = blockIdx.x;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  // Everything that does not depend on the live length is requested first: the (m, l) pairs
-  // of every split of the grid and the first partial outputs.  Splits beyond the active
-  // ones hold stale values; they are masked (m) or skipped (O) below, never multiplied.
-  float2_t ml[TPW];
+__global__ __launch_bounds__(256) void causal_add_kernel(const half_t* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                         half_t* __restrict__ out, int H, int nsplit, const int32_t* __restrict__ len_dev,
+                                                         long cap, int pp, int units) {
+  constexpr int VR = HD / 8, MOST = 8;
+  const int piece = blockIdx.z, pieces = gridDim.z;
+  const int rows = causal_rows(len_dev, piece / pp * pp, pp, pieces, cap);
+  const int nact = causal_splits((rows + CAUSAL_TILE - 1) / CAUSAL_TILE, nsplit, units);
+  if (nact == 1) return;                           // written by the workgroup itself
+  const int id = blockIdx.x * 256 + threadIdx.x;   // (head, row, vector)
+  const int hr = id / VR, c = id % VR;
+  if (hr >= H * 32) return;
+  const int head = hr >> 5, row = hr & 31;
+  const long slot = ((long)piece * H + head) * nsplit * 32 + row;
+  float m_run = M_FLOOR, l_run = 0.f;
+  float acc[8];
 #pragma unroll
-  for (int k = 0; k < TPW; ++k) {
-    const int t = blockIdx.y * MERGE_TOK + wave * TPW + k;
-    const int sp = lane < nsplit ? lane : nsplit - 1;
-    ml[k] = *reinterpret_cast<const float2_t*>(part_ml + (((long)head * nsplit + sp) * 32 + t) * 2);
-  }
-  const int tl = tid / QW;
-  const int dq = tid % QW;
-  const int t = blockIdx.y * MERGE_TOK + tl;
-  const half_t* src = part_o + ((long)head * nsplit * 32 + t) * HD + dq * 4;
-  // One or two pieces of query rows (most splits of the grid are active): every split's partial output is requested before
-  // the length is known.  More pieces (a few active splits out of a grid sized for the longest cache): only the active
-  // ones, after it (8B shape, 16 pieces behind 1536 cache rows: 20 -> 9 us).
-  const bool eager = gridDim.z <= 2;
-  half4_t pre[PRE];
-  if (eager) {
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  for (int s0 = 0; s0 < nact; s0 += MOST) {
+    float2_t ml[MOST];
+    half8_t o[MOST];
 #pragma unroll
-    for (int k = 0; k < PRE; ++k)
-      if (k < nsplit) pre[k] = *reinterpret_cast<const half4_t*>(src + (long)k * 32 * HD);
-  }
-
-  int P = len_dev[piece];
-  if (P > cap - 32) P = (int)(cap - 32);    // as in the split kernel
-  if (P < 0) P = 0;
-  const int nact = active_splits((P + 32 + KT * sub - 1) / (KT * sub), nsplit, groups * gridDim.z,
-                                 split_slots(H / groups, HD), 3 - sub);   // as in the split kernel
-  if (!eager) {
-#pragma unroll
-    for (int k = 0; k < PRE; ++k)
-      if (k < nact) pre[k] = *reinterpret_cast<const half4_t*>(src + (long)k * 32 * HD);
-  }
-#pragma unroll
-  for (int k = 0; k < TPW; ++k) {
-    const float m = lane < nact ? ml[k][0] : -INFINITY;
-    const float l = lane < nact ? ml[k][1] : 0.f;
-    const float mx = wave_max(m);
-    const float w = m == -INFINITY ? 0.f : exp2f(m - mx);
-    const float den = wave_sum(w * l);
-    wts[wave * TPW + k][lane] = den > 0.f ? w / den : 0.f;
-  }
-  __syncthreads();
-  float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int k = 0; k < PRE; ++k)
-    if (k < nact) {
-      const float wk = wts[tl][k];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] += wk * (float)pre[k][e];
-    }
-  for (int s0 = PRE; s0 < nact; s0 += 8) {
-    half4_t v[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int sp = s0 + k < nact ? s0 + k : nact - 1;
-      v[k] = *reinterpret_cast<const half4_t*>(src + (long)sp * 32 * HD);
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
+    for (int k = 0; k < MOST; ++k)
       if (s0 + k < nact) {
-        const float wk = wts[tl][s0 + k];
+        const long at = slot + (long)(s0 + k) * 32;
+        ml[k] = *reinterpret_cast<const float2_t*>(part_ml + at * 2);
+        o[k] = *reinterpret_cast<const half8_t*>(part_o + at * HD + c * 8);
+      }
+    float mx = m_run;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] += wk * (float)v[k][e];
+    for (int k = 0; k < MOST; ++k)
+      if (s0 + k < nact) mx = fmaxf(mx, ml[k][0]);
+    const float alpha = __builtin_amdgcn_exp2f(m_run - mx);
+    m_run = mx;
+    l_run *= alpha;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] *= alpha;
+#pragma unroll
+    for (int k = 0; k < MOST; ++k)
+      if (s0 + k < nact) {
+        const float f = __builtin_amdgcn_exp2f(ml[k][0] - mx);
+        l_run += f * ml[k][1];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = fmaf(f, (float)o[k][e], acc[e]);
       }
   }
-  half4_t o = half4_t{(half_t)acc[0], (half_t)acc[1], (half_t)acc[2], (half_t)acc[3]};
-  *reinterpret_cast<half4_t*>(out + ((long)t * H + head) * HD + dq * 4) = o;
-}
-
-// Key splits of the grid (gridDim.y), sized for the longest length; how many of them get work
-// follows the live length inside the kernels (active_splits).
-int splits_for(int max_len) {
-  const int ntiles = (max_len + KT - 1) / KT;
-  int n = (ntiles + 1) / 2;            // two tiles per workgroup at the longest length
-  if (n > 64) n = 64;                  // one split per lane in the merge
-  if (n < 1) n = 1;
-  return n;
+  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+  half8_t r;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) r[e] = (half_t)(acc[e] * inv);
+  *reinterpret_cast<half8_t*>(out + ((long)(piece * 32 + row) * H + head) * HD + c * 8) = r;
 }
 
 template <int HD>
 int launch_causal(const void* q, const void* kc, const void* vc, const int32_t* len, void* out, int pieces, int H, int G,
                   long cap, int max_len, float scale, void* workspace, hipStream_t st) {
-  // The grid holds as many splits as the longest length makes active: a workgroup without
-  // work still takes a slot for the 2 us in which it learns that from the cache length, and
-  // thousands of them ahead of the last pieces' workgroups (a chunk of 16 pieces in a grid of 36
-  // splits for 4 active ones) held those back by 18 of 44 us.
-  const int rep = H / G;
-  // 64 keys per tile where a tile's 16-byte vectors are at most four per thread (three or more
-  // waves per workgroup at head dimension 128, two or more at 64), 32 keys otherwise
-  const int need64 = (2 * KT * (HD / 8) + rep * 64 - 1) / (rep * 64);
-  const int sub = need64 <= 4 ? 2 : 1;
-  const int ktt = KT * sub;
-  const int nsplit = active_splits((max_len + ktt - 1) / ktt, splits_for(max_len), G * pieces, split_slots(rep, HD), 3 - sub);
+  const int rep = H / G, hp = rep < 4 ? rep : 4, gx = G * ((rep + hp - 1) / hp);
+  // with fewer than four heads per group a workgroup takes several pieces, unless that leaves compute units without one
+  int pp = 4 / hp;
+  while (pp > 1 && gx * ((pieces + pp - 1) / pp) < 256) --pp;
+  const int nz = (pieces + pp - 1) / pp, units = gx * nz;
+  const int nsplit = causal_splits((max_len + CAUSAL_TILE - 1) / CAUSAL_TILE, MAX_CAUSAL_SPLITS, units);
   float* part_ml = static_cast<float*>(workspace);
   half_t* part_o = reinterpret_cast<half_t*>(part_ml + (size_t)pieces * H * nsplit * 32 * 2);
-  const float sl2 = scale * 1.4426950408889634f;
-  const size_t lds = 2 * ktt * (HD * 2 + 16);
-  // vectors of a tile per thread (a power of two) and the tiles in flight that its registers allow
-  const int need = (ktt * (HD / 8) + rep * 64 - 1) / (rep * 64);
-#define EAGLE_ATTN_SPLIT(NVU, DEPTH, SUB)                                                                         \
-  hipLaunchKernelGGL((causal_split_kernel<HD, NVU, DEPTH, SUB>), dim3(G, nsplit, pieces), dim3(rep * 64), lds, st, \
-                     static_cast<const half_t*>(q), static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), len, part_o, \
-                     part_ml, H, G, cap, sl2, pieces * 32)
-  if (sub == 2) {
-    if (need <= 1) EAGLE_ATTN_SPLIT(1, 3, 2);
-    else if (need <= 2) EAGLE_ATTN_SPLIT(2, 2, 2);
-    else EAGLE_ATTN_SPLIT(4, 1, 2);
-  } else {
-    if (need <= 4) EAGLE_ATTN_SPLIT(4, 2, 1);
-    else EAGLE_ATTN_SPLIT(8, 1, 1);
-  }
-#undef EAGLE_ATTN_SPLIT
-  hipLaunchKernelGGL(causal_merge_kernel<HD>, dim3(H, 32 / MERGE_TOK, pieces), dim3(MERGE_TOK * HD / 4), 0, st, part_o, part_ml,
-                     static_cast<half_t*>(out), H, nsplit, len, cap, G, sub);
+  hipLaunchKernelGGL((causal_attn_kernel<HD, HD == 64 ? 2 : 1>), dim3(gx, nsplit, nz), dim3(512), 0, st, static_cast<const half_t*>(q),
+                     static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), len, static_cast<half_t*>(out), part_o, part_ml, H, G,
+                     cap, scale * 1.4426950408889634f, pieces, hp, pp);
+  if (nsplit > 1)
+    hipLaunchKernelGGL(causal_add_kernel<HD>, dim3((H * 32 * (HD / 8) + 255) / 256, 1, pieces), dim3(256), 0, st, part_o, part_ml,
+                       static_cast<half_t*>(out), H, nsplit, len, cap, pp, units);
   return eagle_launch_status();
 }
 

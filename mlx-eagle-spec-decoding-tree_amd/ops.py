@@ -681,7 +681,7 @@ def scaled_dot_product_attention(queries, keys, values, cache=None, scale=None, 
 
 
 def causal_attention(q, k_cache, v_cache, piece_len_dev, scale, max_len=None, out=None):
-    """Causal attention of a prompt chunk in pieces of 32 rows, one launch pair for all pieces:
+    """Causal attention of a prompt chunk in pieces of 32 rows, one launch for all pieces (two with few rows behind many):
     q [H,R,hd] (R a multiple of 32); piece j sits at cache rows piece_len_dev[j] .. +31.
     Returns [R, H*hd]."""
     _need_cuda(q, k_cache, v_cache, piece_len_dev)

@@ -1,0 +1,39 @@
+"""Attention of a prompt chunk over its divisions of the work (heads and pieces per workgroup, key splits) against 64-bit
+attention: lengths around tiles of 128 keys and their halves, pieces that are not consecutive, a cache that ends with the chunk."""
+import math
+
+import pytest
+import torch
+
+from mlx_eagle_spec_decoding_tree_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+# probabilities and the result rounded to fp16 and, with key splits, partial results too: each 2^-11 relative, averaged
+# over keys and elements (2^-11 / sqrt(3) each), and some room
+REL = 9e-4
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("H,G", [(1, 1), (4, 2), (6, 2), (4, 1), (5, 1), (14, 2), (28, 4), (16, 2)])
+@pytest.mark.parametrize("pieces,P,spare", [(1, 0, 0), (2, 31, 0), (3, 64, 7), (5, 97, 0), (16, 0, 0), (2, 1500, 40), (9, 700, 3)])
+def test_causal_chunk(dev, H, G, hd, pieces, P, spare):
+    g = torch.Generator(device=dev).manual_seed(H * 100 + pieces)
+    R = 32 * pieces
+    cap = P + R + spare
+    print(f"H={H} G={G} hd={hd} pieces={pieces} P={P} cap={cap}", flush=True)
+    q = torch.randn(H, R, hd, generator=g, device=dev).half()
+    k, v = (torch.randn(G, cap, hd, generator=g, device=dev).half() for _ in range(2))
+    starts = P + 32 * torch.arange(pieces, device=dev)
+    if pieces == 5:
+        starts[3] = 5                          # a piece somewhere else in the cache
+    got = ops.causal_attention(q, k, v, starts.int(), hd ** -0.5, max_len=cap)
+    rows = (starts[:, None] + torch.arange(32, device=dev)[None]).reshape(-1)
+    seen = torch.arange(cap, device=dev)[None] <= rows[:, None]
+    want = torch.empty(R, H, hd, dtype=torch.float64, device=dev)
+    for h in range(H):
+        s = q[h].double() @ k[h // (H // G)].double().t().contiguous() * hd ** -0.5
+        want[:, h] = torch.softmax(s.masked_fill(~seen, -math.inf), -1) @ v[h // (H // G)].double()
+    want = want.reshape(R, H * hd)
+    assert bool(torch.isfinite(got).all())
+    assert ((got.double() - want).norm() / want.norm()).item() <= REL
