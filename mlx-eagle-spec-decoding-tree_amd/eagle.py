@@ -553,7 +553,7 @@ class TreeVerifier:
         self.V = total_tokens
         self.T = T = total_tokens + 1
         # above 32 tree tokens: q|k|v, o, down and gate|up in the slab form with 64-row tiles where the shapes
-        # allow it, the tiled head in two passes, other products on the kernels of `ops.quantized_matmul`; two
+        # allow it, the head and other products on the kernels of `ops.quantized_matmul`; two
         # mask words per token
         self.wide = T > MAXT
         if self.wide and not fuse:
@@ -577,7 +577,8 @@ class TreeVerifier:
         self.head_tiled = None
         if (tiled or tiled is None) and fuse:
             self.tiled = tiled_projections(model, self.qkv_w, self.gu_w, self.slab, self.swiglu)
-            self.head_tiled = tiled_head(model)
+            # (one launch of the rows kernel reads the head once: 40 rows of 3584 -> 152064 80 us, two of the tiled form 117)
+            self.head_tiled = None if self.wide else tiled_head(model)
         i32 = dict(dtype=torch.int32, device=dev)
         f16 = dict(dtype=torch.float16, device=dev)
         self.tokens = torch.zeros(T, **i32)
