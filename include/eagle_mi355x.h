@@ -613,6 +613,9 @@ int eagle_fill_i32(int32_t* dst, int32_t value, long n, eagle_stream_t stream);
 /* positions[t] = *cache_len_dev + tree_position_ids[t] (mlx_eagle.py:343). */
 int eagle_tree_positions(const int32_t* tree_position_ids, const int32_t* cache_len_dev,
                          int32_t* positions, int T, eagle_stream_t stream);
+/* The rows of a prompt chunk of R rows (a multiple of 32, at most EAGLE_MAX_CHUNK) appended at *cache_len_dev:
+ * positions[i] = *cache_len_dev + i, and piece_len[j] = positions[32 j] for eagle_causal_attention_f16. */
+int eagle_chunk_positions(const int32_t* cache_len_dev, int32_t* positions, int32_t* piece_len, int R, eagle_stream_t stream);
 /* *cache_len_dev += delta (KVCache.offset bookkeeping after an append). */
 int eagle_advance_len(int32_t* cache_len_dev, int delta, eagle_stream_t stream);
 

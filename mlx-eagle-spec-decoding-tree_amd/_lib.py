@@ -109,6 +109,7 @@ SIGNATURES = {
     "eagle_kv_compact_f16": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_long, c_void_p]),
     "eagle_fill_i32": (c_int, [c_void_p, c_int32, c_long, c_void_p]),
     "eagle_tree_positions": (c_int, [c_void_p] * 3 + [c_int, c_void_p]),
+    "eagle_chunk_positions": (c_int, [c_void_p] * 3 + [c_int, c_void_p]),
     "eagle_advance_len": (c_int, [c_void_p, c_int, c_void_p]),
 }
 

@@ -332,6 +332,16 @@ __global__ void tree_positions_kernel(const int32_t* __restrict__ pos_ids,
   if (i < T) positions[i] = *len_dev + pos_ids[i];
 }
 
+// rows *len .. *len + R - 1 of a prompt chunk and the first row of each of its pieces of 32
+__global__ void chunk_positions_kernel(const int32_t* __restrict__ len_dev, int32_t* __restrict__ positions,
+                                       int32_t* __restrict__ piece_len, int R) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= R) return;
+  const int at = *len_dev + i;
+  positions[i] = at;
+  if ((i & 31) == 0) piece_len[i >> 5] = at;
+}
+
 __global__ void advance_len_kernel(int32_t* len_dev, int delta) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *len_dev += delta;
 }
@@ -473,6 +483,15 @@ EAGLE_EXPORT int eagle_tree_positions(const int32_t* tree_position_ids,
   hipLaunchKernelGGL(tree_positions_kernel, dim3(1), dim3(64), 0,
                      static_cast<hipStream_t>(stream), tree_position_ids, cache_len_dev, positions,
                      T);
+  return eagle_launch_status();
+}
+
+EAGLE_EXPORT int eagle_chunk_positions(const int32_t* cache_len_dev, int32_t* positions, int32_t* piece_len, int R,
+                                       eagle_stream_t stream) {
+  if (!cache_len_dev || !positions || !piece_len) return EAGLE_ERR_NULL;
+  if (R < 32 || (R % 32) != 0 || R > EAGLE_MAX_CHUNK) return EAGLE_ERR_SHAPE;
+  hipLaunchKernelGGL(chunk_positions_kernel, dim3((R + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), cache_len_dev,
+                     positions, piece_len, R);
   return eagle_launch_status();
 }
 

@@ -173,9 +173,7 @@ class ChunkPass:
         self.act = torch.empty((R, I), **f16)
         self.down = torch.empty((R, D), **f16)
         self.logits = torch.empty((P, args.vocab_size), **f16)      # of the last piece only
-        self.piece_off = (torch.arange(self.pieces, **i32) * P).contiguous()
         self.piece_len = torch.zeros(self.pieces, **i32)
-        self.arange = torch.arange(P, **i32)
         self.positions = torch.zeros(R, **i32)
         self.len_dev = cache[0].len_dev
         L = _lib.lib()
@@ -193,12 +191,8 @@ class ChunkPass:
         layers = m.model.layers
         at0 = layers[0].self_attn
         # cache length, positions and rotary table of every piece, once for all layers
-        _lib.check(L.eagle_tree_positions(_ptr(self.piece_off), _ptr(self.len_dev), _ptr(self.piece_len),
-                                          self.pieces, st), "piece lengths")
-        for j in range(self.pieces):
-            pos = self.positions[j * P:(j + 1) * P]
-            _lib.check(L.eagle_tree_positions(_ptr(self.arange), _ptr(self.piece_len[j:j + 1]), _ptr(pos),
-                                              P, st), "positions")
+        _lib.check(L.eagle_chunk_positions(_ptr(self.len_dev), _ptr(self.positions), _ptr(self.piece_len), self.R, st),
+                   "chunk positions")
         ops.rope_table(self.positions, at0._inv_freqs, at0._scaling_factor, out=self.rope_cs)
         emb = m.model.embed_tokens
         ops.embed(self.tokens, emb.weight, emb.scales, emb.biases, out=self.h)
