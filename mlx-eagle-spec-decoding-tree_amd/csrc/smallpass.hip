@@ -18,8 +18,8 @@
 //   * The norm is folded into x as it was loaded (whole rows, every lane columns of its own; in the operand layout
 //     half the lanes hold nothing when T <= 8): each wave sums the squares of its columns, the row
 //     sums are added across the waves in LDS; no launch and no pass over memory for it.  Every
-//     workgroup repeats it, so it is kept short: v_dot2 for the sums, one square root and division per lane,
-//     mixed-precision products (8 rows, K 896: gate|up 5.8 -> 5.3 us, 4.5 without a norm; q|k|v 4.1 -> 3.9).
+//     workgroup repeats it, so it is kept short: v_dot2 for the sums, one reciprocal root per lane,
+//     mixed-precision products (8 rows, K 896: gate|up 4.7 us, 4.0 without a norm).
 //   * The weights are never rounded: the matrix instructions multiply x with the integers q (exact in
 //     fp16, through the fp8 conversion) a quantisation group at a time, and with ones for the group's
 //     sum of x; scale and bias are applied to the two sums in fp32.
@@ -38,8 +38,6 @@
 
 namespace {
 
-typedef __attribute__((address_space(3))) float4_t sp_lds_float4;
-
 struct SmallArgs {
   const half_t* x;          // [T, K]
   const half_t* norm_w;     // [K] or nullptr
@@ -49,7 +47,7 @@ struct SmallArgs {
   const half_t* bias;       // [N] or nullptr
   const half_t* residual;   // [T, N] or nullptr
   half_t* out;              // [T, N] ([T, N / 2] for SwiGLU)
-  float eps;
+  float eps, inv_k;         // inv_k = 1 / K
   int T, N, K;
   // rope form: (cos, sin) table [T, hd / 2, 2], rotated q [H, T, hd], caches [G, cap, hd], *len_dev = row of
   // the first new K / V row
@@ -76,14 +74,24 @@ enum { SMALL_PLAIN = 0, SMALL_SWIGLU = 1, SMALL_ROPE = 2 };
 // weights are B: the accumulator of lane (r, kq) is x rows 4 kq .. + 4 of weight row r, whose scale and
 // bias are one value per lane.
 //
-// What bounds this kernel is the number of cache lines its load instructions touch per compute
+// What bounds this kernel is the instructions of a wave, one after the other at about five cycles each (weights that are in the L2
+// already save 0.3 us of 5): wave-uniform values are kept scalar, addresses are a uniform base and 32 bits per lane, the
+// epilogue is spread over the threads.  8 rows of the 0.5B shapes, us before / after that: gate|up + norm 5.4 / 4.7, q|k|v 3.9 / 3.5,
+// down 4.7 / 4.55, 2048 -> 8192 5.45 / 5.1, one row of 3584 -> 3584 4.4 / 4.0.
+// Next to that it is the number of cache lines its load instructions touch per compute
 // unit, so every request is shaped for few lines: x is read with whole rows of a chunk per
 // instruction (four rows x 256 bytes) and brought into the operand layout through a per-wave LDS
 // buffer; the two scales (biases) of a chunk come as one 4-byte load for the three chunks of a
 // wave at once and are handed to the lanes that need them with a lane shuffle.
 constexpr int SMALL_MAXC = 3;
-constexpr int SMALL_RED = 64 + 4;          // floats per four weight rows of a wave's tile
+constexpr int SMALL_RED = 16 + 4;          // floats per x row of a wave's tile
 constexpr int SMALL_XROW = 256 + 16;       // bytes per staged x row: 128 columns, padded against bank conflicts
+
+// a load at a uniform address plus 32 bits of a lane's own
+template <typename T>
+__device__ inline T small_load(const void* base, uint32_t at) {
+  return *reinterpret_cast<const T*>(static_cast<const char*>(base) + at);
+}
 
 // the sum over sixteen neighbouring lanes, in all of them
 __device__ inline float row16_sum(float v) {
@@ -94,25 +102,29 @@ __device__ inline float row16_sum(float v) {
   return v;
 }
 
+// (four waves per SIMD in the launch bounds: with more registers to give away the compiler puts the products into accumulation registers
+// and reads them back, 48 instructions of gate|up; the builds that need more than 128 take two)
 template <int NW, int MAXC, int RP, int MODE, bool NORM>
-__global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
+__global__ __launch_bounds__(NW * 64, NW <= 8 && RP == 4 && MAXC == 3 ? 2 : 4) void qmm_small_kernel(SmallArgs a) {
   constexpr int NT = MODE == SMALL_PLAIN ? 1 : 2;
   // a slice per wave: first its x, then (written by the same wave) its weights, then its tiles
   // Whether weights are loaded by whole 64-byte pieces (four lanes of a row next to each other, a quarter of the cache
-  // lines per load) and dealt to the lanes through LDS: where a wave has several loads in flight and one tile (8 rows, us
-  // without / with: 2048 -> 8192 5.6 / 5.3, 3072 -> 4096 4.9 / 4.7; gate|up with two tiles a wave 5.4 / 5.5, one chunk 2.4 / 2.5)
+  // lines per load) and dealt to the lanes through LDS: where a wave has several loads in flight and one tile (8 rows, us when it
+  // came, without / with: 2048 -> 8192 5.6 / 5.3, 3072 -> 4096 4.9 / 4.7; gate|up with two tiles a wave 5.4 / 5.5, one chunk 2.4 / 2.5)
   constexpr bool WHOLE = MAXC > 1 && NT == 1;
-  constexpr int XB = RP * 4 * SMALL_XROW, WB = WHOLE ? MAXC * 1024 : 0, TB = NT * 16 * SMALL_RED;
+  constexpr int XB = RP * 4 * SMALL_XROW, WB = WHOLE ? MAXC * 1024 : 0, TB = NT * 16 * SMALL_RED * 4;
   constexpr int XW = XB > WB ? XB : WB, SLICE = XW > TB ? XW : TB;
   __shared__ __attribute__((aligned(16))) unsigned char slices[NW][SLICE];
   __shared__ float ssq[NORM ? NW : 1][16];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, kq = lane >> 4;
   const int K = a.K, KW = K >> 3, G = K >> 6;
   // chunks dealt over the waves as evenly as they go
   const int chunks = K >> 7;
   const int per = chunks / NW, rem = chunks % NW;
   const int nch = per + (wave < rem ? 1 : 0);
+  // every build serves only K of which each wave owns all its chunks but perhaps the last (small_launch)
+  auto owned = [&](int c) { return MAXC > 1 && c < MAXC - 1 ? true : c < nch; };
   const int k0 = (wave * per + (wave < rem ? wave : rem)) * 128;
   int row0, second;                       // first row of tile 0, distance of tile 1
   if (MODE == SMALL_ROPE) {
@@ -136,61 +148,53 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
     const int xr = lane >> 4, xc = lane & 15;
 #pragma unroll
     for (int p = 0; p < RP; ++p) {
-      int row = 4 * p + xr;
-      row = row < a.T ? row : a.T - 1;
-      const half_t* xp = a.x + (long)row * K + kb + xc * 8;
+      const int row = 4 * p + xr < a.T ? 4 * p + xr : a.T - 1;
+      const uint32_t at = (uint32_t)row * (K * 2) + xc * 16;
 #pragma unroll
-      for (int c = 0; c < MAXC; ++c) xg[c][p] = *reinterpret_cast<const uint4_t*>(xp + (c < nch ? c : 0) * 128);
+      for (int c = 0; c < MAXC; ++c) xg[c][p] = small_load<uint4_t>(a.x + kb + (owned(c) ? c : 0) * 128, at);
     }
   }
   half8_t nw[MAXC];
   if (NORM && a.norm_w) {
-    const half_t* np = a.norm_w + kb + (lane & 15) * 8;
 #pragma unroll
-    for (int c = 0; c < MAXC; ++c) nw[c] = *reinterpret_cast<const half8_t*>(np + (c < nch ? c : 0) * 128);
+    for (int c = 0; c < MAXC; ++c) nw[c] = small_load<half8_t>(a.norm_w + kb + (owned(c) ? c : 0) * 128, (lane & 15) * 16);
   }
   __builtin_amdgcn_sched_barrier(0);
   uint4_t wv[NT][MAXC];
   uint32_t spair[NT], bpair[NT];          // lane (r, c): the two scales (biases) of row r in chunk c
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    long row = row0 + second * t + r;
-    if (MODE == SMALL_PLAIN && row > a.N - 1) row = a.N - 1;         // (N a multiple of 8: never stored)
-    long wrow = WHOLE ? row0 + second * t + (lane >> 2) : row;
-    if (WHOLE && wrow > a.N - 1) wrow = a.N - 1;
-    const uint32_t* wp = a.w + wrow * KW + (kb >> 3) + (WHOLE ? lane & 3 : kq) * 4;
+    // (rows past the end read the last one: N is a multiple of 8, their values are never stored)
+    const int first = row0 + second * t, last = MODE == SMALL_PLAIN ? a.N - 1 - first : 15;
+    const int lr = r < last ? r : last, wr = WHOLE ? (lane >> 2 < last ? lane >> 2 : last) : lr;
+    const uint32_t* wp = a.w + (long)first * KW + (kb >> 3);
+    const uint32_t wat = (uint32_t)wr * (KW * 4) + (WHOLE ? lane & 3 : kq) * 16;
 #pragma unroll
-    for (int c = 0; c < MAXC; ++c) wv[t][c] = *reinterpret_cast<const uint4_t*>(wp + (c < nch ? c : 0) * 16);
-    const int cpair = MAXC > 1 && kq < nch ? kq : 0;
-    spair[t] = *reinterpret_cast<const uint32_t*>(a.s + row * G + (kb >> 6) + cpair * 2);
-    bpair[t] = *reinterpret_cast<const uint32_t*>(a.b + row * G + (kb >> 6) + cpair * 2);
+    for (int c = 0; c < MAXC; ++c) wv[t][c] = small_load<uint4_t>(wp + (owned(c) ? c : 0) * 16, wat);
+    const uint32_t sat = (uint32_t)lr * (G * 2) + (MAXC > 1 && kq < nch ? kq : 0) * 4;
+    spair[t] = small_load<uint32_t>(a.s + (long)first * G + (kb >> 6), sat);
+    bpair[t] = small_load<uint32_t>(a.b + (long)first * G + (kb >> 6), sat);
   }
-  // what the epilogue of wave 0 adds (bias, residual, the rotation's cos / sin, the cache length)
-  // is requested here with everything else, not after the product: a load behind the product is
-  // a microsecond of latency on the critical path of a kernel that takes four.  The values are
-  // only read under the conditions they were loaded under.
-  half4_t e_bias0, e_bias1, e_res;
-  float4_t e_cs[2];
+  // What the epilogue adds (bias, residual, the rotation's cos / sin, the cache length) is requested here with everything
+  // else, not after the product: a load behind the product is a microsecond of latency on the critical path of a
+  // kernel that takes four.  Thread (m, n) of the first 16 T holds x row m of weight row n of the tile (and of the other).
+  const int em = threadIdx.x >> 4, en = threadIdx.x & 15;
+  const bool epi = em < a.T && (MODE != SMALL_PLAIN || row0 + en < a.N);
+  half_t e_bias0 = (half_t)0.f, e_bias1 = (half_t)0.f, e_res = (half_t)0.f;
+  float2_t e_cs = {1.f, 0.f};
   long e_len = 0;
-  const int e_rope_head = MODE == SMALL_ROPE ? row0 / a.hd : 0;
-  if (wave == 0) {
-    const int bn = MODE == SMALL_PLAIN && row0 + 4 * kq >= a.N ? 0 : row0 + 4 * kq;
+  const int e_head = MODE == SMALL_ROPE ? row0 / a.hd : 0;
+  const int e_d = MODE == SMALL_ROPE ? row0 - e_head * a.hd : 0;
+  if (epi) {
     if (a.bias) {
-      e_bias0 = *reinterpret_cast<const half4_t*>(a.bias + bn);
-      if (NT == 2) e_bias1 = *reinterpret_cast<const half4_t*>(a.bias + bn + second);
+      e_bias0 = a.bias[row0 + en];
+      if (NT == 2) e_bias1 = a.bias[row0 + second + en];
     }
-    if (MODE == SMALL_PLAIN && a.residual && r < a.T)
-      e_res = *reinterpret_cast<const half4_t*>(a.residual + (long)r * a.N + bn);
-    if (MODE == SMALL_ROPE) {
-      e_len = *a.len_dev;
-      if (r < a.T && e_rope_head < a.H + a.G) {
-        const int d = row0 - e_rope_head * a.hd + 4 * kq;
-        const float4_t* cs = reinterpret_cast<const float4_t*>(a.rope_cs + ((long)r * (a.hd >> 1) + d) * 2);
-        e_cs[0] = cs[0];
-        e_cs[1] = cs[1];
-      }
-    }
+    if (MODE == SMALL_PLAIN && a.residual) e_res = a.residual[(long)em * a.N + row0 + en];
+    if (MODE == SMALL_ROPE && e_head < a.H + a.G)
+      e_cs = *reinterpret_cast<const float2_t*>(a.rope_cs + ((long)em * (a.hd >> 1) + e_d + en) * 2);
   }
+  if (MODE == SMALL_ROPE) e_len = *a.len_dev;
   __builtin_amdgcn_sched_barrier(0);
   // ---- RMSNorm folded into x, as it was loaded: lane l holds columns 8 (l % 16) .. + 8 of rows 4 p + l / 16 ----
   if (NORM && a.norm_w) {
@@ -200,7 +204,7 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
       ss[p] = 0.f;
 #pragma unroll
       for (int c = 0; c < MAXC; ++c) {
-        if (c < nch) {
+        if (owned(c)) {
           const half8_t v = __builtin_bit_cast(half8_t, xg[c][p]);
 #pragma unroll
           for (int e = 0; e < 8; e += 2) {
@@ -217,13 +221,14 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
     float tot = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) tot += ssq[w][mr];
-    const float rinv_r = 1.0f / sqrtf(tot / (float)K + a.eps);         // of row r: one square root and division per lane
+    // (the hardware's reciprocal square root, 1 ulp, as a square root and a division round it too: a fifth of their chain)
+    const float rinv_r = __builtin_amdgcn_rsqf(__builtin_fmaf(tot, a.inv_k, a.eps));       // of row r
 #pragma unroll
     for (int p = 0; p < RP; ++p) {
       const float rinv = __shfl(rinv_r, 4 * p + (lane >> 4), 64);
 #pragma unroll
       for (int c = 0; c < MAXC; ++c) {
-        if (c < nch) {
+        if (owned(c)) {
           const half8_t v = __builtin_bit_cast(half8_t, xg[c][p]);
           half8_t o;
 #pragma unroll
@@ -275,7 +280,7 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
   for (int t = 0; t < NT; ++t) acc[t] = zero;
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) {
-    if (c < nch) {
+    if (owned(c)) {
       float4_t sx[2];
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
@@ -318,101 +323,54 @@ __global__ __launch_bounds__(NW * 64) void qmm_small_kernel(SmallArgs a) {
     }
   }
   __builtin_amdgcn_wave_barrier();
-  // Into LDS so that a lane of the epilogue reads four weight rows of one x row with one load: x row m,
-  // weight row n at 4 m + 68 (n / 4) + n % 4 (68: the sixteen weight rows of a store in different banks).
+  // The waves' tiles meet in LDS, x row m of weight row n at 20 m + n (the four rows of a store in different banks), and
+  // every thread of the first 16 T finishes one output: one wave that finished all of them was a tail of 200 instructions.
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    float* red = reinterpret_cast<float*>(slices[wave]) + t * (4 * SMALL_RED);
+    float* red = reinterpret_cast<float*>(slices[wave]) + t * (16 * SMALL_RED);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[4 * (4 * kq + i) + SMALL_RED * (r >> 2) + (r & 3)] = acc[t][i];
+    for (int i = 0; i < 4; ++i) red[SMALL_RED * (4 * kq + i) + r] = acc[t][i];
   }
   __syncthreads();
-  if (wave != 0) return;
+  if (!epi) return;
+  float sum[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int at = t * (4 * SMALL_RED) + 4 * r + SMALL_RED * kq;
-    float4_t sum = zero;
+    sum[t] = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) sum += *(const sp_lds_float4*)(reinterpret_cast<const float*>(slices[w]) + at);
-    acc[t] = sum;
+    for (int w = 0; w < NW; ++w) sum[t] += reinterpret_cast<const float*>(slices[w])[t * (16 * SMALL_RED) + SMALL_RED * em + en];
   }
-
-  // ---- epilogue: lane (m, q4) holds weight rows row0 (+ 16) + 4 q4 .. + 4 of x row m ----
-  const int m = r, q4 = kq;
-  if (m >= a.T) return;
+  half_t lo = (half_t)sum[0], hi = (half_t)sum[NT - 1];
+  if (a.bias) {
+    lo = lo + e_bias0;
+    hi = hi + e_bias1;
+  }
   if (MODE == SMALL_ROPE) {
     // the linear output rounded to fp16 (bias added in fp16), rotated with the table's (cos, sin)
     // exactly as the separate rope launch does; v rows pass through
-    const int half = a.hd >> 1;
-    const int hb = e_rope_head;
-    const int d = row0 - hb * a.hd + 4 * q4;            // < hd / 2
-    half4_t lo, hi;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      lo[i] = (half_t)acc[0][i];
-      hi[i] = (half_t)acc[NT - 1][i];
-      if (a.bias) {
-        lo[i] = lo[i] + e_bias0[i];
-        hi[i] = hi[i] + e_bias1[i];
-      }
-    }
     const long P = e_len;
-    if (P + m >= a.cap) return;                         // the host checks capacity; never write past the buffer
+    if (P + em >= a.cap) return;                        // the host checks capacity; never write past the buffer
     half_t* dst;
-    if (hb < a.H) {
-      dst = a.q_out + ((long)hb * a.T + m) * a.hd;
+    if (e_head < a.H) {
+      dst = a.q_out + ((long)e_head * a.T + em) * a.hd;
     } else {
-      const int g = hb < a.H + a.G ? hb - a.H : hb - a.H - a.G;
-      dst = (hb < a.H + a.G ? a.k_cache : a.v_cache) + ((long)g * a.cap + P + m) * a.hd;
+      const int g = e_head < a.H + a.G ? e_head - a.H : e_head - a.H - a.G;
+      dst = (e_head < a.H + a.G ? a.k_cache : a.v_cache) + ((long)g * a.cap + P + em) * a.hd;
     }
-    if (hb < a.H + a.G) {
-      half4_t olo, ohi;
-#pragma unroll
-      for (int j2 = 0; j2 < 2; ++j2) {
-        const float4_t v = e_cs[j2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const int j = 2 * j2 + e;
-          const float co = v[2 * e], sn = v[2 * e + 1];
-          const float x1 = (float)lo[j], x2 = (float)hi[j];
-          olo[j] = (half_t)__builtin_fmaf(x1, co, -(x2 * sn));
-          ohi[j] = (half_t)__builtin_fmaf(x1, sn, x2 * co);
-        }
-      }
-      lo = olo;
-      hi = ohi;
+    if (e_head < a.H + a.G) {
+      const float x1 = (float)lo, x2 = (float)hi;
+      lo = (half_t)__builtin_fmaf(x1, e_cs[0], -(x2 * e_cs[1]));
+      hi = (half_t)__builtin_fmaf(x1, e_cs[1], x2 * e_cs[0]);
     }
-    *reinterpret_cast<half4_t*>(dst + d) = lo;
-    *reinterpret_cast<half4_t*>(dst + half + d) = hi;
+    dst[e_d + en] = lo;
+    dst[(a.hd >> 1) + e_d + en] = hi;
   } else if (MODE == SMALL_SWIGLU) {
-    const int n_g = row0 + 4 * q4;                      // gate rows; the matching up rows are 16 further
-    half4_t o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      half_t g = (half_t)acc[0][i], u = (half_t)acc[NT - 1][i];
-      if (a.bias) {
-        g = g + e_bias0[i];
-        u = u + e_bias1[i];
-      }
-      const float gf = (float)g;
-      const half_t act = (half_t)(gf / (1.0f + expf(-gf)));
-      o[i] = (half_t)((float)act * (float)u);
-    }
-    *reinterpret_cast<half4_t*>(a.out + (long)m * (a.N >> 1) + (row0 >> 1) + 4 * q4) = o;
+    const float gf = (float)lo;
+    const half_t act = (half_t)(gf / (1.0f + expf(-gf)));
+    a.out[(long)em * (a.N >> 1) + (row0 >> 1) + en] = (half_t)((float)act * (float)hi);
   } else {
-    const int n = row0 + 4 * q4;
-    if (n >= a.N) return;
-    half4_t o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      o[i] = (half_t)acc[0][i];
-      if (a.bias) o[i] = o[i] + e_bias0[i];
-    }
-    if (a.residual) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = (half_t)((float)o[i] + (float)e_res[i]);
-    }
-    *reinterpret_cast<half4_t*>(a.out + (long)m * a.N + n) = o;
+    if (a.residual) lo = (half_t)((float)lo + (float)e_res);
+    a.out[(long)em * a.N + row0 + en] = lo;
   }
 }
 
@@ -420,7 +378,7 @@ constexpr int SMALL_K16 = 16 * SMALL_MAXC * 128;      // sixteen waves, three ch
 
 template <int NW, int MAXC, int MODE, bool NORM>
 void small_go(const SmallArgs& a, int grid, hipStream_t st) {
-  // (up to four rows in one pass: 1 x 3584 -> 3584 4.5 -> 4.3 us)
+  // (up to four rows in one pass: 1 x 3584 -> 3584 4.5 -> 4.3 us when it came)
   if (MODE == SMALL_PLAIN && a.T <= 4)
     hipLaunchKernelGGL((qmm_small_kernel<NW, MAXC, 1, MODE, NORM>), dim3(grid), dim3(NW * 64), 0, st, a);
   else if (a.T > 8)
@@ -508,6 +466,7 @@ EAGLE_EXPORT int eagle_qmm_small_w4g64_f16(const void* x, const void* norm_w, fl
   a.residual = static_cast<const half_t*>(residual);
   a.out = static_cast<half_t*>(out);
   a.eps = eps;
+  a.inv_k = 1.0f / (float)K;
   a.T = T;
   a.N = N;
   a.K = K;
@@ -553,6 +512,7 @@ EAGLE_EXPORT int eagle_qkv_rope_small_w4g64_f16(const void* x, const void* norm_
   a.residual = nullptr;
   a.out = nullptr;
   a.eps = eps;
+  a.inv_k = 1.0f / (float)D;
   a.T = T;
   a.N = (H + 2 * G) * hd;
   a.K = D;
