@@ -27,6 +27,22 @@ __device__ inline half4_t lds_read_tr16(const unsigned char* p) {
   return __builtin_bit_cast(half4_t, v);
 }
 
+// A value and that of the lane 16 or 32 away, in both lanes (one of them in each half of the pair), without a trip through LDS.
+__device__ inline float2_t swap_pair32(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t a = r[0], b = r[1];
+  return float2_t{__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)};
+}
+__device__ inline float2_t swap_pair16(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const uint32_t a = r[0], b = r[1];
+  return float2_t{__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)};
+}
+__device__ inline float swap_max(float2_t p) { return fmaxf(p[0], p[1]); }
+__device__ inline float swap_add(float2_t p) { return p[0] + p[1]; }
+
 // ---- 1..64 query rows (a tree, a draft pass): queries packed over heads and tokens ----
 //
 // A workgroup owns 16 NC columns of S^T = K Q^T, (query head, token) pairs of one KV group, and a range of the keys.  Its
@@ -34,20 +50,21 @@ __device__ inline half4_t lds_read_tr16(const unsigned char* p) {
 // their (m, l, O) meet in LDS in fp32: no barrier in the loop.  A block comes in by whole rows and goes through the wave's slice of
 // LDS (K for the operand layout, V for the transposing read); the first is requested before the length is known.
 //
-// What bounds it: the launch, the round trip of the length and of the first block (3.3 us on a short cache), then 0.10
-// (head dimension 64) or 0.18 us per block and compute unit, about half of that the block's way through LDS and back.
-// (K straight from memory into the operand layout, 16 bytes of 64 lines per load, 0.14 / 0.28; sixteen waves, two blocks ahead
-// or 32 columns per workgroup: slower; K and V one after the other in one buffer: no gain at 64, spills at 128.)
+// What bounds it: the launch, the round trip of the length and of the first block (3.0 us on a short cache), then 0.10
+// (head dimension 64) or 0.18 us per block and compute unit, about half of that the block's way through LDS and back, the rest its
+// instructions (a scalar wave index, 32-bit lane offsets and lane swaps instead of shuffles took 5 % off).
+// (K straight from memory into the operand layout, 16 bytes of 64 lines per load, 0.14 / 0.28; ten, twelve or sixteen waves, two blocks
+// ahead or 32 columns per workgroup: slower; K and V one after the other in one buffer: no gain at 64, spills at 128.)
 // Against one wave per query head with up to 33 key splits, partial results in fp16 and a merge of them, us per
-// call in a graph (start / now): 14 heads of 64 in 2 groups, 8 rows behind 560 keys 10.1 / 5.2, behind 2048 11.5 / 9.8 (one split),
-// 32 rows behind 4000 16.0 / 8.2; 28 heads of 128 in 4 groups, 32 rows behind 1024 14.6 / 9.2, 2048 17.3 / 10.8, 40 rows 15.6 / 11.7.
+// call in a graph (before / now): 14 heads of 64 in 2 groups, 8 rows behind 560 keys 10.1 / 4.9, behind 2048 11.5 / 9.0 (one split),
+// 32 rows behind 4000 16.0 / 8.0; 28 heads of 128 in 4 groups, 32 rows behind 1024 14.6 / 9.1, 2048 17.3 / 10.9, 40 rows 15.6 / 11.3.
 constexpr int NW = 8;                   // waves per workgroup
 
 template <int HD, int NC, bool WIDE>
 __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ kc, const half_t* __restrict__ vc,
     const uint32_t* __restrict__ mask_bits, const int32_t* __restrict__ len_dev, half_t* __restrict__ out, float* __restrict__ part,
-    int T, int H, int G, long cap, float scale_log2e, int Tk) {
+    int T, int H, int G, long cap, float scale_log2e, int Tk, uint32_t inv_T) {
   constexpr int KSTEPS = HD / 32;       // MFMA steps over the head dimension for S
   constexpr int DB = HD / 16;           // 16-wide blocks of the head dimension for O
   constexpr int STR = HD * 2 + 16;      // LDS row stride in bytes of a wave's V block
@@ -59,31 +76,31 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
   __shared__ __attribute__((aligned(16))) unsigned char slices[NW][SLICE];
   __shared__ float2_t ml[NW][16 * NC];
   const int g = blockIdx.x, rep = H / G;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 15, kq = lane >> 4;
   const int cols = rep * T;
   const int nsplit = gridDim.z;
   const int first = blockIdx.z * NW + wave, stride = nsplit * NW;     // this wave's blocks: first, first + stride, ...
   const int col0 = blockIdx.y * 16 * NC;
-  const half_t* kb_ptr = kc + (long)g * cap * HD;
-  const half_t* vb_ptr = vc + (long)g * cap * HD;
+  const char* kb_ptr = reinterpret_cast<const char*>(kc + (long)g * cap * HD);
+  const char* vb_ptr = reinterpret_cast<const char*>(vc + (long)g * cap * HD);
 
   half8_t kreg[NV], vreg[NV];
   const int vrow = lane / VR, vcol = lane % VR;
   auto fetch = [&](int blk, int last) {              // rows past `last` read row `last`
-    const int kb = blk * 32;
+    const int kb = blk * 32 < last ? blk * 32 : last, most = last - kb;
+    const char* kp = kb_ptr + (long)kb * (HD * 2);   // uniform, with 32 bits of a lane's own
+    const char* vp = vb_ptr + (long)kb * (HD * 2);
+    uint32_t at[NV];
 #pragma unroll
     for (int it = 0; it < NV; ++it) {
-      int row = kb + it * (64 / VR) + vrow;
-      if (row > last) row = last;
-      kreg[it] = *reinterpret_cast<const half8_t*>(kb_ptr + (long)row * HD + vcol * 8);
+      const int row = it * (64 / VR) + vrow;
+      at[it] = (uint32_t)(row < most ? row : most) * (HD * 2) + vcol * 16;
     }
 #pragma unroll
-    for (int it = 0; it < NV; ++it) {
-      int row = kb + it * (64 / VR) + vrow;
-      if (row > last) row = last;
-      vreg[it] = *reinterpret_cast<const half8_t*>(vb_ptr + (long)row * HD + vcol * 8);
-    }
+    for (int it = 0; it < NV; ++it) kreg[it] = *reinterpret_cast<const half8_t*>(kp + at[it]);
+#pragma unroll
+    for (int it = 0; it < NV; ++it) vreg[it] = *reinterpret_cast<const half8_t*>(vp + at[it]);
   };
   // A wave's first block is requested before the length is known: rows of the buffer, whatever they hold
   // (scores of rows past the end are masked, their V rows replaced by zeros).
@@ -95,8 +112,8 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
   for (int n = 0; n < NC; ++n) {
     int col = col0 + 16 * n + c;
     if (col > cols - 1) col = cols - 1;              // columns past the end repeat the last one and are not stored
-    const int hr = col / T, t = col - hr * T;
-    const half_t* qp = q + ((long)(g * rep + hr) * T + t) * HD + kq * 8;
+    const int t = col - (int)((uint32_t)col * inv_T >> 16) * T;
+    const half_t* qp = q + (long)g * cols * HD + col * HD + kq * 8;       // [group][head, token]
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) qreg[n][kk] = *reinterpret_cast<const half8_t*>(qp + kk * 32);
     lo_bits[n] = mask_bits[WIDE ? 2 * t : t];
@@ -175,8 +192,7 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < 4; ++i) bm = fmaxf(bm, sacc[n][h][i]);
-      bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
-      bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+      bm = swap_max(swap_pair32(swap_max(swap_pair16(bm))));
       const float m_new = fmaxf(m_run[n], bm * scale_log2e);
       const float alpha = __builtin_amdgcn_exp2f(m_run[n] - m_new);
       float psum = 0.f;
@@ -206,8 +222,7 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
   // (m, l, O) of the waves with blocks through LDS
 #pragma unroll
   for (int n = 0; n < NC; ++n) {
-    l_run[n] += __shfl_xor(l_run[n], 16, 64);
-    l_run[n] += __shfl_xor(l_run[n], 32, 64);
+    l_run[n] = swap_add(swap_pair32(swap_add(swap_pair16(l_run[n]))));
     if (kq == 0) ml[wave][16 * n + c] = float2_t{m_run[n], l_run[n]};
   }
   __builtin_amdgcn_wave_barrier();
@@ -247,7 +262,7 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
       *reinterpret_cast<float4_t*>(part + (long)H * T * nsplit * 2 + slot * HD + dq * 4) = acc;
     } else {
       const float inv = den > 0.f ? 1.f / den : 0.f;
-      const int hr = col / T, t = col - hr * T;
+      const int hr = (uint32_t)col * inv_T >> 16, t = col - hr * T;
       *reinterpret_cast<half4_t*>(out + ((long)t * H + g * rep + hr) * HD + dq * 4) =
           half4_t{(half_t)(acc[0] * inv), (half_t)(acc[1] * inv), (half_t)(acc[2] * inv), (half_t)(acc[3] * inv)};
     }
@@ -313,11 +328,12 @@ int launch_tree(const void* q, const void* kc, const void* vc, const uint32_t* b
   const int nc = HD > 64 && T > 32 ? 2 : 1;
   const dim3 grid(G, (H / G * T + 16 * nc - 1) / (16 * nc), nsplit);
   const float sl2 = scale * 1.4426950408889634f;
+  const uint32_t inv_T = (65536 + T - 1) / T;          // col / T = col inv_T >> 16 for the at most 512 columns of a group
   float* part = static_cast<float*>(workspace);
   half_t* o = static_cast<half_t*>(out);
 #define EAGLE_ATTN(NC)                                                                                              \
   hipLaunchKernelGGL((tree_attn_kernel<HD, NC, WIDE>), grid, dim3(NW * 64), 0, st, static_cast<const half_t*>(q),   \
-                     static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), bits, len, o, part, T, H, G, cap, sl2, Tk)
+                     static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), bits, len, o, part, T, H, G, cap, sl2, Tk, inv_T)
   if constexpr (HD > 64) {
     if (nc == 2) EAGLE_ATTN(2);
     else EAGLE_ATTN(1);
@@ -509,7 +525,7 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 16; ++i) bm = fmaxf(bm, sacc[h][i]);
-    bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+    bm = swap_max(swap_pair32(bm));
     const float m_new = fmaxf(m_run, bm * scale_log2e);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     float psum = 0.f;
@@ -549,7 +565,7 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
   }
   if constexpr (DEPTH > 1)
     if (t0 < ntiles) do_tile(Stage<0>{}, t0);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = swap_add(swap_pair32(l_run));
   // the second half of the waves hands its (m, l, O) to the first through LDS
   __syncthreads();
   constexpr int OS = HD + 4;
