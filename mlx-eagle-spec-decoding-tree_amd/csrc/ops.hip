@@ -76,7 +76,12 @@ __global__ void rope_arrayed_scalar_kernel(const half_t* __restrict__ x,
 }
 
 // Token-major projections -> rotated q [H,T,hd] and K/V cache rows P + t.
-// grid.x covers T * (H + 2G) * (hd/16) threads.
+// One token per grid row, (H + 2G) * (hd/16) threads of it along x.  The launch is a chain of latencies (length, table,
+// row, store) around index arithmetic: with one index over tokens, heads and columns taken apart by three 64-bit
+// divisions, eight tokens of 28 + 2 * 4 heads of 128 took 3.1 us in a graph, so 2.55 (a launch that only loads and
+// stores once: 2.4), and 2048 tokens 9.6 against 9.1.  One wave to a workgroup: the few rows of a tree reach more CUs
+// (256 threads: 2.7, and 12 for 2048 tokens, whose last workgroup of each row is nearly empty).
+constexpr int ROPE_THREADS = 64;
 __global__ void rope_kv_append_kernel(const half_t* __restrict__ q_lin,
                                       const half_t* __restrict__ k_lin,
                                       const half_t* __restrict__ v_lin,
@@ -89,13 +94,11 @@ __global__ void rope_kv_append_kernel(const half_t* __restrict__ q_lin,
                                       const float* __restrict__ rope_cs) {
   const int half = hd >> 1;
   const int per_row = half >> 3;
-  const int heads = H + 2 * G;
-  const long total = (long)T * heads * per_row;
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= total) return;
-  const int c = (int)(idx % per_row);
-  const int hh = (int)((idx / per_row) % heads);
-  const int t = (int)(idx / ((long)per_row * heads));
+  const unsigned idx = blockIdx.x * blockDim.x + threadIdx.x;
+  const int hh = (int)(idx / (unsigned)per_row);
+  if (hh >= H + 2 * G) return;
+  const int c = (int)(idx - (unsigned)hh * per_row);
+  const int t = blockIdx.y;
   const long P = *len_dev;
   if (P + t >= cap) return;   // host checks capacity; never write past the buffer
   if (hh < H + G) {
@@ -140,7 +143,8 @@ __global__ void rope_kv_append_kernel(const half_t* __restrict__ q_lin,
 // [slab][32][(H + 2G) hd] with a row = [q heads | k heads | v heads]: every value is
 // fp16(sum of the slabs) + bias before the rotation.  One thread per four column pairs
 // (half of the work of a thread above, twice the threads: all its slab loads are in flight
-// together and the launch is a few dozen workgroups either way).
+// together), tokens and threads dealt as above: 8 tokens of 28 + 2 * 4 heads of 128 from 14 slabs 4.55 -> 3.7 us,
+// 40 from 7 3.97 -> 3.65.
 __global__ void rope_kv_append_slabs_kernel(const float* __restrict__ partial, int nslab,
                                             const half_t* __restrict__ bias,
                                             const float* __restrict__ rope_cs,
@@ -151,12 +155,11 @@ __global__ void rope_kv_append_slabs_kernel(const float* __restrict__ partial, i
   const int half = hd >> 1;
   const int per_row = half >> 2;
   const int heads = H + 2 * G;
-  const long total = (long)T * heads * per_row;
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= total) return;
-  const int c = (int)(idx % per_row) * 4;
-  const int hh = (int)((idx / per_row) % heads);
-  const int t = (int)(idx / ((long)per_row * heads));
+  const unsigned idx = blockIdx.x * blockDim.x + threadIdx.x;
+  const int hh = (int)(idx / (unsigned)per_row);
+  if (hh >= heads) return;
+  const int c = (int)(idx - (unsigned)hh * per_row) * 4;
+  const int t = blockIdx.y;
   const size_t ld = (size_t)heads * hd;
   const size_t stride = (size_t)eagle_slab_rows(T) * ld;
   const float* p = partial + (size_t)t * ld + (size_t)hh * hd + c;
@@ -539,8 +542,8 @@ EAGLE_EXPORT int eagle_rope_kv_append_f16(const void* q_lin, const void* k_lin, 
   if (!eagle_aligned16(q_lin) || !eagle_aligned16(k_lin) || !eagle_aligned16(v_lin) ||
       !eagle_aligned16(q_out) || !eagle_aligned16(k_cache) || !eagle_aligned16(v_cache))
     return EAGLE_ERR_ALIGN;
-  const long total = (long)T * (H + 2 * G) * (hd / 16);
-  hipLaunchKernelGGL(rope_kv_append_kernel, dim3(blocks_for(total, 256)), dim3(256), 0,
+  const long row = (long)(H + 2 * G) * (hd / 16);
+  hipLaunchKernelGGL(rope_kv_append_kernel, dim3(blocks_for(row, ROPE_THREADS), T), dim3(ROPE_THREADS), 0,
                      static_cast<hipStream_t>(stream), (const half_t*)q_lin, (const half_t*)k_lin,
                      (const half_t*)v_lin, positions, inv_freqs, scaling_factor, (half_t*)q_out,
                      (half_t*)k_cache, (half_t*)v_cache, cache_len_dev, T, H, G, hd, capacity,
@@ -565,8 +568,8 @@ EAGLE_EXPORT int eagle_rope_kv_append_table_f16(const void* q_lin, const void* k
       !eagle_aligned16(rope_cs) || !eagle_aligned16(q_out) || !eagle_aligned16(k_cache) ||
       !eagle_aligned16(v_cache))
     return EAGLE_ERR_ALIGN;
-  const long total = (long)T * (H + 2 * G) * (hd / 16);
-  hipLaunchKernelGGL(rope_kv_append_kernel, dim3(blocks_for(total, 256)), dim3(256), 0,
+  const long row = (long)(H + 2 * G) * (hd / 16);
+  hipLaunchKernelGGL(rope_kv_append_kernel, dim3(blocks_for(row, ROPE_THREADS), T), dim3(ROPE_THREADS), 0,
                      static_cast<hipStream_t>(stream), (const half_t*)q_lin, (const half_t*)k_lin,
                      (const half_t*)v_lin, (const int32_t*)nullptr, (const float*)nullptr, 1.0f,
                      (half_t*)q_out, (half_t*)k_cache, (half_t*)v_cache, cache_len_dev, T, H, G, hd,
@@ -587,8 +590,8 @@ EAGLE_EXPORT int eagle_rope_kv_append_slabs_f16(const float* partial, int slabs,
   if (!eagle_aligned16(partial) || !eagle_aligned16(rope_cs) || !eagle_aligned16(q_out) ||
       !eagle_aligned16(k_cache) || !eagle_aligned16(v_cache) || (bias && !eagle_aligned16(bias)))
     return EAGLE_ERR_ALIGN;
-  const long total = (long)T * (H + 2 * G) * (hd / 8);
-  hipLaunchKernelGGL(rope_kv_append_slabs_kernel, dim3(blocks_for(total, 256)), dim3(256), 0,
+  const long row = (long)(H + 2 * G) * (hd / 8);
+  hipLaunchKernelGGL(rope_kv_append_slabs_kernel, dim3(blocks_for(row, ROPE_THREADS), T), dim3(ROPE_THREADS), 0,
                      static_cast<hipStream_t>(stream), partial, slabs, (const half_t*)bias, rope_cs,
                      (half_t*)q_out, (half_t*)k_cache, (half_t*)v_cache, cache_len_dev, T, H, G, hd,
                      capacity);
