@@ -14,30 +14,7 @@ constexpr int TOPK_MAX = 8;          // k of the expansion (candidates per node)
 constexpr int CHUNK = 4096;          // logits per workgroup
 constexpr int THREADS = 256;
 
-// Reductions over a wave without the LDS shuffles: halves and rows of sixteen lanes by half-wave swaps, then rotations
-// within a row.  Every lane gets the result; sums are formed in the order of a butterfly from 32 lanes down.
-template <int ROR>
-__device__ inline int row_ror(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x120 + ROR, 0xf, 0xf, false); }
-template <typename Op>
-__device__ inline uint32_t wave_reduce(uint32_t v, Op op) {
-  const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  v = op(a[0], a[1]);
-  const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  v = op(b[0], b[1]);
-  v = op(v, (uint32_t)row_ror<8>((int)v));
-  v = op(v, (uint32_t)row_ror<4>((int)v));
-  v = op(v, (uint32_t)row_ror<2>((int)v));
-  return op(v, (uint32_t)row_ror<1>((int)v));
-}
-__device__ inline float f32(uint32_t v) { return __builtin_bit_cast(float, v); }
-__device__ inline uint32_t u32(float v) { return __builtin_bit_cast(uint32_t, v); }
-__device__ inline float sum64(float v) {
-  return f32(wave_reduce(u32(v), [](uint32_t a, uint32_t b) { return u32(f32(a) + f32(b)); }));
-}
-__device__ inline float max64(float v) {
-  return f32(wave_reduce(u32(v), [](uint32_t a, uint32_t b) { return u32(fmaxf(f32(a), f32(b))); }));
-}
-__device__ inline uint32_t max64(uint32_t v) {
+__device__ inline uint32_t wave_max(uint32_t v) {
   return wave_reduce(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
 }
 
@@ -65,7 +42,7 @@ __device__ inline uint32_t wave_topk(uint32_t (&key)[N], int k) {
     uint32_t best = key[0];
 #pragma unroll
     for (int j = 1; j < N; ++j) best = key[j] > best ? key[j] : best;
-    best = max64(best);
+    best = wave_max(best);
 #pragma unroll
     for (int j = 0; j < N; ++j) key[j] = key[j] == best ? 0u : key[j];
     if (lane == n) mine = best;
@@ -95,14 +72,14 @@ __global__ __launch_bounds__(THREADS) void lse_partial_kernel(
     x[j] = i < V ? (float)r[i] : -INFINITY;
     m = fmaxf(m, x[j]);
   }
-  m = max64(m);
+  m = wave_max(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   float s = 0.f;
 #pragma unroll
   for (int j = 0; j < CHUNK / THREADS; ++j) s += x[j] == -INFINITY ? 0.f : expf(x[j] - m);
-  s = sum64(s);
+  s = wave_sum(s);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
@@ -132,7 +109,7 @@ __device__ inline void row_stats(const float* pm, const float* ps, int row, int 
       t[j] = c < nch ? rs[c] : 0.f;
       m = fmaxf(m, v[j]);
     }
-    m = max64(m);
+    m = wave_max(m);
 #pragma unroll
     for (int j = 0; j < STATS / 64; ++j)             // (every wave writes the same values)
       shared[lane + 64 * j] = v[j] == -INFINITY ? 0.f : t[j] * expf(v[j] - m);
