@@ -252,6 +252,9 @@ int eagle_qmm_slab_count(int K, int steps_per_slab);
 /* K steps per slab recommended for this product, 0 where eagle_qmm_w4g64_f16 is the faster form
  * (few rows, very many weight rows, or K not a multiple of 512). */
 int eagle_qmm_slab_steps(int M, int N, int K);
+/* The same, and above 32 rows longer slabs where those would be more workgroups than the GPU runs side by side (a plan
+ * of whole passes asks this one; the partial sums are then fewer, too). */
+int eagle_qmm_slab_steps_one_round(int M, int N, int K);
 size_t eagle_qmm_slab_partial_bytes(int N, int K, int steps_per_slab);             /* M <= 32 */
 size_t eagle_qmm_slab_partial_bytes_rows(int M, int N, int K, int steps_per_slab); /* M <= 64 */
 int eagle_qmm_slab_partial_w4g64(const void* x, const uint32_t* wq, const void* scales,

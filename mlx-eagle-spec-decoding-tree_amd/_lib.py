@@ -51,6 +51,7 @@ SIGNATURES = {
     "eagle_qmm_gemm_split_w4g64_f16": (c_int, [c_void_p] * 6 + [c_int] * 6 + [c_void_p, c_size_t, c_void_p]),
     "eagle_qmm_slab_count": (c_int, [c_int] * 2),
     "eagle_qmm_slab_steps": (c_int, [c_int] * 3),
+    "eagle_qmm_slab_steps_one_round": (c_int, [c_int] * 3),
     "eagle_qmm_slab_partial_bytes": (c_size_t, [c_int] * 3),
     "eagle_qmm_slab_partial_bytes_rows": (c_size_t, [c_int] * 4),
     "eagle_qmm_slab_partial_w4g64": (c_int, [c_void_p] * 5 + [c_size_t] + [c_int] * 6 + [c_void_p]),

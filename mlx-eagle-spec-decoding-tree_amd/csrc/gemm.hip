@@ -1477,6 +1477,20 @@ EAGLE_EXPORT int eagle_qmm_slab_steps(int M, int N, int K) {
   return G <= 64 ? 8 : G <= 128 ? 16 : 32;
 }
 
+EAGLE_EXPORT int eagle_qmm_slab_steps_one_round(int M, int N, int K) {
+  // Above 32 rows the x chunks of a slab of more than one chunk take most of a compute unit's LDS, so it holds one workgroup:
+  // longer slabs until the launch is no more workgroups than compute units, or a nearly empty second round of them takes as
+  // long as the first (40 rows, us at the length above and at this one: 3584 x 18944 20.8 in 280 workgroups, 18.4 in 224;
+  // 5120 x 13824 25.0 and 18.7, 8192 x 8192 19.7 and 17.2, 8192 x 28672 59.6 and 50.2, 8192 x 5120 16.4 and 12.0; eight steps
+  // beyond it 20.0, 19.8, 18.5, 52.9, 13.9).  Up to 32 rows two fit, and the length above is the better one (3584 x 18944:
+  // 13.6, with 40 steps 14.9).
+  int steps = eagle_qmm_slab_steps(M, N, K);
+  if (M <= SLAB_ROWS || steps <= SLAB_RING) return steps;
+  const long blocks = (N + 127) / 128;
+  while (steps < K / 64 && blocks * eagle_qmm_slab_count(K, steps) > NUM_CU) steps += SLAB_RING;
+  return steps;
+}
+
 EAGLE_EXPORT size_t eagle_qmm_slab_partial_bytes(int N, int K, int steps_per_slab) {
   if (N < 1) return 0;
   return (size_t)eagle_qmm_slab_count(K, steps_per_slab) * SLAB_ROWS * N * sizeof(float);

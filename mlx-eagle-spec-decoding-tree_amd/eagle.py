@@ -486,7 +486,7 @@ def slab_plan(model, T, forced=None, fused=True):
     shapes = {"qkv": ((H + 2 * G) * hd, D), "o": (D, H * hd), "down": (D, I)}
     plan = {}
     for name, (n, k) in shapes.items():
-        s = ops.slab_steps(T, n, k) if forced is None else int(forced.get(name, 0))
+        s = ops.slab_steps_one_round(T, n, k) if forced is None else int(forced.get(name, 0))
         ok = fused and s > 0 and ops.slab_count(k, s) > 0
         if name == "o":
             ok = ok and layer.self_attn.o_proj.bias is None

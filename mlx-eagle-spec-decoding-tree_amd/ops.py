@@ -144,6 +144,11 @@ def slab_steps(M, N, K):
     return _lib.lib().eagle_qmm_slab_steps(int(M), int(N), int(K))
 
 
+def slab_steps_one_round(M, N, K):
+    """`slab_steps`, and above 32 rows as many more as put the launch into one round of workgroups."""
+    return _lib.lib().eagle_qmm_slab_steps_one_round(int(M), int(N), int(K))
+
+
 def slab_rows(M):
     """Rows of a partial tile of the slab form for M rows of x."""
     if M < 1 or M > 64:
