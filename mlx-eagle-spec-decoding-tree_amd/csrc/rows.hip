@@ -21,14 +21,16 @@
 //     group of weight rows next to each other in the grid, so that an XCD's L2 gives the weights to several of them.
 //
 // What bounds it: the bytes a compute unit takes in, its weights and all of its x (the loads and the x path alone
-// 58 .. 65 of those 71 us), then the vector instructions of the expansion.  Against the streaming kernel (us, launches
-// back to back over rotating weights): 32 x 3584 x 152064 71 / 80, 27 x 18944 x 3584 18 / 23, 32 x 2048 x 8192 8.2 / 11.0,
-// 64 x 8192 x 8192 24 / 40.  With many rows the vector instructions (expansion per block, a multiply-add per group and
+// 58 .. 65 us there), then the vector instructions of the expansion.  Against the streaming kernel (us, launches
+// back to back over rotating weights): 32 x 3584 x 152064 68.5 / 80, 27 x 18944 x 3584 17.5 / 23, 32 x 2048 x 8192 7.5 / 11.0,
+// 64 x 8192 x 8192 23 / 40.  With many rows the vector instructions (expansion per block, a multiply-add per group and
 // output) about equal the matrix instructions: 2048 x 37888 x 3584 675 us = 0.82 PFLOP/s, 512 x 3584 x 18944 114 us; the
 // GEMM, which rounds the weights to fp16 and expands them once per 256 rows, takes 580 and 93 (128 x 3584 x 37888 58 us
 // with the sums of a tile added behind its matrix instructions, 55 under the next tile's).  In a prompt pass, weights
 // not in a cache: 732 and (2048 x 3584 x 18944) 372 us against 553 and 263; matrix pipes 37 % busy at 2.05 GHz.
 #include "common.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -74,7 +76,7 @@ constexpr int rows_block(int MT, int KP) { return (MT > 2 ? 2 : 4) / KP > 0 ? (M
 // bytes of LDS: two blocks of x, its sums, scales (and biases); at the end the sums of the K parts
 size_t rows_lds_bytes(int RT, int MT, int KP, int nu, bool both) {
   const size_t rows = 16 * MT, B = rows_block(MT, KP), wrows = ROWS_WAVES / KP * RT * 16;
-  const size_t stage = 2 * KP * B * rows * ROWS_XROW + KP * (4 * nu + B) * rows * 8 +
+  const size_t stage = 2 * KP * B * rows * ROWS_XROW + KP * 4 * nu * rows * 8 +
                        (both ? 2 : 1) * (size_t)ROWS_WAVES * RT * 16 * rows_stride(nu);
   const size_t epi = KP * rows * (wrows + 4) * 4;
   return stage > epi ? stage : epi;
@@ -108,7 +110,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
   };
   const int NU = (uhi - ulo + KP - 1) / KP;        // units of the longest K part
   const int c0 = first(kp), nch = first(kp + 1) - c0;
-  const int XC = 4 * NU + B;                       // (the block staged past the end included)
+  const int XC = 4 * NU;
   half2_t* xsum = reinterpret_cast<half2_t*>(rows_lds + 2 * BUF);      // [KP][XC][ROWS][2]: (hi, lo) of a group's sum
   // scales of this wave's rows for its K part [RT * 16][stride], then the biases if a.both
   const int stride = rows_stride(NU);
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
   };
   // Scales and biases: 16 bytes are a row's groups in four chunks.  A wave reads all that its rows and K part
   // need in one go, whole lines of memory once, and keeps them in LDS.  Values past the part become zero.
-  constexpr int SBN = 10;                          // loads in one go
+  constexpr int SBN = RT * MT < 15 ? 10 : 9;       // loads in one go (the registers of the largest form hold nine)
   const int pieces = RT * 16 * NU;
   const uint32_t inv = (65536u + NU - 1) / NU;
   uint4_t sreg[SBN], breg[SBN];
@@ -242,8 +244,8 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
 
   const int xcol = 4 * (kq & 1) + 2 * (kq >> 1);
   const int alane = kp * (B * SLOT) + r * ROWS_XROW + xcol * 16;
-  // one chunk: `u` its place among four (static)
-  auto chunk = [&](int u, int c) {
+  // one chunk: `u` its place among four (static), `last` in the last unit (nothing is requested past its end)
+  auto chunk = [&](int u, int c, auto last) {
     const unsigned char* xa = rows_lds + (c / B & 1) * BUF + (c % B) * SLOT + alane;
     uint32_t s2[RT];
 #pragma unroll
@@ -255,7 +257,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
       v = uint4_t{w02[0], w13[0], w02[1], w13[1]};
     };
     auto reload = [&](int t) {                     // both halves of a line together
-      if (u & 1) {
+      if ((u & 1) && (!last() || u - 1 + AH < 4)) {
         rows_pin();
         request_w((u - 1) % AH, t, c - 1 + AH);
         request_w(u % AH, t, c + AH);
@@ -337,20 +339,35 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
       }
     }
   };
-  auto step = [&](int u, int c) {
-    if (u % B == 0) request_x(c / B + 1);
+  auto step = [&](int u, int c, auto last) {
+    const bool more = !last() || u / B * B + B < 4;          // another block of x follows
+    if (u % B == 0 && more) request_x(c / B + 1);
     rows_pin();
-    chunk(u, c);
-    rows_pin();
-    if (u % B == B - 1) {
+    chunk(u, c, last);
+    if (last())
+      __builtin_amdgcn_sched_barrier(0);       // (nothing is requested between these chunks: keep them apart all the same)
+    else
+      rows_pin();
+    if (u % B == B - 1 && more) {
       store_x(c / B + 1);
       rows_barrier();
     }
   };
-  for (int j = 0; j < NU; ++j) {
+  // The last unit by itself: what it would request, no chunk uses.  With the block of x and the ring of weights past the end
+  // fetched all the same, a workgroup of one unit spent a round trip to memory and a barrier on them (us before / now:
+  // 32 x 3584 x 4608 left as seven partial sums 7.06 / 6.59, 40 x 3584 x 37888 32.4 / 30.8, 40 x 3584 x 152064 87.6 / 79.2,
+  // 128 x 3584 x 37888 58.8 / 54.6).
+  for (int j = 0; j + 1 < NU; ++j) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) step(u, 4 * j + u);
+    for (int u = 0; u < 4; ++u) step(u, 4 * j + u, std::false_type{});
   }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) step(u, 4 * (NU - 1) + u, std::true_type{});
+  // (or the compiler sinks the accumulation of the unit behind it, into the block that uses the sums, and runs out of registers)
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(acc[t][mt]));
 
   // ---- the biases times the sums of x: eight chunks per matrix instruction, each sum as hi + lo ----
   const unsigned char* bl = sbl + RT * 16 * stride;
