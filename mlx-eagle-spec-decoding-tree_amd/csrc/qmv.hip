@@ -195,6 +195,7 @@ EAGLE_EXPORT int eagle_qmv_rows_supported(int M, int N, int K) {
 //   M = 2: 7.2 / 8.5, 5.8 / 6.9, 16.3 / 15.9, 6.6 / 7.2: the vector ALU up to a few thousand rows;
 //   M = 4: 9.4 / 8.6, 8.4 / 7.0, 28.7 / 16.1, 8.9 / 7.3; M = 8: 15.1 / 8.7, 14.3 / 7.1, 44.2 / 16.1,
 //          14.2 / 7.4: matrix tiles everywhere (5 + 4 M vector instructions per packed word).
+// (The small-row kernel is asked before: what is left to this one is N past its lines.)
 EAGLE_EXPORT int eagle_qmv_preferred(int M, int N, int K) {
   if (M > 2 || K > 4096 || !eagle_qmv_rows_supported(M, N, K)) return 0;
   return M == 1 ? N <= 65536 : N <= 16384;

@@ -424,23 +424,21 @@ EAGLE_EXPORT int eagle_qmm_small_supported(int T, int N, int K, int norm, int sw
          K <= SMALL_K16;
 }
 
-// Where this kernel beats the vector kernel and the streaming kernel for a plain (or SwiGLU) product:
-// measured over K 384 .. 6144, N 512 .. 18944, 1 .. 16 rows, launches back to back over rotating weights.
-// Its workgroups have no loop over N and share nothing, so it holds as long as they fit the compute units in
-// a few rounds: sixteen waves (K above 3072) are one workgroup per unit, eight two, four five.  Eight rows
-// against the streaming kernel: 3584 x 3584 4.9 / 8.6 us, 2048 -> 8192 5.5 / 7.5, 4864 -> 896 5.1 / 8.0;
-// just past the line, 4096 -> 12288 13.1 / 12.9.  One row where the vector kernel runs: only at K above
-// 3072 (3584 x 3584 4.7 / 5.4; 2048 -> 2048 3.7 / 3.7).
+// Where this kernel beats the vector kernel, the streaming kernel and the rows kernel for a plain (or SwiGLU) product:
+// measured over K 512 .. 6144, N 512 .. 37888, 1 .. 16 rows, launches back to back over rotating weights.  Its
+// workgroups have no loop over N and share nothing, so it holds for so many rounds of 256 workgroups of 16 weight rows, fewer
+// the more K and rows of x each has to itself.  Inside and just past the lines, this / the fastest other, us:
+//   1 row  (vector kernel)   2048 -> 8192 4.4 / 5.2, 3584 -> 4608 5.1 / 6.1, 3584 -> 18944 11.3 / 11.5; 3584 -> 28672 15.4 / 14.8
+//   4 rows                   2048 -> 28672 9.7 / 10.2, 3584 -> 18944 12.1 / 14.7, 6144 -> 8192 10.4 / 11.6; 3072 -> 28672 14.7 / 13.3
+//   8 rows                   896 -> 37888 7.2 / 9.1, 2048 -> 18944 8.6 / 9.3, 3584 -> 12288 9.7 / 10.6; 2560 -> 18944 11.6 / 10.7
+//   16 rows                  896 -> 28672 6.6 / 6.8, 3584 -> 8192 7.9 / 9.3; 4096 -> 8192 10.0 / 9.3, 3584 -> 12288 13.0 / 10.9
 EAGLE_EXPORT int eagle_qmm_small_preferred(int M, int N, int K) {
   if (!eagle_qmm_small_supported(M, N, K, 0, 0)) return 0;
-  const int groups = (N + 15) / 16, cus = 256;
-  if (M == 1 && eagle_qmv_preferred(M, N, K)) return K > 3072 && groups <= cus;
-  const bool few = M <= 8;
-  if (K <= 1536) return groups <= 5 * cus;
-  if (K <= 2048) return groups <= (few ? 3 : 2) * cus;
-  if (K <= 3072) return groups <= 2 * cus;
-  if (K <= 4992) return groups <= (few ? 2 : 1) * cus;
-  return groups <= cus;
+  int rounds;
+  if (M <= 4) rounds = K <= 2048 ? 10 : K <= 3584 ? 5 : K <= 4992 ? 3 : 2;      // (x in one pass of rows)
+  else if (M <= 8) rounds = K <= 1536 ? 10 : K <= 2048 ? 5 : K <= 3584 ? 3 : 2;
+  else rounds = K <= 1024 ? 7 : K <= 1536 ? 5 : K <= 3584 ? 2 : 1;
+  return (N + 15) / 16 <= rounds * 256;
 }
 
 EAGLE_EXPORT int eagle_qmm_small_w4g64_f16(const void* x, const void* norm_w, float eps, const uint32_t* wq,

@@ -1,0 +1,17 @@
+"""quantized_matmul at both sides of the lines of the small-row kernel: the last product it takes and the first it does not."""
+import pytest
+
+from mlx_eagle_spec_decoding_tree_amd import _lib
+from test_gpu_small_dispatch import run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,K,rounds", [(1, 512, 10), (1, 4096, 3), (2, 2176, 5), (4, 4992, 3), (3, 6144, 2), (5, 1536, 10), (8, 2048, 5),
+                                        (8, 2560, 3), (7, 5120, 2), (9, 1024, 7), (16, 1152, 5), (16, 3584, 2), (12, 6144, 1)])
+@pytest.mark.parametrize("past", [0, 8])
+def test_lines(dev, M, K, rounds, past):
+    N = rounds * 256 * 16 + past
+    assert _lib.lib().eagle_qmm_small_preferred(M, N, K) == (past == 0)
+    print(f"M={M} N={N} K={K}", flush=True)
+    run(dev, M, N, K, bias=past == 0)
