@@ -547,12 +547,20 @@ struct RowsPlan {
 // unit ingests them (40 and 72 GB/s), and 0.22 us per unit of four chunks, tile and 16 rows of x.  What the whole
 // grid reads counts a little, a split as much as its second launch and the partial sums (the sums alone where
 // the consumer of the product adds them).  For 65 .. 2048 rows the same formula over the blocks of x.  Its choice against
-// the best of all forms and splits of 4600 and 12600 random products: 17 .. 64 rows 1.4 % longer on
-// average, 8 % at the 95th percentile (up to 16 rows, most of which other kernels serve, 4 and 16); 65 .. 2048 rows 1.2 and 7.5.
+// the best of all forms and splits of 6000 and 12600 random products: 17 .. 64 rows 1.3 % longer on
+// average, 8 % at the 95th percentile; 65 .. 2048 rows 1.2 and 7.5.  Up to 16 rows (one tile, other constants: a unit costs its
+// weights and the barriers of its K parts rather than its matrix instructions, a split more than the few rows say) 0.9 and 7.3,
+// where the constants of the others gave 3.2 and 14 (4 x 8192 -> 3584 two tiles a wave in 16 splits 12.0 us, one in 8 9.9).
 enum { ROWS_WHOLE = 0, ROWS_SPLIT = 1, ROWS_PARTIAL = 2 };
+struct RowsCost {
+  double start, w, x, unit, parts, whole, second, sums, rows;
+};
+constexpr RowsCost rows_cost_one = {2.11, 0.0309, 0.0107, 0.0448, 0.419, 0.0018, 2.60, 1.353, 5.};
+constexpr RowsCost rows_cost = {1.03, 0.0246, 0.0138, 0.221, 0., 0.0107, 2.93, 0.49, 0.};
 RowsPlan rows_find_plan(int M, int N, int K, int mode) {
   const int units = ((K >> 7) + 3) / 4;
   const int least_zb = (M + 63) / 64, mt = (M + 16 * least_zb - 1) / (16 * least_zb), zb = (M + 16 * mt - 1) / (16 * mt);
+  const RowsCost& cost = mt == 1 ? rows_cost_one : rows_cost;
   RowsPlan best = {-1, 1};
   double least = 1e30;
   for (int f = 0; f < ROWS_FORMS; ++f) {
@@ -568,8 +576,9 @@ RowsPlan rows_find_plan(int M, int N, int K, int mode) {
       if (rows_lds_bytes(form.rt, mt, form.kp, nu, false) > ROWS_LDS) continue;
       const double rounds = (double)((blocks * z + 255) / 256);
       const double w = wrows * (double)nu * form.kp * (512 * 0.5625 / 1e3), x = 16. * mt * nu * form.kp * (1024 / 1e3);
-      double t = rounds * (1.03 + 0.0246 * w + 0.0138 * x + 0.221 * nu * form.rt * mt) + 0.0107 * (blocks * z / 256.) * (w + 0.5 * x);
-      if (z > 1) t += (mode == ROWS_SPLIT ? 2.93 : 0.) + 0.49 * 4e-6 * z * (double)M * N;
+      double t = rounds * (cost.start + cost.w * w + cost.x * x + (cost.unit * form.rt * mt + cost.parts * (form.kp - 1)) * nu) +
+                 cost.whole * (blocks * z / 256.) * (w + 0.5 * x);
+      if (z > 1) t += (mode == ROWS_SPLIT ? cost.second : 0.) + cost.sums * 4e-6 * z * (M + cost.rows) * N;
       if (t < least) {
         least = t;
         best = {f, z};
