@@ -13,9 +13,9 @@
  *
  * Two groups.  DEFAULT: what the library's own verification step, draft loop and prompt pass
  * call when nothing is chosen by hand: eagle_qmm_w4g64_f16 (+ _workspace_bytes), eagle_qmm_swiglu_*,
- * eagle_qmm_rows_* (17 rows up, and every product of a prompt of the module path), eagle_pass_begin_f16,
+ * eagle_qmm_rows_* (17 rows up, fewer past the lines of the small-row kernel, and every product of a prompt of the module path), eagle_pass_begin_f16,
  * eagle_qmm_slab_* (partial sums, SwiGLU, their tiled forms and eagle_qmm_tile_w4g64),
- * eagle_qmv_w4g64_f16 / eagle_qmv_rows_w4g64_f16 (one and two rows), eagle_qmm_small_* and
+ * eagle_qmv_w4g64_f16 / eagle_qmv_rows_w4g64_f16 (one row, very many weight rows), eagle_qmm_small_* and
  * eagle_qkv_rope_small_* (a drafter's passes), eagle_qmm_gemm_* (prompt chunks), every rope, norm,
  * attention, embedding, argmax, tree and loop-state entry point.  ON REQUEST: complete and tested,
  * but picked by a caller only: eagle_qmm_plan / eagle_qmm_w4g64_f16_tuned (a launch shape chosen by

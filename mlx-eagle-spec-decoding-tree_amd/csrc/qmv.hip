@@ -188,17 +188,12 @@ EAGLE_EXPORT int eagle_qmv_rows_supported(int M, int N, int K) {
   return M >= 1 && M <= 8 && N >= 8 && K >= 512 && (K % 512) == 0 && qmv_lds_bytes(qmv_rows_of(M), K) <= 150 * 1024;
 }
 
-// Measured on the projection shapes of the 7B model, vector ALU against matrix tiles, us per launch:
-//   M = 1: 5.8 / 8.5 (3584 x 3584), 4.4 / 6.7 (512 x 3584), 12.6 / 16.1 (18944 x 3584), 5.3 / 7.1
-//          (8192 x 2048); a long K over few rows (3584 x 18944: 28.3 / 18.9) and the vocabulary
-//          projection (66.6 / 63.2) stay on the matrix kernel;
-//   M = 2: 7.2 / 8.5, 5.8 / 6.9, 16.3 / 15.9, 6.6 / 7.2: the vector ALU up to a few thousand rows;
-//   M = 4: 9.4 / 8.6, 8.4 / 7.0, 28.7 / 16.1, 8.9 / 7.3; M = 8: 15.1 / 8.7, 14.3 / 7.1, 44.2 / 16.1,
-//          14.2 / 7.4: matrix tiles everywhere (5 + 4 M vector instructions per packed word).
-// (The small-row kernel is asked before: what is left to this one is N past its lines.)
+// Measured on the projection shapes of the 7B model, vector ALU against the matrix kernels, us per launch.  The small-row kernel is
+// asked before: what is left is N past its lines.  M = 1: 14.8 / 15.4 (28672 x 3584), 17.9 / 19.4 (37888 x 3584); a long K over few
+// rows (3584 x 18944: 28.3 / 18.9) and the vocabulary projection (66.6 / 63.2) stay on the matrix kernels.  M = 2: behind
+// everywhere (12288 x 4096 12.6 / 10.6, 28672 x 3584 20.7 / 14.3): 5 + 4 M vector instructions per packed word.
 EAGLE_EXPORT int eagle_qmv_preferred(int M, int N, int K) {
-  if (M > 2 || K > 4096 || !eagle_qmv_rows_supported(M, N, K)) return 0;
-  return M == 1 ? N <= 65536 : N <= 16384;
+  return M == 1 && K <= 4096 && N <= 65536 && eagle_qmv_rows_supported(M, N, K);
 }
 
 EAGLE_EXPORT int eagle_qmv_supported(int N, int K) { return eagle_qmv_rows_supported(1, N, K); }

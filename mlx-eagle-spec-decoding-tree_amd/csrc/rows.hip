@@ -614,20 +614,15 @@ EAGLE_EXPORT int eagle_qmm_rows_supported(int M, int N, int K, int swiglu) {
 
 // Where it beats the other forms (us, against the streaming kernel unless noted).  33 rows on: everywhere (two
 // passes of the streaming kernel; 48 x 3584 x 18944 23 / 38, 64 x 896 x 512 8.1 / 10.8).  17 .. 32 rows: from about
-// 4 MB of weights or K above 4608 (2048 -> 3584 7.9 / 9.1, 896 -> 8192 6.6 / 6.8, 8192 -> 512 10.4 / 12.2, but 2048 ->
-// 1152 7.7 / 7.5).  Up to 16 rows the streaming kernel's waves hold all of x and its weights come in whole lines:
-// even at K up to 2048 and in a middle range (3584 -> 37888 24.2 / 23.3, 4864 -> 18944 21.0 / 20.3), behind below
-// (3584 -> 18944 15.6 / 16.7) and above it (8192 -> 37888 42 / 50, 3584 -> 152064 61 / 66, 18944 -> 3584 16 / 20).
+// 4 MB of weights or K above 4608 (2048 -> 3584 7.4 / 9.1, 896 -> 8192 6.3 / 6.8, 8192 -> 512 9.9 / 12.2, but 2560 ->
+// 512 7.7 / 5.7).  Up to 16 rows, past the lines of the small-row kernel: everywhere (512 -> 152064 12.4 / 18.3, 2048 -> 18944
+// 9.3 / 10.8, 3584 -> 28672 14.3 / 17.2, 3584 -> 65536 26 / 29, 14336 -> 896 9.5 / 12.1; of 467 products it is more than 3 %
+// ahead in 285 and behind in 88, most in 11008 -> 18944, 36 / 29, and 4864 -> 37888, 28 / 26).
 // The forms for one or a few rows come first where they apply (the caller asks them before).  Above 64 rows the GEMM is
 // faster; who must not round a weight asks for this kernel.
 EAGLE_EXPORT int eagle_qmm_rows_preferred(int M, int N, int K) {
   if (M < 1 || M > 2 * EAGLE_MAX_M) return 0;
-  const double size = (double)N * K;
-  if (M <= 16) {
-    if (K <= 2048 || (size > 7e7 && size < 2.5e8 && K <= 8192)) return 0;
-  } else if (M <= 32) {
-    if (size < 7e6 && K <= 4608) return 0;
-  }
+  if (M > 16 && M <= 32 && (double)N * K < 7e6 && K <= 4608) return 0;
   return eagle_qmm_rows_supported(M, N, K, 0);
 }
 

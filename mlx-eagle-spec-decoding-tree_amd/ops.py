@@ -78,8 +78,8 @@ def quantized_matmul(x, w_q, scales, biases, transpose=True, group_size=64, bits
                      out=None, tuned=None, gemm=None):
     """`mx.quantized_matmul(x, w, scales, biases, transpose=True, group_size=64, bits=4)`
     (any leading dims, flattened as qmm_kernel.py:99-100,136): the small-row kernel for up to 16 rows
-    where the library prefers it (eagle_qmm_small_preferred), the vector-ALU kernel for one row (or
-    two) where `qmv_preferred` says so, up to 64 rows the kernel of csrc/rows.hip where the library prefers
+    where the library prefers it (eagle_qmm_small_preferred), the vector-ALU kernel for one row
+    where `qmv_preferred` says so, up to 64 rows the kernel of csrc/rows.hip where the library prefers
     it (eagle_qmm_rows_preferred), else the streaming kernel in passes of 32 rows, a tiled GEMM above that.  `bias` ([N] fp16) is added after rounding, as the patched linear layer does
     (mlx_model_fwd_bench.py:70-71).  `tuned` forces a launch shape of the streaming kernel,
     `gemm=True` the tiled GEMM whatever the row count.  The default path is native code

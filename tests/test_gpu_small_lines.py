@@ -1,4 +1,5 @@
-"""quantized_matmul at both sides of the lines of the small-row kernel: the last product it takes and the first it does not."""
+"""quantized_matmul at both sides of the lines of the small-row kernel, the last product it takes and the first it does not, and up to
+16 rows past them, where the rows kernel takes over."""
 import pytest
 
 from mlx_eagle_spec_decoding_tree_amd import _lib
@@ -15,3 +16,12 @@ def test_lines(dev, M, K, rounds, past):
     assert _lib.lib().eagle_qmm_small_preferred(M, N, K) == (past == 0)
     print(f"M={M} N={N} K={K}", flush=True)
     run(dev, M, N, K, bias=past == 0)
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 8200, 6144), (2, 12296, 4096), (4, 20488, 2560), (8, 20488, 2048), (16, 8200, 2048), (9, 28680, 512),
+                                   (16, 24, 8192)])
+def test_past_the_lines(dev, M, N, K):
+    L = _lib.lib()
+    assert L.eagle_qmm_rows_preferred(M, N, K) == 1 and not L.eagle_qmm_small_preferred(M, N, K) and not L.eagle_qmv_preferred(M, N, K)
+    print(f"M={M} N={N} K={K}", flush=True)
+    run(dev, M, N, K, bias=True)
