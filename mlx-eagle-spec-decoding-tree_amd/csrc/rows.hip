@@ -22,11 +22,11 @@
 //
 // What bounds it: the bytes a compute unit takes in, its weights and all of its x (the loads and the x path alone
 // 58 .. 65 us there), then the vector instructions of the expansion.  Against the streaming kernel (us, launches
-// back to back over rotating weights): 32 x 3584 x 152064 68.5 / 80, 27 x 18944 x 3584 17.5 / 23, 32 x 2048 x 8192 7.5 / 11.0,
+// back to back over rotating weights): 32 x 3584 x 152064 69.5 / 80, 27 x 18944 x 3584 17.5 / 23, 32 x 2048 x 8192 7.5 / 11.0,
 // 64 x 8192 x 8192 23 / 40.  With many rows the vector instructions (expansion per block, a multiply-add per group and
 // output) about equal the matrix instructions: 2048 x 37888 x 3584 675 us = 0.82 PFLOP/s, 512 x 3584 x 18944 114 us; the
 // GEMM, which rounds the weights to fp16 and expands them once per 256 rows, takes 580 and 93 (128 x 3584 x 37888 58 us
-// with the sums of a tile added behind its matrix instructions, 55 under the next tile's).  In a prompt pass, weights
+// with the sums of a tile added behind its matrix instructions, 54 under the next tile's).  In a prompt pass, weights
 // not in a cache: 732 and (2048 x 3584 x 18944) 372 us against 553 and 263; matrix pipes 37 % busy at 2.05 GHz.
 #include "common.h"
 
@@ -354,9 +354,9 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
     }
   };
   // The last unit by itself: what it would request, no chunk uses.  With the block of x and the ring of weights past the end
-  // fetched all the same, a workgroup of one unit spent a round trip to memory and a barrier on them (us before / now:
-  // 32 x 3584 x 4608 left as seven partial sums 7.06 / 6.59, 40 x 3584 x 37888 32.4 / 30.8, 40 x 3584 x 152064 87.6 / 79.2,
-  // 128 x 3584 x 37888 58.8 / 54.6).
+  // fetched all the same, a workgroup of one unit spent a round trip to memory and a barrier on them (us before / now, timed in turn:
+  // 32 x 3584 x 4608 left as seven partial sums 7.07 / 6.53, 40 rows 8.0 / 7.7; 32 x 3584 x 37888 with SwiGLU 27.3 / 26.5, 40 x 3584 x
+  // 152064 80.2 / 78.8, 128 x 3584 x 37888 55.0 / 53.9).
   for (int j = 0; j + 1 < NU; ++j) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) step(u, 4 * j + u, std::false_type{});
@@ -615,9 +615,9 @@ EAGLE_EXPORT int eagle_qmm_rows_supported(int M, int N, int K, int swiglu) {
 // Where it beats the other forms (us, against the streaming kernel unless noted).  33 rows on: everywhere (two
 // passes of the streaming kernel; 48 x 3584 x 18944 23 / 38, 64 x 896 x 512 8.1 / 10.8).  17 .. 32 rows: from about
 // 4 MB of weights or K above 4608 (2048 -> 3584 7.4 / 9.1, 896 -> 8192 6.3 / 6.8, 8192 -> 512 9.9 / 12.2, but 2560 ->
-// 512 7.7 / 5.7).  Up to 16 rows, past the lines of the small-row kernel: everywhere (512 -> 152064 12.4 / 18.3, 2048 -> 18944
-// 9.3 / 10.8, 3584 -> 28672 14.3 / 17.2, 3584 -> 65536 26 / 29, 14336 -> 896 9.5 / 12.1; of 467 products it is more than 3 %
-// ahead in 285 and behind in 88, most in 11008 -> 18944, 36 / 29, and 4864 -> 37888, 28 / 26).
+// 512 7.7 / 5.7).  Up to 16 rows, past the lines of the small-row kernel: everywhere.  Timed in
+// turn over 222 products of K up to 2048 or 70 .. 250 M weights it is 8 % faster on average (512 -> 152064 12.4 / 18.3, 2048 -> 18944
+// 9.2 / 10.8, 3584 -> 28672 14.3 / 17.2, 4096 -> 32768 16.8 / 21.5), more than 3 % behind in 18 (two rows 4864 -> 18944 18.6 / 16.5).
 // The forms for one or a few rows come first where they apply (the caller asks them before).  Above 64 rows the GEMM is
 // faster; who must not round a weight asks for this kernel.
 EAGLE_EXPORT int eagle_qmm_rows_preferred(int M, int N, int K) {
