@@ -344,7 +344,7 @@ def main():
     kv_bytes = 2 * L * G * (PREFIX + NODES) * hd * 2
     achieved = alg / (qmm_ms * 1e-3) / 1e9
     traffic, traffic_source = read_traffic_record()
-    stream_kernel = "qmm_w4g64_kernel"          # (above 32 tree tokens: two launches of it per product)
+    stream_kernel = "qmm_rows_kernel" if ver.wide else "qmm_w4g64_kernel"      # (above 32 tree tokens the head, in one launch)
     burst = (not ver.wide) and any(l[6] is True and l[7] is not None for l in launches)
     rows_form = any(l[6] == "rows" for l in launches)
     kernels = ((stream_kernel if any(not l[6] for l in launches) else "qmm_rows_tiled_kernel")
@@ -594,7 +594,7 @@ def attention_bench(opt):
         rows.append({"prefix": P, **{k: round(v, 2) for k, v in t.items()}, "kv_bytes": kv,
                      "attention_frac_of_hbm_peak": round(kv / t["attention_us"] / 1e3 / HBM_PEAK_GBS, 4)})
     # causal attention of a prompt chunk (mlx_llama.py:185-192 with the causal mask of :275-276):
-    # all 32-row pieces of the chunk in one launch pair, behind P0 cache rows
+    # all 32-row pieces of the chunk in one launch, behind P0 cache rows
     causal = []
     for name, (Hc, Gc, hdc) in (("8B target", (32, 8, 128)), ("7B target", (28, 4, 128)), ("0.5B drafter", (14, 2, 64))):
         for R, P0 in ((512, 0), (512, 1536), (2048, 0)):

@@ -547,9 +547,9 @@ struct RowsPlan {
 // unit ingests them (40 and 72 GB/s), and 0.22 us per unit of four chunks, tile and 16 rows of x.  What the whole
 // grid reads counts a little, a split as much as its second launch and the partial sums (the sums alone where
 // the consumer of the product adds them).  For 65 .. 2048 rows the same formula over the blocks of x.  Its choice against
-// the best of all forms and splits of 6000 and 12600 random products: 17 .. 64 rows 1.3 % longer on
+// the best of all forms and splits of 1400 and 12600 random products: 17 .. 64 rows 1.2 % longer on
 // average, 8 % at the 95th percentile; 65 .. 2048 rows 1.2 and 7.5.  Up to 16 rows (one tile, other constants: a unit costs its
-// weights and the barriers of its K parts rather than its matrix instructions, a split more than the few rows say) 0.9 and 7.3,
+// weights and the barriers of its K parts rather than its matrix instructions, a split more than the few rows say) 1.0 and 7.3,
 // where the constants of the others gave 3.2 and 14 (4 x 8192 -> 3584 two tiles a wave in 16 splits 12.0 us, one in 8 9.9).
 enum { ROWS_WHOLE = 0, ROWS_SPLIT = 1, ROWS_PARTIAL = 2 };
 struct RowsCost {
