@@ -367,8 +367,8 @@ int launch_tree(const void* q, const void* kc, const void* vc, const uint32_t* b
 // runs the online softmax on its accumulator (a lane owns one row, its partner lane + 32 the other half of the keys) and feeds
 // exp(S^T) straight back as the B operand of O^T += V^T P^T; only V needs a transposed read from LDS (ds_read_b64_tr_b16).
 //
-// A chunk has hundreds of pairs, so the keys are split over workgroups only where a few pairs would leave most of the GPU idle (fp16
-// partial results, added by a second kernel).  What bounds it: 2.5 us per tile of a workgroup, of which the matrix instructions are 0.9,
+// A chunk has hundreds of pairs, so the keys are split over workgroups only where a few pairs would leave most of the GPU idle (O / l of
+// a split in fp16, added by a second kernel: in fp32 128 rows behind 1536 keys, seven splits, take 20.6 us, so 17.3).  What bounds it: 2.5 us per tile of a workgroup, of which the matrix instructions are 0.9,
 // and the last workgroups of a causal triangle.  Before, a workgroup held all heads of a group (seven waves) on tiles of 64 keys, one
 // per compute unit, the longest twice the average, and every result went through partials and a merge; us per chunk
 // (28 heads of 128 in 4 groups; before / now): 2048 rows 101 / 52, 512 rows 24.8 / 15.7, 128 rows 13.4 / 8.1, 512 rows behind 1536
@@ -604,13 +604,16 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
       part_ml[slot * 2 + 0] = m_run;
       part_ml[slot * 2 + 1] = l_run;
     }
+    // O / l, a weighted mean of values: O itself grows with the keys of the split, past what fp16 holds
+    const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
     half_t* po = part_o + slot * HD;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4)
         *reinterpret_cast<half4_t*>(po + db * 32 + 8 * i4 + 4 * hb) =
-            half4_t{(half_t)o_acc[db][4 * i4 + 0], (half_t)o_acc[db][4 * i4 + 1], (half_t)o_acc[db][4 * i4 + 2], (half_t)o_acc[db][4 * i4 + 3]};
+            half4_t{(half_t)(o_acc[db][4 * i4 + 0] * inv), (half_t)(o_acc[db][4 * i4 + 1] * inv), (half_t)(o_acc[db][4 * i4 + 2] * inv),
+                    (half_t)(o_acc[db][4 * i4 + 3] * inv)};
     return;
   }
   // one split: the rows as they lie in memory, through the wave's part of LDS
@@ -674,8 +677,8 @@ __global__ __launch_bounds__(256) void causal_add_kernel(const half_t* __restric
 #pragma unroll
     for (int k = 0; k < MOST; ++k)
       if (s0 + k < nact) {
-        const float f = __builtin_amdgcn_exp2f(ml[k][0] - mx);
-        l_run += f * ml[k][1];
+        const float f = __builtin_amdgcn_exp2f(ml[k][0] - mx) * ml[k][1];
+        l_run += f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = fmaf(f, (float)o[k][e], acc[e]);
       }

@@ -37,3 +37,18 @@ def test_causal_chunk(dev, H, G, hd, pieces, P, spare):
     want = want.reshape(R, H * hd)
     assert bool(torch.isfinite(got).all())
     assert ((got.double() - want).norm() / want.norm()).item() <= REL
+
+
+@pytest.mark.parametrize("H,G,hd,R,P,value", [(16, 16, 128, 128, 16000, 20.), (32, 32, 64, 64, 16000, 20.), (28, 4, 128, 512, 32000, 20.),
+                                              (14, 2, 64, 32, 5000, 32768.)])
+def test_partial_results_of_long_splits(dev, H, G, hd, R, P, value):
+    """A split of thousands of keys with equal scores holds thousands of times their values before they are divided by the sum of
+    the probabilities.  The sums are whole numbers below 2^24 (times the value), so the result is the value itself."""
+    cap = P + R
+    print(f"H={H} G={G} hd={hd} R={R} P={P} value={value}", flush=True)
+    q = torch.zeros(H, R, hd, device=dev).half()
+    k = torch.randn(G, cap, hd, generator=torch.Generator(device=dev).manual_seed(P), device=dev).half()
+    v = torch.full((G, cap, hd), value, device=dev).half()
+    starts = (P + 32 * torch.arange(R // 32, device=dev)).int()
+    got = ops.causal_attention(q, k, v, starts, hd ** -0.5, max_len=cap)
+    assert torch.equal(got, torch.full_like(got, value))
