@@ -408,7 +408,9 @@ constexpr int MAX_CAUSAL_SPLITS = 64;     // what the workspace holds
 template <int V>
 struct Stage { static constexpr int value = V; };
 
-template <int HD, int DEPTH>
+// SEVERAL: more than one piece in a workgroup (pp > 1).  The tiles then hold rows past the end of a wave's own piece.  Their probabilities
+// are zero, but zero times an infinity is not: the lanes that fetch such a row for the transposing read of V fetch zeros instead.
+template <int HD, int DEPTH, bool SEVERAL>
 __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ kc, const half_t* __restrict__ vc,
     const int32_t* __restrict__ len_dev, half_t* __restrict__ out, half_t* __restrict__ part_o, float* __restrict__ part_ml, int H,
@@ -419,8 +421,10 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
   constexpr int VEC_ROW = HD / 8;       // 16-byte vectors per K/V row
   constexpr int KTT = CAUSAL_TILE;
   constexpr int NVU = KTT * VEC_ROW / 512;        // vectors of K (or V) per thread
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * KTT * STR];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * KTT * STR + (SEVERAL ? HD * 2 : 0)];
   __shared__ float2_t ml_half[4][32];
+  const unsigned char* zeros = lds + 2 * KTT * STR;
+  if (SEVERAL && threadIdx.x < HD / 2) reinterpret_cast<uint32_t*>(lds + 2 * KTT * STR)[threadIdx.x] = 0u;   // (read behind the barriers of a tile)
   unsigned char* ldsK = lds;
   unsigned char* ldsV = lds + KTT * STR;
   const int rep = H / G, quads = (rep + hp - 1) / hp;
@@ -453,8 +457,8 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
   float m_run = M_FLOOR, l_run = 0.f;
   // this lane's address for the transposing loads of V: within 16 lanes, lane s asks for key row s / 4 at the four d
   // columns 4 (s % 4) .. + 3 of the group's 16 and gets four keys of its own d
-  const unsigned char* vt_base =
-      ldsV + (64 * khalf + 4 * hb + ((lane & 15) >> 2)) * STR + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+  const int vt_row = 4 * hb + ((lane & 15) >> 2);
+  const unsigned char* vt_base = ldsV + (64 * khalf + vt_row) * STR + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   float16_t o_acc[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -546,14 +550,16 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) o_acc[db][i] *= alpha;
     }
+    const int left = own - kb;                    // rows of this half tile before the wave's end
+    auto v_rows = [&](int c) { return !SEVERAL || vt_row < left - c ? vt_base + c * STR : zeros; };
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-          const half4_t lo = lds_read_tr16(vt_base + (32 * h + 16 * u) * STR + db * 64);
-          const half4_t hi = lds_read_tr16(vt_base + (32 * h + 16 * u + 8) * STR + db * 64);
+          const half4_t lo = lds_read_tr16(v_rows(32 * h + 16 * u) + db * 64);
+          const half4_t hi = lds_read_tr16(v_rows(32 * h + 16 * u + 8) + db * 64);
           const half8_t a = half8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
           o_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bp[h][u], o_acc[db], 0, 0, 0);
         }
@@ -701,9 +707,13 @@ int launch_causal(const void* q, const void* kc, const void* vc, const int32_t* 
   const int nsplit = causal_splits((max_len + CAUSAL_TILE - 1) / CAUSAL_TILE, MAX_CAUSAL_SPLITS, units);
   float* part_ml = static_cast<float*>(workspace);
   half_t* part_o = reinterpret_cast<half_t*>(part_ml + (size_t)pieces * H * nsplit * 32 * 2);
-  hipLaunchKernelGGL((causal_attn_kernel<HD, HD == 64 ? 2 : 1>), dim3(gx, nsplit, nz), dim3(512), 0, st, static_cast<const half_t*>(q),
-                     static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), len, static_cast<half_t*>(out), part_o, part_ml, H, G,
-                     cap, scale * 1.4426950408889634f, pieces, hp, pp);
+#define EAGLE_CAUSAL(SEVERAL)                                                                                                              \
+  hipLaunchKernelGGL((causal_attn_kernel<HD, HD == 64 ? 2 : 1, SEVERAL>), dim3(gx, nsplit, nz), dim3(512), 0, st,                          \
+                     static_cast<const half_t*>(q), static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), len,                   \
+                     static_cast<half_t*>(out), part_o, part_ml, H, G, cap, scale * 1.4426950408889634f, pieces, hp, pp)
+  if (pp > 1) EAGLE_CAUSAL(true);
+  else EAGLE_CAUSAL(false);
+#undef EAGLE_CAUSAL
   if (nsplit > 1)
     hipLaunchKernelGGL(causal_add_kernel<HD>, dim3((H * 32 * (HD / 8) + 255) / 256, 1, pieces), dim3(256), 0, st, part_o, part_ml,
                        static_cast<half_t*>(out), H, nsplit, len, cap, pp, units);

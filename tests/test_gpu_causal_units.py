@@ -52,3 +52,24 @@ def test_partial_results_of_long_splits(dev, H, G, hd, R, P, value):
     starts = (P + 32 * torch.arange(R // 32, device=dev)).int()
     got = ops.causal_attention(q, k, v, starts, hd ** -0.5, max_len=cap)
     assert torch.equal(got, torch.full_like(got, value))
+
+
+@pytest.mark.parametrize("bad", [math.inf, math.nan])
+@pytest.mark.parametrize("H,G,hd,pieces,P", [(32, 32, 64, 32, 0), (32, 32, 128, 32, 40), (16, 16, 64, 64, 1), (16, 8, 128, 64, 100), (32, 16, 64, 32, 7)])
+def test_rows_of_later_pieces_stay_out(dev, H, G, hd, pieces, P, bad):
+    """Fewer than four heads per group and enough pieces that a workgroup holds several: rows of the cache past a piece's end, which
+    no row of it sees, may hold anything, whether they lie in a later piece or behind all of them."""
+    g = torch.Generator(device=dev).manual_seed(pieces + H)
+    R = 32 * pieces
+    cap = P + R + 50
+    print(f"H={H} G={G} hd={hd} pieces={pieces} P={P} bad={bad}", flush=True)
+    q = torch.randn(H, R, hd, generator=g, device=dev).half()
+    k, v = (torch.randn(G, cap, hd, generator=g, device=dev).half() for _ in range(2))
+    starts = (P + 32 * torch.arange(pieces, device=dev)).int()
+    want = ops.causal_attention(q, k, v, starts, hd ** -0.5, max_len=cap)
+    assert bool(torch.isfinite(want).all())
+    for end in (1, 2, 3, 5, pieces - 1, pieces):          # everything from the end of this many pieces on is bad
+        kk, vv = k.clone(), v.clone()
+        kk[:, P + 32 * end:], vv[:, P + 32 * end:] = math.nan, bad
+        got = ops.causal_attention(q, kk, vv, starts, hd ** -0.5, max_len=cap)
+        assert torch.equal(got[:32 * end], want[:32 * end]), end
