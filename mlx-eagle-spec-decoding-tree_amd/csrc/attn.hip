@@ -394,10 +394,12 @@ __device__ inline int causal_rows(const int32_t* len_dev, int p, int n, int piec
 // Splits in use for `ntiles` tiles in a grid of `nsplit`, `units` workgroups beside each other: as many as fill the GPU, with
 // at least four tiles each (two where there are few units): a split costs its partial results and the second launch (28
 // heads of 128, us with no split / at least 4 / 2 / 1 tiles: 512 rows 15.7 / 15.7 / 19.1 / 21.1, 256 rows behind 1792 41.6 / 25.3 / 25.9 /
-// 26.2, 64 rows behind 2000 46 / 21.4 / 17.7 / 17.5).
+// 26.2, 64 rows behind 2000 46 / 21.4 / 17.7 / 17.5).  Three tiles of few units: one split each (32 rows behind 300 12.2, in two
+// splits 14.2), at head dimension 64 no split, if that spares the second launch (8.5; 9.1 and 10.4).
+template <int HD>
 __host__ __device__ inline int causal_splits(int ntiles, int nsplit, int units) {
   int tpw = (ntiles + nsplit - 1) / nsplit;
-  const int fill = (units * ntiles + 255) / 256, least = units <= 32 ? 2 : 4;
+  const int fill = (units * ntiles + 255) / 256, least = units > 32 ? 4 : HD > 64 && ntiles == 3 ? 1 : 2;
   tpw = tpw > fill ? tpw : fill;
   tpw = tpw > least ? tpw : least;
   return (ntiles + tpw - 1) / tpw;
@@ -447,7 +449,7 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
   const int Ltot = causal_rows(len_dev, group * pp, pp, pieces, cap);
   const int ntiles = (Ltot + KTT - 1) / KTT;
   const int own = live ? P + 32 : 0;       // keys up to here concern this wave's rows
-  const int nactive = causal_splits(ntiles, nsplit, gridDim.x * gridDim.z);
+  const int nactive = causal_splits<HD>(ntiles, nsplit, gridDim.x * gridDim.z);
   if (split >= nactive) return;
   half8_t qreg[KSTEPS];
   const half_t* qp = q + ((long)head * pieces * 32 + piece * 32 + ql) * HD;
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(256) void causal_add_kernel(const half_t* __restric
   constexpr int VR = HD / 8, MOST = 8;
   const int piece = blockIdx.z, pieces = gridDim.z;
   const int rows = causal_rows(len_dev, piece / pp * pp, pp, pieces, cap);
-  const int nact = causal_splits((rows + CAUSAL_TILE - 1) / CAUSAL_TILE, nsplit, units);
+  const int nact = causal_splits<HD>((rows + CAUSAL_TILE - 1) / CAUSAL_TILE, nsplit, units);
   if (nact == 1) return;                           // written by the workgroup itself
   const int id = blockIdx.x * 256 + threadIdx.x;   // (head, row, vector)
   const int hr = id / VR, c = id % VR;
@@ -700,11 +702,25 @@ template <int HD>
 int launch_causal(const void* q, const void* kc, const void* vc, const int32_t* len, void* out, int pieces, int H, int G,
                   long cap, int max_len, float scale, void* workspace, hipStream_t st) {
   const int rep = H / G, hp = rep < 4 ? rep : 4, gx = G * ((rep + hp - 1) / hp);
-  // with fewer than four heads per group a workgroup takes several pieces, unless that leaves compute units without one
-  int pp = 4 / hp;
-  while (pp > 1 && gx * ((pieces + pp - 1) / pp) < 256) --pp;
-  const int nz = (pieces + pp - 1) / pp, units = gx * nz;
-  const int nsplit = causal_splits((max_len + CAUSAL_TILE - 1) / CAUSAL_TILE, MAX_CAUSAL_SPLITS, units);
+  const int tiles = (max_len + CAUSAL_TILE - 1) / CAUSAL_TILE;
+  // With fewer than four heads per group a workgroup can take several pieces, so that its waves share the tiles, and the keys are split
+  // instead.  By the least of: a tile takes 2.2 us (128) or 1.25 (64) whatever part of the waves is busy with it, splits 3.2 and 1.2 per
+  // MB of partial results (16 heads in 16 groups of 128, us for one piece / four: 512 rows behind 0 14.5 / 15.2, 1536 39 / 25, 8000 154 / 60;
+  // 64 rows behind 300, one / two, 12.7 / 13.3, 8000 30 / 26).
+  int pp = 1, nz = pieces, units = gx * pieces, nsplit = 1;
+  double least = 1e30;
+  for (int n = 1; n <= 4 / hp && n <= pieces; ++n) {
+    const int z = (pieces + n - 1) / n, u = gx * z;
+    const int s = HD == 64 && tiles <= 3 ? 1 : causal_splits<HD>(tiles, MAX_CAUSAL_SPLITS, u);
+    const double t = (HD > 64 ? 2.2 : 1.25) * ((u * s + 255) / 256) * ((tiles + s - 1) / s) + (s > 1 ? 3.2 + 2.4e-6 * pieces * 32 * H * HD * s : 0.);
+    if (t < least) {
+      least = t;
+      pp = n;
+      nz = z;
+      units = u;
+      nsplit = s;
+    }
+  }
   float* part_ml = static_cast<float*>(workspace);
   half_t* part_o = reinterpret_cast<half_t*>(part_ml + (size_t)pieces * H * nsplit * 32 * 2);
 #define EAGLE_CAUSAL(SEVERAL)                                                                                                              \

@@ -73,3 +73,11 @@ def test_rows_of_later_pieces_stay_out(dev, H, G, hd, pieces, P, bad):
         kk[:, P + 32 * end:], vv[:, P + 32 * end:] = math.nan, bad
         got = ops.causal_attention(q, kk, vv, starts, hd ** -0.5, max_len=cap)
         assert torch.equal(got[:32 * end], want[:32 * end]), end
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("H,G,pieces,P,spare", [(16, 16, 5, 1500, 0), (16, 16, 7, 3000, 5), (16, 8, 3, 5000, 0), (8, 8, 2, 9000, 3), (8, 8, 11, 700, 1),
+                                                (9, 3, 3, 5000, 0), (1, 1, 1, 300, 0), (4, 2, 2, 290, 40), (16, 16, 17, 40, 0)])
+def test_several_pieces_and_splits(dev, H, G, hd, pieces, P, spare):
+    """Few heads per group: two, three and four pieces per workgroup, the last workgroup with fewer, and one, on split keys."""
+    test_causal_chunk(dev, H, G, hd, pieces, P, spare)
