@@ -465,8 +465,9 @@ int eagle_draft_attention_f16(const void* q, const void* k_cache, const void* v_
  * forward (mlx_eagle.py:329-346 through mlx_llama.py:185-192) of a tree above 32 tokens needs
  * (the reference's default is 39 draft nodes, mlx_eagle.py:390,510; there Tk = T): T queries
  * against the P = *cache_len_dev prefix rows and the Tk <= 64 rows P .. P+Tk-1, of which query t
- * sees row j iff bit (j % 32) of mask_words[2*t + j/32] is set.  q [H,T,hd], out [T, H*hd].  A query's result does not
- * depend on the queries beside it (the other two forms give the same bits). */
+ * sees row j iff bit (j % 32) of mask_words[2*t + j/32] is set.  q [H,T,hd], out [T, H*hd].  For max_len up
+ * to 6144 a query's result does not depend on the queries beside it; above, the keys of a long cache are split by what the
+ * queries leave idle, and it may, by the rounding of sums.  The other two forms give the same bits for the same T. */
 size_t eagle_tree_attention_wide_workspace_bytes(int T, int H, int hd, int max_len);
 int eagle_tree_attention_wide_f16(const void* q, const void* k_cache, const void* v_cache,
                                   const uint32_t* mask_words, const int32_t* cache_len_dev, void* out,

@@ -60,11 +60,24 @@ __device__ inline float swap_add(float2_t p) { return p[0] + p[1]; }
 // 32 rows behind 4000 16.0 / 8.0; 28 heads of 128 in 4 groups, 32 rows behind 1024 14.6 / 9.1, 2048 17.3 / 10.9, 40 rows 15.6 / 11.3.
 constexpr int NW = 8;                   // waves per workgroup
 
+// Key splits in use behind a prefix of P rows, of a grid that holds `most`: no fewer than `least`, no more than one per 512 keys, so that
+// a short prefix in a large cache pays for few partial results.
+__device__ inline int tree_splits_in_use(int P, int least, int most) {
+  const int n = P >> 9 < most ? P >> 9 : most;
+  return n > least ? n : least;
+}
+// cached rows before the masked ones: never past the cache, whatever the counter says
+__device__ inline int tree_prefix(const int32_t* len_dev, long cap, int Tk) {
+  int P = len_dev[0];
+  if (P > cap - Tk) P = (int)(cap - Tk);
+  return P < 0 ? 0 : P;
+}
+
 template <int HD, int NC, bool WIDE>
 __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ kc, const half_t* __restrict__ vc,
     const uint32_t* __restrict__ mask_bits, const int32_t* __restrict__ len_dev, half_t* __restrict__ out, float* __restrict__ part,
-    int T, int H, int G, long cap, float scale_log2e, int Tk, uint32_t inv_T) {
+    int T, int H, int G, long cap, float scale_log2e, int Tk, uint32_t inv_T, int least) {
   constexpr int KSTEPS = HD / 32;       // MFMA steps over the head dimension for S
   constexpr int DB = HD / 16;           // 16-wide blocks of the head dimension for O
   constexpr int STR = HD * 2 + 16;      // LDS row stride in bytes of a wave's V block
@@ -80,7 +93,7 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
   const int c = lane & 15, kq = lane >> 4;
   const int cols = rep * T;
   const int nsplit = gridDim.z;
-  const int first = blockIdx.z * NW + wave, stride = nsplit * NW;     // this wave's blocks: first, first + stride, ...
+  const int first = blockIdx.z * NW + wave;          // this wave's first block
   const int col0 = blockIdx.y * 16 * NC;
   const char* kb_ptr = reinterpret_cast<const char*>(kc + (long)g * cap * HD);
   const char* vb_ptr = reinterpret_cast<const char*>(vc + (long)g * cap * HD);
@@ -120,11 +133,11 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
     hi_bits[n] = WIDE ? mask_bits[2 * t + 1] : 0u;
   }
   __builtin_amdgcn_sched_barrier(0);
-  int P = len_dev[0];
-  if (P > cap - Tk) P = (int)(cap - Tk);             // never past the cache, whatever the counter says
-  if (P < 0) P = 0;
+  const int P = tree_prefix(len_dev, cap, Tk);
   const int Ltot = P + Tk;
   const int nblk = (Ltot + 31) >> 5;
+  const int in_use = tree_splits_in_use(P, least, nsplit), stride = in_use * NW;
+  if ((int)blockIdx.z >= in_use) return;
 
   float m_run[NC], l_run[NC];
   float4_t o_acc[NC][DB];
@@ -269,15 +282,18 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
   }
 }
 
-// Adds the key splits: one thread per four output elements, everything requested at once.
-template <int HD, int NS>
-__global__ __launch_bounds__(256) void tree_attn_add_kernel(const float* __restrict__ part, half_t* __restrict__ out, int T, int H) {
-  constexpr int QW = HD / 4;
+// Adds the key splits: one thread per four output elements, the NS splits that are always in use requested at once; those that a long
+// prefix adds (LONG: a grid of most > NS splits) eight at a time behind them.
+template <int HD, int NS, bool LONG>
+__global__ __launch_bounds__(256) void tree_attn_add_kernel(const float* __restrict__ part, half_t* __restrict__ out, int T, int H, int most,
+                                                            const int32_t* __restrict__ len_dev, long cap, int Tk) {
+  constexpr int QW = HD / 4, MORE = 8;
   const int id = blockIdx.x * 256 + threadIdx.x;
   const int row = id / QW, dq = id % QW;             // row = head * T + token
   if (row >= H * T) return;
-  const float* ml = part + (long)row * NS * 2;
-  const float* po = part + (long)H * T * NS * 2 + (long)row * NS * HD + dq * 4;
+  if (!LONG) most = NS;
+  const float* ml = part + (long)row * most * 2;
+  const float* po = part + (long)H * T * most * 2 + (long)row * most * HD + dq * 4;
   float2_t w[NS];
   float4_t o[NS];
 #pragma unroll
@@ -285,6 +301,7 @@ __global__ __launch_bounds__(256) void tree_attn_add_kernel(const float* __restr
     w[i] = *reinterpret_cast<const float2_t*>(ml + 2 * i);
     o[i] = *reinterpret_cast<const float4_t*>(po + i * HD);
   }
+  const int in_use = LONG ? tree_splits_in_use(tree_prefix(len_dev, cap, Tk), NS, most) : NS;
   float mx = M_FLOOR;
 #pragma unroll
   for (int i = 0; i < NS; ++i) mx = fmaxf(mx, w[i][0]);
@@ -297,21 +314,43 @@ __global__ __launch_bounds__(256) void tree_attn_add_kernel(const float* __restr
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] = fmaf(f, o[i][e], acc[e]);
   }
+  for (int s0 = NS; s0 < in_use; s0 += MORE) {
+    float2_t wm[MORE];
+    float4_t om[MORE];
+#pragma unroll
+    for (int i = 0; i < MORE; ++i) {                 // (past the end the last one again, with a weight of zero)
+      const int at = s0 + i < in_use ? s0 + i : in_use - 1;
+      wm[i] = *reinterpret_cast<const float2_t*>(ml + 2 * at);
+      om[i] = *reinterpret_cast<const float4_t*>(po + (long)at * HD);
+    }
+    float m_new = mx;
+#pragma unroll
+    for (int i = 0; i < MORE; ++i) m_new = fmaxf(m_new, wm[i][0]);
+    const float alpha = __builtin_amdgcn_exp2f(mx - m_new);
+    mx = m_new;
+    den *= alpha;
+    acc *= alpha;
+#pragma unroll
+    for (int i = 0; i < MORE; ++i) {
+      const float f = s0 + i < in_use ? __builtin_amdgcn_exp2f(wm[i][0] - mx) : 0.f;
+      den += f * wm[i][1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(f, om[i][e], acc[e]);
+    }
+  }
   const float inv = den > 0.f ? 1.f / den : 0.f;
   const int head = row / T, t = row - head * T;
   *reinterpret_cast<half4_t*>(out + ((long)t * H + head) * HD + dq * 4) =
       half4_t{(half_t)(acc[0] * inv), (half_t)(acc[1] * inv), (half_t)(acc[2] * inv), (half_t)(acc[3] * inv)};
 }
 
-
 // Key splits of a launch.  One where the keys are few: a second launch that adds the splits costs 2.0 us, a compute unit takes
 // 3.2 us per 1000 keys of head dimension 64 and 5.7 of 128, and the live length is usually well below the capacity that
 // the rule sees (14 heads of 64 in a cache of 2048: one split 5.2 / 6.8 / 9.9 us at 560 / 1024 / 2048 keys, eight 6.4 / 6.6 / 7.1; 28 heads
 // of 128: one 8.2 / 11.1 / 16.9, four 8.9 / 9.2 / 10.8).  Otherwise as many as give every compute unit a workgroup at 32 query rows
-// and a wave a block.  It does not look at the rows, so a query's result is the same bits whatever else is in the launch: above
-// 32 rows of head dimension 128, where LDS holds one workgroup per compute unit, a workgroup takes 32 columns
+// and a wave a block.  It does not look at the rows, so a query's result is the same bits whatever else is in the launch (but for long
+// caches, launch_tree): above 32 rows of head dimension 128, where LDS holds one workgroup per compute unit, a workgroup takes 32 columns
 // instead (40 rows behind 2048 keys, four splits: 13.4 us against 16.7 for 288 workgroups of 16).
-constexpr int MAX_SPLITS = 16;
 int key_splits(int max_len, int H, int hd) {
   if (max_len <= (hd > 64 ? 768 : 2048)) return 1;
   const int fit = 256 / (2 * H), len = (max_len + 32 * NW - 1) / (32 * NW);
@@ -324,27 +363,38 @@ int key_splits(int max_len, int H, int hd) {
 template <int HD, bool WIDE>
 int launch_tree(const void* q, const void* kc, const void* vc, const uint32_t* bits, const int32_t* len, void* out, int T,
                 int Tk, int H, int G, long cap, int max_len, float scale, void* workspace, hipStream_t st) {
-  const int nsplit = key_splits(max_len, H, HD);
-  const int nc = HD > 64 && T > 32 ? 2 : 1;
-  const dim3 grid(G, (H / G * T + 16 * nc - 1) / (16 * nc), nsplit);
+  constexpr int LONG_CACHE = 6144, KEYS = HD > 64 ? 1536 : 3072, MAX_LONG_SPLITS = 32;
+  const int least = key_splits(max_len, H, HD), rep_T = H / G * T;
+  int nsplit = least, nc = HD > 64 && T > 32 ? 2 : 1;
+  // Long caches: key_splits gives a few rows a handful of workgroups, each with thousands of keys (32 heads of 128 in 8 groups, one row
+  // behind 8192 keys 27 us, 32768 84; 64 heads 45 and 152).  The rows then say how many splits fill the compute units, the prefix how many of
+  // those are used, and from twice that length on many rows go 32 columns to a workgroup (14.3, 31; 14.7, 31; 32 rows of 28 heads behind 16384
+  // keys 36 -> 27; behind 600 in so large a cache 9.1 -> 11).
+  if (max_len > LONG_CACHE && max_len > least * KEYS) {
+    const int b16 = G * ((rep_T + 15) / 16), b32 = G * ((rep_T + 31) / 32);
+    if (b16 > 32 && max_len > 2 * least * KEYS) nc = 2;
+    const int fill = 256 / (nc == 2 ? b32 : b16) < MAX_LONG_SPLITS ? 256 / (nc == 2 ? b32 : b16) : MAX_LONG_SPLITS;
+    if (fill > nsplit) nsplit = fill;
+  }
+  const dim3 grid(G, (rep_T + 16 * nc - 1) / (16 * nc), nsplit);
   const float sl2 = scale * 1.4426950408889634f;
   const uint32_t inv_T = (65536 + T - 1) / T;          // col / T = col inv_T >> 16 for the at most 512 columns of a group
   float* part = static_cast<float*>(workspace);
   half_t* o = static_cast<half_t*>(out);
 #define EAGLE_ATTN(NC)                                                                                              \
   hipLaunchKernelGGL((tree_attn_kernel<HD, NC, WIDE>), grid, dim3(NW * 64), 0, st, static_cast<const half_t*>(q),   \
-                     static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), bits, len, o, part, T, H, G, cap, sl2, Tk, inv_T)
-  if constexpr (HD > 64) {
-    if (nc == 2) EAGLE_ATTN(2);
-    else EAGLE_ATTN(1);
-  } else {
-    EAGLE_ATTN(1);
-  }
+                     static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), bits, len, o, part, T, H, G, cap, sl2, Tk, inv_T, least)
+  if (nc == 2) EAGLE_ATTN(2);
+  else EAGLE_ATTN(1);
 #undef EAGLE_ATTN
   const dim3 add((H * T * (HD / 4) + 255) / 256);
-#define EAGLE_ATTN_ADD(NS) \
-  case NS: hipLaunchKernelGGL((tree_attn_add_kernel<HD, NS>), add, dim3(256), 0, st, part, o, T, H); break
-  switch (nsplit) {
+#define EAGLE_ATTN_ADD(NS)                                                                                                              \
+  case NS:                                                                                                                              \
+    if (nsplit > NS) hipLaunchKernelGGL((tree_attn_add_kernel<HD, NS, true>), add, dim3(256), 0, st, part, o, T, H, nsplit, len, cap, Tk); \
+    else hipLaunchKernelGGL((tree_attn_add_kernel<HD, NS, false>), add, dim3(256), 0, st, part, o, T, H, nsplit, len, cap, Tk);            \
+    break
+  if (nsplit > 1) switch (least) {
+    EAGLE_ATTN_ADD(1);
     EAGLE_ATTN_ADD(2);
     EAGLE_ATTN_ADD(3);
     EAGLE_ATTN_ADD(4);

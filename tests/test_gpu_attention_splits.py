@@ -55,3 +55,27 @@ def test_splits(dev, H, G, hd, cap):
         if T > 8:                              # a row's result does not depend on the rows beside it
             few = ops.draft_attention(q[:, 3:8].contiguous(), kk, vv, words[3:8].contiguous(), len_dev, Tk, hd ** -0.5, max_len=cap)
             assert torch.equal(few, got[3:8])
+
+
+# around the length from which the splits follow the rows, and from which many rows go 32 columns to a workgroup (28 and 32 heads of 128:
+# four splits at least, 6144 and 12288; 64 heads two, 6144; 32 of 64 four, 12288 and 24576; 160 of 64 one), up to 32 splits
+@pytest.mark.parametrize("H,G,hd", [(28, 4, 128), (32, 8, 128), (64, 8, 128), (32, 4, 64), (160, 20, 64), (1, 1, 64)])
+@pytest.mark.parametrize("cap", [6144, 6145, 12289, 24577])
+def test_long_caches(dev, H, G, hd, cap):
+    g = torch.Generator(device=dev).manual_seed(H + cap)
+    k, v = (torch.randn(G, cap, hd, generator=g, device=dev).half() for _ in range(2))
+    for T, P in ((1, cap - 1), (1, 5), (3, 1100), (8, cap - 8), (8, 2559), (8, 5000), (16, cap - 20), (24, 3000), (32, cap - 33), (33, 4099), (64, cap - 64)):
+        print(f"H={H} G={G} hd={hd} cap={cap} T={T} P={P}", flush=True)
+        q = torch.randn(H, T, hd, generator=g, device=dev).half()
+        vis = torch.rand(T, T, generator=g, device=dev) < 0.5
+        vis[0] = False
+        kk, vv = k.clone(), v.clone()
+        kk[:, P + T:], vv[:, P + T:] = math.nan, math.inf
+        words, len_dev = ops.mask_to_words(vis), torch.tensor([P], dtype=torch.int32, device=dev)
+        # partial results of another length in the workspace: what is not in use now must not be read
+        ops.draft_attention(q, k, v, words, torch.tensor([cap - T], dtype=torch.int32, device=dev), T, hd ** -0.5, max_len=cap)
+        got = ops.draft_attention(q, kk, vv, words, len_dev, T, hd ** -0.5, max_len=cap)
+        want = attention64(q, k, v, vis, P, T, hd ** -0.5)
+        assert bool(torch.isfinite(got).all())
+        assert ((got.double() - want).norm() / want.norm()).item() <= REL
+        assert torch.equal(ops.tree_attention(q, kk, vv, words, len_dev, hd ** -0.5, max_len=cap), got)
