@@ -123,6 +123,24 @@ def link_host(compiles):
     os.replace(tmp, HOST)
 
 
+def run_all(cmds, logs, jobs):
+    """Run the commands, at most `jobs` at once, and return (return code, what it printed) of each.  They print into files: more
+    than a pipe holds would stop a command while another one is waited for."""
+    procs = []
+    for cmd, path in zip(cmds, logs):
+        running = [p for p in procs if p.poll() is None]
+        if len(running) >= jobs:
+            running[0].wait()
+        with open(path, "wb") as log:
+            procs.append(subprocess.Popen(cmd, stdout=log, stderr=subprocess.STDOUT))
+    out = []
+    for p, path in zip(procs, logs):
+        p.wait()
+        with open(path, "rb") as log:
+            out.append((p.returncode, log.read().decode(errors="replace")))
+    return out
+
+
 def build(verbose=False, jobs=8):
     """Compile every csrc/*.hip to an object (in parallel) and link the library, then the host
     module on top of it."""
@@ -130,26 +148,17 @@ def build(verbose=False, jobs=8):
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     host = start_host(objdir)
-    procs = []
-    objs = []
     flags = [f for f in FLAGS if f != "-shared"]
-    for src in sources():
-        obj = os.path.join(objdir, os.path.basename(src) + ".o")
-        objs.append(obj)
-        cmd = [cc, *flags, "-c", src, "-o", obj]
-        if verbose:
-            print(" ".join(cmd))
-        procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
-        while sum(p.poll() is None for _, p in procs) >= jobs:
-            procs[0][1].wait()
+    objs = [os.path.join(objdir, os.path.basename(src) + ".o") for src in sources()]
+    cmds = [[cc, *flags, "-c", src, "-o", obj] for src, obj in zip(sources(), objs)]
+    if verbose:
+        print("\n".join(" ".join(cmd) for cmd in cmds))
     report = {}
-    for src, p in procs:
-        out, _ = p.communicate()
-        text = out.decode(errors="replace")
+    for src, (code, text) in zip(sources(), run_all(cmds, [obj + ".log" for obj in objs], jobs)):
         report.update(scratch_report(text))
         noise = ("is not a recognized feature for this target", "-Rpass-analysis=kernel-resource-usage")
         text = "\n".join(l for l in text.splitlines() if not any(n in l for n in noise))
-        if p.returncode != 0:
+        if code != 0:
             raise RuntimeError(f"hipcc failed on {src}:\n{text}")
         if verbose and text.strip():
             print(text)

@@ -294,3 +294,12 @@ def test_rows_form_takes_a_prompt_but_leaves_partial_sums_for_64_rows():
     for M in (65, 512, 2048):                   # room for every split that the plan can take, without overflow
         for N, K in ((512, 18944), (3584, 3584), (152064, 3584), (16, 128)):
             assert L.eagle_qmm_rows_workspace_bytes(M, N, K) % (4 * M * N) == 0
+
+
+def test_build_commands_may_print_more_than_a_pipe_holds(tmp_path):
+    """The compiler's remarks on one source are some 150 KB; with more sources than jobs the build waits for one compile at a time."""
+    import sys
+    from mlx_eagle_spec_decoding_tree_amd import build
+    cmds = [[sys.executable, "-c", f"import sys; print('{n}' * 200000); sys.exit({n})"] for n in range(5)]
+    done = build.run_all(cmds, [str(tmp_path / f"{n}.log") for n in range(5)], jobs=2)
+    assert [(code, text.strip()) for code, text in done] == [(n, str(n) * 200000) for n in range(5)]
