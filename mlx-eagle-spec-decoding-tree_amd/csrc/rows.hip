@@ -539,6 +539,7 @@ constexpr int ROWS_FORMS = sizeof(rows_forms) / sizeof(rows_forms[0]);
 
 struct RowsPlan {
   int form, splits;
+  bool behind;         // the streaming kernel is expected to be faster
 };
 
 // The division of the work with the least predicted time (us), from a model fitted to timings of every form, launches
@@ -557,11 +558,34 @@ struct RowsCost {
 };
 constexpr RowsCost rows_cost_one = {2.11, 0.0309, 0.0107, 0.0448, 0.419, 0.0018, 2.60, 1.353, 5.};
 constexpr RowsCost rows_cost = {1.03, 0.0246, 0.0138, 0.221, 0., 0.0107, 2.93, 0.49, 0.};
+
+// Up to 16 rows of x, K up to 2048 or 70 .. 250 M weights: whether the streaming kernel is faster than this one by the form (rt tiles, kp
+// parts, no splits).  That kernel deals the tiles of 16 weight rows evenly over the compute units, where this one has whole rounds of 128 .. 640
+// weight rows a workgroup: at 100000 weight rows half of the second round idles (3 x 1152 -> 102016 22.8 us, 18.9; 10 x 640 -> 99944 17.2, 14.9;
+// 4 x 2816 -> 34496 17.9, 16.9), while 28672 or 152064 fill theirs (8 x 512 -> 152064 12.4, 18.3; 8 x 3584 -> 28672 14.3, 17.2).  Both times (us) from
+// fits to 1779 such products of 16000 weight rows up, 2.7 and 3 % rms: the streaming kernel's by its waves, one per 256 columns, and the tiles of
+// a workgroup, which come in steps of four.  This kernel is more than 3 % behind in 345 of them, with the rule in 76 (8 %: 93, 6), and the rule
+// loses more than 3 % in 20.  (The streaming kernel's result is further from the exact one before it is rounded: 0.02 .. 0.5 % more error after.)
+bool rows_behind_streaming(int M, int N, int K, int rt, int kp) {
+  const double size = (double)N * K;
+  if (M > 16 || N <= 16000 || K > 3584 || (K > 2048 && (size <= 7e7 || size >= 2.5e8))) return false;
+  const int waves = (K + 255) >> 8, all = (N + 15) >> 4, tiles = (all + 255) / 256, steps = (tiles + 3) / 4;
+  static const double start[] = {4.02, 5.08, 5.86}, tile[] = {0.313, 0.454, 0.864}, step[] = {0.094, 0.282, 0.343}, more[] = {0.152, 0.343, 0.444};
+  static const int least[] = {2, 5, 9};
+  const int b = waves <= 4 ? 0 : waves <= 8 ? 1 : 2;
+  const double stream = start[b] + (tile[b] + (K % 256 ? 0.028 : 0.) + 0.0037 * M) * tiles + (step[b] + more[b] * (waves - least[b])) * steps;
+  const int units = ((K >> 7) + 3) / 4, nu = (units + kp - 1) / kp, wrows = ROWS_WAVES / kp * rt * 16;
+  const int blocks = (N + wrows - 1) / wrows, rounds = (blocks + 255) / 256;
+  const double rows = 1.32 + rounds * (1.94 + 0.396 * rt + (0.517 + 0.0065 * M) * nu * rt + 0.197 * nu * kp + (K % 512 ? 0.104 * rt : 0.)) +
+                      blocks / 256. * 0.519 * nu * rt + 0.027e-6 * size;
+  return stream < 0.98 * rows;
+}
+
 RowsPlan rows_find_plan(int M, int N, int K, int mode) {
   const int units = ((K >> 7) + 3) / 4;
   const int least_zb = (M + 63) / 64, mt = (M + 16 * least_zb - 1) / (16 * least_zb), zb = (M + 16 * mt - 1) / (16 * mt);
   const RowsCost& cost = mt == 1 ? rows_cost_one : rows_cost;
-  RowsPlan best = {-1, 1};
+  RowsPlan best = {-1, 1, false};
   double least = 1e30;
   for (int f = 0; f < ROWS_FORMS; ++f) {
     const RowsForm& form = rows_forms[f];
@@ -581,10 +605,11 @@ RowsPlan rows_find_plan(int M, int N, int K, int mode) {
       if (z > 1) t += (mode == ROWS_SPLIT ? cost.second : 0.) + cost.sums * 4e-6 * z * (M + cost.rows) * N;
       if (t < least) {
         least = t;
-        best = {f, z};
+        best = {f, z, false};
       }
     }
   }
+  if (best.form >= 0 && best.splits == 1) best.behind = rows_behind_streaming(M, N, K, rows_forms[best.form].rt, rows_forms[best.form].kp);
   return best;
 }
 
@@ -615,15 +640,14 @@ EAGLE_EXPORT int eagle_qmm_rows_supported(int M, int N, int K, int swiglu) {
 // Where it beats the other forms (us, against the streaming kernel unless noted).  33 rows on: everywhere (two
 // passes of the streaming kernel; 48 x 3584 x 18944 23 / 38, 64 x 896 x 512 8.1 / 10.8).  17 .. 32 rows: from about
 // 4 MB of weights or K above 4608 (2048 -> 3584 7.4 / 9.1, 896 -> 8192 6.3 / 6.8, 8192 -> 512 9.9 / 12.2, but 2560 ->
-// 512 7.7 / 5.7).  Up to 16 rows, past the lines of the small-row kernel: everywhere.  Timed in
-// turn over 222 products of K up to 2048 or 70 .. 250 M weights it is 8 % faster on average (512 -> 152064 12.4 / 18.3, 2048 -> 18944
-// 9.2 / 10.8, 3584 -> 28672 14.3 / 17.2, 4096 -> 32768 16.8 / 21.5), more than 3 % behind in 18 (two rows 4864 -> 18944 18.6 / 16.5).
+// 512 7.7 / 5.7).  Up to 16 rows, past the lines of the small-row kernel: everywhere but where
+// rows_behind_streaming expects it to be slower (2048 -> 18944 9.2 / 10.8, 4096 -> 32768 16.8 / 21.5, 4864 -> 18944 17.1 / 19.0).
 // The forms for one or a few rows come first where they apply (the caller asks them before).  Above 64 rows the GEMM is
 // faster; who must not round a weight asks for this kernel.
 EAGLE_EXPORT int eagle_qmm_rows_preferred(int M, int N, int K) {
   if (M < 1 || M > 2 * EAGLE_MAX_M) return 0;
   if (M > 16 && M <= 32 && (double)N * K < 7e6 && K <= 4608) return 0;
-  return eagle_qmm_rows_supported(M, N, K, 0);
+  return eagle_qmm_rows_supported(M, N, K, 0) && !rows_plan(M, N, K, ROWS_SPLIT).behind;
 }
 
 EAGLE_EXPORT size_t eagle_qmm_rows_workspace_bytes(int M, int N, int K) {

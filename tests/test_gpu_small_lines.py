@@ -2,8 +2,9 @@
 16 rows past them, where the rows kernel takes over."""
 import pytest
 
-from mlx_eagle_spec_decoding_tree_amd import _lib
+from mlx_eagle_spec_decoding_tree_amd import _lib, ops
 from test_gpu_small_dispatch import run
+from util import close_fp16
 
 pytestmark = pytest.mark.gpu
 
@@ -25,3 +26,16 @@ def test_past_the_lines(dev, M, N, K):
     assert L.eagle_qmm_rows_preferred(M, N, K) == 1 and not L.eagle_qmm_small_preferred(M, N, K) and not L.eagle_qmv_preferred(M, N, K)
     print(f"M={M} N={N} K={K}", flush=True)
     run(dev, M, N, K, bias=True)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 102016, 1152), (10, 99944, 640), (4, 34496, 2816), (2, 71944, 1664), (1, 116528, 1280), (16, 99968, 640)])
+def test_where_the_streaming_kernel_takes_over(dev, M, N, K):
+    """The rows kernel's second round of workgroups is half empty at these numbers of weight rows."""
+    L = _lib.lib()
+    assert L.eagle_qmm_rows_preferred(M, N, K) == 0 and L.eagle_qmm_rows_supported(M, N, K, 0) == 1 and L.eagle_qmm_rows_preferred(M, 152064, 512) == 1
+    print(f"M={M} N={N} K={K}", flush=True)
+    d, x, got = run(dev, M, N, K, bias=N % 32 == 8)
+    if N % 32 == 0:                                # (gate, up) tiles of 16 rows in turn
+        act = ops.quantized_matmul_swiglu(x, d["weight"], d["scales"], d["biases"]).cpu().numpy()
+        g, u = (got.astype("float64").reshape(M, N // 32, 2, 16)[:, :, i].reshape(M, N // 2) for i in (0, 1))
+        close_fp16(act, g / (1 + 2.718281828459045 ** -g) * u)
