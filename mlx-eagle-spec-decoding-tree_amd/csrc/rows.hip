@@ -551,7 +551,8 @@ struct RowsPlan {
 // the best of all forms and splits of 1400 and 12600 random products: 17 .. 64 rows 1.2 % longer on
 // average, 8 % at the 95th percentile; 65 .. 2048 rows 1.2 and 7.5.  Up to 16 rows (one tile, other constants: a unit costs its
 // weights and the barriers of its K parts rather than its matrix instructions, a split more than the few rows say) 1.0 and 7.3,
-// where the constants of the others gave 3.2 and 14 (4 x 8192 -> 3584 two tiles a wave in 16 splits 12.0 us, one in 8 9.9).
+// where the constants of the others gave 3.2 and 14 (4 x 8192 -> 3584 two tiles a wave in 16 splits 12.0 us, one in 8 9.9).  Splits of up to
+// three rows count as those of four (2 x 11008 -> 18944 chose another division: 36.1 us, 33.1).
 enum { ROWS_WHOLE = 0, ROWS_SPLIT = 1, ROWS_PARTIAL = 2 };
 struct RowsCost {
   double start, w, x, unit, parts, whole, second, sums, rows;
@@ -602,7 +603,7 @@ RowsPlan rows_find_plan(int M, int N, int K, int mode) {
       const double w = wrows * (double)nu * form.kp * (512 * 0.5625 / 1e3), x = 16. * mt * nu * form.kp * (1024 / 1e3);
       double t = rounds * (cost.start + cost.w * w + cost.x * x + (cost.unit * form.rt * mt + cost.parts * (form.kp - 1)) * nu) +
                  cost.whole * (blocks * z / 256.) * (w + 0.5 * x);
-      if (z > 1) t += (mode == ROWS_SPLIT ? cost.second : 0.) + cost.sums * 4e-6 * z * (M + cost.rows) * N;
+      if (z > 1) t += (mode == ROWS_SPLIT ? cost.second : 0.) + cost.sums * 4e-6 * z * ((M > 4 ? M : 4) + cost.rows) * N;
       if (t < least) {
         least = t;
         best = {f, z, false};
