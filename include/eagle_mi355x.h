@@ -531,8 +531,9 @@ int eagle_post_process_draft_tree(const int32_t* tree_position_ids, const int32_
                                   int total, int32_t* retrieve_indices, int32_t* shape_out,
                                   eagle_stream_t stream);
 /* The same with the rows packed: leaf_num rows of max_depth + 1 entries, nothing between them
- * (retrieve_indices still holds 64 * 64 entries).  shape_out (8-byte aligned) is written last, as one
- * 8-byte store, and may be pinned host memory: a caller that has cleared it and sees it change may use the rows on any stream. */
+ * (retrieve_indices still holds 64 * 64 entries).  shape_out may be pinned host memory, for a caller that waits for the stream
+ * to learn the shape.  Where it is 8-byte aligned it is written last, as one 8-byte store: a caller that has cleared it and sees it
+ * change may use the rows on any stream. */
 int eagle_post_process_draft_tree_packed(const int32_t* tree_position_ids, const int32_t* mask_index,
                                          int total, int32_t* retrieve_indices, int32_t* shape_out,
                                          eagle_stream_t stream);

@@ -177,7 +177,8 @@ __global__ __launch_bounds__(TREE_THREADS) void process_draft_tree_kernel(
 
 // mlx_eagle.py:254-295 in one wave (a lane per token, T <= 64).  retrieve [64][64], shape {leaf_num,
 // max_depth + 1}; PACKED: rows of max_depth + 1 entries, leaf_num of them, without padding, and the shape last, as one 8-byte
-// store to memory that the host may be watching: who sees it may use the rows, on any stream, as after a wait for this one.
+// store to memory that the host may be watching: who sees it may use the rows, on any stream, as after a wait for this one.  (A shape
+// that is not aligned for that store is written as two words, for a caller that waits for the stream.)
 template <bool PACKED>
 __global__ __launch_bounds__(64) void post_process_kernel(const int32_t* __restrict__ pos_ids,
                                                          const int32_t* __restrict__ mask_index,
@@ -225,9 +226,14 @@ __global__ __launch_bounds__(64) void post_process_kernel(const int32_t* __restr
   }
   if (PACKED) {
     __syncthreads();
-    if (tid == 0)
+    if (tid != 0) return;
+    if (reinterpret_cast<uintptr_t>(shape) & 7u) {
+      shape[0] = leaves;
+      shape[1] = cols;
+    } else {
       __hip_atomic_store(reinterpret_cast<unsigned long long*>(shape),
                          (unsigned long long)(uint32_t)cols << 32 | (uint32_t)leaves, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 }
 
@@ -415,7 +421,6 @@ static int post_process(const int32_t* tree_position_ids, const int32_t* mask_in
                         int32_t* retrieve_indices, int32_t* shape_out, bool packed, eagle_stream_t stream) {
   if (!tree_position_ids || !mask_index || !retrieve_indices || !shape_out) return EAGLE_ERR_NULL;
   if (total < 1 || total >= MAXT) return EAGLE_ERR_SHAPE;
-  if (packed && (reinterpret_cast<uintptr_t>(shape_out) & 7u)) return EAGLE_ERR_ALIGN;     // one 8-byte store
   if (packed)
     hipLaunchKernelGGL(post_process_kernel<true>, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream),
                        tree_position_ids, mask_index, total, retrieve_indices, shape_out);

@@ -191,3 +191,24 @@ def test_topk_and_search_sorted_mirror(dev):
         tgt = rng.choice(arr, 12)
         got = eagle.search_sorted(torch.from_numpy(arr).to(dev), torch.from_numpy(tgt).to(dev))
         assert np.array_equal(got.cpu().numpy(), to.search_sorted(arr, tgt))
+
+
+@pytest.mark.parametrize("where", ["device", "pinned"])
+def test_packed_post_process_takes_a_shape_at_any_word(dev, where):
+    """shape_out of the packed form at a word that is not 8-byte aligned, and at one that is."""
+    rng = np.random.default_rng(5)
+    scores, tokens, parents_list, _ = simulate_draft(rng, 4)
+    pos_w, midx_w, _, _ = to.process_draft_tree(scores, tokens, parents_list, np.array([[9]]), 8, 31)
+    want = to.post_process_draft_tree(pos_w, 31, midx_w)
+    pos, midx = to_dev(pos_w.astype(np.int32), dev), to_dev(midx_w.astype(np.int32), dev)
+    for at in (0, 1, 2, 3):
+        buf = torch.zeros(8, dtype=torch.int32, device=dev) if where == "device" else torch.zeros(8, dtype=torch.int32, pin_memory=True)
+        ri = torch.full((64 * 64,), 77, dtype=torch.int32, device=dev)
+        rc = _lib.lib().eagle_post_process_draft_tree_packed(pos.data_ptr(), midx.data_ptr(), 31, ri.data_ptr(), buf.data_ptr() + 4 * at,
+                                                             torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        got = buf.cpu().tolist()
+        assert got[at:at + 2] == list(want.shape) and got[:at] == [0] * at and got[at + 2:] == [0] * (6 - at)
+        ri = ri.cpu().numpy()
+        assert np.array_equal(ri[:want.size].reshape(want.shape), want) and (ri[want.size:] == 77).all()
