@@ -543,8 +543,9 @@ class TreeVerifier:
         through the slab form of the matmul (their consumer adds the slabs), 0 for the
         streaming kernel; None: the library's choice for this shape.
         tiled: the slab products (and gate|up + SwiGLU) read a copy of their weights in the tiled
-        layout (`ops.tile_weights`; doubles the memory of those matrices).  None: on for the fused
-        step."""
+        layout (`ops.tile_weights`; doubles the memory of those matrices), and up to 32 tree tokens the vocabulary
+        projection too; a larger tree reads that from the checkpoint's layout (`head_tiled` stays None).
+        None: on for the fused step."""
         args = model.args
         self.model, self.cache, self.args = model, cache, args
         if total_tokens + 1 > TREE_SLOTS:

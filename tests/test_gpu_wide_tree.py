@@ -163,3 +163,10 @@ def test_device_loop_with_the_reference_default_tree(dev, same, graph):
     assert_greedy_stream(target, prompt, [first] + more, dev)
     with pytest.raises(ValueError):
         spec.SpeculativeDecoder(target2, draft2, capacity=256, k=8, depth=5, verify_num_tokens=64)
+
+
+def test_tiled_copies_of_a_wide_tree_leave_the_head_out(dev):
+    s = build(dev, "qwen_like", 50, 40, seed=1)
+    ver = eagle.TreeVerifier(s["model"], s["cache"], total_tokens=39, tiled=True)
+    assert ver.tiled is not None and ver.head_tiled is None
+    assert ver.qmm_launches()[-1][-2:] == (False, None)
