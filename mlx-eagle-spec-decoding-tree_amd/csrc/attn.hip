@@ -269,10 +269,10 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
       for (int e = 0; e < 4; ++e) acc[e] = fmaf(f, o[e], acc[e]);
     }
     if (nsplit > 1) {
-      // partials: (m, l) [H * T][nsplit][2], then O [H * T][nsplit][HD]
+      // partials: O [H * T][nsplit][HD], then (m, l) [H * T][nsplit][2] (behind O, so that O is 16-byte aligned whatever their number)
       const long slot = ((long)g * cols + col) * nsplit + blockIdx.z;
-      if (dq == 0) *reinterpret_cast<float2_t*>(part + slot * 2) = float2_t{mx, den};
-      *reinterpret_cast<float4_t*>(part + (long)H * T * nsplit * 2 + slot * HD + dq * 4) = acc;
+      if (dq == 0) *reinterpret_cast<float2_t*>(part + (long)H * T * nsplit * HD + slot * 2) = float2_t{mx, den};
+      *reinterpret_cast<float4_t*>(part + slot * HD + dq * 4) = acc;
     } else {
       const float inv = den > 0.f ? 1.f / den : 0.f;
       const int hr = (uint32_t)col * inv_T >> 16, t = col - hr * T;
@@ -292,8 +292,8 @@ __global__ __launch_bounds__(256) void tree_attn_add_kernel(const float* __restr
   const int row = id / QW, dq = id % QW;             // row = head * T + token
   if (row >= H * T) return;
   if (!LONG) most = NS;
-  const float* ml = part + (long)row * most * 2;
-  const float* po = part + (long)H * T * most * 2 + (long)row * most * HD + dq * 4;
+  const float* ml = part + (long)H * T * most * HD + (long)row * most * 2;
+  const float* po = part + (long)row * most * HD + dq * 4;
   float2_t w[NS];
   float4_t o[NS];
 #pragma unroll

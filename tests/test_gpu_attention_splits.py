@@ -24,9 +24,10 @@ def attention64(q, k, v, vis, P, Tk, scale):
     return torch.matmul(p, v).transpose(0, 1).reshape(q.shape[1], -1)
 
 
-# (query heads, KV groups, head dimension): 16, 12, 8, 6, 4, 3, 2 and 1 splits at the longer caches
+# (query heads, KV groups, head dimension): 16, 12, 8, 6, 4, 3, 2 and 1 splits at the longer caches; with 35 heads and an odd
+# number of rows the partial results are an odd number of (m, l) pairs
 @pytest.mark.parametrize("H,G,hd", [(2, 1, 64), (10, 2, 128), (14, 2, 64), (20, 5, 128), (28, 4, 128), (36, 9, 64),
-                                    (64, 8, 128), (160, 20, 64), (1, 1, 128)])
+                                    (64, 8, 128), (160, 20, 64), (1, 1, 128), (35, 5, 128)])
 @pytest.mark.parametrize("cap", [64, 768, 769, 2049, 5000])
 def test_splits(dev, H, G, hd, cap):
     g = torch.Generator(device=dev).manual_seed(H * 1000 + cap)
