@@ -674,7 +674,8 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
                     (half_t)(o_acc[db][4 * i4 + 3] * inv)};
     return;
   }
-  // one split: the rows as they lie in memory, through the wave's part of LDS
+  // one split: the rows as they lie in memory, through the wave's part of LDS (other lanes' reads of half_o come first)
+  __builtin_amdgcn_wave_barrier();
   unsigned char* mine = lds + wave * (32 * OS * 4);
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
 #pragma unroll
