@@ -421,8 +421,9 @@ int launch_tree(const void* q, const void* kc, const void* vc, const uint32_t* b
 // a split in fp16, added by a second kernel: in fp32 128 rows behind 1536 keys, seven splits, take 20.6 us, so 17.3).  What bounds it: 2.5 us per tile of a workgroup, of which the matrix instructions are 0.9,
 // and the last workgroups of a causal triangle.  Before, a workgroup held all heads of a group (seven waves) on tiles of 64 keys, one
 // per compute unit, the longest twice the average, and every result went through partials and a merge; us per chunk
-// (28 heads of 128 in 4 groups; before / now): 2048 rows 101 / 52, 512 rows 24.8 / 15.7, 128 rows 13.4 / 8.1, 512 rows behind 1536
-// 41 / 36; 14 heads of 64 in 2 groups, 2048 rows 37 / 27.
+// (28 heads of 128 in 4 groups, K and V of 28 layers in turn in a graph; before / now): 2048 rows 98 / 52, 512 rows 24.8 / 14.8, 128 rows
+// 13.9 / 7.6, 512 rows behind 1536 40 / 31; 14 heads of 64 in 2 groups, 2048 rows 37 / 26.  With K and V from HBM 2048 rows take 98 / 51, 512
+// 24.7 / 15.4.
 constexpr int CAUSAL_TILE = 128;
 
 // cached rows before piece p (never past the cache, whatever the counter says: a graph replayed beyond the capacity
@@ -441,16 +442,10 @@ __device__ inline int causal_rows(const int32_t* len_dev, int p, int n, int piec
   return most;
 }
 
-// Splits in use for `ntiles` tiles in a grid of `nsplit`, `units` workgroups beside each other: as many as fill the GPU, with
-// at least four tiles each (two where there are few units): a split costs its partial results and the second launch (28
-// heads of 128, us with no split / at least 4 / 2 / 1 tiles: 512 rows 15.7 / 15.7 / 19.1 / 21.1, 256 rows behind 1792 41.6 / 25.3 / 25.9 /
-// 26.2, 64 rows behind 2000 46 / 21.4 / 17.7 / 17.5).  Three tiles of few units: one split each (32 rows behind 300 12.2, in two
-// splits 14.2), at head dimension 64 no split, if that spares the second launch (8.5; 9.1 and 10.4).
-template <int HD>
-__host__ __device__ inline int causal_splits(int ntiles, int nsplit, int units) {
+// Key splits in use for `ntiles` tiles in a grid of `nsplit`, of `least` tiles or more: a cache much shorter than the launch was sized for,
+// and the shorter pieces of a chunk, pay for few partial results.
+__device__ inline int causal_splits(int ntiles, int nsplit, int least) {
   int tpw = (ntiles + nsplit - 1) / nsplit;
-  const int fill = (units * ntiles + 255) / 256, least = units > 32 ? 4 : HD > 64 && ntiles == 3 ? 1 : 2;
-  tpw = tpw > fill ? tpw : fill;
   tpw = tpw > least ? tpw : least;
   return (ntiles + tpw - 1) / tpw;
 }
@@ -466,7 +461,7 @@ template <int HD, int DEPTH, bool SEVERAL>
 __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ kc, const half_t* __restrict__ vc,
     const int32_t* __restrict__ len_dev, half_t* __restrict__ out, half_t* __restrict__ part_o, float* __restrict__ part_ml, int H,
-    int G, long cap, float scale_log2e, int pieces, int hp, int pp) {
+    int G, long cap, float scale_log2e, int pieces, int hp, int pp, int least) {
   constexpr int KSTEPS = HD / 16;       // MFMA steps over the head dimension for S
   constexpr int DB = HD / 32;           // 32-wide blocks of the head dimension for O
   constexpr int STR = HD * 2 + 16;      // LDS row stride in bytes (pad: conflict-free reads)
@@ -481,8 +476,8 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
   unsigned char* ldsV = lds + KTT * STR;
   const int rep = H / G, quads = (rep + hp - 1) / hp;
   const int g = blockIdx.x / quads, hq = blockIdx.x % quads;
-  const int split = blockIdx.y, nsplit = gridDim.y;
-  const int group = gridDim.z - 1 - blockIdx.z;   // (the last pieces see the most keys: dispatched first)
+  const int split = blockIdx.z, nsplit = gridDim.z;      // (the slowest: splits that are not in use leave no gaps between the others)
+  const int group = gridDim.y - 1 - blockIdx.y;   // (the last pieces see the most keys: dispatched first)
   const int tid = threadIdx.x;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wave = wid & 3, khalf = wid >> 2;
@@ -499,7 +494,7 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
   const int Ltot = causal_rows(len_dev, group * pp, pp, pieces, cap);
   const int ntiles = (Ltot + KTT - 1) / KTT;
   const int own = live ? P + 32 : 0;       // keys up to here concern this wave's rows
-  const int nactive = causal_splits<HD>(ntiles, nsplit, gridDim.x * gridDim.z);
+  const int nactive = causal_splits(ntiles, nsplit, least);
   if (split >= nactive) return;
   half8_t qreg[KSTEPS];
   const half_t* qp = q + ((long)head * pieces * 32 + piece * 32 + ql) * HD;
@@ -699,11 +694,11 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
 template <int HD>
 __global__ __launch_bounds__(256) void causal_add_kernel(const half_t* __restrict__ part_o, const float* __restrict__ part_ml,
                                                          half_t* __restrict__ out, int H, int nsplit, const int32_t* __restrict__ len_dev,
-                                                         long cap, int pp, int units) {
+                                                         long cap, int pp, int least) {
   constexpr int VR = HD / 8, MOST = 8;
   const int piece = blockIdx.z, pieces = gridDim.z;
   const int rows = causal_rows(len_dev, piece / pp * pp, pp, pieces, cap);
-  const int nact = causal_splits<HD>((rows + CAUSAL_TILE - 1) / CAUSAL_TILE, nsplit, units);
+  const int nact = causal_splits((rows + CAUSAL_TILE - 1) / CAUSAL_TILE, nsplit, least);
   if (nact == 1) return;                           // written by the workgroup itself
   const int id = blockIdx.x * 256 + threadIdx.x;   // (head, row, vector)
   const int hr = id / VR, c = id % VR;
@@ -753,37 +748,51 @@ template <int HD>
 int launch_causal(const void* q, const void* kc, const void* vc, const int32_t* len, void* out, int pieces, int H, int G,
                   long cap, int max_len, float scale, void* workspace, hipStream_t st) {
   const int rep = H / G, hp = rep < 4 ? rep : 4, gx = G * ((rep + hp - 1) / hp);
-  const int tiles = (max_len + CAUSAL_TILE - 1) / CAUSAL_TILE;
-  // With fewer than four heads per group a workgroup can take several pieces, so that its waves share the tiles, and the keys are split
-  // instead.  By the least of: a tile takes 2.2 us (128) or 1.25 (64) whatever part of the waves is busy with it, splits 3.2 and 1.2 per
-  // MB of partial results (16 heads in 16 groups of 128, us for one piece / four: 512 rows behind 0 14.5 / 15.2, 1536 39 / 25, 8000 154 / 60;
-  // 64 rows behind 300, one / two, 12.7 / 13.3, 8000 30 / 26).
-  int pp = 1, nz = pieces, units = gx * pieces, nsplit = 1;
-  double least = 1e30;
+  // With fewer than four heads per group a workgroup can take several pieces, so that its waves share the tiles; the keys can be split.  The
+  // division with the least predicted time (us): a workgroup costs its start and its tiles, whatever part of its waves is busy with
+  // them, the launch as many of those as there are rounds (fewer where a causal triangle leaves later workgroups short), splits a second
+  // launch and their partial results.  Fitted to 2424 shapes timed in all their divisions (32 .. 2048 rows behind 16 .. 32768 keys), 7.4 % rms;
+  // its choice is 0.5 % longer than the best of them on average, 3 % at the 95th percentile, where filling the compute units once
+  // took 2.6 and 16, and counting on a part of a round 14 and 100 (28 heads, 224 rows behind 8000, 280 workgroups 73 us, 224 51).
+  struct Cost {
+    double tile, start, add, parts, several;
+  };
+  constexpr Cost cost = HD > 64 ? Cost{2.27, 0.89, 4.0, 1.34e-6, 0.} : Cost{1.33, 0.43, 2.8, 1.48e-6, 0.058};
+  const int rows = pieces * 32, tiles = (max_len + CAUSAL_TILE - 1) / CAUSAL_TILE;
+  const double triangle = rows < max_len ? 1.5 * rows / max_len : 1.5;
+  int pp = 1, nsplit = 1, least = 1;
+  double least_us = 1e30;
   for (int n = 1; n <= 4 / hp && n <= pieces; ++n) {
-    const int z = (pieces + n - 1) / n, u = gx * z;
-    const int s = HD == 64 && tiles <= 3 ? 1 : causal_splits<HD>(tiles, MAX_CAUSAL_SPLITS, u);
-    const double t = (HD > 64 ? 2.2 : 1.25) * ((u * s + 255) / 256) * ((tiles + s - 1) / s) + (s > 1 ? 3.2 + 2.4e-6 * pieces * 32 * H * HD * s : 0.);
-    if (t < least) {
-      least = t;
-      pp = n;
-      nz = z;
-      units = u;
-      nsplit = s;
+    const int units = gx * ((pieces + n - 1) / n);
+    for (int tpw = tiles, s = 1; s <= MAX_CAUSAL_SPLITS;) {
+      const double fill = units * s / 256., whole = (units * s + 255) / 256, rounds = whole > 1. ? whole - triangle * (whole - fill) : 1.;
+      const double us = rounds * (cost.start + (cost.tile + (n > 1 ? cost.several : 0.)) * tpw) +
+                        (s > 1 ? cost.add + cost.parts * rows * H * HD * s : 0.);
+      if (us < least_us) {
+        least_us = us;
+        pp = n;
+        nsplit = s;
+        least = units * s > 256 ? 12 : 4;            // (more than one round of workgroups only while the splits are long)
+        least = tpw < least ? tpw : least;
+      }
+      if (tpw == 1) break;
+      s = (tiles + tpw - 2) / (tpw - 1);             // the fewest splits with fewer tiles each
+      tpw = (tiles + s - 1) / s;
     }
   }
+  const int nz = (pieces + pp - 1) / pp;
   float* part_ml = static_cast<float*>(workspace);
   half_t* part_o = reinterpret_cast<half_t*>(part_ml + (size_t)pieces * H * nsplit * 32 * 2);
 #define EAGLE_CAUSAL(SEVERAL)                                                                                                              \
-  hipLaunchKernelGGL((causal_attn_kernel<HD, HD == 64 ? 2 : 1, SEVERAL>), dim3(gx, nsplit, nz), dim3(512), 0, st,                          \
+  hipLaunchKernelGGL((causal_attn_kernel<HD, HD == 64 ? 2 : 1, SEVERAL>), dim3(gx, nz, nsplit), dim3(512), 0, st,                          \
                      static_cast<const half_t*>(q), static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), len,                   \
-                     static_cast<half_t*>(out), part_o, part_ml, H, G, cap, scale * 1.4426950408889634f, pieces, hp, pp)
+                     static_cast<half_t*>(out), part_o, part_ml, H, G, cap, scale * 1.4426950408889634f, pieces, hp, pp, least)
   if (pp > 1) EAGLE_CAUSAL(true);
   else EAGLE_CAUSAL(false);
 #undef EAGLE_CAUSAL
   if (nsplit > 1)
     hipLaunchKernelGGL(causal_add_kernel<HD>, dim3((H * 32 * (HD / 8) + 255) / 256, 1, pieces), dim3(256), 0, st, part_o, part_ml,
-                       static_cast<half_t*>(out), H, nsplit, len, cap, pp, units);
+                       static_cast<half_t*>(out), H, nsplit, len, cap, pp, least);
   return eagle_launch_status();
 }
 

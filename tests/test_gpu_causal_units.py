@@ -77,7 +77,9 @@ def test_rows_of_later_pieces_stay_out(dev, H, G, hd, pieces, P, bad):
 
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("H,G,pieces,P,spare", [(16, 16, 5, 1500, 0), (16, 16, 7, 3000, 5), (16, 8, 3, 5000, 0), (8, 8, 2, 9000, 3), (8, 8, 11, 700, 1),
-                                                (9, 3, 3, 5000, 0), (1, 1, 1, 300, 0), (4, 2, 2, 290, 40), (16, 16, 17, 40, 0)])
+                                                (9, 3, 3, 5000, 0), (1, 1, 1, 300, 0), (4, 2, 2, 290, 40), (16, 16, 17, 40, 0),
+                                                (32, 16, 34, 30, 3000), (8, 8, 2, 50, 9000), (16, 16, 9, 4000, 0)])
 def test_several_pieces_and_splits(dev, H, G, hd, pieces, P, spare):
-    """Few heads per group: two, three and four pieces per workgroup, the last workgroup with fewer, and one, on split keys."""
+    """Few heads per group: two, three and four pieces per workgroup, the last workgroup with fewer, and one, on split keys; splits
+    that a cache much longer than the chunk leaves unused, and more than a round of workgroups."""
     test_causal_chunk(dev, H, G, hd, pieces, P, spare)
