@@ -57,14 +57,20 @@ __device__ inline float swap_add(float2_t p) { return p[0] + p[1]; }
 // ahead or 32 columns per workgroup: slower; K and V one after the other in one buffer: no gain at 64, spills at 128.)
 // Against one wave per query head with up to 33 key splits, partial results in fp16 and a merge of them, us per
 // call in a graph (before / now): 14 heads of 64 in 2 groups, 8 rows behind 560 keys 10.1 / 4.9, behind 2048 11.5 / 9.0 (one split),
-// 32 rows behind 4000 16.0 / 8.0; 28 heads of 128 in 4 groups, 32 rows behind 1024 14.6 / 9.1, 2048 17.3 / 10.9, 40 rows 15.6 / 11.3.
+// 32 rows behind 4000 15.8 / 7.7; 28 heads of 128 in 4 groups, 32 rows behind 1024 14.6 / 9.1, 2048 17.0 / 10.8, 40 rows behind 1000 15.9 / 11.3.
+// Those are of K and V of 28 layers in turn; from HBM (2 GiB of them in turn) 8 rows behind 2048 11.6 / 11.0, 32 behind 1024 14.7 / 9.3, 2048 17.3 / 11.3.
 constexpr int NW = 8;                   // waves per workgroup
 
-// Key splits in use behind a prefix of P rows, of a grid that holds `most`: no fewer than `least`, no more than one per 512 keys, so that
-// a short prefix in a large cache pays for few partial results.
-__device__ inline int tree_splits_in_use(int P, int least, int most) {
-  const int n = P >> 9 < most ? P >> 9 : most;
-  return n > least ? n : least;
+// Key splits of a launch: `most` in the grid; `least` always in use, behind a prefix of P rows no more than one per 512 keys and, up to `half`
+// rows, than `few`, so that a short prefix in a large cache pays for few partial results.
+struct TreeSplits {
+  int least, few, most, half;
+};
+__device__ inline int tree_splits_in_use(int P, const TreeSplits& s) {
+  int n = P >> 9;
+  const int top = P > s.half ? s.most : s.few;
+  n = n < top ? n : top;
+  return n > s.least ? n : s.least;
 }
 // cached rows before the masked ones: never past the cache, whatever the counter says
 __device__ inline int tree_prefix(const int32_t* len_dev, long cap, int Tk) {
@@ -77,7 +83,7 @@ template <int HD, int NC, bool WIDE>
 __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ kc, const half_t* __restrict__ vc,
     const uint32_t* __restrict__ mask_bits, const int32_t* __restrict__ len_dev, half_t* __restrict__ out, float* __restrict__ part,
-    int T, int H, int G, long cap, float scale_log2e, int Tk, uint32_t inv_T, int least) {
+    int T, int H, int G, long cap, float scale_log2e, int Tk, uint32_t inv_T, TreeSplits splits, uint32_t inv_G) {
   constexpr int KSTEPS = HD / 32;       // MFMA steps over the head dimension for S
   constexpr int DB = HD / 16;           // 16-wide blocks of the head dimension for O
   constexpr int STR = HD * 2 + 16;      // LDS row stride in bytes of a wave's V block
@@ -88,12 +94,21 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
   static_assert(NC * 16 * OSTR * 4 <= SLICE, "a wave's O tile does not fit over its blocks");
   __shared__ __attribute__((aligned(16))) unsigned char slices[NW][SLICE];
   __shared__ float2_t ml[NW][16 * NC];
-  const int g = blockIdx.x, rep = H / G;
+  const int nsplit = splits.most;
+  // this workgroup's KV group and key split; with inv_G the grid is 8 x columns x eighths of the (split, group) pairs, which puts
+  // the columns that read the same keys on one XCD
+  int g = blockIdx.x, split = blockIdx.z;
+  if (inv_G) {
+    const int pair = blockIdx.z * 8 + blockIdx.x;
+    split = (int)((uint32_t)pair * inv_G >> 16);
+    g = pair - split * G;
+  }
+  if (split >= nsplit) return;
+  const int rep = H / G;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 15, kq = lane >> 4;
   const int cols = rep * T;
-  const int nsplit = gridDim.z;
-  const int first = blockIdx.z * NW + wave;          // this wave's first block
+  const int first = split * NW + wave;          // this wave's first block
   const int col0 = blockIdx.y * 16 * NC;
   const char* kb_ptr = reinterpret_cast<const char*>(kc + (long)g * cap * HD);
   const char* vb_ptr = reinterpret_cast<const char*>(vc + (long)g * cap * HD);
@@ -136,8 +151,8 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
   const int P = tree_prefix(len_dev, cap, Tk);
   const int Ltot = P + Tk;
   const int nblk = (Ltot + 31) >> 5;
-  const int in_use = tree_splits_in_use(P, least, nsplit), stride = in_use * NW;
-  if ((int)blockIdx.z >= in_use) return;
+  const int in_use = tree_splits_in_use(P, splits), stride = in_use * NW;
+  if (split >= in_use) return;
 
   float m_run[NC], l_run[NC];
   float4_t o_acc[NC][DB];
@@ -270,7 +285,7 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
     }
     if (nsplit > 1) {
       // partials: O [H * T][nsplit][HD], then (m, l) [H * T][nsplit][2] (behind O, so that O is 16-byte aligned whatever their number)
-      const long slot = ((long)g * cols + col) * nsplit + blockIdx.z;
+      const long slot = ((long)g * cols + col) * nsplit + split;
       if (dq == 0) *reinterpret_cast<float2_t*>(part + (long)H * T * nsplit * HD + slot * 2) = float2_t{mx, den};
       *reinterpret_cast<float4_t*>(part + slot * HD + dq * 4) = acc;
     } else {
@@ -285,13 +300,13 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
 // Adds the key splits: one thread per four output elements, the NS splits that are always in use requested at once; those that a long
 // prefix adds (LONG: a grid of most > NS splits) eight at a time behind them.
 template <int HD, int NS, bool LONG>
-__global__ __launch_bounds__(256) void tree_attn_add_kernel(const float* __restrict__ part, half_t* __restrict__ out, int T, int H, int most,
+__global__ __launch_bounds__(256) void tree_attn_add_kernel(const float* __restrict__ part, half_t* __restrict__ out, int T, int H, TreeSplits splits,
                                                             const int32_t* __restrict__ len_dev, long cap, int Tk) {
   constexpr int QW = HD / 4, MORE = 8;
   const int id = blockIdx.x * 256 + threadIdx.x;
   const int row = id / QW, dq = id % QW;             // row = head * T + token
   if (row >= H * T) return;
-  if (!LONG) most = NS;
+  const int most = LONG ? splits.most : NS;
   const float* ml = part + (long)H * T * most * HD + (long)row * most * 2;
   const float* po = part + (long)row * most * HD + dq * 4;
   float2_t w[NS];
@@ -301,7 +316,7 @@ __global__ __launch_bounds__(256) void tree_attn_add_kernel(const float* __restr
     w[i] = *reinterpret_cast<const float2_t*>(ml + 2 * i);
     o[i] = *reinterpret_cast<const float4_t*>(po + i * HD);
   }
-  const int in_use = LONG ? tree_splits_in_use(tree_prefix(len_dev, cap, Tk), NS, most) : NS;
+  const int in_use = LONG ? tree_splits_in_use(tree_prefix(len_dev, cap, Tk), splits) : NS;
   float mx = M_FLOOR;
 #pragma unroll
   for (int i = 0; i < NS; ++i) mx = fmaxf(mx, w[i][0]);
@@ -346,7 +361,7 @@ __global__ __launch_bounds__(256) void tree_attn_add_kernel(const float* __restr
 
 // Key splits of a launch.  One where the keys are few: a second launch that adds the splits costs 2.0 us, a compute unit takes
 // 3.2 us per 1000 keys of head dimension 64 and 5.7 of 128, and the live length is usually well below the capacity that
-// the rule sees (14 heads of 64 in a cache of 2048: one split 5.2 / 6.8 / 9.9 us at 560 / 1024 / 2048 keys, eight 6.4 / 6.6 / 7.1; 28 heads
+// the rule sees (14 heads of 64: one split 4.9 / 9.1 us at 560 / 2040 keys, eight 6.2 / 6.6; 28 heads
 // of 128: one 8.2 / 11.1 / 16.9, four 8.9 / 9.2 / 10.8).  Otherwise as many as give every compute unit a workgroup at 32 query rows
 // and a wave a block.  It does not look at the rows, so a query's result is the same bits whatever else is in the launch (but for long
 // caches, launch_tree): above 32 rows of head dimension 128, where LDS holds one workgroup per compute unit, a workgroup takes 32 columns
@@ -363,37 +378,68 @@ int key_splits(int max_len, int H, int hd) {
 template <int HD, bool WIDE>
 int launch_tree(const void* q, const void* kc, const void* vc, const uint32_t* bits, const int32_t* len, void* out, int T,
                 int Tk, int H, int G, long cap, int max_len, float scale, void* workspace, hipStream_t st) {
-  constexpr int LONG_CACHE = 6144, KEYS = HD > 64 ? 1536 : 3072, MAX_LONG_SPLITS = 32;
+  constexpr int LONG_CACHE = 6144, MAX_LONG_SPLITS = 32;
   const int least = key_splits(max_len, H, HD), rep_T = H / G * T;
-  int nsplit = least, nc = HD > 64 && T > 32 ? 2 : 1;
+  int nc = HD > 64 && T > 32 ? 2 : 1;
+  TreeSplits splits = {least, least, least, 0};
+  uint32_t inv_G = 0;
   // Long caches: key_splits gives a few rows a handful of workgroups, each with thousands of keys (32 heads of 128 in 8 groups, one row
-  // behind 8192 keys 27 us, 32768 84; 64 heads 45 and 152).  The rows then say how many splits fill the compute units, the prefix how many of
-  // those are used, and from twice that length on many rows go 32 columns to a workgroup (14.3, 31; 14.7, 31; 32 rows of 28 heads behind 16384
-  // keys 36 -> 27; behind 600 in so large a cache 9.1 -> 11).
-  if (max_len > LONG_CACHE && max_len > least * KEYS) {
-    const int b16 = G * ((rep_T + 15) / 16), b32 = G * ((rep_T + 31) / 32);
-    if (b16 > 32 && max_len > 2 * least * KEYS) nc = 2;
-    const int fill = 256 / (nc == 2 ? b32 : b16) < MAX_LONG_SPLITS ? 256 / (nc == 2 ? b32 : b16) : MAX_LONG_SPLITS;
-    if (fill > nsplit) nsplit = fill;
+  // behind 8192 keys 27 us, 32768 84; 64 heads 45 and 152).  The rows then say how many splits fill the compute units and how many columns
+  // a workgroup takes, the prefix how many of those splits are used.  The workgroups of a group and split read the same keys and go to
+  // one XCD (35 heads in 5 groups, 27 rows behind 31451: 42 us, 75 spread over all of them).  By the least predicted time (us), fitted to 549
+  // shapes in all their divisions (1 .. 64 rows behind 6 .. 32 thousand keys): rounds of the workgroups of an XCD, each the blocks of a wave,
+  // the bytes that all of them read, a second launch and its partial results.  A cache is seldom full: the splits of three quarters of it are
+  // used from half of it up, those of a quarter below, and the columns are those with the smaller loss in both.
+  if (max_len > LONG_CACHE) {
+    struct Cost {
+      double start, block[2], add, parts, read;
+    };
+    constexpr Cost cost = HD > 64 ? Cost{1.63, {1.53, 1.79}, 6.9, 2.1e-6, 2.1e-9} : Cost{0., {0.66, 0.95}, 2.8, 4.9e-6, 0.55e-9};
+    double us[2][2];
+    int best[2][2];
+    for (int c = 0; c < 2; ++c) {
+      const int ny = (rep_T + 16 * c + 15) / (16 * c + 16);
+      for (int l = 0; l < 2; ++l) {
+        const int blocks = max_len / 128 * (l ? 3 : 1);
+        us[c][l] = 1e30;
+        for (int n = least; n <= MAX_LONG_SPLITS && (n == least || n * 16 <= blocks); ++n) {
+          const int rounds = ((G * n + 7) / 8 * ny + 31) / 32, each = (blocks + n * NW - 1) / (n * NW);
+          const double t = rounds * (cost.start + cost.block[c] * each) + (n > 1 ? cost.add + cost.parts * T * H * HD * n : 0.) +
+                           cost.read * ny * G * blocks * (32. * HD * 4);
+          if (t < us[c][l]) {
+            us[c][l] = t;
+            best[c][l] = n;
+          }
+        }
+      }
+    }
+    const int c = us[1][0] / us[0][0] + us[1][1] / us[0][1] < 2. ? 1 : 0;
+    nc = c + 1;
+    splits.few = best[c][0];
+    splits.most = best[c][1] > best[c][0] ? best[c][1] : best[c][0];
+    splits.half = max_len / 2;
+    if (G <= 48) inv_G = (65536 + G - 1) / G;          // (pair / G = pair inv_G >> 16 for up to 32 G + 7 pairs of up to 50 groups)
   }
-  const dim3 grid(G, (rep_T + 16 * nc - 1) / (16 * nc), nsplit);
+  const int ny = (rep_T + 16 * nc - 1) / (16 * nc);
+  const dim3 grid = inv_G ? dim3(8, ny, (G * splits.most + 7) / 8) : dim3(G, ny, splits.most);
   const float sl2 = scale * 1.4426950408889634f;
   const uint32_t inv_T = (65536 + T - 1) / T;          // col / T = col inv_T >> 16 for the at most 512 columns of a group
   float* part = static_cast<float*>(workspace);
   half_t* o = static_cast<half_t*>(out);
 #define EAGLE_ATTN(NC)                                                                                              \
   hipLaunchKernelGGL((tree_attn_kernel<HD, NC, WIDE>), grid, dim3(NW * 64), 0, st, static_cast<const half_t*>(q),   \
-                     static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), bits, len, o, part, T, H, G, cap, sl2, Tk, inv_T, least)
+                     static_cast<const half_t*>(kc), static_cast<const half_t*>(vc), bits, len, o, part, T, H, G, cap, sl2, Tk, inv_T, \
+                     splits, inv_G)
   if (nc == 2) EAGLE_ATTN(2);
   else EAGLE_ATTN(1);
 #undef EAGLE_ATTN
   const dim3 add((H * T * (HD / 4) + 255) / 256);
 #define EAGLE_ATTN_ADD(NS)                                                                                                              \
   case NS:                                                                                                                              \
-    if (nsplit > NS) hipLaunchKernelGGL((tree_attn_add_kernel<HD, NS, true>), add, dim3(256), 0, st, part, o, T, H, nsplit, len, cap, Tk); \
-    else hipLaunchKernelGGL((tree_attn_add_kernel<HD, NS, false>), add, dim3(256), 0, st, part, o, T, H, nsplit, len, cap, Tk);            \
+    if (splits.most > NS) hipLaunchKernelGGL((tree_attn_add_kernel<HD, NS, true>), add, dim3(256), 0, st, part, o, T, H, splits, len, cap, Tk); \
+    else hipLaunchKernelGGL((tree_attn_add_kernel<HD, NS, false>), add, dim3(256), 0, st, part, o, T, H, splits, len, cap, Tk);            \
     break
-  if (nsplit > 1) switch (least) {
+  if (splits.most > 1) switch (least) {
     EAGLE_ATTN_ADD(1);
     EAGLE_ATTN_ADD(2);
     EAGLE_ATTN_ADD(3);

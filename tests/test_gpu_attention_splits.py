@@ -58,9 +58,10 @@ def test_splits(dev, H, G, hd, cap):
             assert torch.equal(few, got[3:8])
 
 
-# around the length from which the splits follow the rows, and from which many rows go 32 columns to a workgroup (28 and 32 heads of 128:
-# four splits at least, 6144 and 12288; 64 heads two, 6144; 32 of 64 four, 12288 and 24576; 160 of 64 one), up to 32 splits
-@pytest.mark.parametrize("H,G,hd", [(28, 4, 128), (32, 8, 128), (64, 8, 128), (32, 4, 64), (160, 20, 64), (1, 1, 64)])
+# around the length from which the splits and the columns of a workgroup follow the rows, up to 32 splits, and the grid is dealt by XCD:
+# groups that do and do not divide eight, fewer and more than eight, more than the division by multiplication serves
+@pytest.mark.parametrize("H,G,hd", [(28, 4, 128), (32, 8, 128), (64, 8, 128), (32, 4, 64), (160, 20, 64), (1, 1, 64), (35, 5, 128),
+                                    (60, 60, 64)])
 @pytest.mark.parametrize("cap", [6144, 6145, 12289, 24577])
 def test_long_caches(dev, H, G, hd, cap):
     g = torch.Generator(device=dev).manual_seed(H + cap)
