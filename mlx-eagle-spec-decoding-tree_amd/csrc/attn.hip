@@ -27,21 +27,11 @@ __device__ inline half4_t lds_read_tr16(const unsigned char* p) {
   return __builtin_bit_cast(half4_t, v);
 }
 
-// A value and that of the lane 16 or 32 away, in both lanes (one of them in each half of the pair), without a trip through LDS.
-__device__ inline float2_t swap_pair32(float v) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  const uint32_t a = r[0], b = r[1];
-  return float2_t{__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)};
-}
-__device__ inline float2_t swap_pair16(float v) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  const uint32_t a = r[0], b = r[1];
-  return float2_t{__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)};
-}
-__device__ inline float swap_max(float2_t p) { return fmaxf(p[0], p[1]); }
-__device__ inline float swap_add(float2_t p) { return p[0] + p[1]; }
+// over the lane 32 away, and over the four lanes sixteen apart: without a trip through LDS
+__device__ inline float max32(float v) { return wave_f32(wave_reduce32(wave_u32(v), WaveMax())); }
+__device__ inline float sum32(float v) { return wave_f32(wave_reduce32(wave_u32(v), WaveAdd())); }
+__device__ inline float max16_32(float v) { return max32(wave_f32(wave_reduce16(wave_u32(v), WaveMax()))); }
+__device__ inline float sum16_32(float v) { return sum32(wave_f32(wave_reduce16(wave_u32(v), WaveAdd()))); }
 
 // ---- 1..64 query rows (a tree, a draft pass): queries packed over heads and tokens ----
 //
@@ -220,7 +210,7 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < 4; ++i) bm = fmaxf(bm, sacc[n][h][i]);
-      bm = swap_max(swap_pair32(swap_max(swap_pair16(bm))));
+      bm = max16_32(bm);
       const float m_new = fmaxf(m_run[n], bm * scale_log2e);
       const float alpha = __builtin_amdgcn_exp2f(m_run[n] - m_new);
       float psum = 0.f;
@@ -250,7 +240,7 @@ __global__ __launch_bounds__(NW * 64) void tree_attn_kernel(
   // (m, l, O) of the waves with blocks through LDS
 #pragma unroll
   for (int n = 0; n < NC; ++n) {
-    l_run[n] = swap_add(swap_pair32(swap_add(swap_pair16(l_run[n]))));
+    l_run[n] = sum16_32(l_run[n]);
     if (kq == 0) ml[wave][16 * n + c] = float2_t{m_run[n], l_run[n]};
   }
   __builtin_amdgcn_wave_barrier();
@@ -622,7 +612,7 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 16; ++i) bm = fmaxf(bm, sacc[h][i]);
-    bm = swap_max(swap_pair32(bm));
+    bm = max32(bm);
     const float m_new = fmaxf(m_run, bm * scale_log2e);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     float psum = 0.f;
@@ -664,7 +654,7 @@ __global__ __launch_bounds__(512, 2) void causal_attn_kernel(
   }
   if constexpr (DEPTH > 1)
     if (t0 < ntiles) do_tile(Stage<0>{}, t0);
-  l_run = swap_add(swap_pair32(l_run));
+  l_run = sum32(l_run);
   // the second half of the waves hands its (m, l, O) to the first through LDS
   __syncthreads();
   constexpr int OS = HD + 4;

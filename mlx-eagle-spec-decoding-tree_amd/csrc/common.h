@@ -29,27 +29,40 @@ static inline int eagle_launch_status() {
 // and 12.65.
 template <int ROR>
 __device__ inline uint32_t wave_row_ror(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + ROR, 0xf, 0xf, false);
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + ROR, 0xf, 0xf, true);
+}
+// over the lanes 32 and 16 apart, and over the sixteen lanes of a row
+template <typename Op>
+__device__ inline uint32_t wave_reduce32(uint32_t v, Op op) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return op(a[0], a[1]);
 }
 template <typename Op>
-__device__ inline uint32_t wave_reduce(uint32_t v, Op op) {
-  const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  v = op(a[0], a[1]);
-  const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  v = op(b[0], b[1]);
+__device__ inline uint32_t wave_reduce16(uint32_t v, Op op) {
+  const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return op(a[0], a[1]);
+}
+template <typename Op>
+__device__ inline uint32_t wave_reduce_row(uint32_t v, Op op) {
   v = op(v, wave_row_ror<8>(v));
   v = op(v, wave_row_ror<4>(v));
   v = op(v, wave_row_ror<2>(v));
   return op(v, wave_row_ror<1>(v));
 }
+template <typename Op>
+__device__ inline uint32_t wave_reduce(uint32_t v, Op op) {
+  return wave_reduce_row(wave_reduce16(wave_reduce32(v, op), op), op);
+}
 __device__ inline float wave_f32(uint32_t v) { return __builtin_bit_cast(float, v); }
 __device__ inline uint32_t wave_u32(float v) { return __builtin_bit_cast(uint32_t, v); }
-__device__ inline float wave_sum(float v) {
-  return wave_f32(wave_reduce(wave_u32(v), [](uint32_t a, uint32_t b) { return wave_u32(wave_f32(a) + wave_f32(b)); }));
-}
-__device__ inline float wave_max(float v) {
-  return wave_f32(wave_reduce(wave_u32(v), [](uint32_t a, uint32_t b) { return wave_u32(fmaxf(wave_f32(a), wave_f32(b))); }));
-}
+struct WaveAdd {
+  __device__ uint32_t operator()(uint32_t a, uint32_t b) const { return wave_u32(wave_f32(a) + wave_f32(b)); }
+};
+struct WaveMax {
+  __device__ uint32_t operator()(uint32_t a, uint32_t b) const { return wave_u32(fmaxf(wave_f32(a), wave_f32(b))); }
+};
+__device__ inline float wave_sum(float v) { return wave_f32(wave_reduce(wave_u32(v), WaveAdd())); }
+__device__ inline float wave_max(float v) { return wave_f32(wave_reduce(wave_u32(v), WaveMax())); }
 
 // Eight nibbles -> fp16 q, exact, in the order q0 q2 q4 q6 q1 q3 q5 q7.  A byte that holds a nibble is, read as OCP e4m3,
 // q * 2^-9 (subnormals up to 7, the first exponents up to 15), so the fp8 conversion gives the fp16 values of q two at a

@@ -93,15 +93,6 @@ __device__ inline T small_load(const void* base, uint32_t at) {
   return *reinterpret_cast<const T*>(static_cast<const char*>(base) + at);
 }
 
-// the sum over sixteen neighbouring lanes, in all of them
-__device__ inline float row16_sum(float v) {
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true));   // row_ror:8
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x124, 0xf, 0xf, true));
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x122, 0xf, 0xf, true));
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xf, 0xf, true));
-  return v;
-}
-
 // (four waves per SIMD in the launch bounds: with more registers to give away the compiler puts the products into accumulation registers
 // and reads them back, 48 instructions of gate|up; the builds that need more than 128 take two)
 template <int NW, int MAXC, int RP, int MODE, bool NORM>
@@ -213,7 +204,7 @@ __global__ __launch_bounds__(NW * 64, NW <= 8 && RP == 4 && MAXC == 3 ? 2 : 4) v
           }
         }
       }
-      ss[p] = row16_sum(ss[p]);
+      ss[p] = wave_f32(wave_reduce_row(wave_u32(ss[p]), WaveAdd()));
       if ((lane & 15) == 0) ssq[wave][4 * p + (lane >> 4)] = ss[p];
     }
     __syncthreads();
