@@ -850,7 +850,8 @@ __global__ void rope_table_kernel(const int32_t* __restrict__ pos, const float* 
 
 EAGLE_EXPORT size_t eagle_tree_attention_workspace_bytes(int H, int hd, int max_len) {
   if (H < 1 || hd < 1 || max_len < 1) return 0;
-  return (size_t)H * 64 * 32 * (hd + 2) * sizeof(float);   // at most 64 key splits
+  // 64 key splits of 32 rows: what a piece of a prompt chunk may use (a tree up to 32 splits)
+  return (size_t)H * 64 * 32 * (hd + 2) * sizeof(float);
 }
 
 EAGLE_EXPORT int eagle_tree_attention_f16(const void* q, const void* k_cache, const void* v_cache,

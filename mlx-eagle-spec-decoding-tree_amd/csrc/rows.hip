@@ -642,7 +642,10 @@ EAGLE_EXPORT int eagle_qmm_rows_supported(int M, int N, int K, int swiglu) {
 // passes of the streaming kernel; 48 x 3584 x 18944 23 / 38, 64 x 896 x 512 8.1 / 10.8).  17 .. 32 rows: from about
 // 4 MB of weights or K above 4608 (2048 -> 3584 7.4 / 9.1, 896 -> 8192 6.3 / 6.8, 8192 -> 512 9.9 / 12.2, but 2560 ->
 // 512 7.7 / 5.7).  Up to 16 rows, past the lines of the small-row kernel: everywhere but where
-// rows_behind_streaming expects it to be slower (2048 -> 18944 9.2 / 10.8, 4096 -> 32768 16.8 / 21.5, 4864 -> 18944 17.1 / 19.0).
+// rows_behind_streaming expects it to be slower (2048 -> 18944 9.2 / 10.8, 4096 -> 32768 16.8 / 21.5, 4864 -> 18944 17.1 / 19.0).  Of 2943
+// products with K 4096 .. 8192 and 70 .. 250 M weights 151 are more than 3 % behind, 11 % at most, nearly all at K above 6912 (4 x 8192 -> 11488
+// 19.3 / 17.5), the mean is 0.87; fits to both times do not tell those apart.  Of 3312 with K 8193 .. 11264 332, 25 % at most (4 x 11008 -> 16928
+// 34.1 / 27.3), the mean is 0.94: there a division of K into 22 units is uneven whatever the splits.
 // The forms for one or a few rows come first where they apply (the caller asks them before).  Above 64 rows the GEMM is
 // faster; who must not round a weight asks for this kernel.
 EAGLE_EXPORT int eagle_qmm_rows_preferred(int M, int N, int K) {

@@ -76,8 +76,8 @@ enum { SMALL_PLAIN = 0, SMALL_SWIGLU = 1, SMALL_ROPE = 2 };
 //
 // What bounds this kernel is the instructions of a wave, one after the other at about five cycles each (weights that are in the L2
 // already save 0.3 us of 5): wave-uniform values are kept scalar, addresses are a uniform base and 32 bits per lane, the
-// epilogue is spread over the threads.  8 rows of the 0.5B shapes, us before / after that: gate|up + norm 5.4 / 4.7, q|k|v 3.9 / 3.5,
-// down 4.7 / 4.55, 2048 -> 8192 5.45 / 5.1, one row of 3584 -> 3584 4.4 / 4.0.
+// epilogue is spread over the threads.  8 rows of the 0.5B shapes, us in a graph before / after that: gate|up + norm 5.4 / 4.7, q|k|v 3.9 / 3.5,
+// down 4.7 / 4.55, 2048 -> 8192 5.45 / 5.1, one row of 3584 -> 3584 4.4 / 4.0 (from the host a call takes as long: 4.8 and 4.4 .. 4.75, no shorter than before).
 // Next to that it is the number of cache lines its load instructions touch per compute
 // unit, so every request is shaped for few lines: x is read with whole rows of a chunk per
 // instruction (four rows x 256 bytes) and brought into the operand layout through a per-wave LDS

@@ -623,7 +623,8 @@ class TreeVerifier:
         # size every workspace before any capture
         L = _lib.lib()
         head = model.lm_head if not args.tie_word_embeddings else model.model.embed_tokens
-        # (what the streaming kernel needs of it: a tree above 32 tokens takes that in two passes)
+        # (what the streaming kernel needs of it: products of a tree above 32 tokens that the rows kernel does not take go
+        # through it in two passes)
         need = max(L.eagle_qmm_workspace_bytes(rows, n, k) for n, k in
                    ((H * hd, D), (G * hd, D), ((H + 2 * G) * hd, D), (D, H * hd), (I, D), (2 * I, D),
                     (D, I), (head.weight.shape[0], D))

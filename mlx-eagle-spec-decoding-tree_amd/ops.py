@@ -655,8 +655,7 @@ def draft_attention(q, k_cache, v_cache, mask_words, cache_len_dev, Tk, scale, m
 
 def scaled_dot_product_attention(queries, keys, values, cache=None, scale=None, mask=None):
     """Drop-in for the call at mlx_llama.py:185-192 on the tree and draft paths:
-    queries [1,H,T,hd] with T <= 64 (32 query rows per launch set), keys/values [1,G,S,hd],
-    mask [1,1,T,S] additive.  Only
+    queries [1,H,T,hd] with T <= 64, keys/values [1,G,S,hd], mask [1,1,T,S] additive.  Only
     the last min(S, 64) columns of the mask are looked at: every earlier column has to be zero
     (a prefix that all queries see), which holds for the verification mask
     (mlx_eagle.py:337-338), the expansion masks up to depth 8 (mlx_eagle.py:143-171) and causal

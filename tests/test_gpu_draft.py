@@ -253,8 +253,8 @@ def test_generate_step_stream_equals_target_greedy(dev, same):
 
 def test_generate_step_with_the_reference_default_tree(dev):
     """depth 5, 39 draft nodes (the reference's defaults, mlx_eagle.py:509-510): a tree of 40 tokens
-    on the module path (tiled GEMMs for 40 rows, attention in two pieces of query rows inside one
-    launch pair); the emitted stream is the target's greedy stream."""
+    on the module path (the rows kernel for 40 rows, attention over two mask words per query); the
+    emitted stream is the target's greedy stream."""
     (targs, tw, target), (dargs, dw, draft) = tiny_pair(dev, same=True, seed=6)
     rng = np.random.default_rng(9)
     prompt = rng.integers(0, targs.vocab_size, 40).astype(np.int32)
@@ -421,7 +421,7 @@ def test_draft_attention_random_shapes(dev):
 
 
 def test_causal_attention_pieces(dev):
-    """All 32-row pieces of a chunk in one launch pair against per-piece causal attention."""
+    """All 32-row pieces of a chunk in one call against per-piece causal attention."""
     rng = np.random.default_rng(77)
     for (H, G, hd, P, R) in ((4, 2, 64, 0, 64), (14, 2, 64, 100, 96), (32, 8, 128, 37, 160), (8, 8, 128, 500, 32)):
         print(f"chunk attention H={H} G={G} hd={hd} P={P} R={R}", flush=True)

@@ -110,8 +110,8 @@ def test_one_layer_at_7b_width(dev):
 
 def test_one_layer_at_7b_width_with_the_default_tree(dev):
     """The same layer on a tree of 40 tokens (the reference's default of 39 draft nodes,
-    mlx_eagle.py:390,510): 64-row partial tiles in the slab form, gate|up and the vocabulary
-    projection as two passes of 32 rows, attention in two pieces of query rows."""
+    mlx_eagle.py:390,510): 64-row partial tiles in the slab form, the vocabulary
+    projection in one launch of the rows kernel, attention over two mask words per query."""
     P, T = 2048, 40
     s = setup_step(dev, synth.qwen25_7b(), 1, 6, P, T)
     mask = np.concatenate([np.zeros((T, P), np.float16), tree_oracle.additive_mask(s["anc"])], axis=1)

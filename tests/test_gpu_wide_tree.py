@@ -1,6 +1,6 @@
 """Trees of 33..64 tokens (the reference's default is 39 draft nodes, mlx_eagle.py:390,510) on the
-fused verification step and the device loop: attention in pieces of 32 query rows inside one
-launch pair, the projections as tiled GEMMs."""
+fused verification step and the device loop: attention over two mask words per query, the projections in the
+slab form with 64-row tiles, the head on the rows kernel."""
 import numpy as np
 import pytest
 import torch
@@ -16,8 +16,8 @@ pytestmark = pytest.mark.gpu
 
 
 def test_attention_of_up_to_64_queries(dev):
-    """One launch pair for 33..64 queries: against the oracle, and bit for bit against the
-    32-query form called once per piece of rows."""
+    """33..64 queries in one call: against the oracle, and bit for bit against the form for up to
+    32 queries called once per 32 rows."""
     rng = np.random.default_rng(4040)
     for case in range(16):
         hd = int(rng.choice([64, 128]))
