@@ -326,6 +326,12 @@ __device__ inline void rows_wave(const RowsArgs& a, int nb, int m0, int wave, in
   }
 #pragma unroll
   for (int u = 0; u < REM; ++u) step(u, 4 * (NU - 1) + u, std::true_type{});
+  // The chunks that a short last unit leaves in the ring count as used: with the ring's last place read in the loop alone, the compiler fetched it
+  // into other registers and copied it at the end of each unit, behind a wait for every load in flight
+#pragma unroll
+  for (int u = REM; u < AH; ++u)
+#pragma unroll
+    for (int t = 0; t < RT; ++t) asm volatile("" ::"v"(ring[u][t]));
   // (or the compiler sinks the accumulation of the unit behind it, into the block that uses the sums, and runs out of registers)
 #pragma unroll
   for (int t = 0; t < RT; ++t)
