@@ -19,6 +19,7 @@ struct RowsArgs {
   int both;               // scales and biases fit LDS together
   int pitch;              // rows of x per split in `partial`
   int zb;                 // blocks of 16 MT rows of x
+  int pairs;              // K is dealt in pairs of chunks (1), or chunk by chunk (0)
 };
 
 constexpr int ROWS_WAVES = 8;
@@ -69,9 +70,13 @@ __device__ inline void rows_wave(const RowsArgs& a, int nb, int m0, int wave, in
   const int r = lane & 15, kq = lane >> 4;
   const int K = a.K, M = MANY && a.M - m0 > ROWS ? ROWS : a.M - m0, N = a.N;
   const int all = K >> 7;
-  // chunks of 128 columns, dealt over the K parts of all workgroups along y; worked off in units of four, the last of REM
+  // chunks of 128 columns, dealt over the K parts of all workgroups along y; worked off in units of four, the last of REM.
+  // In pairs (the two halves of a line; the longest part has the units it has chunk by chunk), unless a.pairs is 0
   const int parts = gridDim.y * KP;
-  auto first = [&](int p) { return (int)((unsigned)all * (blockIdx.y * KP + p) / parts); };
+  auto first = [&](int p) {
+    const int c = (int)((unsigned)((all + a.pairs) >> a.pairs) * (blockIdx.y * KP + p) / parts) << a.pairs;
+    return c < all ? c : all;
+  };
   const int NU = ((all + parts - 1) / parts + 3) >> 2;         // units of the longest part
   const int c0 = first(kp), nch = first(kp + 1) - c0;
   const int XC = 4 * NU;

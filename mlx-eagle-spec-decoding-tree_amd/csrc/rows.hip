@@ -9,8 +9,12 @@
 //     three and a half units of the loop, not four (32 x 3584 -> 37888 with SwiGLU 28.1 us -> 24.0, 40 rows 32.0 -> 29.2, 64 rows 38.9 -> 32.8;
 //     40 x 18944 -> 3584 left as partial sums 19.6 -> 18.7).  Wide matrices take many tiles per workgroup (x is read by fewer), narrow
 //     ones few tiles and K split over workgroups, whose fp32 partial sums a second launch adds (rows_plan).
+//   * A product whose parts are added here deals K in pairs of chunks, the two 64-byte halves of a line: a part that begins with a second half
+//     requests no line whole, and the line at each seam twice (8 x 10240 -> 21064 in three parts 35.5 us chunk by chunk, 30.7 in pairs; 3 x 13568 ->
+//     17888 39.2, 34.4; 40 x 18944 -> 3584 23.0, 22.4).  One that is left as partial sums deals single chunks: alone it gains as much, but in the
+//     middle of a tree pass's weights the longer parts cost more (40 tokens 2519 us, 2533 in pairs).
 //   * Weights go from memory to registers, 16 bytes per lane, a ring of AH chunks of 128 columns ahead; both 64-byte
-//     halves of a line are requested together.  Two half-wave swaps deal the words of a lane so that a matrix
+//     halves of a line are requested together (of two lines, where a part begins at an odd chunk).  Two half-wave swaps deal the words of a lane so that a matrix
 //     instruction works in one quantisation group; nibbles become fp16 integers through the fp8 conversion (exact).
 //     The group's sum enters the accumulators times its scale in fp32: no weight is rounded.
 //   * x (MT tiles of 16 rows) goes through LDS in blocks, two in turn, one barrier per block that leaves the loads
@@ -246,6 +250,7 @@ EAGLE_EXPORT int eagle_qmm_rows_w4g64_f16(const void* x, const uint32_t* wq, con
   a.swiglu = swiglu != 0;
   a.both = 0;
   a.pitch = M;
+  a.pairs = 1;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int rc = p.form->run(a, p.splits, st);
   if (rc != EAGLE_OK || p.splits == 1) return rc;
@@ -280,6 +285,7 @@ EAGLE_EXPORT int eagle_qmm_rows_partial_w4g64(const void* x, const uint32_t* wq,
   a.N = N;
   a.K = K;
   a.pitch = eagle_slab_rows(M);
+  a.pairs = 0;
   if (partial_bytes < (size_t)splits * a.pitch * N * sizeof(float)) return EAGLE_ERR_WORKSPACE;
   return rows_plan(M, N, K, ROWS_PARTIAL).form->run(a, splits, static_cast<hipStream_t>(stream));
 }
