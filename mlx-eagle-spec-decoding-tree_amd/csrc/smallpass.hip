@@ -152,7 +152,7 @@ __global__ __launch_bounds__(NW * 64, NW <= 8 && RP == 4 && MAXC == 3 ? 2 : 4) v
     }
   }
   half8_t nw[MAXC];
-  if (NORM && a.norm_w) {
+  if (NORM) {
 #pragma unroll
     for (int c = 0; c < MAXC; ++c) nw[c] = small_load<half8_t>(a.norm_w + kb + (owned(c) ? c : 0) * 128, (lane & 15) * 16);
   }
@@ -204,8 +204,7 @@ __global__ __launch_bounds__(NW * 64, NW <= 8 && RP == 4 && MAXC == 3 ? 2 : 4) v
   // x w of each wave's own columns, brought near one by a power of two (exact; by the row's mean square over these columns, so that x w keeps
   // fp16's range whatever x is), and is rounded once as w x / rms would be.  The power and the row's 1 / rms go onto the sums at the end: no
   // wave waits for another's squares before its matrix instructions. ----
-  const bool normed = NORM && a.norm_w;
-  if (normed) {
+  if (NORM) {
 #pragma unroll
     for (int p = 0; p < RP; ++p) {
       float ss = 0.f;
@@ -349,7 +348,7 @@ __global__ __launch_bounds__(NW * 64, NW <= 8 && RP == 4 && MAXC == 3 ? 2 : 4) v
   if (!epi) return;
   float sum[NT];
   float2_t wave_ss[NW];
-  if (normed) {
+  if (NORM) {
 #pragma unroll
     for (int w = 0; w < NW; ++w) wave_ss[w] = ssq[w][em];
   }
@@ -360,10 +359,10 @@ __global__ __launch_bounds__(NW * 64, NW <= 8 && RP == 4 && MAXC == 3 ? 2 : 4) v
     for (int w = 0; w < NW; ++w) {
       const float* red = reinterpret_cast<const float*>(slices[w]) + t * (16 * SMALL_RED);
       const float v = HALF ? red[SMALL_RED * em + en] + red[SMALL_RED * (8 + em) + en] : red[SMALL_RED * em + en];
-      sum[t] = normed ? __builtin_fmaf(v, wave_ss[w][1], sum[t]) : sum[t] + v;
+      sum[t] = NORM ? __builtin_fmaf(v, wave_ss[w][1], sum[t]) : sum[t] + v;
     }
   }
-  if (normed) {
+  if (NORM) {
     float tot = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) tot += wave_ss[w][0];
@@ -432,6 +431,14 @@ void small_go(const SmallArgs& a, int grid, hipStream_t st) {
     hipLaunchKernelGGL((qmm_small_kernel<NW, MAXC, 2, MODE, NORM, false>), dim3(grid), dim3(NW * 64), 0, st, a);
 }
 
+template <int NW, int MAXC, int MODE>
+void small_norm(const SmallArgs& a, int grid, hipStream_t st) {
+  if (a.norm_w)
+    small_go<NW, MAXC, MODE, true>(a, grid, st);
+  else
+    small_go<NW, MAXC, MODE, false>(a, grid, st);
+}
+
 template <int MODE>
 void small_launch(const SmallArgs& a, int grid, hipStream_t st) {
   // A load that a wave makes for a chunk it does not own costs what any other does, so the waves are chosen
@@ -439,20 +446,18 @@ void small_launch(const SmallArgs& a, int grid, hipStream_t st) {
   // 3.28 / 3.51; the other way round for the many workgroups of gate|up, 9728 rows: 6.2 / 5.8), 4 x 2 against
   // 4 x 3 (gate|up 5.8 / 6.3), 16 x 2 against 16 x 3 for K = 3584 (4.9 / 5.7), 13 x 3 against 16 x 3 for
   // K = 4864 (5.08 / 5.18).  By N and K alone: a SwiGLU product gives the bits of the plain one.
+  // Products with a norm and without one (o, down, the plain operator) have builds of their own: the norm weights of a wave's chunks take registers.
+  // (One build for both left 2 x 2048 -> 28712 three workgroups to a compute unit for four, 10.4 us for 9.2, and cost 896 -> 896 2.5 %.)
   const int chunks = a.K >> 7;
-  if (chunks <= 4) return small_go<4, 1, MODE, true>(a, grid, st);
-  if (chunks <= 7 && a.N <= 8192) return small_go<7, 1, MODE, true>(a, grid, st);
-  if (chunks <= 8) return small_go<4, 2, MODE, true>(a, grid, st);
-  if (chunks <= 12) return small_go<4, 3, MODE, true>(a, grid, st);
-  if (chunks <= 16) return small_go<8, 2, MODE, true>(a, grid, st);
-  if (chunks <= 24) return small_go<8, 3, MODE, true>(a, grid, st);
-  // Sixteen waves leave a wave 128 registers: the norm weights of its chunks (48 of them) only
-  // have room in a build of their own, so the products without a norm (o, down) get one that
-  // does not hold them.
-  const bool norm = a.norm_w != nullptr;
-  if (chunks <= 32) return norm ? small_go<16, 2, MODE, true>(a, grid, st) : small_go<16, 2, MODE, false>(a, grid, st);
-  if (chunks <= 39) return norm ? small_go<13, 3, MODE, true>(a, grid, st) : small_go<13, 3, MODE, false>(a, grid, st);
-  return norm ? small_go<16, 3, MODE, true>(a, grid, st) : small_go<16, 3, MODE, false>(a, grid, st);
+  if (chunks <= 4) return small_norm<4, 1, MODE>(a, grid, st);
+  if (chunks <= 7 && a.N <= 8192) return small_norm<7, 1, MODE>(a, grid, st);
+  if (chunks <= 8) return small_norm<4, 2, MODE>(a, grid, st);
+  if (chunks <= 12) return small_norm<4, 3, MODE>(a, grid, st);
+  if (chunks <= 16) return small_norm<8, 2, MODE>(a, grid, st);
+  if (chunks <= 24) return small_norm<8, 3, MODE>(a, grid, st);
+  if (chunks <= 32) return small_norm<16, 2, MODE>(a, grid, st);
+  if (chunks <= 39) return small_norm<13, 3, MODE>(a, grid, st);
+  return small_norm<16, 3, MODE>(a, grid, st);
 }
 
 // two scales or biases of a row are one load, four values of the bias another
