@@ -20,11 +20,12 @@
 //     workgroups, each with half the instructions of a product; half of the products, x of one group with weights of the
 //     other, is dropped.  The sums are the same bits: a tile of 16 keeps two sums, of the even and of the odd groups.
 //   * The norm is folded into x as it was loaded (whole rows, every lane columns of its own; in the operand layout
-//     half the lanes hold nothing when T <= 8): each wave multiplies x with the norm weights and a power of two that brings its
-//     columns of a row near one, and sums their squares; the power and the row's 1 / rms go onto the sums at the end, where the
+//     half the lanes hold nothing when T <= 8): each wave multiplies x with the norm weights and with powers of two that keep
+//     its columns in fp16's range, and sums their squares; the powers and the row's 1 / rms go onto the sums at the end, where the
 //     waves meet anyway.  No launch, no pass over memory and no barrier for it (8 rows, us in a graph, with the row sums added across
-//     the waves before the product / so: gate|up of K 896 4.68 / 4.55, q|k|v 2.76 / 2.66, 16 rows of 2048 -> 11008 9.9 / 9.0;
-//     4.0 without a norm).  Error against 64 bits as before: 0.999 of it over 24 kinds of rows and widths, 1.004 at most.
+//     the waves before the product / so: gate|up of K 896 4.68 / 4.46, q|k|v with the rotation 3.44 / 3.18, 16 rows of 2048 -> 22016 13.4 / 12.3;
+//     4.0 without a norm).  Error against 64 bits: that of w x / rms rounded once, 2.9e-4 of the result, also beside a column of 30000 where
+//     the others are 0.004 (with w x / rms itself in fp16 1.6e-3 .. 4e-3 there: subnormal numbers).
 //   * The weights are never rounded: the matrix instructions multiply x with the integers q (exact in
 //     fp16, through the fp8 conversion) a quantisation group at a time, and with ones for the group's
 //     sum of x; scale and bias are applied to the two sums in fp32.
@@ -201,31 +202,46 @@ __global__ __launch_bounds__(NW * 64, NW <= 8 && RP == 4 && MAXC == 3 ? 2 : 4) v
   if (MODE == SMALL_ROPE) e_len = *a.len_dev;
   __builtin_amdgcn_sched_barrier(0);
   // ---- RMSNorm folded into x, as it was loaded: lane l holds columns 8 (l % 16) .. + 8 of rows 4 p + l / 16.  The product takes
-  // x w of each wave's own columns, brought near one by a power of two (exact; by the row's mean square over these columns, so that x w keeps
-  // fp16's range whatever x is), and is rounded once as w x / rms would be.  The power and the row's 1 / rms go onto the sums at the end: no
-  // wave waits for another's squares before its matrix instructions. ----
+  // x w of each wave's own columns, either factor times a power of two, and is rounded once as w x / rms would be.  The powers and the row's 1 / rms
+  // go onto the sums at the end: no wave waits for another's squares before its matrix instructions.  The powers bring the roots of both sums of
+  // squares, which bound the factors, to 2^10 .. 2^11 (x) and 2^3.5 .. 2^4.5 (w): no product leaves fp16's range, and what is small beside the
+  // largest keeps its bits (the factors themselves are exact down to 2^-24 and 2^-17 of those roots).  With x alone brought near one by its mean
+  // square a large column cost the small ones beside it bits: 8 rows of 2048, one 30000 beside 0.05, error 1.3 times that of w x / rms. ----
   if (NORM) {
+    auto squares = [&](half8_t v, float sum) {       // exact products, fp32 sum
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const half2_t p2 = half2_t{v[e], v[e + 1]};
+        sum = __builtin_amdgcn_fdot2(p2, p2, sum, false);
+      }
+      return sum;
+    };
+    // the exponent that brings a root of `sum` below 2^(top / 2), inside fp16's powers, and 2^-k
+    auto exponent = [](float sum, int top) {
+      const int k = (__builtin_amdgcn_frexp_expf(sum) - top + 1) >> 1;
+      return k < -14 ? -14 : k > 14 ? 14 : k;
+    };
+    auto power8 = [](int k) {
+      const half_t d = __builtin_bit_cast(half_t, (unsigned short)((15 - k) << 10));
+      return half8_t{d, d, d, d, d, d, d, d};
+    };
+    float sw = 0.f;
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c)
+      if (owned(c)) sw = squares(nw[c], sw);
+    const int kw = exponent(wave_f32(wave_reduce_row(wave_u32(sw), WaveAdd())), 9);
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) nw[c] = nw[c] * power8(kw);
 #pragma unroll
     for (int p = 0; p < RP; ++p) {
       float ss = 0.f;
 #pragma unroll
-      for (int c = 0; c < MAXC; ++c) {
-        if (owned(c)) {
-          const half8_t v = __builtin_bit_cast(half8_t, xg[c][p]);
-#pragma unroll
-          for (int e = 0; e < 8; e += 2) {
-            const half2_t p2 = half2_t{v[e], v[e + 1]};
-            ss = __builtin_amdgcn_fdot2(p2, p2, ss, false);      // exact products, fp32 sum
-          }
-        }
-      }
+      for (int c = 0; c < MAXC; ++c)
+        if (owned(c)) ss = squares(__builtin_bit_cast(half8_t, xg[c][p]), ss);
       ss = wave_f32(wave_reduce_row(wave_u32(ss), WaveAdd()));
-      // half the exponent of the mean square over about 128 MAXC columns, inside fp16's powers
-      int k = (__builtin_amdgcn_frexp_expf(ss) - (MAXC > 2 ? 9 : MAXC > 1 ? 8 : 7)) >> 1;
-      k = k < -14 ? -14 : k > 14 ? 14 : k;
-      const half_t down = __builtin_bit_cast(half_t, (unsigned short)((15 - k) << 10));
-      if ((lane & 15) == 0) ssq[wave][4 * p + (lane >> 4)] = float2_t{ss, wave_f32((uint32_t)(127 + k) << 23)};
-      const half8_t d8 = {down, down, down, down, down, down, down, down};
+      const int k = exponent(ss, 22);
+      if ((lane & 15) == 0) ssq[wave][4 * p + (lane >> 4)] = float2_t{ss, wave_f32((uint32_t)(127 + k + kw) << 23)};
+      const half8_t d8 = power8(k);
 #pragma unroll
       for (int c = 0; c < MAXC; ++c)
         if (owned(c)) xg[c][p] = __builtin_bit_cast(uint4_t, __builtin_bit_cast(half8_t, xg[c][p]) * d8 * nw[c]);
@@ -332,7 +348,7 @@ __global__ __launch_bounds__(NW * 64, NW <= 8 && RP == 4 && MAXC == 3 ? 2 : 4) v
   }
   __builtin_amdgcn_wave_barrier();
   // The waves' tiles meet in LDS, x row m of weight row n at 20 m + n (the four rows of a store in different banks), and
-  // every thread of the first 16 T finishes one output: one wave that finished all of them was a tail of 200 instructions.
+  // every thread of the first TR T finishes one output: one wave that finished all of them was a tail of 200 instructions.
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     float* red = reinterpret_cast<float*>(slices[wave]) + t * (16 * SMALL_RED);

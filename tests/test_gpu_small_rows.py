@@ -120,6 +120,53 @@ def test_norm_folded_in_at_any_scale(dev, T, K):
         assert (got.double() - want).norm() <= 6.9e-4 * want.norm()
 
 
+def norm_error(dev, g, x, nw, dead=None):
+    """Error of the product with the norm folded in, relative to the result, whose size the scales make 0.1 or, themselves normal numbers, more; the weights of the
+    quantisation group `dead` are zero."""
+    K, N = x.shape[1], 48
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 8), dtype=torch.int32, device=dev, generator=g)
+    xn = x.double() * torch.rsqrt((x.double() ** 2).mean(1, keepdim=True) + EPS) * nw.double()
+    live = torch.arange(K, device=dev) // 64 != dead if dead is not None else torch.ones(K, dtype=torch.bool, device=dev)
+    size = xn[:, live].square().mean().sqrt()
+    s = ((torch.rand((N, K // 64), device=dev, generator=g) * 0.02 + 0.005) / (0.6 * size * K ** 0.5).clamp(max=50)).half()
+    if dead is not None:
+        s[:, dead] = 0
+    b = (-7.5 * s.float()).half()
+    assert s.isfinite().all() and b.isfinite().all()
+    q = ((w[..., None] >> (4 * torch.arange(8, device=dev, dtype=torch.int32))) & 15).reshape(N, K).double()
+    wide = q * s.double().repeat_interleave(64, 1) + b.double().repeat_interleave(64, 1)
+    want = xn @ wide.T
+    got = ops.quantized_matmul_small(x, w, s, b, norm_weight=nw, eps=EPS)
+    return ((got.double() - want).norm() / want.norm()).item()
+
+
+# (below: two independent roundings of at most 2^-11 each, as above)
+@pytest.mark.parametrize("T,K", [(1, 128), (8, 896), (4, 2048), (16, 2048), (8, 4864), (2, 6144)])
+@pytest.mark.parametrize("large,small,gain", [(3000., 0.5, 1.0), (30000., 0.05, 1.0), (30000., 0.004, 1.0), (30000., 0.002, 20.0), (30000., 0.01, 400.0)])
+def test_norm_folded_in_beside_one_large_column(dev, T, K, large, small, gain):
+    """One column outweighs the row and its weights are zero: the small columns decide the result and keep their bits, for norm weights of any
+    size (with less than 2^24 between them, products with a norm weight are normal numbers of fp16)."""
+    g = torch.Generator(device=dev).manual_seed(T + K)
+    at = 5 if K == 128 else 133
+    x = (torch.randn((T, K), device=dev, generator=g) * small).half()
+    x[:, at] = large
+    nw = (gain * (1 + 0.3 * torch.randn(K, device=dev, generator=g))).half()
+    assert norm_error(dev, g, x, nw, dead=at // 64) <= 6.9e-4
+
+
+@pytest.mark.parametrize("T,K", [(8, 128), (1, 896), (8, 2944), (16, 6144)])
+@pytest.mark.parametrize("size", [2.0 ** -14, 1.0, 60000.0])
+@pytest.mark.parametrize("weight", [2.0 ** -10, 1.0, 600.0, 60000.0])
+def test_norm_folded_in_keeps_the_range(dev, T, K, size, weight):
+    """Rows and norm weights at both ends of fp16's range, and one column far above the others in both: nothing leaves the range."""
+    g = torch.Generator(device=dev).manual_seed(T + K)
+    sign = torch.randint(0, 2, (T, K), device=dev, generator=g) * 2.0 - 1
+    x, nw = (size * sign).half(), torch.full((K,), weight, device=dev).half()
+    assert norm_error(dev, g, x, nw) <= 6.9e-4
+    x[:, 70], nw[70] = min(1000 * size, 60000.0), min(1000 * weight, 60000.0)
+    assert norm_error(dev, g, x, nw) <= 6.9e-4
+
+
 @pytest.mark.parametrize("I,K,bias", [(4864, 896, False), (16, 128, True), (272, 1280, True), (1536, 512, False),
                                       (48, 2560, True), (8960, 1536, False)])
 @pytest.mark.parametrize("T", [1, 8, 16])
