@@ -79,6 +79,15 @@ __device__ inline half8_t eagle_expand8(uint32_t w) {
 // eight values of x in that order
 __device__ inline half8_t eagle_permute8(half8_t v) { return half8_t{v[0], v[2], v[4], v[6], v[1], v[3], v[5], v[7]}; }
 
+// A pair (x1, x2) turned by an angle: a fused multiply-add on a product rounded to fp32, then fp16.  Every rotation in the library is this one, so
+// that they agree bit for bit.  The sums are held in fp32 registers: folded into mixed-precision instructions by the compiler's choice
+// they were rounded once to fp16, other elements of the same kernel twice (three values of a million differ).
+__device__ inline half2_t eagle_rotate(float x1, float x2, float co, float sn) {
+  float lo = __builtin_fmaf(x1, co, -(x2 * sn)), hi = __builtin_fmaf(x1, sn, x2 * co);
+  asm("" : "+v"(lo), "+v"(hi));
+  return half2_t{(half_t)lo, (half_t)hi};
+}
+
 // Rows of a partial tile of the slab form: 32 for up to 32 rows of x, 64 for 33..64.
 __host__ __device__ inline int eagle_slab_rows(int M) { return M > 32 ? 64 : 32; }
 

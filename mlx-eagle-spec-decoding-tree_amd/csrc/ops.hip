@@ -19,12 +19,9 @@ __device__ inline void rotate8(const half8_t lo, const half8_t hi, const float* 
     const float theta = lf * pos;
     float sn, cs;
     sincosf(theta, &sn, &cs);
-    const float x1 = (float)lo[j];
-    const float x2 = (float)hi[j];
-    // one fused multiply-add on an explicitly rounded product: every rotation in the library
-    // uses this form, so that they agree bit for bit
-    (*olo)[j] = (half_t)__builtin_fmaf(x1, cs, -(x2 * sn));
-    (*ohi)[j] = (half_t)__builtin_fmaf(x1, sn, x2 * cs);
+    const half2_t o = eagle_rotate((float)lo[j], (float)hi[j], cs, sn);
+    (*olo)[j] = o[0];
+    (*ohi)[j] = o[1];
   }
 }
 
@@ -69,10 +66,9 @@ __global__ void rope_arrayed_scalar_kernel(const half_t* __restrict__ x,
   const float theta = lf * (float)pos[(long)b * L + t];
   float sn, cs;
   sincosf(theta, &sn, &cs);
-  const float x1 = (float)x[row * hd + i];
-  const float x2 = (float)x[row * hd + i + half];
-  out[row * hd + i] = (half_t)__builtin_fmaf(x1, cs, -(x2 * sn));
-  out[row * hd + i + half] = (half_t)__builtin_fmaf(x1, sn, x2 * cs);
+  const half2_t o = eagle_rotate((float)x[row * hd + i], (float)x[row * hd + i + half], cs, sn);
+  out[row * hd + i] = o[0];
+  out[row * hd + i + half] = o[1];
 }
 
 // Token-major projections -> rotated q [H,T,hd] and K/V cache rows P + t.
@@ -114,10 +110,9 @@ __global__ void rope_kv_append_kernel(const half_t* __restrict__ q_lin,
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const int j = 2 * j2 + e;
-        const float co = v[2 * e], sn = v[2 * e + 1];
-        const float x1 = (float)lo[j], x2 = (float)hi[j];
-        olo[j] = (half_t)__builtin_fmaf(x1, co, -(x2 * sn));
-        ohi[j] = (half_t)__builtin_fmaf(x1, sn, x2 * co);
+        const half2_t o = eagle_rotate((float)lo[j], (float)hi[j], v[2 * e], v[2 * e + 1]);
+        olo[j] = o[0];
+        ohi[j] = o[1];
       }
     }
     *reinterpret_cast<half8_t*>(dst + c * 8) = olo;
@@ -168,9 +163,9 @@ __global__ __launch_bounds__(ROPE_THREADS) void rope_kv_append_angles_kernel(
       const float lf = scale * freq[j];
       float sn, cs;
       sincosf(lf * p, &sn, &cs);
-      const float x1 = (float)lo[j], x2 = (float)hi[j];
-      lo[j] = (half_t)__builtin_fmaf(x1, cs, -(x2 * sn));
-      hi[j] = (half_t)__builtin_fmaf(x1, sn, x2 * cs);
+      const half2_t o = eagle_rotate((float)lo[j], (float)hi[j], cs, sn);
+      lo[j] = o[0];
+      hi[j] = o[1];
     }
   }
 #pragma unroll
@@ -253,9 +248,9 @@ __global__ void rope_kv_append_slabs_kernel(const float* __restrict__ partial, i
     for (int j = 0; j < 4; ++j) {
       const float co = j < 2 ? cs0[2 * j] : cs1[2 * (j - 2)];
       const float sn = j < 2 ? cs0[2 * j + 1] : cs1[2 * (j - 2) + 1];
-      const float x1 = (float)xlo[j], x2 = (float)xhi[j];
-      olo[j] = (half_t)__builtin_fmaf(x1, co, -(x2 * sn));
-      ohi[j] = (half_t)__builtin_fmaf(x1, sn, x2 * co);
+      const half2_t o = eagle_rotate((float)xlo[j], (float)xhi[j], co, sn);
+      olo[j] = o[0];
+      ohi[j] = o[1];
     }
     *reinterpret_cast<half4_t*>(dst + c) = olo;
     *reinterpret_cast<half4_t*>(dst + half + c) = ohi;

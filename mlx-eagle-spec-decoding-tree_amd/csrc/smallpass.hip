@@ -405,9 +405,9 @@ __global__ __launch_bounds__(NW * 64, NW <= 8 && RP == 4 && MAXC == 3 ? 2 : 4) v
       dst = (e_head < a.H + a.G ? a.k_cache : a.v_cache) + ((long)g * a.cap + P + em) * a.hd;
     }
     if (e_head < a.H + a.G) {
-      const float x1 = (float)lo, x2 = (float)hi;
-      lo = (half_t)__builtin_fmaf(x1, e_cs[0], -(x2 * e_cs[1]));
-      hi = (half_t)__builtin_fmaf(x1, e_cs[1], x2 * e_cs[0]);
+      const half2_t o = eagle_rotate((float)lo, (float)hi, e_cs[0], e_cs[1]);
+      lo = o[0];
+      hi = o[1];
     }
     dst[e_d + en] = lo;
     dst[(a.hd >> 1) + e_d + en] = hi;

@@ -40,3 +40,37 @@ def test_every_column_of_every_row(dev, H, G, hd, form, T):
     assert torch.equal(v[:, P:P + T].double(), rows[H + G:])
     for cache in (k, v):
         assert (cache[:, :P] == 9).all() and (cache[:, P + T:] == 9).all()
+
+
+def test_every_rotation_rounds_alike(dev):
+    """The sums in fp32 on a product rounded to fp32, then fp16, bit for bit, in every kernel that rotates and in each of its elements (rounded to
+    fp16 at once three in a million differ: the largest launch has nine million)."""
+    g = torch.Generator().manual_seed(5)
+    H, G, hd, P, half = 28, 4, 128, 3, 64
+    N = (H + 2 * G) * hd
+    inv = ops.default_inv_freqs(hd, 1e6, device=dev)
+    ln = torch.tensor([P], dtype=torch.int32, device=dev)
+    for form, T in (("table", 2048), ("plain", 32), ("slabs", 64), ("arrayed", 2048)):
+        qkv = torch.randn((T, N), generator=g).half().to(dev)
+        pos = (torch.arange(T) + 40).int().to(dev)
+        cs = ops.rope_table(pos, inv, 1.0)
+        q = torch.empty((H, T, hd), dtype=torch.float16, device=dev)
+        k, v = (torch.empty((G, P + T, hd), dtype=torch.float16, device=dev) for _ in range(2))
+        rows = qkv.view(T, H + 2 * G, hd).transpose(0, 1)[:H + G]
+        if form == "slabs":
+            partial = torch.zeros((1, ops.slab_rows(T), N), device=dev)
+            partial[0, :T] = qkv.float()
+            ops.rope_kv_append_slabs(partial, 1, None, cs, q, k, v, ln, T, H, G, hd)
+        elif form == "arrayed":
+            out = ops.arrayed_rope(rows.contiguous()[None], pos[None], inv, 1.0)[0]
+            q, k[:, P:] = out[:H], out[H:]
+        else:
+            ops.rope_kv_append(qkv, qkv[:, H * hd:], qkv[:, (H + G) * hd:], pos, inv, 1.0, q, k, v, ln, H, G, hd, row_stride=N,
+                               rope_cs=cs if form == "table" else None)
+        x1, x2 = rows[..., :half].float(), rows[..., half:].float()
+        co, sn = cs[..., 0], cs[..., 1]
+        # (a product of 11 and 24 bits is exact in 64 bits, and so is its sum with one of 24, or rounded 29 bits below fp32)
+        lo = (x1.double() * co.double() - (x2 * sn).double()).float().half()
+        hi = (x1.double() * sn.double() + (x2 * co).double()).float().half()
+        want = torch.cat([lo, hi], -1)
+        assert torch.equal(q, want[:H]) and torch.equal(k[:, P:P + T], want[H:]), (form, int((q != want[:H]).sum()))
