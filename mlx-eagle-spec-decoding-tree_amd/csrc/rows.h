@@ -82,7 +82,9 @@ __device__ inline void rows_wave(const RowsArgs& a, int nb, int m0, int wave, in
     const int c = (int)((unsigned long)n * a.inv >> 31) << a.pairs;
     return c < all ? c : all;
   };
-  const int NU = a.units;
+  // (Three tiles of x: the counters that the compiler makes of the addresses when the kernel works the units out itself are the faster loop, 34 x 4352 ->
+  // 76632 48.6 us, 51.6 from the host; with one, two and four tiles the other way round, 32 x 3584 -> 152064 67.7, 67.2.)
+  const int NU = MT == 3 ? ((all + (int)gridDim.y * KP - 1) / ((int)gridDim.y * KP) + 3) >> 2 : a.units;
   const int c0 = first(kp), nch = first(kp + 1) - c0;
   const int XC = 4 * NU;
   half2_t* xsum = reinterpret_cast<half2_t*>(rows_lds + 2 * BUF);      // [KP][XC][ROWS][2]: (hi, lo) of a group's sum
