@@ -42,7 +42,7 @@ namespace {
 // The partial sums of a split product added in split order: fp16 (+ bias), or silu(g) * u of interleaved gate|up
 // rows.  Four outputs per thread and one wave per workgroup, every load in flight before the first add.  What a compute unit takes in of
 // its partial sums bounds it: with eight outputs and 256 threads 27 x 18944 -> 3584 had 48 workgroups with 73 KB each (the product with it 17.4 us,
-// 16.9 with 378).  (The model below was fitted before that: it counts the second launch 0.4 us too long.)
+// 16.9 with 378).
 constexpr int SUM_WAVE = 64;
 __device__ inline float4_t rows_sum4(const float* __restrict__ p, int splits, size_t stride) {
   float4_t sum = {0.f, 0.f, 0.f, 0.f};
@@ -94,21 +94,24 @@ struct RowsPlan {
 // back to back over rotating weights in a graph.  A compute unit takes its workgroups one after the other; each costs its start, its
 // share of the weights and its x, with more K parts more barriers.  What the whole grid reads counts a little, a split as much as
 // its second launch and the partial sums (the sums alone where the consumer of the product adds them).  Constants by the
-// rows: up to 16, 17 .. 32, 33 .. 48, more; above 64 the last over the blocks of x.  The choice against the best of all forms and
-// splits of 6976 products (178000 timings): 1.2, 0.6, 0.8 and 1.4 % longer on average, 7, 4, 5 and 10 at the 95th
-// percentile; of 4724 products of 65 .. 2048 rows (93000 timings) 0.5 and 4.  Splits of up to three rows count as those of four (2 x 11008 -> 18944
-// chose another division: 36.1 us, 33.1).
+// rows: up to 16, 17 .. 32, 33 .. 48, more; above 64 the last over the blocks of x.  The second launch counts 0.6 us less from 17 rows on than the fit
+// gave for its first kernel: of 9900 products of 17 .. 64 rows that take another division for it the mean is 0.94, 0.94 and 0.98 of the time, one in ten
+// loses more than 3 %, 21 at most (46 x 2432 -> 5720).  The choice against the best of the divisions within 1.35 of the least predicted time, this kernel
+// and this launch, 16950 products (141000 timings): 0.7, 0.8, 1.1 and 0.8 % longer on average, 5, 6, 7 and 6 at the 95th percentile; of 1620
+// products of 65 .. 512 rows (13500 timings) 1.0 and 6.  Splits of up to three rows count as those of four (2 x 11008 -> 18944 chose another division: 36.1 us, 33.1).
 enum { ROWS_WHOLE = 0, ROWS_SPLIT = 1, ROWS_PARTIAL = 2 };
 struct RowsCost {
   double start, w, x, unit, parts, whole, second, sums, rows;
 };
 constexpr RowsCost rows_cost_one = {2.11, 0.0309, 0.0107, 0.0448, 0.419, 0.0018, 2.60, 1.353, 5.};
-constexpr RowsCost rows_cost_two = {3.89, 0.0416, 0.0058, 0., 0.293, 0.0068, 3.22, 0.459, 0.};
-constexpr RowsCost rows_cost_three = {4.23, 0.0484, 0.0104, 0., 0.0887, 0.0070, 3.46, 0.336, 0.};
-constexpr RowsCost rows_cost = {1.03, 0.0246, 0.0138, 0.221, 0., 0.0107, 2.93, 0.49, 0.};
+constexpr RowsCost rows_cost_two = {3.89, 0.0416, 0.0058, 0., 0.293, 0.0068, 2.62, 0.459, 0.};
+constexpr RowsCost rows_cost_three = {4.23, 0.0484, 0.0104, 0., 0.0887, 0.0070, 2.86, 0.336, 0.};
+constexpr RowsCost rows_cost = {1.03, 0.0246, 0.0138, 0.221, 0., 0.0107, 2.33, 0.49, 0.};
 
 // What the norm or rope launch that adds the partial sums takes for them, us per MB: 40 rows of 18944 -> 3584 are left as nine instead of thirteen
-// (19.1 us either way; the norm behind them reads 5.2 instead of 7.5 MB).  At 0.37 32 x 3584 -> 4608 would lose 1.3 us on the product for 0.9 behind it.
+// (19.1 us either way; the norm behind them reads 5.2 instead of 7.5 MB: 4.1 for 5.3 us).  Timed over 1 .. 16 parts that launch takes 0.24 .. 0.6 a MB as a
+// norm (64 .. 18 rows of 3584; nearly nothing up to five parts, most past nine) and 0.1 .. 0.23 as a rotation (18 .. 64 rows of 4608).  The line lies low
+// on purpose: at 0.37 32 x 3584 -> 4608, which a rotation adds, would lose 1.3 us on the product for 0.9 behind it.
 constexpr double rows_read = 0.18;
 
 // Up to 16 rows of x, K up to 2048 or 70 .. 250 M weights: whether the streaming kernel is faster than this one by the form (rt tiles, kp
