@@ -5,7 +5,8 @@
 
 #include <type_traits>
 
-namespace {
+// What rows.hip and the sources of forms share; the kernel and its launches are each source's own.
+namespace eagle_rows {
 
 struct RowsArgs {
   const half_t* x;        // [M, K]
@@ -29,6 +30,47 @@ constexpr int ROWS_LDS = 160 * 1024;
 constexpr int ROWS_RSRC = 0x00020000;      // buffer descriptor: untyped bytes
 constexpr int ROWS_XROW = 256 + 16;        // bytes of a staged x row: a chunk of 128 columns, padded against bank conflicts
 
+// bytes of a row's scales in LDS for `units` units of four chunks: an odd multiple of 16, so that sixteen rows
+// sit in different banks
+__host__ __device__ constexpr int rows_stride(int units) { return (units | 1) * 16; }
+
+constexpr int rows_block(int MT, int KP) { return (MT > 2 ? 2 : 4) / KP > 0 ? (MT > 2 ? 2 : 4) / KP : 1; }
+
+// bytes of LDS: two blocks of x, its sums, scales (and biases); at the end the sums of the K parts
+inline size_t rows_lds_bytes(int RT, int RT2, int MT, int KP, int nu, bool both) {
+  const size_t rows = 16 * MT, B = rows_block(MT, KP), wrows = ROWS_WAVES / KP / 2 * (RT + RT2) * 16;
+  const size_t stage = 2 * KP * B * rows * ROWS_XROW + KP * 4 * nu * rows * 8 +
+                       (both ? 2 : 1) * (size_t)ROWS_WAVES * RT * 16 * rows_stride(nu);
+  const size_t epi = KP * rows * (wrows + 4) * 4;
+  return stage > epi ? stage : epi;
+}
+
+// chunks in the last unit of the longest K part (of all workgroups along y and all parts)
+inline int rows_last(int K, int parts) { return (((K >> 7) + parts - 1) / parts - 1) % 4 + 1; }
+
+struct RowsForm {
+  int rt, rt2, mt, kp;
+  int (*launch)(const RowsArgs&, int, hipStream_t);
+  int (*launch_half)(const RowsArgs&, int, hipStream_t);      // the last unit of a K part has at most two chunks
+  int (*launch_many)(const RowsArgs&, int, hipStream_t);      // more than 64 rows (blocks of 48 or 64), or nullptr
+  int (*launch_many_half)(const RowsArgs&, int, hipStream_t);
+  int run(const RowsArgs& a, int splits, hipStream_t st) const {
+    const bool half = rows_last(a.K, splits * kp) <= 2;
+    return (a.M > 2 * EAGLE_MAX_M ? half ? launch_many_half : launch_many : half ? launch_half : launch)(a, splits, st);
+  }
+  int wrows() const { return ROWS_WAVES / kp / 2 * (rt + rt2) * 16; }
+};
+struct RowsTable {
+  const RowsForm* forms;
+  int count;
+};
+RowsTable forms_1();
+RowsTable forms_2();
+RowsTable forms_3();
+RowsTable forms_4();
+
+namespace {
+
 // a barrier that leaves the loads from memory in flight
 __device__ inline void rows_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -43,24 +85,9 @@ __device__ inline float rows_sum8(float v) {
   return v;
 }
 
-// bytes of a row's scales in LDS for `units` units of four chunks: an odd multiple of 16, so that sixteen rows
-// sit in different banks
-__host__ __device__ constexpr int rows_stride(int units) { return (units | 1) * 16; }
-
-constexpr int rows_block(int MT, int KP) { return (MT > 2 ? 2 : 4) / KP > 0 ? (MT > 2 ? 2 : 4) / KP : 1; }
-
-// bytes of LDS: two blocks of x, its sums, scales (and biases); at the end the sums of the K parts
-size_t rows_lds_bytes(int RT, int RT2, int MT, int KP, int nu, bool both) {
-  const size_t rows = 16 * MT, B = rows_block(MT, KP), wrows = ROWS_WAVES / KP / 2 * (RT + RT2) * 16;
-  const size_t stage = 2 * KP * B * rows * ROWS_XROW + KP * 4 * nu * rows * 8 +
-                       (both ? 2 : 1) * (size_t)ROWS_WAVES * RT * 16 * rows_stride(nu);
-  const size_t epi = KP * rows * (wrows + 4) * 4;
-  return stage > epi ? stage : epi;
-}
-
 // The part of a workgroup's wave: RT tiles from row0 on (the waves of a workgroup may differ in RT), then its sums in LDS.
 template <int RT, int MOST, int WROWS, int MT, int KP, int AH, bool MANY, int REM>
-__device__ inline void rows_wave(const RowsArgs& a, int nb, int m0, int wave, int rg, int kp, int row0) {
+__device__ inline void rows_wave(const RowsArgs& a, int nb, int m0, int wave, int kp, int row0) {
   constexpr int B = rows_block(MT, KP);            // chunks per K part and block of staged x
   constexpr int ROWS = 16 * MT;                    // rows of x
   constexpr int SLOT = ROWS * ROWS_XROW;           // bytes of a staged chunk
@@ -398,6 +425,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
   constexpr int ROWS = 16 * MT;
   constexpr int RG = ROWS_WAVES / KP;              // groups of tiles side by side
   constexpr int WROWS = RG / 2 * (RT + RT2) * 16;  // weight rows per workgroup
+  static_assert(WROWS % 32 == 0, "SwiGLU pairs the tiles of a workgroup");
   constexpr int OROW = WROWS + 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -407,9 +435,9 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void qmm_rows_kernel(RowsArgs a) {
   const int M = MANY && a.M - m0 > ROWS ? ROWS : a.M - m0, N = a.N;
   const int row0 = nb * WROWS + (rg < RG / 2 ? rg * RT : RG / 2 * RT + (rg - RG / 2) * RT2) * 16;
   if (RT == RT2 || rg < RG / 2)
-    rows_wave<RT, RT, WROWS, MT, KP, AH, MANY, REM>(a, nb, m0, wave, rg, kp, row0);
+    rows_wave<RT, RT, WROWS, MT, KP, AH, MANY, REM>(a, nb, m0, wave, kp, row0);
   else
-    rows_wave<RT2, RT, WROWS, MT, KP, AH, MANY, REM>(a, nb, m0, wave, rg, kp, row0);
+    rows_wave<RT2, RT, WROWS, MT, KP, AH, MANY, REM>(a, nb, m0, wave, kp, row0);
   const float* red = reinterpret_cast<const float*>(rows_lds);
   rows_barrier();
   const int base = nb * WROWS;
@@ -489,21 +517,6 @@ static int rows_launch(const RowsArgs& a, int splits, hipStream_t st) {
   return eagle_launch_status();
 }
 
-// chunks in the last unit of the longest K part (of all workgroups along y and all parts)
-inline int rows_last(int K, int parts) { return (((K >> 7) + parts - 1) / parts - 1) % 4 + 1; }
-
-struct RowsForm {
-  int rt, rt2, mt, kp;
-  int (*launch)(const RowsArgs&, int, hipStream_t);
-  int (*launch_half)(const RowsArgs&, int, hipStream_t);      // the last unit of a K part has at most two chunks
-  int (*launch_many)(const RowsArgs&, int, hipStream_t);      // more than 64 rows (blocks of 48 or 64), or nullptr
-  int (*launch_many_half)(const RowsArgs&, int, hipStream_t);
-  int run(const RowsArgs& a, int splits, hipStream_t st) const {
-    const bool half = rows_last(a.K, splits * kp) <= 2;
-    return (a.M > 2 * EAGLE_MAX_M ? half ? launch_many_half : launch_many : half ? launch_half : launch)(a, splits, st);
-  }
-  int wrows() const { return ROWS_WAVES / kp / 2 * (rt + rt2) * 16; }
-};
 template <int RT, int RT2, int MT, int KP, int AH>
 constexpr RowsForm rows_form() {
   constexpr auto whole = rows_launch<RT, RT2, MT, KP, AH, false, 4>, half = rows_launch<RT, RT2, MT, KP, AH, false, 2>;
@@ -514,12 +527,4 @@ constexpr RowsForm rows_form() {
 }
 
 }  // namespace
-
-struct RowsTable {
-  const RowsForm* forms;
-  int count;
-};
-RowsTable eagle_rows_forms_1();
-RowsTable eagle_rows_forms_2();
-RowsTable eagle_rows_forms_3();
-RowsTable eagle_rows_forms_4();
+}  // namespace eagle_rows

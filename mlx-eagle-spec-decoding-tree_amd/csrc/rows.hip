@@ -37,6 +37,8 @@
 // not in a cache: 732 and (2048 x 3584 x 18944) 372 us against 553 and 263; matrix pipes 37 % busy at 2.05 GHz.
 #include "rows.h"
 
+using namespace eagle_rows;
+
 namespace {
 
 // The partial sums of a split product added in split order: fp16 (+ bias), or silu(g) * u of interleaved gate|up
@@ -144,7 +146,7 @@ RowsPlan rows_find_plan(int M, int N, int K, int mode) {
   const RowsCost& cost = mt == 1 ? rows_cost_one : mt == 2 ? rows_cost_two : M <= 48 ? rows_cost_three : rows_cost;
   RowsPlan best = {nullptr, 1, false}, even = best;
   double least = 1e30, least_even = 1e30;
-  const RowsTable table = mt == 1 ? eagle_rows_forms_1() : mt == 2 ? eagle_rows_forms_2() : mt == 3 ? eagle_rows_forms_3() : eagle_rows_forms_4();
+  const RowsTable table = mt == 1 ? forms_1() : mt == 2 ? forms_2() : mt == 3 ? forms_3() : forms_4();
   for (int f = 0; f < table.count; ++f) {
     const RowsForm& form = table.forms[f];
     const int wrows = form.wrows();

@@ -2,6 +2,8 @@
 // tiles of x, K parts, chunks requested ahead.
 #include "rows.h"
 
+using namespace eagle_rows;
+
 static const RowsForm forms[] = {
     rows_form<1, 1, 2, 1, 4>(),
     rows_form<1, 1, 2, 2, 4>(),
@@ -15,4 +17,4 @@ static const RowsForm forms[] = {
     rows_form<3, 2, 2, 2, 4>(),
     rows_form<2, 1, 2, 2, 4>(),
 };
-RowsTable eagle_rows_forms_2() { return {forms, (int)(sizeof(forms) / sizeof(forms[0]))}; }
+RowsTable eagle_rows::forms_2() { return {forms, (int)(sizeof(forms) / sizeof(forms[0]))}; }

@@ -33,7 +33,7 @@ def test_short_last_units_leave_the_loads_in_flight(tmp_path):
         pytest.skip("no hipcc")
     src, asm = tmp_path / "forms.hip", tmp_path / "forms.s"
     calls = "".join(f"  rc |= rows_launch<{a}, {b}, {mt}, {kp}, 4, false, {rem}>(a, 1, s);\n" for a, b, mt, kp in FORMS for rem in (2, 4))
-    src.write_text(f'#include "rows.h"\nint forms(const RowsArgs& a, hipStream_t s) {{\n  int rc = 0;\n{calls}  return rc;\n}}\n')
+    src.write_text(f'#include "rows.h"\nusing namespace eagle_rows;\nint forms(const RowsArgs& a, hipStream_t s) {{\n  int rc = 0;\n{calls}  return rc;\n}}\n')
     flags = [f for f in build.FLAGS if f not in ("-shared", "-Rpass-analysis=kernel-resource-usage")]
     subprocess.run([cc, *flags, f"-I{build.CSRC}", "-S", "--cuda-device-only", str(src), "-o", str(asm)], check=True,
                    stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
@@ -43,3 +43,14 @@ def test_short_last_units_leave_the_loads_in_flight(tmp_path):
         whole, short = waits[a, b, mt, kp, 4], waits[a, b, mt, kp, 2]
         assert len(whole) == len(short) == (1 if a == b else 2)
         assert min(whole) > 0 and short == whole, (a, b, mt, kp, short, whole)
+
+
+def test_the_sources_of_forms_share_one_definition_of_their_types():
+    """The launches that rows.hip calls take an argument type of all sources, not one of each source's unnamed namespace."""
+    objects = [os.path.join(build.HERE, "build", f"rows_{i}.hip.o") for i in range(1, 5)]
+    if not all(os.path.exists(o) for o in objects):
+        pytest.skip("no objects of a build here")
+    for obj in objects:
+        names = subprocess.run(["nm", "-C", obj], check=True, stdout=subprocess.PIPE).stdout.decode()
+        launches = [line for line in names.splitlines() if "::rows_launch<" in line]
+        assert launches and all("(eagle_rows::RowsArgs const&" in line for line in launches), launches[:1]
