@@ -120,6 +120,11 @@ int eagle_qmm_rows_w4g64_f16(const void* x, const uint32_t* wq, const void* scal
                              const void* bias, void* out, int M, int N, int K, int group_size, int bits,
                              int swiglu, void* workspace, size_t workspace_bytes, eagle_stream_t stream);
 
+/* How the rows kernel divides a product: mode 0 in one pass (no workspace), 1 with its workspace, 2 left as partial sums.  plan6 = {16-row
+ * weight tiles of a wave in the first and in the second half of a workgroup, 16-row tiles of x in a block, K parts inside
+ * a workgroup, workgroups along K, chunks of 128 columns in the last unit of the build (2 or 4)}.  Not 0 if no division fits. */
+int eagle_qmm_rows_plan(int M, int N, int K, int mode, int* plan6);
+
 /* The same product left as fp32 partial sums for its consumer (eagle_rmsnorm_slabs_f16,
  * eagle_rope_kv_append_slabs_f16): partial [splits][R][N] with splits = eagle_qmm_rows_partial_splits (0: shape not
  * taken) and R = 32 up to 32 rows, 64 above. */
@@ -225,10 +230,12 @@ int eagle_qmm_gemm_swiglu_w4g64_f16(const void* x, const uint32_t* wq, const voi
  * weight rows, a long K): several workgroups then share an output block, each over a part of K, and a second
  * launch adds their fp32 sums in order.  The library decides; workspace bytes 0: no split.  Same
  * roundings; workspace 16-byte aligned.  The bytes serve any alignment of scales and biases; eagle_qmm_gemm_plan tells
- * what is chosen for one (a power of two, in bytes): plan4 = {block (0..3: 64 x 128, 96 or 128 x 128, 128 x 256, 160 .. 256
- * x 256 rows of x by weight rows), K groups inside a workgroup, workgroups along K, scales per fetch}. */
+ * what is chosen for one (a power of two, in bytes): plan4 = {kind of block (0..3: 64 x 128, 96 or 128 x 128, 128 x 256, 160 .. 256
+ * x 256 rows of x by weight rows), K groups inside a workgroup, workgroups along K, scales per fetch}; eagle_qmm_gemm_block
+ * the block itself, block2 = {rows of x, weight rows}. */
 size_t eagle_qmm_gemm_workspace_bytes(int M, int N, int K, int swiglu);
 int eagle_qmm_gemm_plan(int M, int N, int K, int swiglu, int sb_align, int may_split, int* plan4);
+int eagle_qmm_gemm_block(int M, int N, int K, int swiglu, int sb_align, int may_split, int* block2);
 int eagle_qmm_gemm_split_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
                                    const void* biases, const void* bias, void* out, int M, int N,
                                    int K, int group_size, int bits, int swiglu, void* workspace,

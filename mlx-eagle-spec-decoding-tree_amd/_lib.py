@@ -27,6 +27,7 @@ SIGNATURES = {
     "eagle_qmm_small_preferred": (c_int, [c_int] * 3),
     "eagle_qmm_rows_supported": (c_int, [c_int] * 4),
     "eagle_qmm_rows_preferred": (c_int, [c_int] * 3),
+    "eagle_qmm_rows_plan": (c_int, [c_int] * 4 + [c_void_p]),
     "eagle_qmm_rows_partial_splits": (c_int, [c_int] * 3),
     "eagle_qmm_rows_partial_w4g64": (c_int, [c_void_p] * 5 + [c_size_t] + [c_int] * 5 + [c_void_p]),
     "eagle_qmm_rows_workspace_bytes": (c_size_t, [c_int] * 3),
@@ -48,6 +49,7 @@ SIGNATURES = {
     "eagle_qmm_gemm_swiglu_w4g64_f16": (c_int, [c_void_p] * 6 + [c_int] * 5 + [c_void_p]),
     "eagle_qmm_gemm_workspace_bytes": (c_size_t, [c_int] * 4),
     "eagle_qmm_gemm_plan": (c_int, [c_int] * 6 + [c_void_p]),
+    "eagle_qmm_gemm_block": (c_int, [c_int] * 6 + [c_void_p]),
     "eagle_qmm_gemm_split_w4g64_f16": (c_int, [c_void_p] * 6 + [c_int] * 6 + [c_void_p, c_size_t, c_void_p]),
     "eagle_qmm_slab_count": (c_int, [c_int] * 2),
     "eagle_qmm_slab_steps": (c_int, [c_int] * 3),

@@ -1955,14 +1955,27 @@ EAGLE_EXPORT size_t eagle_qmm_gemm_workspace_bytes(int M, int N, int K, int swig
   return need;
 }
 
+static bool gemm_plan_takes(int M, int N, int K, int sb_align) {
+  return M >= 1 && N >= 8 && K >= 64 && (K % 64) == 0 && sb_align >= 2 && (sb_align & (sb_align - 1)) == 0;
+}
+
 EAGLE_EXPORT int eagle_qmm_gemm_plan(int M, int N, int K, int swiglu, int sb_align, int may_split, int* plan4) {
   if (!plan4) return EAGLE_ERR_NULL;
-  if (M < 1 || N < 8 || K < 64 || (K % 64) != 0 || sb_align < 2 || (sb_align & (sb_align - 1)) != 0) return EAGLE_ERR_SHAPE;
+  if (!gemm_plan_takes(M, N, K, sb_align)) return EAGLE_ERR_SHAPE;
   const GemmPlan p = gemm_plan(M, N, K, (uintptr_t)sb_align, swiglu != 0, may_split != 0);
   plan4[0] = p.block < 4 ? p.block : p.block == 6 ? 1 : 3;
   plan4[1] = p.kgrp;
   plan4[2] = p.splits;
   plan4[3] = p.sbw;
+  return EAGLE_OK;
+}
+
+EAGLE_EXPORT int eagle_qmm_gemm_block(int M, int N, int K, int swiglu, int sb_align, int may_split, int* block2) {
+  if (!block2) return EAGLE_ERR_NULL;
+  if (!gemm_plan_takes(M, N, K, sb_align)) return EAGLE_ERR_SHAPE;
+  const GemmPlan p = gemm_plan(M, N, K, (uintptr_t)sb_align, swiglu != 0, may_split != 0);
+  block2[0] = 32 * GEMM_MT[p.block];
+  block2[1] = 128 * GEMM_NTW[p.block];
   return EAGLE_OK;
 }
 

@@ -267,6 +267,17 @@ EAGLE_EXPORT int eagle_qmm_rows_w4g64_f16(const void* x, const uint32_t* wq, con
   return eagle_launch_status();
 }
 
+EAGLE_EXPORT int eagle_qmm_rows_plan(int M, int N, int K, int mode, int* plan6) {
+  if (!plan6) return EAGLE_ERR_NULL;
+  if (mode < ROWS_WHOLE || mode > ROWS_PARTIAL) return EAGLE_ERR_UNSUPPORTED;
+  if (!eagle_qmm_rows_supported(M, N, K, 0) || (mode == ROWS_PARTIAL && M > 2 * EAGLE_MAX_M)) return EAGLE_ERR_SHAPE;
+  const RowsPlan p = rows_plan(M, N, K, mode);
+  if (!p.form) return EAGLE_ERR_SHAPE;
+  const int plan[] = {p.form->rt, p.form->rt2, p.form->mt, p.form->kp, p.splits, rows_last(K, p.splits * p.form->kp) <= 2 ? 2 : 4};
+  for (int i = 0; i < 6; ++i) plan6[i] = plan[i];
+  return EAGLE_OK;
+}
+
 EAGLE_EXPORT int eagle_qmm_rows_partial_splits(int M, int N, int K) {
   return M <= 2 * EAGLE_MAX_M && eagle_qmm_rows_supported(M, N, K, 0) ? rows_plan(M, N, K, ROWS_PARTIAL).splits : 0;
 }

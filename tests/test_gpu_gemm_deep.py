@@ -70,14 +70,18 @@ def test_swiglu(dev, M, I, K):
 
 # sizes whose least predicted time is that of blocks of 160, of 192 and of 96 rows: scales in fetches of four and eight groups, whole and split
 # over K, the last block of rows and of columns ragged (no K of 1024: unsplit, that may be the shallow loop and its rounding)
-@pytest.mark.parametrize("M,N,K,bias", [(1738, 4616, 256, True), (1680, 4744, 512, False), (778, 1168, 7936, False), (133, 5528, 6656, True),
-                                        (1937, 5272, 256, False), (1791, 5384, 512, True),
-                                        (1608, 1200, 768, False), (908, 648, 2304, True), (1848, 1040, 512, True), (777, 592, 3584, False)])
+BETWEEN = [(1738, 4616, 256, True), (1680, 4744, 512, False), (778, 1168, 7936, False), (133, 5528, 6656, True), (1937, 5272, 256, False),
+           (1791, 5384, 512, True), (1608, 1200, 768, False), (908, 648, 2304, True), (1848, 1040, 512, True), (777, 592, 3584, False),
+           (162, 4104, 11776, True)]
+SWIGLU_BETWEEN = [(1477, 2704, 256), (1871, 2192, 512), (131, 2720, 6656), (1542, 3280, 256), (1977, 2448, 512), (1479, 656, 768),
+                  (1490, 656, 512), (920, 336, 2304)]
+
+
+@pytest.mark.parametrize("M,N,K,bias", BETWEEN)
 def test_products_in_blocks_between(dev, M, N, K, bias):
     test_products(dev, M, N, K, bias)
 
 
-@pytest.mark.parametrize("M,I,K", [(1477, 2704, 256), (1871, 2192, 512), (131, 2720, 6656), (1542, 3280, 256), (1977, 2448, 512), (1479, 656, 768),
-                                   (1490, 656, 512), (920, 336, 2304)])
+@pytest.mark.parametrize("M,I,K", SWIGLU_BETWEEN)
 def test_swiglu_in_blocks_between(dev, M, I, K):
     test_swiglu(dev, M, I, K)
