@@ -1557,10 +1557,16 @@ EAGLE_EXPORT int eagle_qmm_slab_swiglu_preferred(int M, int N, int K) {
   //   7B stream  23.5   22.7   27.6   28.7   48.5   56.1      (40, 64: two launches)
   //   8B slab    23.5   24.1   24.8   24.3   30.7   31.3      (224 workgroups of four waves)
   //   8B stream  20.8   21.2   26.1   27.0   45.5   52.8
-  // (eagle_qmm_rows_w4g64_f16, graph-timed as 29.7, 37.8 and 39.1 are for the 7B slab form at 32, 40 and 64 rows: 28.3,
-  // 36.1 and 42.4.  Up to 32 rows the operator's rule asks for that one first.)
   // so: always above 32 rows; from 24 rows where workgroups of four waves fill at least half of
   // the compute units and at most all of them.
+  // The rows kernel (eagle_qmm_rows_w4g64_f16), which rounds no weight, has overtaken this form since (graphs over rotating weights, us):
+  //   rows               33     40     48     49     56     64
+  //   7B slab / rows  36.7/27.3  37.3/27.3  38.0/28.1  37.7/31.9  38.0/32.0  38.3/32.4
+  //   8B slab / rows  31.0/26.5  31.1/26.4  31.9/26.6  32.7/33.4  33.8/35.1  33.7/37.5
+  // Of 14900 shapes of 33 .. 64 rows this form is the faster one for K up to 512 (1.14 and 1.25 times, to and past 48 rows), up to 1.15 times
+  // for K to 1536 past 48 rows, and 1.5 times slower on average.  The operator keeps it at 33 .. 64 rows all the same: its
+  // bits there are those of the step on tiled weights, which runs this kernel, and are tested.  Up to 32 rows it asks for the rows kernel first, the
+  // native decoder at any number of rows.
   if (!eagle_qmm_slab_swiglu_supported(M, N, K)) return 0;
   if (M > SLAB_ROWS) return 1;
   const long blocks = (N + 127) / 128;

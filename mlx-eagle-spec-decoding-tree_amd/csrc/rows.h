@@ -356,7 +356,8 @@ __device__ inline void rows_wave(const RowsArgs& a, int nb, int m0, int wave, in
     }
   };
   // The last unit by itself: what it would request, no chunk uses.  With the block of x and the ring of weights past the end
-  // fetched all the same, a workgroup of one unit spent a round trip to memory and a barrier on them (us before / now, timed in turn:
+  // fetched all the same, a workgroup of one unit spent a round trip to memory and a barrier on them (us with / without, timed in turn with equal shares
+  // of the waves and whole last units:
   // 32 x 3584 x 4608 left as seven partial sums 7.07 / 6.53, 40 rows 8.0 / 7.7; 32 x 3584 x 37888 with SwiGLU 27.3 / 26.5, 40 x 3584 x
   // 152064 80.2 / 78.8, 128 x 3584 x 37888 55.0 / 53.9).
   for (int j = 0; j + 1 < NU; ++j) {

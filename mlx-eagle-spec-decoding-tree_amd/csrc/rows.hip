@@ -33,7 +33,7 @@
 // 64 x 8192 x 8192 23 / 40.  With many rows the vector instructions (expansion per block, a multiply-add per group and
 // output) about equal the matrix instructions: 2048 x 37888 x 3584 675 us = 0.82 PFLOP/s, 512 x 3584 x 18944 114 us; the
 // GEMM, which rounds the weights to fp16 and expands them once per 256 rows, takes 580 and 93 (128 x 3584 x 37888 58 us
-// with the sums of a tile added behind its matrix instructions, 54 under the next tile's).  In a prompt pass, weights
+// with the sums of a tile added behind its matrix instructions, 54 under the next tile's, 49 with unequal shares of the waves).  In a prompt pass, weights
 // not in a cache: 732 and (2048 x 3584 x 18944) 372 us against 553 and 263; matrix pipes 37 % busy at 2.05 GHz.
 #include "rows.h"
 
