@@ -274,7 +274,7 @@ int eagle_qmm_slab_partial_w4g64(const void* x, const uint32_t* wq, const void* 
  * For 33..64 rows (a tree above 32 tokens) one launch in place of two of the 32-row kernel. */
 int eagle_qmm_slab_swiglu_supported(int M, int N, int K);
 /* 1 where this form measured faster than eagle_qmm_swiglu_w4g64_f16 (always above 32 rows).  It rounds the weights to
- * fp16; eagle_qmm_rows_w4g64_f16 does not, and is faster above 32 rows too but for K up to 512 (49 rows on: some K up to 1536). */
+ * fp16; eagle_qmm_rows_w4g64_f16 does not, and is faster above 32 rows too but for K up to 512 (past 48 rows: and some shapes of larger K). */
 int eagle_qmm_slab_swiglu_preferred(int M, int N, int K);
 int eagle_qmm_slab_swiglu_w4g64_f16(const void* x, const uint32_t* wq, const void* scales,
                                     const void* biases, const void* bias, void* out, int M, int N, int K,

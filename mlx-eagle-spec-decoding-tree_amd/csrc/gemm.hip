@@ -1563,8 +1563,8 @@ EAGLE_EXPORT int eagle_qmm_slab_swiglu_preferred(int M, int N, int K) {
   //   rows               33     40     48     49     56     64
   //   7B slab / rows  36.7/27.3  37.3/27.3  38.0/28.1  37.7/31.9  38.0/32.0  38.3/32.4
   //   8B slab / rows  31.0/26.5  31.1/26.4  31.9/26.6  32.7/33.4  33.8/35.1  33.7/37.5
-  // Of 14900 shapes of 33 .. 64 rows this form is the faster one for K up to 512 (1.14 and 1.25 times, to and past 48 rows), up to 1.15 times
-  // for K to 1536 past 48 rows, and 1.5 times slower on average.  The operator keeps it at 33 .. 64 rows all the same: its
+  // Of 14900 shapes of 33 .. 64 rows this form is the faster one for K up to 512 (1.10 and 1.20 times on average, to and past 48 rows),
+  // past 48 rows for some shapes of any K (1.2 times at most to 1024, 1.15 above), and 1.5 times slower on average.  The operator keeps it at 33 .. 64 rows all the same: its
   // bits there are those of the step on tiled weights, which runs this kernel, and are tested.  Up to 32 rows it asks for the rows kernel first, the
   // native decoder at any number of rows.
   if (!eagle_qmm_slab_swiglu_supported(M, N, K)) return 0;
