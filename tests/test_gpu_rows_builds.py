@@ -52,7 +52,8 @@ def product(dev, M, N, K, swiglu=False):
     rc = L.eagle_qmm_rows_w4g64_f16(x.data_ptr(), w.data_ptr(), s.data_ptr(), b.data_ptr(), None, out.data_ptr(), M, N, K, 64, 4,
                                     int(swiglu), ws.data_ptr() if need else None, need, torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and bool(out[M].isnan().all())
-    pick = torch.unique(torch.cat([torch.arange(min(N, 96)), torch.randint(0, N, (300,)), torch.arange(max(0, N - 700), N)])).to(dev)
+    pick = torch.unique(torch.cat([torch.arange(min(N, 96)),
+                                   torch.randint(0, N, (300,), generator=torch.Generator().manual_seed(N)), torch.arange(max(0, N - 700), N)])).to(dev)
     shift = 4 * torch.arange(8, device=dev, dtype=torch.int32)
 
     def wide(rows):
@@ -79,7 +80,8 @@ def test_every_build(dev, M, N, K):
 def test_gate_up_of_the_7b_target(dev, M):
     N, K = 37888, 3584
     got, x, wide, _ = product(dev, M, N, K, swiglu=True)
-    at = torch.unique(torch.cat([torch.arange(64), torch.randint(0, N // 2, (300,)), torch.arange(N // 2 - 400, N // 2)])).to(dev)
+    at = torch.unique(torch.cat([torch.arange(64),
+                                 torch.randint(0, N // 2, (300,), generator=torch.Generator().manual_seed(M)), torch.arange(N // 2 - 400, N // 2)])).to(dev)
     gate = at // 16 * 32 + at % 16
     g, u = x @ wide(gate).T, x @ wide(gate + 16).T
     act = torch.nn.functional.silu(g)
